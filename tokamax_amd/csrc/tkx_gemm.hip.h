@@ -15,9 +15,9 @@
 // k-atom, and fragments are double-buffered in registers. Operands that are contraction-contiguous
 // are read from LDS with ds_read_b128; operands that are contiguous along the other axis are read
 // with the gfx950 transposing LDS loads (ds_read_b64_tr_b16 / _tr_b8), so no operand is ever
-// transposed in memory. The 32x32 MFMA is issued with its operands swapped (B-fragment first) so
-// that each lane ends up holding runs of 4 consecutive C columns of one C row; the epilogue applies
-// scales, bias and activation in registers and writes whole row segments through LDS.
+// transposed in memory. The MFMA (32x32, or 16x16 in the larger 16-bit tiles) is issued with its operands swapped
+// (B-fragment first) so that each lane ends up holding runs of 4 consecutive C columns of one C row; the epilogue
+// applies scales, bias and activation in registers and writes whole row segments through LDS.
 #pragma once
 
 #include <type_traits>
@@ -55,14 +55,53 @@ enum OperandLayout { kKC = 0 /* contraction-contiguous */, kMC = 1 /* contiguous
 
 __host__ __device__ constexpr int elem_bytes(int e) { return e == kEF32 ? 4 : (e == kEBF16 || e == kEF16) ? 2 : 1; }
 
+// The 16 accumulators a lane has of a 32x32 block of C, as four groups of 4 consecutive columns of one row: one MFMA
+// result register tuple of the 32x32 instructions, four of the 16x16 ones.
+struct Acc4 { f32x4 q[4]; };
+__device__ __forceinline__ f32x4 get4(const f32x16& c, int t) { return f32x4{c[4 * t], c[4 * t + 1], c[4 * t + 2], c[4 * t + 3]}; }
+__device__ __forceinline__ f32x4 get4(const Acc4& c, int t) { return c.q[t]; }
+__device__ __forceinline__ void set4(f32x16& c, int t, f32x4 v) {
+#pragma unroll
+  for (int e = 0; e < 4; ++e) c[4 * t + e] = v[e];
+}
+__device__ __forceinline__ void set4(Acc4& c, int t, f32x4 v) { c.q[t] = v; }
+
 // MFMA flavour chosen by the A element kind: contraction elements per 32x32 atom and fragment bytes.
-template <int EA> struct Mma;
+// M16 (bf16, f16): a 32x32 block is four 16x16x32 MFMAs, 32 deep, instead of one 32x32x16. Both forms have the same
+// nominal rate, but under a sustained load of random operands the chip's power limit sets the clock, and the 16x16
+// form spends less on its accumulators (a quarter of their register traffic per product): a register-resident loop
+// of it holds 1770 TFLOP/s on all CUs where 32x32x16 holds 1537, with two waves per SIMD. (fp8: 3330 against 3400
+// TFLOP/s for 16x16x128 and 32x32x64; those kernels keep the 32x32 form.) In the GEMM, whose other bound is the operand
+// stream: the gate-up product of 16384 rows, k = 4096, 2 n = 28672 over 8 groups 3074 -> 2907 us (1325 TFLOP/s), the
+// down product 1560 -> 1484 us, a 256-expert prefill (65536 rows, k = 7168, n = 2048) 2289 -> 2192 us.
+template <int EA, bool M16 = false> struct Mma;
 template <> struct Mma<kEBF16> { static constexpr int KA = 16; typedef i32x4 Frag; };
 template <> struct Mma<kEF16> { static constexpr int KA = 16; typedef i32x4 Frag; };
+template <> struct Mma<kEBF16, true> { static constexpr int KA = 32; typedef i32x8 Frag; };
+template <> struct Mma<kEF16, true> { static constexpr int KA = 32; typedef i32x8 Frag; };
 template <> struct Mma<kEF32> { static constexpr int KA = 8; typedef i32x4 Frag; };
 template <> struct Mma<kEF8> { static constexpr int KA = 64; typedef i32x8 Frag; };
 // int8 x int8 -> int32: the accumulator registers hold int32 bits (kept in the f32x16 type the kernel uses).
 template <> struct Mma<kEI8> { static constexpr int KA = 32; typedef i32x4 Frag; };
+
+// One 32x32x32 block product as four 16x16x32 MFMAs. A fragment's halves are its rows (columns) 0-15 and 16-31, each
+// lane holding row lane % 16, contraction entries 8 (lane / 16) .. + 7. Group 2 r + c of the accumulators is row half
+// r (of `second`, the A fragment), column half c (of `first`).
+template <int EA>
+__device__ __forceinline__ Acc4 mma_atom(const i32x8& first, const i32x8& second, Acc4 acc) {
+#pragma unroll
+  for (int r = 0; r < 2; ++r)
+#pragma unroll
+    for (int c = 0; c < 2; ++c) {
+      const i32x4 f = {first[4 * c], first[4 * c + 1], first[4 * c + 2], first[4 * c + 3]};
+      const i32x4 g = {second[4 * r], second[4 * r + 1], second[4 * r + 2], second[4 * r + 3]};
+      if constexpr (EA == kEBF16)
+        acc.q[2 * r + c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, f), __builtin_bit_cast(bf16x8, g), acc.q[2 * r + c], 0, 0, 0);
+      else
+        acc.q[2 * r + c] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, f), __builtin_bit_cast(f16x8, g), acc.q[2 * r + c], 0, 0, 0);
+    }
+  return acc;
+}
 
 template <int EA>
 __device__ __forceinline__ f32x16 mma_atom(const typename Mma<EA>::Frag& first, const typename Mma<EA>::Frag& second,
@@ -172,11 +211,36 @@ __device__ __forceinline__ i32x4 i4x8_to_bf16x8_times16(int w) {
 // `PAIRED` (contraction-contiguous 16-bit tiles): atoms 2 d and 2 d + 1 share their 32 contraction entries the way a
 // lane's eight packed int4 bytes hold them: lanes 0-31 own entries 0-15 (first half in the even atom, second in the
 // odd one) and lanes 32-63 entries 16-31, instead of 8 entries per half-wave and atom in ascending order.
-template <int LAYOUT, int ES, int EC, int ROW_BYTES, bool PAIRED = false>
-__device__ __forceinline__ typename Mma<EC>::Frag load_frag(const unsigned char* tile, int rc0, int kk, int lane, int rc_step = 0) {
-  typedef typename Mma<EC>::Frag Frag;
-  constexpr int KA = Mma<EC>::KA;
-  if constexpr (LAYOUT == kKC) {
+// `M16`: the fragment of four 16x16x32 MFMAs (see mma_atom): halves of 16 rows / columns, 16 lanes each.
+template <int LAYOUT, int ES, int EC, int ROW_BYTES, bool PAIRED = false, bool M16 = false>
+__device__ __forceinline__ typename Mma<EC, M16>::Frag load_frag(const unsigned char* tile, int rc0, int kk, int lane, int rc_step = 0) {
+  typedef typename Mma<EC, M16>::Frag Frag;
+  constexpr int KA = Mma<EC, M16>::KA;
+  if constexpr (M16) {
+    const int q = lane >> 4, s = lane & 15;
+    Frag f;
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      i32x4 v;
+      if constexpr (LAYOUT == kKC) {
+        // (16 rows further on the swizzle is the same: a constant distance)
+        v = lds_read_b128(tile + (rc_step + 16 * h) * ROW_BYTES,
+                          kc_offset<ROW_BYTES>(rc0 + s, PAIRED ? (kk >> 1) * 8 + 2 * q + (kk & 1) : kk * 4 + q));
+      } else if constexpr (ES == kEI8) {
+        const int krow = kk * KA + 8 * q + (s >> 1), col = rc0 + rc_step + 16 * h + 8 * (s & 1);
+        v = i8x8_to_bf16x8(lds_read_tr8(tile + mc_offset<ROW_BYTES, ES>(krow, col)));
+      } else {
+        // (the transposing read of 16-bit elements: see below; a block of 16 lanes covers 4 k-rows of 16 columns)
+        const int krow = kk * KA + 8 * q + (s >> 2), col = rc0 + rc_step + 16 * h + 4 * (s & 3);
+        const i32x2 lo = lds_read_tr16(tile + mc_offset<ROW_BYTES, ES>(krow, col * 2));
+        const i32x2 hi = lds_read_tr16(tile + mc_offset<ROW_BYTES, ES>(krow + 4, col * 2));
+        v = i32x4{lo[0], lo[1], hi[0], hi[1]};
+      }
+#pragma unroll
+      for (int e = 0; e < 4; ++e) f[4 * h + e] = v[e];
+    }
+    return f;
+  } else if constexpr (LAYOUT == kKC) {
     static_assert(ES == EC, "contraction-contiguous operands are stored in the compute type");
     const int row = rc0 + (lane & 31), q = lane >> 5;
     tile += rc_step * ROW_BYTES;
@@ -609,9 +673,27 @@ struct GemmKernel {
   // factor 16 is taken out where they become floats.
   static constexpr bool I4I = I4 && EA == kEI8;
   static constexpr int EBS = I4 ? (int)kEI8 : EB;  // element kind of a B stage in LDS
-  static constexpr int KA = Mma<EC>::KA;
   static constexpr int WTM = BM / WM, WTN = BN / WN;
   static constexpr int TM = WTM / 32, TN = WTN / 32;
+  // 16x16x32 MFMAs (see Mma). An atom is then 32 deep and its fragments are 32 bytes per lane, so they are kept once
+  // where the order of an atom's blocks allows it: the blocks go outer index by outer index, the inner index (the one
+  // with four blocks or more, if there is one) fastest. An outer fragment is free after its last inner block and is
+  // next needed an outer index less than an atom later; an inner fragment is free in the last outer pass and needed
+  // NI blocks later. With NI >= 4 that is at least four blocks (sixteen MFMAs, 256 cycles of the matrix pipe for one
+  // wave, twice that with the SIMD's other wave) between the LDS read of a fragment and its first use. Smaller wave
+  // tiles double-buffer what does not have that distance, which takes an even number of atoms per k-step.
+  // Wave tiles of fewer than four blocks and classic pipelines with 32-deep k-steps keep the 32x32x16 form: their
+  // launches are bound by the operand stream, and the 16x16 form measured even or 2-3 % slower there (a 256-row gated
+  // unit on 256x256x32: 117.1 against 114.2 us).
+  static constexpr bool kColsOuter = TM >= 4 || TN < 4;
+  static constexpr int NI = kColsOuter ? TM : TN, NO = kColsOuter ? TN : TM;
+  static constexpr bool kDoubleInner = NI < 4, kDoubleOuter = (NO - 1) * NI < 4;
+  static constexpr bool M16 = (EA == kEBF16 || EA == kEF16) && EB == EA && TM * TN >= 4 && (BKC % 64 == 0 || SPLIT);
+  static constexpr int FA_COPIES = (kColsOuter ? kDoubleInner : kDoubleOuter) ? 2 : 1;
+  static constexpr int FB_COPIES = (kColsOuter ? kDoubleOuter : kDoubleInner) ? 2 : 1;
+  static constexpr int KA = Mma<EC, M16>::KA;
+  typedef typename Mma<EC, M16>::Frag Frag;
+  typedef typename std::conditional<M16, Acc4, f32x16>::type Acc;
   // Kernels that can quantise their result to fp8 with one scale per (row, 128 columns): the plain forward of bf16 and
   // fp8 operands, with whole quantisation tiles inside a workgroup's tile and inside or across whole wave columns.
   static constexpr bool QOUT = MODE == kFwd && (EA == kEBF16 || EA == kEF8) && EB == EA && BN % 128 == 0 &&
@@ -631,8 +713,8 @@ struct GemmKernel {
   // c >= 1 at the start of its own atom, while the MFMAs on fragment 0 run. 16 registers fewer than two sets of
   // converted fragments, which is what lets the 256 x 256 x 128 tile live in 256.
   static constexpr bool JOUT = LEAN && I4F && TN >= 2;
-  static_assert(KSTEPS % 2 == 0, "the fragment double buffer assumes an even number of k-atoms per step");
-  static_assert(!SPLIT || (MODE == kFwd && EA == EB && BK % 2 == 0), "split pipeline: plain forward, operands of one type");
+  static_assert(KSTEPS % 2 == 0 || (M16 && FA_COPIES == 1 && FB_COPIES == 1), "the fragment double buffer assumes an even number of k-atoms per step");
+  static_assert(!SPLIT || (MODE == kFwd && M16 && KSTEPS == 1 && BK % 2 == 0), "split pipeline: plain forward of 16-bit operands");
   static_assert(!I4 || (((I4P && (MODE == kFwd || MODE == kFwdGlu || MODE == kFwdSubK)) || (I4F && (MODE == kFwd || MODE == kFwdGlu || MODE == kFwdSubK)) ||
                         (I4I && (MODE == kFwd || MODE == kFwdGlu || MODE == kFwdSubK))) && !SPLIT),
                 "packed int4 weights: forward with bf16, fp8 or int8 activations");
@@ -660,6 +742,62 @@ struct GemmKernel {
   // What the launch bound asks for: waves per SIMD with that many workgroups on the CU.
   static constexpr int kWavesPerSimd = (THREADS / 64 + 3) / 4 * kWorkgroupsPerCu;
   static_assert(NS >= 2 && SMEM_BYTES <= 160 * 1024, "stages must fit the 160 KB LDS");
+
+  // One atom of 16x16x32 MFMAs: its TM x TN blocks in the order described at kColsOuter, with the LDS reads of the next
+  // atom's fragments (`READS`: from A tile `at`, atom `akk`, and B tile `bt`, atom `bkk`) and NL load slots of `issue`
+  // threaded between the blocks. `bar` runs once, before the first of those reads and loads: the barrier of a k-step
+  // whose next fragments come from the next stage. Fragments kept once put it NI blocks into the atom, so that the reads
+  // the previous atom ended on have arrived by then.
+  template <int NV, int PAR, bool READS, int NL, class Bar, class Issue>
+  static __device__ __forceinline__ void atom16(Acc (&acc)[TM][TN], Frag (&fa)[FA_COPIES][TM], Frag (&fb)[FB_COPIES][TN],
+                                                const unsigned char* at, int akk, const unsigned char* bt, int bkk, int wm,
+                                                int wn, int lane, Bar&& bar, Issue&& issue) {
+    constexpr int NM = TM * TN;
+    constexpr int BAR = kDoubleInner || kDoubleOuter ? 0 : NI - 1;
+    constexpr int LPM = (NL + NM - BAR - 1) / (NM - BAR);
+    auto read_a = [&](int i) {
+      if (i < NV) fa[FA_COPIES == 2 ? 1 - PAR : 0][i] = load_frag<LA, EA, EC, StageA::ROW_BYTES, false, true>(at, wm * 32, akk, lane, i * WM * 32);
+    };
+    auto read_b = [&](int j) {
+      if (NV > 0) fb[FB_COPIES == 2 ? 1 - PAR : 0][j] = load_frag<LB, EBS, EC, StageB::ROW_BYTES, false, true>(bt, wn * WTN, bkk, lane, j * 32);
+    };
+#pragma unroll
+    for (int t = 0; t < NM; ++t) {
+      const int o = t / NI, n = t % NI, i = kColsOuter ? n : o, j = kColsOuter ? o : n;
+      if (i < NV) acc[i][j] = mma_atom<EC>(fb[FB_COPIES == 2 ? PAR : 0][j], fa[FA_COPIES == 2 ? PAR : 0][i], acc[i][j]);
+      if (t == BAR) bar();
+      if constexpr (READS) {
+        // a fragment kept once: behind its last block; kept twice: an atom ahead of its first one
+#pragma unroll
+        for (int x = 0; x < NO; ++x)
+          if (t == (kDoubleOuter ? x * NI : x * NI + NI - 1)) kColsOuter ? read_b(x) : read_a(x);
+#pragma unroll
+        for (int x = 0; x < NI; ++x)
+          if (t == (kDoubleInner ? x : (NO - 1) * NI + x)) kColsOuter ? read_a(x) : read_b(x);
+      }
+      if (t >= BAR) {
+#pragma unroll
+        for (int q = 0; q < LPM; ++q)
+          if ((t - BAR) * LPM + q < NL) issue((t - BAR) * LPM + q);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  }
+  // The fragments of atom 0 of the first stage.
+  template <int NV>
+  static __device__ __forceinline__ void first_frags16(Frag (&fa)[FA_COPIES][TM], Frag (&fb)[FB_COPIES][TN], const unsigned char* at,
+                                                       const unsigned char* bt, int wm, int wn, int lane) {
+#pragma unroll
+    for (int i = 0; i < TM; ++i) {
+      fa[0][i] = fa[FA_COPIES - 1][i] = Frag{};
+      if (i < NV) fa[0][i] = load_frag<LA, EA, EC, StageA::ROW_BYTES, false, true>(at, wm * 32, 0, lane, i * WM * 32);
+    }
+#pragma unroll
+    for (int j = 0; j < TN; ++j) {
+      fb[0][j] = fb[FB_COPIES - 1][j] = Frag{};
+      if (NV > 0) fb[0][j] = load_frag<LB, EBS, EC, StageB::ROW_BYTES, false, true>(bt, wn * WTN, 0, lane, j * 32);
+    }
+  }
 
   // QO: the instantiation that stores fp8 with one scale per (row, 128 columns) (QOUT kernels only). It is a kernel of
   // its own so that the plain one carries none of its code or registers.
@@ -781,16 +919,15 @@ struct GemmKernel {
     const unsigned char* Bb = reinterpret_cast<const unsigned char*>(p.B);
     if constexpr (MODE != kDrhs) Bb += (int64_t)group * p.b_group_stride * elem_bytes(EB);
 
-    f32x16 acc[TM][TN];
+    Acc acc[TM][TN];
 #pragma unroll
     for (int i = 0; i < TM; ++i)
 #pragma unroll
       for (int j = 0; j < TN; ++j)
 #pragma unroll
-        for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.f;
+        for (int t = 0; t < 4; ++t) set4(acc[i][j], t, f32x4{0.f, 0.f, 0.f, 0.f});
 
     f32x16 pacc[SUBP ? TM : 1][SUBP ? TN : 1];  // (fp8 x fp8 with k-block scales) the current k-step's products
-    typedef typename Mma<EC>::Frag Frag;
     // Row blocks (32 rows) of this wave that hold at least one row the task stores. A task at a
     // group boundary can have only a few such rows; the blocks without any skip their LDS reads and
     // MFMAs (the wave still takes part in the loads and barriers). `full` selects at compile time
@@ -842,7 +979,7 @@ struct GemmKernel {
       } else if constexpr (I4I) {
         return i4x16_to_i8x16_times16(load_b_raw8(stage, j, kk));
       } else {
-        return load_frag<LB, EBS, EC, StageB::ROW_BYTES>(stage + StageA::BYTES, wn * WTN + j * 32, kk, lane);
+        return load_frag<LB, EBS, EC, StageB::ROW_BYTES, false, M16>(stage + StageA::BYTES, wn * WTN + j * 32, kk, lane);
       }
     };
     const int span = kc_end - kc_begin;
@@ -899,90 +1036,48 @@ struct GemmKernel {
 
       auto k_loop = [&](auto nv_tag) {
         constexpr int NV = decltype(nv_tag)::value;  // row blocks of this wave that hold rows of the task
-        Frag fa[2][TM], fb[2][TN];
-#pragma unroll
-        for (int i = 0; i < TM; ++i) fa[0][i] = fa[1][i] = Frag{};
-#pragma unroll
-        for (int j = 0; j < TN; ++j) fb[0][j] = fb[1][j] = Frag{};
-        // Read number r of an atom, in the order its MFMAs (row block major) first use the fragments.
-        auto read_frag = [&](Frag* a, Frag* b, int r, const unsigned char* atile, int akk, const unsigned char* btile, int bkk) {
-          if (r >= TM + TN) return;
-          const int f = r == 0 ? 0 : r <= TN ? TM + r - 1 : r - TN;
-          if (f < TM) {
-            if (f < NV) a[f] = load_frag<LA, EA, EC, StageA::ROW_BYTES>(atile, wm * 32, akk, lane, f * WM * 32);
-          } else {
-            if (NV > 0) b[f - TM] = load_frag<LB, EB, EC, StageB::ROW_BYTES>(btile, wn * WTN + (f - TM) * 32, bkk, lane);
-          }
-        };
-        constexpr int NM = TM * TN;
-        constexpr int RPM = (TM + TN + NM - 1) / NM;
-        // One atom: its MFMAs with, threaded between them, the reads of the next atom's fragments and (`NL` > 0) load
-        // slots 0 .. NL - 1 of `issue`.
-        auto atom = [&](auto nl_tag, const Frag* a, const Frag* b, Frag* na, Frag* nb, const unsigned char* atile, int akk,
-                        const unsigned char* btile, int bkk, auto issue) {
-          constexpr int NL = decltype(nl_tag)::value;
-          constexpr int LPM = (NL + NM - 1) / NM;
-#pragma unroll
-          for (int t = 0; t < NM; ++t) {
-            const int i = t / TN, j = t % TN;
-            if (i < NV) acc[i][j] = mma_atom<EC>(b[j], a[i], acc[i][j]);
-#pragma unroll
-            for (int r = 0; r < RPM; ++r) read_frag(na, nb, t * RPM + r, atile, akk, btile, bkk);
-#pragma unroll
-            for (int q = 0; q < LPM; ++q)
-              if (t * LPM + q < NL) issue(t * LPM + q);
-            __builtin_amdgcn_sched_barrier(0);
-          }
-        };
-        auto no_loads = [](int) {};
-#pragma unroll
-        for (int f = 0; f < TM + TN; ++f) read_frag(fa[0], fb[0], f, smem, 0, smem + B_REGION, 0);
+        Frag fa[FA_COPIES][TM], fb[FB_COPIES][TN];
+        first_frags16<NV>(fa, fb, smem, smem + B_REGION, wm, wn, lane);
         int a_idx = 0, b_idx = 0;  // stages of the current step
-        // One compute step. ODD: second half of its A stage, which it releases. STEADY: every load this step and the
-        // LOOK steps before it could issue exists, so the loads in flight are known at compile time; the other steps
-        // (the last few of a tile) issue what is left in one piece and wait for everything.
+        // One compute step (one atom). ODD: second half of its A stage, which it releases. STEADY: every load this step
+        // and the LOOK steps before it could issue exists, so the loads in flight are known at compile time; the other
+        // steps (the last few of a tile) issue what is left in one piece and wait for everything.
         auto k_step = [&](auto odd_tag, auto steady_tag, int kt) {
           constexpr bool ODD = decltype(odd_tag)::value, STEADY = decltype(steady_tag)::value;
-          const unsigned char* const a_cur = smem + a_idx * A_BYTES;
-          const unsigned char* const b_cur = smem + B_REGION + b_idx * B_BYTES;
-          constexpr int akk0 = ODD ? KSTEPS : 0;
           const int a_freed = a_idx, b_freed = b_idx;
           if (ODD) a_idx = a_idx + 1 == NS ? 0 : a_idx + 1;
           b_idx = b_idx + 1 == HB ? 0 : b_idx + 1;
           const unsigned char* const a_nxt = smem + a_idx * A_BYTES;
           const unsigned char* const b_nxt = smem + B_REGION + b_idx * B_BYTES;
-          constexpr int nkk0 = ODD ? 0 : KSTEPS;
+          constexpr int nkk = ODD ? 0 : 1;
           // (Pointers of the refills are computed here, far ahead of the MFMAs they are issued between.)
           const unsigned char* const src_b = uniform_pointer(gB0 + (int64_t)(kt + HB) * stepB);
           const unsigned char* const src_a = uniform_pointer(gA0 + (int64_t)((kt - 1) / 2 + NS) * stepA);
           const unsigned dst_b = smem_lds + B_REGION + b_freed * B_BYTES, dst_a = smem_lds + a_freed * A_BYTES;
-#pragma unroll
-          for (int kk = 0; kk + 1 < KSTEPS; ++kk)
-            atom(std::integral_constant<int, 0>{}, fa[kk & 1], fb[kk & 1], fa[(kk + 1) & 1], fb[(kk + 1) & 1], a_cur,
-                 akk0 + kk + 1, b_cur, kk + 1, no_loads);
-          // All LDS reads of this step are issued. After the barrier the next step's operands are complete and this
-          // step's B stage (and, after an odd step, its A stage) is free.
+          // All LDS reads of this step were issued in the step before. After the barrier the next step's operands are
+          // complete and this step's B stage (and, after an odd step, its A stage) is free.
           if constexpr (STEADY) {
-            barrier_after_direct_loads<(ODD ? kOdd : kEven)>();
-            auto issue = [&](int q) {
-              if (ODD && q < PA) da.issue_one(q, src_a, dst_a, wave);
-              else db.issue_one(q - (ODD ? PA : 0), src_b, dst_b, wave);
-            };
-            atom(std::integral_constant<int, (ODD ? PA : 0) + PB>{}, fa[(KSTEPS - 1) & 1], fb[(KSTEPS - 1) & 1], fa[0], fb[0],
-                 a_nxt, nkk0, b_nxt, 0, issue);
+            atom16<NV, 0, true, (ODD ? PA : 0) + PB>(acc, fa, fb, a_nxt, nkk, b_nxt, 0, wm, wn, lane,
+                                                     [&] { barrier_after_direct_loads<(ODD ? kOdd : kEven)>(); },
+                                                     [&](int q) {
+                                                       if (ODD && q < PA) da.issue_one(q, src_a, dst_a, wave);
+                                                       else db.issue_one(q - (ODD ? PA : 0), src_b, dst_b, wave);
+                                                     });
           } else {
-            barrier_after_direct_loads<0>();
-            if (ODD && (kt - 1) / 2 + NS < ndouble) {
+            // (After the last step the reads fetch fragments nobody uses, from LDS that is there.)
+            atom16<NV, 0, true, 0>(acc, fa, fb, a_nxt, nkk, b_nxt, 0, wm, wn, lane,
+                                   [&] {
+                                     barrier_after_direct_loads<0>();
+                                     if (ODD && (kt - 1) / 2 + NS < ndouble) {
 #pragma unroll
-              for (int q = 0; q < PA; ++q) da.issue_one(q, src_a, dst_a, wave);
-            }
-            if (kt + HB < nfull) {
+                                       for (int q = 0; q < PA; ++q) da.issue_one(q, src_a, dst_a, wave);
+                                     }
+                                     if (kt + HB < nfull) {
 #pragma unroll
-              for (int q = 0; q < PB; ++q) db.issue_one(q, src_b, dst_b, wave);
-            }
-            // (After the last step the reads below fetch fragments nobody uses, from LDS that is there.)
-            atom(std::integral_constant<int, 0>{}, fa[(KSTEPS - 1) & 1], fb[(KSTEPS - 1) & 1], fa[0], fb[0], a_nxt, nkk0,
-                 b_nxt, 0, no_loads);
+                                       for (int q = 0; q < PB; ++q) db.issue_one(q, src_b, dst_b, wave);
+                                     }
+                                   },
+                                   [](int) {});
           }
         };
         int kt = 0;
@@ -1081,89 +1176,162 @@ struct GemmKernel {
       // atom's fragments and, in the last atom of a k-step, the global loads that refill the stage
       // just released are threaded between those MFMAs one by one, so that the matrix pipe is
       // never left waiting behind a block of memory instructions.
-      auto k_loop = [&](auto nv_tag) {
-        constexpr int NV = decltype(nv_tag)::value;  // row blocks of this wave that hold rows of the task
-        Frag fa[LEAN ? 1 : 2][TM], fb[2][TN];
-#pragma unroll
-        for (int i = 0; i < TM; ++i) fa[0][i] = fa[LEAN ? 0 : 1][i] = Frag{};
-#pragma unroll
-        for (int j = 0; j < TN; ++j) fb[0][j] = fb[1][j] = Frag{};
-        // Read number r of an atom, in the order the atom's MFMAs (row block major) first use the
-        // fragments: A0, B0, B1, ..., then A1, A2, ... Every fragment is then requested at least
-        // TM*TN - 2 MFMAs before its first use. A fragment f < TM is the A fragment of row block f,
-        // else the B fragment f - TM.
-        // Packed int4 weights: the 8 bytes a lane reads for an even atom hold the B fragments of that atom and of the
-        // next; they are kept as read (`raw`) and converted half by half. The list of an even atom is then A0, the
-        // byte reads, A1, ..., and last the conversions of the first halves; that of an odd atom A0, the conversions
-        // of the second halves, A1, ...
-        [[maybe_unused]] i32x2 raw[I4P ? TN : 1];
-        [[maybe_unused]] i32x4 rawf[I4F ? TN : 1];  // (fp8 activations) a fragment's bytes as read
-        [[maybe_unused]] i32x2 rawi[I4I ? TN : 1];  // (int8 activations) likewise
-        // (kFwdSubK: times the scale of the lane's column for the stage's k-block, like load_b_frag)
-        [[maybe_unused]] auto convert_i4 = [&](int w, const unsigned char* stage, int j) -> i32x4 {
-          if constexpr (SUBK) {
-            const float scale = *reinterpret_cast<const float*>(stage + StageA::BYTES + StageB::BYTES +
-                                                                4 * (wn * WTN + j * 32 + (lane & 31)));
-            return i4x8_to_bf16x8_scaled(w, scale * kPackedInt4Unscale);
-          } else {
-            return i4x8_to_bf16x8_times16(w);
-          }
+      if constexpr (M16) {
+        auto k_loop16 = [&](auto nv_tag) {
+          constexpr int NV = decltype(nv_tag)::value;  // row blocks of this wave that hold rows of the task
+          Frag fa[FA_COPIES][TM], fb[FB_COPIES][TN];
+          first_frags16<NV>(fa, fb, smem, smem + StageA::BYTES, wm, wn, lane);
+          int cur_stage = 0;
+          const StepPtrs none = {};
+          // One k-step, as in k_loop below.
+          auto k_step = [&](auto refill_tag, auto more_tag, int kt) {
+            constexpr bool REFILL = decltype(refill_tag)::value, MORE = decltype(more_tag)::value;
+            const unsigned char* cur = smem + cur_stage * STAGE_BYTES;
+            const int freed = cur_stage;
+            cur_stage = cur_stage + 1 == NS ? 0 : cur_stage + 1;
+            const unsigned char* nxt = smem + cur_stage * STAGE_BYTES;
+            const StepPtrs sp = REFILL ? step_ptrs(kt + NS, freed) : none;
+            auto inner = [&](auto kk_tag) {
+              constexpr int kk = decltype(kk_tag)::value;
+              if constexpr (kk + 1 < KSTEPS)
+                atom16<NV, kk & 1, true, 0>(acc, fa, fb, cur, kk + 1, cur + StageA::BYTES, kk + 1, wm, wn, lane, [] {}, [](int) {});
+            };
+            inner(std::integral_constant<int, 0>{});
+            inner(std::integral_constant<int, 1>{});
+            inner(std::integral_constant<int, 2>{});
+            static_assert(KSTEPS <= 4, "atoms of a k-step are written out");
+            atom16<NV, (KSTEPS - 1) & 1, MORE, REFILL ? NLD : 0>(
+                acc, fa, fb, nxt, 0, nxt + StageA::BYTES, 0, wm, wn, lane, [&] { step_barrier(REFILL || kt + NS - 1 < nfull); },
+                [&](int q) { issue_slot(q, sp); });
+          };
+          int kt = 0;
+          for (; kt + NS < nfull; ++kt) k_step(std::true_type{}, std::true_type{}, kt);
+          for (; kt + 1 < nfull; ++kt) k_step(std::false_type{}, std::true_type{}, kt);
+          for (; kt < nfull; ++kt) k_step(std::false_type{}, std::false_type{}, kt);
         };
-        constexpr int NRD = I4 ? TM + 2 * TN : TM + TN;  // (fp8 activations: A0, the byte reads, A1, ..., the conversions)  // entries of an atom's list
-        auto read_frag = [&](Frag* a, Frag* b, int r, const unsigned char* stage, int kk) {
-          if (r >= NRD) return;
-          const int f = r == 0 ? 0 : r <= TN ? TM + r - 1 : r < TM + TN ? r - TN : r;
-          if (f < TM) {
-            if (f < NV) a[f] = load_frag<LA, EA, EC, StageA::ROW_BYTES, I4P>(stage, wm * 32, kk, lane, f * WM * 32);
-          } else if (f < TM + TN) {
-            if constexpr (I4F) {
-              if (NV > 0) rawf[f - TM] = load_b_raw(stage, f - TM, kk);
-            } else if constexpr (I4I) {
-              if (NV > 0) rawi[f - TM] = load_b_raw8(stage, f - TM, kk);
-            } else if constexpr (I4P) {
-              const int j = f - TM;
-              if (NV > 0) {
-                if (kk & 1) {
-                  b[j] = convert_i4(raw[j][1], stage, j);
-                } else {
-                  const int blk = lane >> 4, s_ = lane & 15;
-                  const int col = wn * WTN + j * 32 + 16 * (blk & 1) + 8 * (s_ & 1);
-                  const int krow = (kk >> 1) * 16 + 8 * (blk >> 1) + (s_ >> 1);
-                  raw[j] = lds_read_tr8(stage + StageA::BYTES + mc_offset<StageB::ROW_BYTES, EBS>(krow, col));
-                }
-              }
+        dispatch_upto<0, TM>(nv_sel, k_loop16);
+      } else {
+        auto k_loop = [&](auto nv_tag) {
+          constexpr int NV = decltype(nv_tag)::value;  // row blocks of this wave that hold rows of the task
+          Frag fa[LEAN ? 1 : 2][TM], fb[2][TN];
+#pragma unroll
+          for (int i = 0; i < TM; ++i) fa[0][i] = fa[LEAN ? 0 : 1][i] = Frag{};
+#pragma unroll
+          for (int j = 0; j < TN; ++j) fb[0][j] = fb[1][j] = Frag{};
+          // Read number r of an atom, in the order the atom's MFMAs (row block major) first use the
+          // fragments: A0, B0, B1, ..., then A1, A2, ... Every fragment is then requested at least
+          // TM*TN - 2 MFMAs before its first use. A fragment f < TM is the A fragment of row block f,
+          // else the B fragment f - TM.
+          // Packed int4 weights: the 8 bytes a lane reads for an even atom hold the B fragments of that atom and of the
+          // next; they are kept as read (`raw`) and converted half by half. The list of an even atom is then A0, the
+          // byte reads, A1, ..., and last the conversions of the first halves; that of an odd atom A0, the conversions
+          // of the second halves, A1, ...
+          [[maybe_unused]] i32x2 raw[I4P ? TN : 1];
+          [[maybe_unused]] i32x4 rawf[I4F ? TN : 1];  // (fp8 activations) a fragment's bytes as read
+          [[maybe_unused]] i32x2 rawi[I4I ? TN : 1];  // (int8 activations) likewise
+          // (kFwdSubK: times the scale of the lane's column for the stage's k-block, like load_b_frag)
+          [[maybe_unused]] auto convert_i4 = [&](int w, const unsigned char* stage, int j) -> i32x4 {
+            if constexpr (SUBK) {
+              const float scale = *reinterpret_cast<const float*>(stage + StageA::BYTES + StageB::BYTES +
+                                                                  4 * (wn * WTN + j * 32 + (lane & 31)));
+              return i4x8_to_bf16x8_scaled(w, scale * kPackedInt4Unscale);
             } else {
-              if (NV > 0) b[f - TM] = load_b_frag(stage, f - TM, kk);
+              return i4x8_to_bf16x8_times16(w);
             }
-          } else if constexpr (I4F) {
-            if (NV > 0) b[f - TM - TN] = i4x32_to_biased_f8x32(rawf[f - TM - TN]);
-          } else if constexpr (I4I) {
-            if (NV > 0) b[f - TM - TN] = i4x16_to_i8x16_times16(rawi[f - TM - TN]);
-          } else if constexpr (I4P) {
-            if (NV > 0 && !(kk & 1)) b[f - TM - TN] = convert_i4(raw[f - TM - TN][0], stage, f - TM - TN);
-          }
-        };
-        constexpr int NM = TM * TN;                      // MFMAs per atom
-        constexpr int RPM = (NRD + NM - 1) / NM;         // list entries threaded after each MFMA
-        constexpr int LPM = (NLD + NM - 1) / NM;         // load slots threaded after each MFMA
-        // (`reads` and `loads` are compile-time tags: a run-time test after every MFMA would put two
-        // branches into each MFMA slot.)
-        auto atom = [&](auto reads_tag, auto loads_tag, const Frag* a, const Frag* b, Frag* na, Frag* nb,
-                        const unsigned char* rd_stage, int rd_kk, const StepPtrs& sp, auto first_tag) {
-          constexpr bool reads = decltype(reads_tag)::value, loads = decltype(loads_tag)::value;
-          constexpr bool first_of_step = decltype(first_tag)::value;  // (SUBP) the partial accumulators start at zero
-          if constexpr (JOUT) {
+          };
+          constexpr int NRD = I4 ? TM + 2 * TN : TM + TN;  // (fp8 activations: A0, the byte reads, A1, ..., the conversions)  // entries of an atom's list
+          auto read_frag = [&](Frag* a, Frag* b, int r, const unsigned char* stage, int kk) {
+            if (r >= NRD) return;
+            const int f = r == 0 ? 0 : r <= TN ? TM + r - 1 : r < TM + TN ? r - TN : r;
+            if (f < TM) {
+              if (f < NV) a[f] = load_frag<LA, EA, EC, StageA::ROW_BYTES, I4P>(stage, wm * 32, kk, lane, f * WM * 32);
+            } else if (f < TM + TN) {
+              if constexpr (I4F) {
+                if (NV > 0) rawf[f - TM] = load_b_raw(stage, f - TM, kk);
+              } else if constexpr (I4I) {
+                if (NV > 0) rawi[f - TM] = load_b_raw8(stage, f - TM, kk);
+              } else if constexpr (I4P) {
+                const int j = f - TM;
+                if (NV > 0) {
+                  if (kk & 1) {
+                    b[j] = convert_i4(raw[j][1], stage, j);
+                  } else {
+                    const int blk = lane >> 4, s_ = lane & 15;
+                    const int col = wn * WTN + j * 32 + 16 * (blk & 1) + 8 * (s_ & 1);
+                    const int krow = (kk >> 1) * 16 + 8 * (blk >> 1) + (s_ >> 1);
+                    raw[j] = lds_read_tr8(stage + StageA::BYTES + mc_offset<StageB::ROW_BYTES, EBS>(krow, col));
+                  }
+                }
+              } else {
+                if (NV > 0) b[f - TM] = load_b_frag(stage, f - TM, kk);
+              }
+            } else if constexpr (I4F) {
+              if (NV > 0) b[f - TM - TN] = i4x32_to_biased_f8x32(rawf[f - TM - TN]);
+            } else if constexpr (I4I) {
+              if (NV > 0) b[f - TM - TN] = i4x16_to_i8x16_times16(rawi[f - TM - TN]);
+            } else if constexpr (I4P) {
+              if (NV > 0 && !(kk & 1)) b[f - TM - TN] = convert_i4(raw[f - TM - TN][0], stage, f - TM - TN);
+            }
+          };
+          constexpr int NM = TM * TN;                      // MFMAs per atom
+          constexpr int RPM = (NRD + NM - 1) / NM;         // list entries threaded after each MFMA
+          constexpr int LPM = (NLD + NM - 1) / NM;         // load slots threaded after each MFMA
+          // (`reads` and `loads` are compile-time tags: a run-time test after every MFMA would put two
+          // branches into each MFMA slot.)
+          auto atom = [&](auto reads_tag, auto loads_tag, const Frag* a, const Frag* b, Frag* na, Frag* nb,
+                          const unsigned char* rd_stage, int rd_kk, const StepPtrs& sp, auto first_tag) {
+            constexpr bool reads = decltype(reads_tag)::value, loads = decltype(loads_tag)::value;
+            constexpr bool first_of_step = decltype(first_tag)::value;  // (SUBP) the partial accumulators start at zero
+            if constexpr (JOUT) {
+#pragma unroll
+              for (int t = 0; t < NM; ++t) {
+                const int j = t / TM, i = t % TM;
+                if (i < NV) acc[i][j] = mma_atom<EC>(fb[0][j], fa[0][i], acc[i][j]);
+                if (t < TN - 1 && NV > 0) fb[0][t + 1] = i4x32_to_biased_f8x32(rawf[t + 1]);
+                if (reads) {
+                  // (the buffer of fragment 0's bytes is free since the previous atom, that of fragment t since the line above)
+                  if (t < TN && NV > 0) rawf[t] = load_b_raw(rd_stage, t, rd_kk);
+                  if (t == TM && NV > 0) fb[0][0] = i4x32_to_biased_f8x32(rawf[0]);
+                  if (j == TN - 1 && i < NV)
+                    fa[0][i] = load_frag<LA, EA, EC, StageA::ROW_BYTES>(rd_stage, wm * 32, rd_kk, lane, i * WM * 32);
+                }
+                if (loads) {
+#pragma unroll
+                  for (int q = 0; q < LPM; ++q) issue_slot(t * LPM + q, sp);
+                }
+                __builtin_amdgcn_sched_barrier(0);
+              }
+              return;
+            }
 #pragma unroll
             for (int t = 0; t < NM; ++t) {
-              const int j = t / TM, i = t % TM;
-              if (i < NV) acc[i][j] = mma_atom<EC>(fb[0][j], fa[0][i], acc[i][j]);
-              if (t < TN - 1 && NV > 0) fb[0][t + 1] = i4x32_to_biased_f8x32(rawf[t + 1]);
+              const int i = t / TN, j = t % TN;
+              if constexpr (SUBP) {
+                if (i < NV) {
+                  f32x16 c = pacc[i][j];
+                  if constexpr (first_of_step) {
+#pragma unroll
+                    for (int e = 0; e < 16; ++e) c[e] = 0.f;
+                  }
+                  pacc[i][j] = mma_atom<EC>(b[j], a[i], c);
+                }
+              } else {
+                if (i < NV) acc[i][j] = mma_atom<EC>(b[j], a[i], acc[i][j]);
+              }
               if (reads) {
-                // (the buffer of fragment 0's bytes is free since the previous atom, that of fragment t since the line above)
-                if (t < TN && NV > 0) rawf[t] = load_b_raw(rd_stage, t, rd_kk);
-                if (t == TM && NV > 0) fb[0][0] = i4x32_to_biased_f8x32(rawf[0]);
-                if (j == TN - 1 && i < NV)
-                  fa[0][i] = load_frag<LA, EA, EC, StageA::ROW_BYTES>(rd_stage, wm * 32, rd_kk, lane, i * WM * 32);
+                if constexpr (LEAN) {
+                  // rhs fragment t after MFMA t; the lhs fragment of a row block after the block's last MFMA
+                  if (t < TN) read_frag(na, nb, t + 1, rd_stage, rd_kk);
+                  if (j == TN - 1) read_frag(na, nb, i == 0 ? 0 : TN + i, rd_stage, rd_kk);
+                  if constexpr (I4F) {
+                    // the bytes of rhs fragment c become fp8 two MFMAs or more after their read was issued
+                    constexpr int LAG = TN == 1 ? 2 : TN;
+                    if (t >= LAG && t < LAG + TN) read_frag(na, nb, TM + TN + t - LAG, rd_stage, rd_kk);
+                  }
+                } else {
+#pragma unroll
+                  for (int r = 0; r < RPM; ++r) read_frag(na, nb, t * RPM + r, rd_stage, rd_kk);
+                }
               }
               if (loads) {
 #pragma unroll
@@ -1171,152 +1339,117 @@ struct GemmKernel {
               }
               __builtin_amdgcn_sched_barrier(0);
             }
-            return;
-          }
-#pragma unroll
-          for (int t = 0; t < NM; ++t) {
-            const int i = t / TN, j = t % TN;
-            if constexpr (SUBP) {
-              if (i < NV) {
-                f32x16 c = pacc[i][j];
-                if constexpr (first_of_step) {
-#pragma unroll
-                  for (int e = 0; e < 16; ++e) c[e] = 0.f;
-                }
-                pacc[i][j] = mma_atom<EC>(b[j], a[i], c);
-              }
-            } else {
-              if (i < NV) acc[i][j] = mma_atom<EC>(b[j], a[i], acc[i][j]);
-            }
-            if (reads) {
-              if constexpr (LEAN) {
-                // rhs fragment t after MFMA t; the lhs fragment of a row block after the block's last MFMA
-                if (t < TN) read_frag(na, nb, t + 1, rd_stage, rd_kk);
-                if (j == TN - 1) read_frag(na, nb, i == 0 ? 0 : TN + i, rd_stage, rd_kk);
-                if constexpr (I4F) {
-                  // the bytes of rhs fragment c become fp8 two MFMAs or more after their read was issued
-                  constexpr int LAG = TN == 1 ? 2 : TN;
-                  if (t >= LAG && t < LAG + TN) read_frag(na, nb, TM + TN + t - LAG, rd_stage, rd_kk);
-                }
-              } else {
-#pragma unroll
-                for (int r = 0; r < RPM; ++r) read_frag(na, nb, t * RPM + r, rd_stage, rd_kk);
-              }
-            }
-            if (loads) {
-#pragma unroll
-              for (int q = 0; q < LPM; ++q) issue_slot(t * LPM + q, sp);
-            }
-            __builtin_amdgcn_sched_barrier(0);
-          }
-        };
+          };
 
-        if constexpr (JOUT) {
+          if constexpr (JOUT) {
 #pragma unroll
-          for (int i = 0; i < TM; ++i)
-            if (i < NV) fa[0][i] = load_frag<LA, EA, EC, StageA::ROW_BYTES>(smem, wm * 32, 0, lane, i * WM * 32);
-#pragma unroll
-          for (int j = 0; j < TN; ++j)
-            if (NV > 0) rawf[j] = load_b_raw(smem, j, 0);
-          if (NV > 0) fb[0][0] = i4x32_to_biased_f8x32(rawf[0]);
-        } else {
-#pragma unroll
-          for (int f = 0; f < NRD; ++f) read_frag(fa[0], fb[0], f, smem, 0);
-        }
-        int cur_stage = 0;
-        const StepPtrs none = {};
-        // One k-step. `refill_tag`: the stage it releases is refilled with k-step kt + NS;
-        // `more_tag`: another k-step follows, so the next stage's first fragments are read.
-        auto k_step = [&](auto refill_tag, auto more_tag, int kt) {
-          const unsigned char* cur = smem + cur_stage * STAGE_BYTES;
-          const int freed = cur_stage;
-          cur_stage = cur_stage + 1 == NS ? 0 : cur_stage + 1;
-          const unsigned char* nxt = smem + cur_stage * STAGE_BYTES;
-          // (Pointers of the refill are computed here, far ahead of the MFMAs they are issued between.)
-          const StepPtrs sp = decltype(refill_tag)::value ? step_ptrs(kt + NS, freed) : none;
-          static_assert(!(SUBP && EC == kEF8) || KSTEPS == 2, "the partial accumulators restart with the first of two atoms");
-          // int8: the int32 sums stay exact over a whole k-block, so they are folded in at the end of the block
-          // only (a fold costs as much vector work as three k-steps of int8 MFMAs); fp8: after every k-step.
-          [[maybe_unused]] bool block_end = true;
-          if constexpr (SUBP && EC == kEI8) {
-            const int mask = (1 << p.log2_block_rows) - 1;
-            const int k0 = kc_begin + kt * BK;
-            block_end = ((k0 + BK) & mask) == 0 || kt + 1 == nfull;
-            if ((k0 & mask) == 0) {
-#pragma unroll
-              for (int i = 0; i < TM; ++i)
-#pragma unroll
-                for (int j = 0; j < TN; ++j)
-#pragma unroll
-                  for (int e = 0; e < 16; ++e) pacc[i][j][e] = 0.f;
-            }
-#pragma unroll
-            for (int kk = 0; kk + 1 < KSTEPS; ++kk)
-              atom(std::true_type{}, std::false_type{}, fa[kk & 1], fb[kk & 1], fa[(kk + 1) & 1], fb[(kk + 1) & 1], cur,
-                   kk + 1, none, std::false_type{});
-          } else if constexpr (SUBP) {
-            atom(std::true_type{}, std::false_type{}, fa[0], fb[0], fa[1], fb[1], cur, 1, none, std::true_type{});
-          } else {
-#pragma unroll
-            for (int kk = 0; kk + 1 < KSTEPS; ++kk)
-              atom(std::true_type{}, std::false_type{}, fa[LEAN ? 0 : kk & 1], fb[kk & 1], fa[LEAN ? 0 : (kk + 1) & 1],
-                   fb[(kk + 1) & 1], cur, kk + 1, none, std::false_type{});
-          }
-          // All LDS reads of `cur` are issued. After the barrier the next stage is complete and `cur`
-          // is free: the last atom's MFMAs cover the first fragment reads of the next stage and the
-          // issue of the loads that refill `cur` with k-step kt + NS.
-          step_barrier(decltype(refill_tag)::value || kt + NS - 1 < nfull);
-          atom(more_tag, refill_tag, fa[LEAN ? 0 : (KSTEPS - 1) & 1], fb[(KSTEPS - 1) & 1], fa[0], fb[0], nxt, 0, sp, std::false_type{});
-          if constexpr (SUBP) if (block_end) {
-            // Fold the products into the result with the scales of their k-block: lane l holds row l % 32
-            // and, for t = 0..3, columns 8 t + 4 (l / 32) + {0..3} of every 32 x 32 block.
-            const unsigned char* slot = smem + NS * STAGE_BYTES + (kt % (NS + 1)) * RING_SLOT;
-            float xs[TM];
-            // (fp8 x packed int4: the weights went in as (w + 8) / 512, so a product sum is 512 part - 8 rowsum(x); with
-            // xs' = 512 xs and xoff = -8 rowsum xs a fold is two fused multiply-adds per element: ws (xs' part + xoff))
-            [[maybe_unused]] float xoff[TM];
-#pragma unroll
-            for (int i = 0; i < TM; ++i) {
-              xs[i] = *reinterpret_cast<const float*>(slot + BN * 4 + 4 * (row_block(i) * 32 + (lane & 31)));
-              if constexpr (I4I) xs[i] *= kPackedInt4Unscale;  // (the weights went into the MFMAs times 16)
-              if constexpr (I4F) {
-                xoff[i] = -8.f * xs[i] * *reinterpret_cast<const float*>(slot + (BN + BM) * 4 + 4 * (row_block(i) * 32 + (lane & 31)));
-                xs[i] *= 512.f;
-              }
-            }
+            for (int i = 0; i < TM; ++i)
+              if (i < NV) fa[0][i] = load_frag<LA, EA, EC, StageA::ROW_BYTES>(smem, wm * 32, 0, lane, i * WM * 32);
 #pragma unroll
             for (int j = 0; j < TN; ++j)
+              if (NV > 0) rawf[j] = load_b_raw(smem, j, 0);
+            if (NV > 0) fb[0][0] = i4x32_to_biased_f8x32(rawf[0]);
+          } else {
 #pragma unroll
-              for (int t = 0; t < 4; ++t) {
-                const f32x4 wsc = *reinterpret_cast<const f32x4*>(slot + 4 * (wn * WTN + j * 32 + 8 * t + 4 * (lane >> 5)));
+            for (int f = 0; f < NRD; ++f) read_frag(fa[0], fb[0], f, smem, 0);
+          }
+          int cur_stage = 0;
+          const StepPtrs none = {};
+          // One k-step. `refill_tag`: the stage it releases is refilled with k-step kt + NS;
+          // `more_tag`: another k-step follows, so the next stage's first fragments are read.
+          auto k_step = [&](auto refill_tag, auto more_tag, int kt) {
+            const unsigned char* cur = smem + cur_stage * STAGE_BYTES;
+            const int freed = cur_stage;
+            cur_stage = cur_stage + 1 == NS ? 0 : cur_stage + 1;
+            const unsigned char* nxt = smem + cur_stage * STAGE_BYTES;
+            // (Pointers of the refill are computed here, far ahead of the MFMAs they are issued between.)
+            const StepPtrs sp = decltype(refill_tag)::value ? step_ptrs(kt + NS, freed) : none;
+            static_assert(!(SUBP && EC == kEF8) || KSTEPS == 2, "the partial accumulators restart with the first of two atoms");
+            // int8: the int32 sums stay exact over a whole k-block, so they are folded in at the end of the block
+            // only (a fold costs as much vector work as three k-steps of int8 MFMAs); fp8: after every k-step.
+            [[maybe_unused]] bool block_end = true;
+            if constexpr (SUBP && EC == kEI8) {
+              const int mask = (1 << p.log2_block_rows) - 1;
+              const int k0 = kc_begin + kt * BK;
+              block_end = ((k0 + BK) & mask) == 0 || kt + 1 == nfull;
+              if ((k0 & mask) == 0) {
 #pragma unroll
                 for (int i = 0; i < TM; ++i)
-                  if (i < NV) {
 #pragma unroll
-                    for (int e = 0; e < 4; ++e) {
-                      float part = pacc[i][j][4 * t + e];
-                      if constexpr (EC == kEI8) part = (float)__builtin_bit_cast(int, part);  // int32 partial sums
-                      if constexpr (I4F) acc[i][j][4 * t + e] = fmaf(wsc[e], fmaf(xs[i], part, xoff[i]), acc[i][j][4 * t + e]);
-                      else acc[i][j][4 * t + e] += part * (xs[i] * wsc[e]);
-                    }
-                  }
+                  for (int j = 0; j < TN; ++j)
+#pragma unroll
+                    for (int e = 0; e < 16; ++e) pacc[i][j][e] = 0.f;
               }
-          }
+#pragma unroll
+              for (int kk = 0; kk + 1 < KSTEPS; ++kk)
+                atom(std::true_type{}, std::false_type{}, fa[kk & 1], fb[kk & 1], fa[(kk + 1) & 1], fb[(kk + 1) & 1], cur,
+                     kk + 1, none, std::false_type{});
+            } else if constexpr (SUBP) {
+              atom(std::true_type{}, std::false_type{}, fa[0], fb[0], fa[1], fb[1], cur, 1, none, std::true_type{});
+            } else {
+#pragma unroll
+              for (int kk = 0; kk + 1 < KSTEPS; ++kk)
+                atom(std::true_type{}, std::false_type{}, fa[LEAN ? 0 : kk & 1], fb[kk & 1], fa[LEAN ? 0 : (kk + 1) & 1],
+                     fb[(kk + 1) & 1], cur, kk + 1, none, std::false_type{});
+            }
+            // All LDS reads of `cur` are issued. After the barrier the next stage is complete and `cur`
+            // is free: the last atom's MFMAs cover the first fragment reads of the next stage and the
+            // issue of the loads that refill `cur` with k-step kt + NS.
+            step_barrier(decltype(refill_tag)::value || kt + NS - 1 < nfull);
+            atom(more_tag, refill_tag, fa[LEAN ? 0 : (KSTEPS - 1) & 1], fb[(KSTEPS - 1) & 1], fa[0], fb[0], nxt, 0, sp, std::false_type{});
+            if constexpr (SUBP) if (block_end) {
+              // Fold the products into the result with the scales of their k-block: lane l holds row l % 32
+              // and, for t = 0..3, columns 8 t + 4 (l / 32) + {0..3} of every 32 x 32 block.
+              const unsigned char* slot = smem + NS * STAGE_BYTES + (kt % (NS + 1)) * RING_SLOT;
+              float xs[TM];
+              // (fp8 x packed int4: the weights went in as (w + 8) / 512, so a product sum is 512 part - 8 rowsum(x); with
+              // xs' = 512 xs and xoff = -8 rowsum xs a fold is two fused multiply-adds per element: ws (xs' part + xoff))
+              [[maybe_unused]] float xoff[TM];
+#pragma unroll
+              for (int i = 0; i < TM; ++i) {
+                xs[i] = *reinterpret_cast<const float*>(slot + BN * 4 + 4 * (row_block(i) * 32 + (lane & 31)));
+                if constexpr (I4I) xs[i] *= kPackedInt4Unscale;  // (the weights went into the MFMAs times 16)
+                if constexpr (I4F) {
+                  xoff[i] = -8.f * xs[i] * *reinterpret_cast<const float*>(slot + (BN + BM) * 4 + 4 * (row_block(i) * 32 + (lane & 31)));
+                  xs[i] *= 512.f;
+                }
+              }
+#pragma unroll
+              for (int j = 0; j < TN; ++j)
+#pragma unroll
+                for (int t = 0; t < 4; ++t) {
+                  const f32x4 wsc = *reinterpret_cast<const f32x4*>(slot + 4 * (wn * WTN + j * 32 + 8 * t + 4 * (lane >> 5)));
+#pragma unroll
+                  for (int i = 0; i < TM; ++i)
+                    if (i < NV) {
+#pragma unroll
+                      for (int e = 0; e < 4; ++e) {
+                        float part = pacc[i][j][4 * t + e];
+                        if constexpr (EC == kEI8) part = (float)__builtin_bit_cast(int, part);  // int32 partial sums
+                        if constexpr (I4F) acc[i][j][4 * t + e] = fmaf(wsc[e], fmaf(xs[i], part, xoff[i]), acc[i][j][4 * t + e]);
+                        else acc[i][j][4 * t + e] += part * (xs[i] * wsc[e]);
+                      }
+                    }
+                }
+            }
+          };
+          // Steady state first (every step refills), then the last NS steps in loops of their own, so
+          // that the hot loop is one straight-line body.
+          int kt = 0;
+          for (; kt + NS < nfull; ++kt) k_step(std::true_type{}, std::true_type{}, kt);
+          for (; kt + 1 < nfull; ++kt) k_step(std::false_type{}, std::true_type{}, kt);
+          for (; kt < nfull; ++kt) k_step(std::false_type{}, std::false_type{}, kt);
         };
-        // Steady state first (every step refills), then the last NS steps in loops of their own, so
-        // that the hot loop is one straight-line body.
-        int kt = 0;
-        for (; kt + NS < nfull; ++kt) k_step(std::true_type{}, std::true_type{}, kt);
-        for (; kt + 1 < nfull; ++kt) k_step(std::false_type{}, std::true_type{}, kt);
-        for (; kt < nfull; ++kt) k_step(std::false_type{}, std::false_type{}, kt);
-      };
-      dispatch_upto<0, TM>(nv_sel, k_loop);
+        dispatch_upto<0, TM>(nv_sel, k_loop);
+      }
       if constexpr (I4P && !SUBK) {
         // (the weights went into the MFMAs times 16)
 #pragma unroll
         for (int i = 0; i < TM; ++i)
 #pragma unroll
-          for (int j = 0; j < TN; ++j) acc[i][j] *= kPackedInt4Unscale;
+          for (int j = 0; j < TN; ++j)
+#pragma unroll
+            for (int t = 0; t < 4; ++t) set4(acc[i][j], t, get4(acc[i][j], t) * kPackedInt4Unscale);
       }
     }
     // (gate-up, per-k-block-scale and packed-int4 problems are taken only with whole k-steps)
@@ -1336,11 +1469,11 @@ struct GemmKernel {
           for (int j = 0; j < TN; ++j) fb[j] = Frag{};
 #pragma unroll
           for (int i = 0; i < TM; ++i)
-            if ((rmask >> i) & 1u) fa[i] = load_frag<LA, EA, EC, TailA::ROW_BYTES>(smem, row_block(i) * 32, kk, lane);
+            if ((rmask >> i) & 1u) fa[i] = load_frag<LA, EA, EC, TailA::ROW_BYTES, false, M16>(smem, row_block(i) * 32, kk, lane);
           if (rmask != 0) {
 #pragma unroll
             for (int j = 0; j < TN; ++j)
-              fb[j] = load_frag<LB, EB, EC, StageB::ROW_BYTES>(smem + TailA::BYTES, wn * WTN + j * 32, kk, lane);
+              fb[j] = load_frag<LB, EB, EC, StageB::ROW_BYTES, false, M16>(smem + TailA::BYTES, wn * WTN + j * 32, kk, lane);
           }
 #pragma unroll
           for (int i = 0; i < TM; ++i)
@@ -1373,7 +1506,7 @@ struct GemmKernel {
           for (int j = 0; j < TN; ++j)
 #pragma unroll
             for (int q = 0; q < 4; ++q) {
-              const f32x4 v = {acc[i][j][4 * q], acc[i][j][4 * q + 1], acc[i][j][4 * q + 2], acc[i][j][4 * q + 3]};
+              const f32x4 v = get4(acc[i][j], q);
               __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(i32x4, v), mine, (int)lane_off,
                                                      ((i * TN + j) * 4 + q) * THREADS * 16, kDeviceScope);
             }
@@ -1406,25 +1539,23 @@ struct GemmKernel {
             for (int q = 0; q < 4; ++q) {
               const f32x4 v = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(
                                                             theirs, (int)lane_off, ((i * TN + j) * 4 + q) * THREADS * 16, kDeviceScope));
-#pragma unroll
-              for (int e = 0; e < 4; ++e) {
-                if constexpr (EC == kEI8 && !SUBP) {
-                  // (int8 x int8: the registers hold the bits of exact int32 sums)
-                  // (scalar copies first: a bit cast applied to a vector's element read element 0)
-                  const float have = acc[i][j][4 * q + e], add = v[e];
-                  const int sum = __builtin_bit_cast(int, have) + __builtin_bit_cast(int, add);
-                  acc[i][j][4 * q + e] = pp == 0 ? add : __builtin_bit_cast(float, sum);
-                } else {
-                  acc[i][j][4 * q + e] = pp == 0 ? v[e] : acc[i][j][4 * q + e] + v[e];
-                }
+              f32x4 sum;
+              const f32x4 have = get4(acc[i][j], q);
+              if constexpr (EC == kEI8 && !SUBP) {
+                // (int8 x int8: the registers hold the bits of exact int32 sums)
+                sum = __builtin_bit_cast(f32x4, __builtin_bit_cast(i32x4, have) + __builtin_bit_cast(i32x4, v));
+              } else {
+                sum = have + v;
               }
+              set4(acc[i][j], q, pp == 0 ? v : sum);
             }
         }
       }
     }
 
-    // Epilogue. After the swapped MFMA, lane l of atom (i, j) holds C row (l % 32) and, for
-    // t = 0..3, columns 8t + 4*(l / 32) + {0,1,2,3} of that atom. Scales and the activation are
+    // Epilogue. After the swapped MFMA, lane l of block (i, j) holds C row (l % 32) and, for
+    // t = 0..3, columns 8t + 4*(l / 32) + {0,1,2,3} of that block (16x16 MFMAs: for group t = 2r + c row
+    // 16 r + l % 16 and columns 16 c + 4 (l / 16) + {0,1,2,3}). Scales and the activation are
     // applied to the accumulators in registers first (each in one pass, with the run-time choices
     // made outside the unrolled loops); the stores then only convert and write. A store's address
     // is the tile's (uniform) base plus one lane offset per row block plus a constant.
@@ -1443,28 +1574,32 @@ struct GemmKernel {
               acc[i][j][e] = (float)__builtin_bit_cast(int, bits) * (I4I ? kPackedInt4Unscale : 1.f);
             }
       }
+      auto lane_row = [&](int t) { return M16 ? (t >> 1) * 16 + (lane & 15) : lane & 31; };             // row in a block
+      auto lane_col = [&](int t) { return M16 ? (t & 1) * 16 + 4 * (lane >> 4) : 8 * t + 4 * (lane >> 5); };  // first column
+      constexpr int LR = M16 ? 2 : 1;  // rows of a block that a lane holds; row r is that of group (4 / LR) r
       const bool inside = col0 + BNO <= p.n_ext;
       // Column of B (of its scales and bias) behind accumulator block j, element group t of this lane.
       auto b_col = [&](int j, int t) {
         const int c = GLU ? (j < TNO ? 0 : p.n_ext) + col0 + wn * WTNO + (j % TNO) * 32 : col0 + wn * WTN + j * 32;
-        return min(c + 4 * (lane >> 5) + 8 * t, p.nb_ext - 4);
+        return min(c + lane_col(t), p.nb_ext - 4);
       };
       if (!SUBP && p.a_scale != nullptr) {  // (SUBP: folded in per k-block)
 #pragma unroll
         for (int i = 0; i < TM; ++i) {
-          const int row = min(row0 + row_block(i) * 32 + (lane & 31), p.m_ext - 1);
-          const float rs = p.a_scale[row];
-          if constexpr (I4F) {
-            const float off = 8.f * p.a_scale[p.m_ext + row];
+#pragma unroll
+          for (int r = 0; r < LR; ++r) {
+            const int row = min(row0 + row_block(i) * 32 + lane_row(r * (4 / LR)), p.m_ext - 1);
+            const float rs = p.a_scale[row];
+            [[maybe_unused]] const float off = I4F ? 8.f * p.a_scale[p.m_ext + row] : 0.f;
 #pragma unroll
             for (int j = 0; j < TN; ++j)
 #pragma unroll
-              for (int e = 0; e < 16; ++e) acc[i][j][e] = 512.f * acc[i][j][e] - off;
+              for (int t = r * (4 / LR); t < (r + 1) * (4 / LR); ++t) {
+                f32x4 v = get4(acc[i][j], t);
+                if constexpr (I4F) v = 512.f * v - off;
+                set4(acc[i][j], t, v * rs);
+              }
           }
-#pragma unroll
-          for (int j = 0; j < TN; ++j)
-#pragma unroll
-            for (int e = 0; e < 16; ++e) acc[i][j][e] *= rs;
         }
       }
       if (!SUBK && p.b_scale != nullptr) {  // (kFwdSubK: applied to the weights on their way into the MFMAs)
@@ -1474,9 +1609,7 @@ struct GemmKernel {
           for (int t = 0; t < 4; ++t) {
             const f32x4 cs = *reinterpret_cast<const f32x4*>(p.b_scale + (int64_t)group * p.nb_ext + b_col(j, t));
 #pragma unroll
-            for (int i = 0; i < TM; ++i)
-#pragma unroll
-              for (int e = 0; e < 4; ++e) acc[i][j][4 * t + e] *= cs[e];
+            for (int i = 0; i < TM; ++i) set4(acc[i][j], t, get4(acc[i][j], t) * cs);
           }
         }
       }
@@ -1487,9 +1620,7 @@ struct GemmKernel {
           for (int t = 0; t < 4; ++t) {
             const f32x4 cb = *reinterpret_cast<const f32x4*>(p.b_bias + (int64_t)group * p.nb_ext + b_col(j, t));
 #pragma unroll
-            for (int i = 0; i < TM; ++i)
-#pragma unroll
-              for (int e = 0; e < 4; ++e) acc[i][j][4 * t + e] += cb[e];
+            for (int i = 0; i < TM; ++i) set4(acc[i][j], t, get4(acc[i][j], t) + cb);
           }
         }
       }
@@ -1504,9 +1635,15 @@ struct GemmKernel {
 #pragma unroll
             for (int j = 0; j < TNO; ++j)
 #pragma unroll
-              for (int e = 0; e < 16; ++e) {
-                acc[i][j][e] = fminf(acc[i][j][e], limit);
-                acc[i][j + TNO][e] = fminf(fmaxf(acc[i][j + TNO][e], -limit), limit) + shift;
+              for (int t = 0; t < 4; ++t) {
+                f32x4 gate = get4(acc[i][j], t), up = get4(acc[i][j + TNO], t);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                  gate[e] = fminf(gate[e], limit);
+                  up[e] = fminf(fmaxf(up[e], -limit), limit) + shift;
+                }
+                set4(acc[i][j], t, gate);
+                set4(acc[i][j + TNO], t, up);
               }
         }
       }
@@ -1520,10 +1657,15 @@ struct GemmKernel {
         for (int i = 0; i < TM; ++i)
 #pragma unroll
           for (int j = 0; j < TNO; ++j) {  // (gate-up: the gate blocks only)
-            f32x16 c = acc[i][j];
+            Acc c = acc[i][j];
             auto apply = [&](auto fn) {
 #pragma unroll
-              for (int e = 0; e < 16; ++e) c[e] = fn(c[e]);
+              for (int t = 0; t < 4; ++t) {
+                f32x4 v = get4(c, t);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) v[e] = fn(v[e]);
+                set4(c, t, v);
+              }
             };
             if (p.activation == TKX_ACT_RELU) apply([](float x) { return x > 0.f ? x : 0.f; });
             else if (p.activation == TKX_ACT_TANH) apply(fast_tanh);
@@ -1544,7 +1686,7 @@ struct GemmKernel {
 #pragma unroll
           for (int j = 0; j < TNO; ++j)
 #pragma unroll
-            for (int e = 0; e < 16; ++e) acc[i][j][e] *= acc[i][j + TNO][e];
+            for (int t = 0; t < 4; ++t) set4(acc[i][j], t, get4(acc[i][j], t) * get4(acc[i][j + TNO], t));
       }
       // The stores go through LDS (free once the k loop is done): as the MFMA leaves them, a
       // lane's values are 4 columns of one row, so a store straight from registers writes 16-byte
@@ -1559,7 +1701,7 @@ struct GemmKernel {
       // a rounding boundary.) A row's 128 columns lie in 128 / WTN wave columns: each wave reduces its part of every
       // row (a lane's 16 TN values, then the lane 32 further on, which holds the row's other columns) and the waves
       // exchange them through LDS.
-      float row_scale[TM][WTN > 128 ? WTN / 128 : 1];
+      float row_scale[TM][LR][WTN > 128 ? WTN / 128 : 1];
       if constexpr (QO) {
         {
           constexpr int QW = WTN >= 128 ? 1 : 128 / WTN;   // wave columns per quantisation tile
@@ -1570,13 +1712,21 @@ struct GemmKernel {
           for (int i = 0; i < TM; ++i)
 #pragma unroll
             for (int q = 0; q < QT; ++q) {
-              float mx = 0.f;
 #pragma unroll
-              for (int j = q * JT; j < (q + 1) * JT; ++j)
+              for (int r = 0; r < LR; ++r) {
+                float mx = 0.f;
 #pragma unroll
-                for (int e = 0; e < 16; ++e) mx = fmaxf(mx, fabsf(acc[i][j][e]));
-              mx = fmaxf(mx, __shfl_xor(mx, 32));
-              if (lane < 32) xchg[(wave * TM * 32 + i * 32 + lane) * QT + q] = mx;
+                for (int j = q * JT; j < (q + 1) * JT; ++j)
+#pragma unroll
+                  for (int t = r * (4 / LR); t < (r + 1) * (4 / LR); ++t) {
+                    const f32x4 v = get4(acc[i][j], t);
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) mx = fmaxf(mx, fabsf(v[e]));
+                  }
+                if (M16) mx = fmaxf(mx, __shfl_xor(mx, 16));
+                mx = fmaxf(mx, __shfl_xor(mx, 32));
+                if (lane < 32 / LR) xchg[(wave * TM * 32 + i * 32 + lane_row(r * (4 / LR))) * QT + q] = mx;
+              }
             }
           __syncthreads();
           const int wn0 = wn / QW * QW;  // first wave column of this wave's quantisation tile
@@ -1584,15 +1734,19 @@ struct GemmKernel {
           for (int i = 0; i < TM; ++i)
 #pragma unroll
             for (int q = 0; q < QT; ++q) {
-              float mx = 0.f;
 #pragma unroll
-              for (int w = 0; w < QW; ++w) mx = fmaxf(mx, xchg[((wm * WN + wn0 + w) * TM * 32 + i * 32 + (lane & 31)) * QT + q]);
-              const float scale = mx == 0.f ? 1.f : mx / 448.f;
-              row_scale[i][q] = 1.f / scale;  // (the values are multiplied by the reciprocal, as the reference's epilogue does)
-              const int row = row0 + row_block(i) * 32 + (lane & 31);
-              const int qcol = (col0 + wn * WTN) / 128 + q;
-              if (lane < 32 && wn == wn0 && row >= act_start && row < act_end && qcol * 128 < p.n_ext)
-                p.c_scale[(int64_t)row * (p.ldc / 128) + qcol] = scale;
+              for (int r = 0; r < LR; ++r) {
+                const int brow = lane_row(r * (4 / LR));
+                float mx = 0.f;
+#pragma unroll
+                for (int w = 0; w < QW; ++w) mx = fmaxf(mx, xchg[((wm * WN + wn0 + w) * TM * 32 + i * 32 + brow) * QT + q]);
+                const float scale = mx == 0.f ? 1.f : mx / 448.f;
+                row_scale[i][r][q] = 1.f / scale;  // (the values are multiplied by the reciprocal, as the reference's epilogue does)
+                const int row = row0 + row_block(i) * 32 + brow;
+                const int qcol = (col0 + wn * WTN) / 128 + q;
+                if (lane < 32 / LR && wn == wn0 && row >= act_start && row < act_end && qcol * 128 < p.n_ext)
+                  p.c_scale[(int64_t)row * (p.ldc / 128) + qcol] = scale;
+              }
             }
           __syncthreads();  // the exchange area is part of the staging slices below
         }
@@ -1625,13 +1779,11 @@ struct GemmKernel {
             for (int j = 0; j < TNO; ++j) {
 #pragma unroll
               for (int t = 0; t < 4; ++t) {
-                f32x4 v;
-#pragma unroll
-                for (int e = 0; e < 4; ++e) v[e] = acc[i][j][4 * t + e];
-                unsigned char* dst = slice + (ii * 32 + (lane & 31)) * PITCH + (j * 32 + 8 * t + 4 * (lane >> 5)) * ESZ;
+                const f32x4 v = get4(acc[i][j], t);
+                unsigned char* dst = slice + (ii * 32 + lane_row(t)) * PITCH + (j * 32 + lane_col(t)) * ESZ;
                 if constexpr (OUT == TKX_F8E4M3FN) {
                   constexpr int JT = TN / (WTN > 128 ? WTN / 128 : 1);
-                  const float inv = row_scale[i][j / JT];
+                  const float inv = row_scale[i][M16 ? t >> 1 : 0][j / JT];
                   float q4[4];
 #pragma unroll
                   for (int e = 0; e < 4; ++e) q4[e] = fminf(fmaxf(v[e] * inv, -448.f), 448.f);
