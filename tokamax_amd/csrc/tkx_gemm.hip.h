@@ -1447,9 +1447,7 @@ struct GemmKernel {
 #pragma unroll
         for (int i = 0; i < TM; ++i)
 #pragma unroll
-          for (int j = 0; j < TN; ++j)
-#pragma unroll
-            for (int t = 0; t < 4; ++t) set4(acc[i][j], t, get4(acc[i][j], t) * kPackedInt4Unscale);
+          for (int j = 0; j < TN; ++j) acc[i][j] *= kPackedInt4Unscale;
       }
     }
     // (gate-up, per-k-block-scale and packed-int4 problems are taken only with whole k-steps)
