@@ -2,14 +2,13 @@
 
   python bench.py [--gpus 1] [--steps K] [--warmup W] [--no-extras] [--no-cpu] [--calibration-copy]
 
-Prints ONE JSON line. A step is one pass of the hot path (scheduler kernel + grouped-GEMM kernel)
+Prints ONE JSON line. A step is one pass of the hot path (one grouped-GEMM launch)
 over one seeded synthetic batch that is already resident in HBM. The headline workload is the
 Mixtral-8x7B-shaped prefill grouped GEMM (m=16384, k=4096, n=14336, G=8, bf16, top-2 router group
 sizes); `value` is its throughput in TFLOP/s with FLOPs = 2 * sum(group_sizes) * k * n.
 
-`roofline` describes the dominant kernel of a step, the grouped GEMM: its average launch duration is
-the HIP-event time of a step (events recorded on the launch stream) minus the separately measured
-duration of the scheduler kernel, the only other kernel in a step. The other measured
+`roofline` describes the kernel of a step, the grouped GEMM: its average launch duration is
+the HIP-event time of a step (events recorded on the launch stream). The other measured
 configurations (DeepSeek-V3 shape, int8-weight decode, fp8, bf16 VJP) are reported under "extras"
 with their own roofline figures; the decode kernel runs for tens of microseconds, less than the
 host needs to issue a launch, so it is timed as a HIP graph of back-to-back launches over rotating
@@ -195,10 +194,7 @@ def main():
   run = lambda: op(w.lhs, w.rhs, group_sizes=gs)
   total_ms, per, wall_ms = _time_steps(run, args.steps, args.warmup, stream)
   ms = total_ms / args.steps
-  # The scheduler kernel alone (the only other kernel of a step), as a graph of back-to-back launches.
-  from tokamax_amd.ragged_dot import hip_ops
-  sched_ms = _time_graph([lambda: hip_ops.schedule(gs, w.m, config.block_m, config.align_tile)], 20)
-  gemm_ms = statistics.mean(per) - sched_ms
+  gemm_ms = statistics.mean(per)  # (the only kernel of a step)
   result = {
       "metric": "ragged_dot TFLOP/s (% MFMA peak) prefill; GB/s (% HBM peak) decode, 1 GPU",
       "value": round(w.flops / ms / 1e9, 2),
@@ -222,7 +218,6 @@ def main():
       },
       "roofline": _roofline("mfma", w.flops, w.algorithmic_bytes(), gemm_ms, "bf16",
                             traffic=_measured_traffic(_gemm_kernel_prefix(0, 1, 1, config), "Mixtral prefill bf16 fwd")),
-      "schedule_kernel_ms": round(sched_ms, 5),
       "ms_median_step": round(statistics.median(per), 5),
       "ms_min_step": round(min(per), 5),
       "wall_ms_per_step": round(wall_ms / args.steps, 5),

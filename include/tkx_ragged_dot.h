@@ -161,9 +161,13 @@ int64_t tkx_ragged_dot_split_workspace_bytes(int64_t m, int64_t num_groups, int3
 int64_t tkx_ragged_dot_workspace_offset(int64_t m, int64_t num_groups, int32_t block_m, int32_t which);
 
 /* Part (1): group-offset prefix sum + tile schedule, one small kernel on `stream`.
- * group_sizes: device int32[G] (negative entries count as 0). Fills `workspace`. */
+ * group_sizes: device int32[G] (negative entries count as 0). Fills `workspace`. (For callers that want the reference's
+ * arrays. The forward and backward kernels do not read them: every wave works out its own tile from group_sizes.) */
 int32_t tkx_ragged_dot_schedule(const int32_t* group_sizes, int64_t num_groups, int64_t m, int32_t block_m,
                                 int32_t align_tile, void* workspace, tkx_stream_t stream);
+/* ... with launch-order spans of up to grid_tile_width tasks. */
+int32_t tkx_ragged_dot_schedule_spans(const int32_t* group_sizes, int64_t num_groups, int64_t m, int32_t block_m,
+                                      int32_t align_tile, int32_t grid_tile_width, void* workspace, tkx_stream_t stream);
 
 /* Parts (2),(3),(4-dlhs): grouped GEMM over the rows of each group.
  *   mode DEFAULT:   lhs [m,k] row-major, rhs [G,k,n] row-major, out [m,n]
@@ -173,7 +177,9 @@ int32_t tkx_ragged_dot_schedule(const int32_t* group_sizes, int64_t num_groups, 
  * Supported (lhs_dtype, rhs_dtype): (f32,f32) (bf16,bf16) (f16,f16) (f8e4m3fn,f8e4m3fn) (bf16,i8), and
  * (bf16,f8e4m3fn) with an rhs scale and (i8,i8) with both scales, in DEFAULT mode.
  * out_dtype: f32, bf16 or f16. Rows >= sum(group_sizes) of `out` are set to zero.
- * Runs the schedule kernel itself (workspace must hold tkx_ragged_dot_workspace_bytes bytes). */
+ * group_sizes may be null in a tiled kernel with one group, which then owns every row.
+ * One launch (`workspace` must hold tkx_ragged_dot_workspace_bytes bytes; a tiled call writes to it with split_k > 1 only,
+ * which also launches a kernel that clears 256 arrival counters). */
 int32_t tkx_ragged_dot_fwd(const void* lhs, const void* rhs, const int32_t* group_sizes,
                            const float* lhs_scale, const float* rhs_scale, void* out, void* workspace,
                            int64_t m, int64_t k, int64_t n, int64_t num_groups, int32_t lhs_dtype,

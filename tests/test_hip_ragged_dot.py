@@ -155,6 +155,44 @@ def test_launch_order_spans(width, device):
     _check(out, _ref(a, b, gs), 1e-5)
 
 
+@pytest.mark.parametrize("num_groups", [1, 3, 255, 256, 257, 700])
+@pytest.mark.parametrize("cfg", [hip_ops.KernelConfig(32, 128, 64, 1, 4, 4), hip_ops.KernelConfig(128, 256, 64, 2, 4, 3, grid_tile_width=2)])
+@pytest.mark.parametrize("kind", ["mixed", "negative", "too many rows", "none"])
+def test_tiles_worked_out_from_group_sizes(num_groups, cfg, kind, device):
+  """Every wave finds its tile from the group sizes, 256 groups at a time: sizes around a lane's four groups and around
+  256 groups, groups of one row and of several tiles (cut into even tasks), empty and negative ones, sizes that add up to
+  more rows than there are, and no sizes at all (one group of every row). Exact products of small integers: the result
+  is exact whatever the order of the sums."""
+  rng = np.random.default_rng(num_groups)
+  if kind == "none" and num_groups > 1:
+    pytest.skip("no sizes: one group")
+  k, n = 64, 264
+  gs = rng.choice([0, 0, 1, 2, 31, 33], num_groups).astype(np.int32)
+  gs[rng.integers(0, num_groups)] = 650
+  gs[-1] = 130
+  if kind == "negative":
+    gs[rng.integers(0, num_groups, 3)] = -(2 ** 31)
+  off = O.group_offsets(gs)
+  m = max(int(off[-1]) - 300 if kind == "too many rows" else int(off[-1]) + 7, 1)
+  lhs = torch.tensor(rng.integers(-2, 3, (m, k)), device=device).to(torch.bfloat16)
+  rhs = torch.tensor(rng.integers(-2, 3, (num_groups, k, n)), device=device).to(torch.bfloat16)
+  if kind == "none":
+    out = torch.full((m, n), 5.0, dtype=torch.float32, device=device)
+    ws = hip_ops.workspace(m, 1, cfg.block_m, device)
+    _lib.check(_lib.load().tkx_ragged_dot_fwd(lhs.data_ptr(), rhs.data_ptr(), None, None, None, out.data_ptr(), ws.data_ptr(), m, k, n,
+                                              1, _lib.TKX_BF16, _lib.TKX_BF16, _lib.TKX_F32, 0, 0, cfg.to_c(),
+                                              torch.cuda.current_stream().cuda_stream))
+    want = lhs.float() @ rhs[0].float()
+  else:
+    out = hip_ops.ragged_dot_fwd(lhs, rhs, torch.tensor(gs, device=device), config=cfg, out_dtype=torch.float32)
+    want = torch.zeros((m, n), dtype=torch.float32, device=device)
+    for g in range(num_groups):
+      lo, hi = min(int(off[g]), m), min(int(off[g + 1]), m)
+      if hi > lo:
+        want[lo:hi] = lhs[lo:hi].float() @ rhs[g].float()
+  assert torch.equal(out, want)
+
+
 def test_padded(device):
   a, b, gs = _inputs("test_padded", 8, 1024, 128, 256, torch.bfloat16, device, random_groups=True)
   out = tokamax_amd.ragged_dot(a, b, torch.tensor(gs, device=device), preferred_element_type=torch.float32)

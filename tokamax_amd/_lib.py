@@ -28,6 +28,7 @@ EXPORTED_SYMBOLS = (
     "tkx_ragged_dot_split_workspace_bytes",
     "tkx_ragged_dot_workspace_offset",
     "tkx_ragged_dot_schedule",
+    "tkx_ragged_dot_schedule_spans",
     "tkx_ragged_dot_fwd",
     "tkx_ragged_dot_fwd_static_workspace",
     "tkx_ragged_dot_fwd_fused",
@@ -105,6 +106,8 @@ def _declare(lib):
   lib.tkx_ragged_dot_workspace_offset.argtypes = [i64, i64, i32, i32]
   lib.tkx_ragged_dot_schedule.restype = i32
   lib.tkx_ragged_dot_schedule.argtypes = [vp, i64, i64, i32, i32, vp, vp]
+  lib.tkx_ragged_dot_schedule_spans.restype = i32
+  lib.tkx_ragged_dot_schedule_spans.argtypes = [vp, i64, i64, i32, i32, i32, vp, vp]
   lib.tkx_ragged_dot_fwd.restype = i32
   lib.tkx_ragged_dot_fwd.argtypes = [vp, vp, vp, vp, vp, vp, vp, i64, i64, i64, i64, i32, i32, i32, i32, i32, cfgp, vp]
   lib.tkx_ragged_dot_fwd_static_workspace.restype = i32

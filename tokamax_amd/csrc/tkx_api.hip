@@ -207,8 +207,17 @@ int32_t tkx_ragged_dot_schedule(const int32_t* group_sizes, int64_t num_groups, 
   if (group_sizes == nullptr || workspace == nullptr) return set_error(TKX_ERR_INVALID, "null pointer argument");
   if (num_groups < 1 || m < 0) return set_error(TKX_ERR_INVALID, "bad sizes m=%lld G=%lld", (long long)m, (long long)num_groups);
   if (block_m < 1 || align_tile < 1) return set_error(TKX_ERR_INVALID, "block_m and align_tile must be positive");
+  return tkx_ragged_dot_schedule_spans(group_sizes, num_groups, m, block_m, align_tile, 1, workspace, stream);
+}
+
+int32_t tkx_ragged_dot_schedule_spans(const int32_t* group_sizes, int64_t num_groups, int64_t m, int32_t block_m,
+                                      int32_t align_tile, int32_t grid_tile_width, void* workspace, tkx_stream_t stream) {
+  if (group_sizes == nullptr || workspace == nullptr) return set_error(TKX_ERR_INVALID, "null pointer argument");
+  if (num_groups < 1 || m < 0) return set_error(TKX_ERR_INVALID, "bad sizes m=%lld G=%lld", (long long)m, (long long)num_groups);
+  if (block_m < 1 || align_tile < 1 || grid_tile_width < 1)
+    return set_error(TKX_ERR_INVALID, "block_m, align_tile and grid_tile_width must be positive");
   const WsLayout L = ws_layout(m, num_groups, block_m);
-  return launch_schedule(group_sizes, num_groups, nullptr, num_groups, m, block_m, align_tile, 1,
+  return launch_schedule(group_sizes, num_groups, nullptr, num_groups, m, block_m, align_tile, grid_tile_width,
                          static_cast<int32_t*>(workspace), L, static_cast<hipStream_t>(stream));
 }
 
@@ -225,8 +234,10 @@ int32_t fwd_impl(const void* lhs, const void* rhs, const int32_t* group_sizes, c
                  int32_t rhs_dtype, int32_t out_dtype, int32_t mode, int32_t activation, bool gateup,
                  int64_t rhs_scale_blocks, const TkxConfig* config, tkx_stream_t stream_, float* out_scale = nullptr) {
   hipStream_t stream = static_cast<hipStream_t>(stream_);
-  if (!lhs || !rhs || !group_sizes || !out || !workspace || !config)
-    return set_error(TKX_ERR_INVALID, "null pointer argument");
+  if (!lhs || !rhs || !out || !workspace || !config) return set_error(TKX_ERR_INVALID, "null pointer argument");
+  // (no group sizes: a single group that owns every row; the tiled kernels only)
+  if (!group_sizes && (num_groups != 1 || group_offset != nullptr || config->block_m == kDecodeBlockM))
+    return set_error(TKX_ERR_INVALID, "null pointer argument: group_sizes (may be null for one group in a tiled kernel)");
   if (group_offset == nullptr) num_group_sizes = num_groups;
   if (num_group_sizes < 1 || num_group_sizes > 0x7fffffffLL)
     return set_error(TKX_ERR_INVALID, "bad number of group sizes %lld", (long long)num_group_sizes);
@@ -370,10 +381,6 @@ int32_t fwd_impl(const void* lhs, const void* rhs, const int32_t* group_sizes, c
     return set_error(TKX_ERR_UNSUPPORTED, "split_k > 1 on a tiled kernel: plain forward and TRANS_RHS only (no gate-up fusion, scales per k-block or quantised result)");
   if (split_k > 16) return set_error(TKX_ERR_INVALID, "split_k must lie in [1, 16], got %d", split_k);
   const WsLayout L = ws_layout(m, num_groups, c.block_m);
-  int32_t st = launch_schedule(group_sizes, num_groups, group_offset, num_group_sizes, m, c.block_m, c.align_tile,
-                               c.grid_tile_width, static_cast<int32_t*>(workspace), L, stream);
-  if (st != TKX_OK) return st;
-
   GemmParams p = {};
   p.A = lhs;
   p.B = rhs;
@@ -382,7 +389,9 @@ int32_t fwd_impl(const void* lhs, const void* rhs, const int32_t* group_sizes, c
   p.b_scale = rhs_scale;
   p.b_bias = rhs_bias;
   p.c_scale = out_scale;
-  p.ws = static_cast<const int32_t*>(workspace);
+  p.group_sizes = group_sizes;
+  p.group_offset = group_offset;
+  p.num_global = (int32_t)num_group_sizes;
   p.lda = dlhs ? n : k;
   p.ldb = n;
   p.ldc = cols;
@@ -399,19 +408,11 @@ int32_t fwd_impl(const void* lhs, const void* rhs, const int32_t* group_sizes, c
   // Whole chunks for every XCD, so that each list entry has a workgroup (see the launch order in run()).
   const int64_t slots = ((int64_t)L.tid_size * p.n_tiles + 8 * kXcdChunk - 1) / (8 * kXcdChunk) * (8 * kXcdChunk);
   p.real_slots = (int32_t)slots;
-  p.tid_size = L.tid_size;
   p.grid_tile_width = c.grid_tile_width;
   p.out_dtype = out_dtype;
   p.activation = activation;
   p.scale_blocks = subk ? (int32_t)rhs_scale_blocks : 1;
   p.log2_block_rows = log2_block_rows;
-  p.ws_offsets = (int32_t)L.offsets;
-  p.ws_gid = (int32_t)L.task[0];
-  p.ws_bstart = (int32_t)L.task[1];
-  p.ws_astart = (int32_t)L.task[2];
-  p.ws_aend = (int32_t)L.task[3];
-  p.ws_span_first = (int32_t)L.task[6];
-  p.ws_span_width = (int32_t)L.task[7];
   if (slots > 0x7fffff00LL) return set_error(TKX_ERR_UNSUPPORTED, "too many tiles");
   // Extra workgroups zero the rows past the last group (and before the first, with a group offset);
   // they exit at once when there are none.
@@ -424,10 +425,12 @@ int32_t fwd_impl(const void* lhs, const void* rhs, const int32_t* group_sizes, c
   int64_t split_wgs = 0;
   if (split_k > 1) {
     int cus = 0;
-    st = device_compute_units(&cus);
+    int32_t st = device_compute_units(&cus);
     if (st != TKX_OK) return st;
     p.split_cus = cus < kSplitUnits ? cus : kSplitUnits;
-    p.ws_split_counters = (int32_t)L.split_counters;
+    p.split_counters = static_cast<int32_t*>(workspace) + L.split_counters;
+    st = launch_clear_words(p.split_counters, kSplitUnits, stream);
+    if (st != TKX_OK) return st;
     p.split_partials = reinterpret_cast<float*>(static_cast<int32_t*>(workspace) + L.words);
     split_wgs = p.split_cus;  // at most that many parts beside the tiles' own workgroups
   }
@@ -477,7 +480,7 @@ int32_t tkx_ragged_dot_fwd_static_workspace(const void* lhs, const void* rhs, co
   int32_t* ws = nullptr;
   const int32_t st = scratch_address(&ws);
   if (st != TKX_OK) return st;
-  // The scheduler kernel writes every word the GEMM kernel reads, so nothing of the last call's contents matters.
+  // (The kernels read nothing from it: only split contractions do, which were declined above.)
   return fwd_impl(lhs, rhs, group_sizes, nullptr, lhs_scale, rhs_scale, nullptr, out, ws, m, k, n, num_groups, num_groups,
                   lhs_dtype, rhs_dtype, out_dtype, mode, activation, false, 1, config, stream);
 }
@@ -521,19 +524,12 @@ int32_t tkx_ragged_dot_drhs(const void* lhs, const void* dout, const int32_t* gr
   if (((uintptr_t)lhs | (uintptr_t)dout | (uintptr_t)out | (uintptr_t)workspace) % 16 != 0)
     return set_error(TKX_ERR_UNSUPPORTED, "pointers must be 16-byte aligned");
 
-  // Only the group offsets are needed; block_m of the schedule is irrelevant here, use a fixed one
-  // so the workspace size depends on (m, G) alone.
-  const int32_t sched_bm = 128;
-  const WsLayout L = ws_layout(m, num_groups, sched_bm);
-  int32_t st = launch_schedule(group_sizes, num_groups, nullptr, num_groups, m, sched_bm, c.align_tile, 1,
-                               static_cast<int32_t*>(workspace), L, stream);
-  if (st != TKX_OK) return st;
-
   GemmParams p = {};
   p.A = lhs;
   p.B = dout;
   p.C = out;
-  p.ws = static_cast<const int32_t*>(workspace);
+  p.group_sizes = group_sizes;
+  p.num_global = (int32_t)num_groups;
   p.lda = k;
   p.ldb = n;
   p.ldc = n;
@@ -548,7 +544,6 @@ int32_t tkx_ragged_dot_drhs(const void* lhs, const void* dout, const int32_t* gr
   p.grid_tile_width = 1;
   p.out_dtype = out_dtype;
   p.activation = TKX_ACT_NONE;
-  p.ws_offsets = (int32_t)L.offsets;
   p.split_k = 1;
   p.split_cus = 1;
   return launch(v, p, (int64_t)num_groups * p.m_tiles * p.n_tiles, stream);

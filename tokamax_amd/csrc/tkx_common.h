@@ -9,19 +9,21 @@
 namespace tkx {
 
 // ---- workspace layout (int32 words) -----------------------------------------------------------
+// What tkx_ragged_dot_schedule fills; the GEMM entry points use the arrival counters and what lies behind them, in calls
+// with split_k > 1.
 // [0] num_tasks  [1] total_rows (end of the last group)  [2] rows before the first group  [kWsHeader ..) group_offsets[G+1]  then eight task arrays of
 // tid_size words each (group_id, block_start, actual_start, actual_end, start_within_block,
 // actual_size, span_first, span_width); every array starts on a 64-word boundary. The last two
 // are not part of the reference's schedule: they cut each group's tasks into spans of at most
-// grid_tile_width tasks (first task and width of the span a task belongs to), which is the unit
-// the GEMM launch order walks n-panel by n-panel.
+// grid_tile_width tasks (first task and width of the span a task belongs to), the unit a launch order
+// walks n-panel by n-panel.
 constexpr int64_t kWsHeader = 64;
 
 struct WsLayout {
   int64_t offsets;   // word offset of group_offsets
   int64_t task[8];   // word offsets of the task arrays
-  int64_t split_counters;  // word offset of kSplitUnits arrival counters (tiled kernels with split_k > 1); the
-                           // scheduler kernel clears them in every call
+  int64_t split_counters;  // word offset of kSplitUnits arrival counters (tiled kernels with split_k > 1); a small
+                           // kernel in front of such a call clears them
   int64_t words;     // total words (the partial tiles of a split launch lie behind them)
   int32_t tid_size;
 };
@@ -60,11 +62,13 @@ int32_t set_error(int32_t code, const char* fmt, ...);
   } while (0)
 
 // ---- schedule -------------------------------------------------------------------------------------
+// The reference's task arrays (the GEMM kernels do not read them: every wave works out its own tile, GroupScan).
 // `group_offset` (device, one int32; null = 0): the G groups are entries [offset, offset + G) of the
 // `num_global` group sizes.
 int32_t launch_schedule(const int32_t* group_sizes, int64_t G, const int32_t* group_offset, int64_t num_global, int64_t m,
                         int32_t block_m, int32_t align_tile, int32_t span_width, int32_t* ws, const WsLayout& L,
                         hipStream_t stream);
+int32_t launch_clear_words(int32_t* words, int32_t count, hipStream_t stream);
 int32_t device_compute_units(int* out);
 
 // ---- grouped GEMM -----------------------------------------------------------------------------
@@ -85,7 +89,9 @@ struct GemmParams {
   const float* b_scale;  // per (group, column of B), or null
   const float* b_bias;   // per (group, column of B), added after the scales, or null
   float* c_scale;        // out_dtype fp8: f32 [m_ext, n_ext / 128], one scale per (row, 128 columns) of the result
-  const int32_t* ws;
+  const int32_t* group_sizes;       // device, num_global entries; null: one group of all m_ext rows
+  const int32_t* group_offset;      // device, one int32, or null: group g is entry offset + g of group_sizes
+  int32_t num_global;
   int64_t lda, ldb, ldc;            // leading dimensions, elements
   int64_t b_group_stride;           // elements between consecutive groups of B (fwd/dlhs)
   int64_t c_group_stride;           // elements between consecutive groups of C (drhs)
@@ -98,14 +104,13 @@ struct GemmParams {
   // Split of the last round (fwd/dlhs, split_k > 1): the launch's tiles beyond the last multiple of `split_cus` are
   // cut along the contraction into floor(split_cus / their number) parts, at most split_k; part 0 belongs to the
   // tile's own workgroup, the others to workgroups behind the zeroing ones. f32 partial tiles in split_partials
-  // ([unit][BM * BN]), arrival counters at ws[ws_split_counters + tile].
-  int32_t split_k, split_cus, ws_split_counters;
+  // ([unit][BM * BN]), arrival counters (zero on entry) in split_counters.
+  int32_t split_k, split_cus;
+  int32_t* split_counters;
   float* split_partials;
-  int32_t tid_size;                 // fwd/dlhs: slots of the schedule's task arrays
   int32_t grid_tile_width;
   int32_t out_dtype, activation;
   int32_t scale_blocks, log2_block_rows;  // kFwdSubK: b_scale is [g, scale_blocks, n]; rows of k per block = 1 << log2
-  int32_t ws_offsets, ws_gid, ws_bstart, ws_astart, ws_aend, ws_span_first, ws_span_width;  // word offsets into ws
 };
 
 struct Variant {

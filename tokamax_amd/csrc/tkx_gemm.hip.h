@@ -594,6 +594,63 @@ __device__ __forceinline__ void store4_as(unsigned char* ptr, f32x4 v) {
   }
 }
 
+// ---- the schedule -------------------------------------------------------------------------------
+// Inclusive scan over the wave with additions that saturate at `limit` (x >= 0): the DPP row shifts inside 16 lanes, then
+// the broadcasts of a row's last lane into the rows behind it.
+__device__ __forceinline__ int wave_scan(int x, int limit) {
+#define TKX_DPP_ADD(CTRL, ROWS) x = min(x + __builtin_amdgcn_update_dpp(0, x, CTRL, ROWS, 0xf, false), limit)
+  TKX_DPP_ADD(0x111, 0xf);  // row_shr:1
+  TKX_DPP_ADD(0x112, 0xf);  // row_shr:2
+  TKX_DPP_ADD(0x114, 0xf);  // row_shr:4
+  TKX_DPP_ADD(0x118, 0xf);  // row_shr:8
+  TKX_DPP_ADD(0x142, 0xa);  // row_bcast:15 into rows 1 and 3
+  TKX_DPP_ADD(0x143, 0xc);  // row_bcast:31 into rows 2 and 3
+#undef TKX_DPP_ADD
+  return x;
+}
+
+// The row ranges and tile counts of 256 groups, four to a lane, as every wave of a GEMM launch works them out for itself
+// from the group sizes: one load and two scans of a few hundred cycles, no more than the dependent loads of a
+// precomputed schedule took, and no scheduler kernel in front of the launch (5.5 us and a launch gap per call).
+// Sizes are device data nobody has checked: each counts as 0 below 0, and rows at or past m do not exist.
+// A group's rows are cut into ceil(rows / BM) tasks of whole units of Q rows (32 rows for every row of waves), as even
+// as they come: the tasks of a group then run at one pace and share its weight panels in L2 to the end.
+// ALIGN: what a task's first row is a multiple of.
+template <int BM, int ALIGN>
+struct GroupScan {
+  int start[4], end[4], tasks[4];  // this lane's groups
+  int tasks_upto;                  // tasks of all groups up to this lane's last one
+  int rows, total;                 // (uniform) the first row and the first task behind these 256 groups
+
+  // Groups c .. c + 255 (c a multiple of 256); `rows0`, `total0`: the rows and tasks in front of them.
+  // `m`: the rows there are.
+  __device__ __forceinline__ void scan(const GemmParams& p, int m, int c, int offset, int lane, int rows0, int total0) {
+    int size[4], sum = 0;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const int g = c + 4 * lane + e;
+      const int64_t j = (int64_t)offset + g;
+      const bool there = g < p.num_groups && j >= 0 && j < p.num_global;
+      int v = m;
+      if (p.group_sizes != nullptr) v = p.group_sizes[there ? (int)j : 0];
+      size[e] = there ? min(max(v, 0), m) : 0;
+      sum = min(sum + size[e], m);
+    }
+    const int upto = wave_scan(sum, m);
+    int at = min(rows0 + __builtin_amdgcn_update_dpp(0, upto, 0x138 /* wave_shr:1 */, 0xf, 0xf, false), m), count = 0;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      start[e] = at;
+      at = end[e] = min(at + size[e], m);
+      tasks[e] = end[e] > start[e] ? (end[e] - (start[e] & -ALIGN) + BM - 1) / BM : 0;
+      count += tasks[e];
+    }
+    tasks_upto = total0 + wave_scan(count, 0x7fffffff);
+    rows = __builtin_amdgcn_readlane(at, 63);
+    total = __builtin_amdgcn_readlane(tasks_upto, 63);
+  }
+};
+
 // ---- the kernel ---------------------------------------------------------------------------------
 // Calls f(integral_constant<int, sel>) for a run-time sel in [I, N].
 template <int I, int N, class Fn>
@@ -816,16 +873,24 @@ struct GemmKernel {
     // tile's rows (a group boundary) then leaves every wave row about the same number of blocks
     // with rows to compute, instead of all of them to one wave row.
     auto row_block = [&](int i) { return i * WM + wm; };
-    const int32_t* ws = p.ws;
     const int b = blockIdx.x;
 
     int group, row0, act_start, act_end, col0, kc_begin, kc_end;
     int part = 0, parts = 1, split_unit = 0;  // (fwd/dlhs) this workgroup contracts part `part` of `parts` of its tile
     if constexpr (MODE != kDrhs) {
-      // (Group sizes are device data nobody has checked: when they add up to more than m_ext rows the schedule
-      // holds more tasks than its arrays have slots for. Every task with a row below m_ext has a slot, so the rest
-      // are dropped here, and the tasks kept store no row at or past m_ext.)
-      const int num_tasks = min(ws[0], p.tid_size);
+      // (kFwdSubK with lhs scales: a tile's scales are fetched four rows at a time)
+      typedef GroupScan<BM, SUBP ? 4 : 1> Scan;
+      const int offset = p.group_offset != nullptr ? __builtin_amdgcn_readfirstlane(p.group_offset[0]) : 0;
+      int lead_rows = 0;  // rows of the groups in front of the first one of this call
+      if (p.group_offset != nullptr) {
+        int rows = 0;
+        for (int j = lane; j < min(max(offset, 0), p.num_global); j += 64) rows = min(rows + min(max(p.group_sizes[j], 0), p.m_ext), p.m_ext);
+        lead_rows = __builtin_amdgcn_readlane(wave_scan(rows, p.m_ext), 63);
+      }
+      Scan sc;
+      sc.scan(p, p.m_ext, 0, offset, lane, lead_rows, 0);
+      for (int c = 256; c < p.num_groups; c += 256) sc.scan(p, p.m_ext, c, offset, lane, sc.rows, sc.total);
+      const int num_tasks = sc.total;
       // Split of the last round: the launch's tiles beyond the last multiple of `split_cus` (a round of workgroups
       // that would leave most CUs idle) are cut along the contraction into `parts` parts. Part 0 is the tile's own
       // workgroup, the others are workgroups behind the zeroing ones.
@@ -849,7 +914,7 @@ struct GemmKernel {
       } else if (b >= p.real_slots) {
         // Tail duty: rows [total_rows, m_ext), and with a group offset the rows before the first
         // group, belong to no group of this call and are defined to be zero.
-        const int total_rows = min(ws[1], p.m_ext), lead_rows = min(ws[2], p.m_ext);
+        const int total_rows = sc.rows;
         const int64_t esz = QO ? 1 : p.out_dtype == TKX_F32 ? 4 : 2;
         const int64_t lo = (int64_t)total_rows * p.ldc * esz, hi = (int64_t)p.m_ext * p.ldc * esz;
         if constexpr (QO) {
@@ -870,8 +935,8 @@ struct GemmKernel {
       // XCD-aware order: consecutive workgroup ids land on different XCDs (id % 8). The tile list is
       // dealt out in chunks of kXcdChunk consecutive tiles, chunk c to XCD c % 8, so that the
       // workgroups an XCD runs at a time are consecutive in the list and the 8 XCDs work on
-      // neighbouring chunks. The list goes span by span (a span = up to `grid_tile_width`
-      // consecutive m-tasks of one group, laid out by the scheduler); inside a span its m-tasks take
+      // neighbouring chunks. The list goes group by group and span by span (a group's tasks are cut into
+      // ceil(tasks / grid_tile_width) spans of nearly equal width); inside a span its m-tasks take
       // an n-panel of the group's weights back to back, then the next n-panel: the tiles of a chunk
       // share panels in their XCD's L2, and neighbouring chunks share the span's lhs panels in the
       // memory-side cache.
@@ -882,17 +947,53 @@ struct GemmKernel {
         if (L < first_split) parts = 1;
       }
       split_unit = (L - first_split) * parts + part;
-      const int t0 = L / p.n_tiles;  // some task of the span that holds L (every task owns n_tiles list entries)
-      const int first = ws[p.ws_span_first + t0], width = ws[p.ws_span_width + t0];
-      const int rem = L - first * p.n_tiles;
+      // The group that owns list entry L (every task owns n_tiles entries), and the entry's place among the group's.
+      int chunk = 0;
+      if (p.num_groups > 256) {
+        sc.scan(p, p.m_ext, 0, offset, lane, lead_rows, 0);
+        while (L >= sc.total * p.n_tiles) sc.scan(p, p.m_ext, chunk += 256, offset, lane, sc.rows, sc.total);
+      }
+      const int owner = __builtin_ctzll(__ballot(L < sc.tasks_upto * p.n_tiles));
+      int tasks = 0, end = 0, first_task = __builtin_amdgcn_readlane(sc.tasks_upto, owner);
+      group = chunk + 4 * owner + 3;
+#pragma unroll
+      for (int e = 3; e >= 0; --e) {  // (the lane's groups from its last one back)
+        if (e == 3 || L < first_task * p.n_tiles) {
+          group = chunk + 4 * owner + e;
+          tasks = __builtin_amdgcn_readlane(sc.tasks[e], owner);
+          act_start = __builtin_amdgcn_readlane(sc.start[e], owner);
+          end = __builtin_amdgcn_readlane(sc.end[e], owner);
+          first_task -= tasks;
+        }
+      }
+      int rem = L - first_task * p.n_tiles, width = tasks, first = 0;
+      if (tasks > p.grid_tile_width) {
+        const int spans = (tasks + p.grid_tile_width - 1) / p.grid_tile_width;
+        const int base = tasks / spans, wider = tasks - base * spans;  // the first `wider` spans are one task wider
+        const int wide_entries = wider * (base + 1) * p.n_tiles;
+        width = base;
+        if (rem < wide_entries) {
+          width = base + 1;
+        } else {
+          rem -= wide_entries;
+          first = wider * (base + 1);
+        }
+        const int span = rem / (width * p.n_tiles);
+        rem -= span * width * p.n_tiles;
+        first += span * width;
+      }
       const int nt = rem / width;
       const int mt = first + (rem - nt * width);
-      if (mt >= p.tid_size) return;  // (a span that runs past the last slot: rows past m_ext only)
-      group = ws[p.ws_gid + mt];
-      row0 = ws[p.ws_bstart + mt];
-      act_end = min(ws[p.ws_aend + mt], p.m_ext);
-      act_start = min(ws[p.ws_astart + mt], act_end);
-      if (act_start >= act_end) return;  // (every row of the task lies at or past m_ext)
+      row0 = act_start & -(SUBP ? 4 : 1);
+      act_end = end;
+      if (tasks > 1) {
+        constexpr int Q = WM * 32;  // rows of a unit
+        const int units = (end - row0 + Q - 1) / Q;
+        const int base = units / tasks, more = units - base * tasks;  // the first `more` tasks are one unit taller
+        row0 += (mt * base + min(mt, more)) * Q;
+        act_end = min(row0 + (base + (mt < more ? 1 : 0)) * Q, end);
+        act_start = max(act_start, row0);
+      }
       col0 = nt * BNO;
       kc_begin = 0;
       kc_end = p.k_ext;
@@ -911,8 +1012,12 @@ struct GemmKernel {
       col0 = nt * BN;
       act_start = row0;
       act_end = min(row0 + BM, p.m_ext);
-      kc_begin = min(ws[p.ws_offsets + group], p.k_ext);
-      kc_end = min(ws[p.ws_offsets + group + 1], p.k_ext);
+      GroupScan<1, 1> sc;  // (rows only)
+      sc.scan(p, p.k_ext, 0, 0, lane, 0, 0);
+      for (int c = 256; c <= group; c += 256) sc.scan(p, p.k_ext, c, 0, lane, sc.rows, 0);
+      const int owner = (group & 255) >> 2, e = group & 3;
+      kc_begin = __builtin_amdgcn_readlane(e < 2 ? (e == 0 ? sc.start[0] : sc.start[1]) : (e == 2 ? sc.start[2] : sc.start[3]), owner);
+      kc_end = __builtin_amdgcn_readlane(e < 2 ? (e == 0 ? sc.end[0] : sc.end[1]) : (e == 2 ? sc.end[2] : sc.end[3]), owner);
     }
 
     const unsigned char* Ab = reinterpret_cast<const unsigned char*>(p.A);
@@ -939,7 +1044,7 @@ struct GemmKernel {
       if (r0 < act_end && r0 + 32 > act_start) rmask |= 1u << i;
     }
     rmask = __builtin_amdgcn_readfirstlane(rmask);
-    // The blocks with rows are the first `nv` of the wave (a task's rows start in the tile's first 8 rows and the
+    // The blocks with rows are the first `nv` of the wave (a task's rows start in the tile's first 4 rows and the
     // blocks of a wave ascend through the tile), so the k loop is compiled once per count: straight-line code for
     // whole and partial tiles alike, no test around an MFMA. (Any other pattern computes every block.)
     const int nv_count = __builtin_popcount(rmask);
@@ -1514,7 +1619,7 @@ struct GemmKernel {
       __syncthreads();  // (also: every wave is done reading the last stage, whose first word carries the verdict below)
       int* verdict = reinterpret_cast<int*>(smem);
       if (tid == 0) {
-        int32_t* counter = const_cast<int32_t*>(ws) + p.ws_split_counters + (split_unit - part) / parts;
+        int32_t* counter = p.split_counters + (split_unit - part) / parts;
         const int arrived = atomicAdd(counter, 1);
         *verdict = arrived == parts - 1;
         if (arrived == parts - 1) atomicExch(counter, 0);

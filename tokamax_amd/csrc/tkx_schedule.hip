@@ -2,7 +2,8 @@
 //
 // Produces, bit for bit, what the reference's GroupInfo.create_aligned computes with XLA ops
 // (tokamax/_src/ops/ragged_dot/pallas_mosaic_gpu_common.py:119-151), plus the group offsets and
-// the number of tasks that belong to non-empty groups, which the GEMM kernels use to skip the rest.
+// the number of tasks that belong to non-empty groups. For callers that want those arrays: the GEMM
+// kernels work out their tiles themselves (tkx_gemm.hip.h, GroupScan).
 #include "tkx_common.h"
 
 namespace tkx {
@@ -43,14 +44,12 @@ __global__ __launch_bounds__(kThreads) void schedule_kernel(const int32_t* __res
                                                              int32_t span_width, int32_t* __restrict__ ws,
                                                              int64_t off_offsets, int64_t off_gid, int64_t off_bstart,
                                                              int64_t off_astart, int64_t off_aend, int64_t off_swb,
-                                                             int64_t off_asize, int64_t off_sfirst, int64_t off_swidth,
-                                                             int64_t off_split_counters) {
+                                                             int64_t off_asize, int64_t off_sfirst, int64_t off_swidth) {
   extern __shared__ int32_t smem[];
   int32_t* scan_buf = smem;                         // 2*kThreads
   int32_t* starts = smem + 2 * kThreads;            // G+1 : exclusive cumsum of clamped sizes
   int32_t* start_tasks = starts + (G + 1);          // G+1 : exclusive cumsum of blocks per group
   const int t = threadIdx.x;
-  for (int i = t; i < kSplitUnits; i += kThreads) ws[off_split_counters + i] = 0;  // arrival counters of a split launch
   const int per = (G + kThreads - 1) / kThreads;
   const int lo = min(t * per, G), hi = min(lo + per, G);
 
@@ -147,7 +146,18 @@ __global__ __launch_bounds__(kThreads) void schedule_kernel(const int32_t* __res
   }
 }
 
+__global__ __launch_bounds__(kThreads) void clear_words_kernel(int32_t* __restrict__ words, int32_t count) {
+  for (int i = threadIdx.x; i < count; i += kThreads) words[i] = 0;
+}
+
 }  // namespace
+
+// (a kernel, not a memset: callers may be capturing a graph)
+int32_t launch_clear_words(int32_t* words, int32_t count, hipStream_t stream) {
+  clear_words_kernel<<<1, kThreads, 0, stream>>>(words, count);
+  TKX_HIP_CHECK(hipGetLastError());
+  return TKX_OK;
+}
 
 int32_t launch_schedule(const int32_t* group_sizes, int64_t G, const int32_t* group_offset, int64_t num_global, int64_t m,
                         int32_t block_m, int32_t align_tile, int32_t span_width, int32_t* ws, const WsLayout& L,
@@ -158,8 +168,7 @@ int32_t launch_schedule(const int32_t* group_sizes, int64_t G, const int32_t* gr
   if (num_global < 0 || num_global > 0x7fffffffLL) return set_error(TKX_ERR_INVALID, "bad number of group sizes");
   schedule_kernel<<<1, kThreads, smem, stream>>>(group_sizes, (int32_t)G, group_offset, (int32_t)num_global, block_m, L.tid_size, align_tile,
                                                 span_width < 1 ? 1 : span_width, ws, L.offsets, L.task[0], L.task[1],
-                                                L.task[2], L.task[3], L.task[4], L.task[5], L.task[6], L.task[7],
-                                                L.split_counters);
+                                                L.task[2], L.task[3], L.task[4], L.task[5], L.task[6], L.task[7]);
   TKX_HIP_CHECK(hipGetLastError());
   return TKX_OK;
 }

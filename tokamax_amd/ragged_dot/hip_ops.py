@@ -208,7 +208,7 @@ def ragged_dot_fwd(lhs, rhs, group_sizes, *, config: KernelConfig, out_dtype: to
   `group_offset` (device int32 tensor of one element): `group_sizes` covers every group of the job, rhs holds the
   groups [offset, offset + g) of them, and the rows of all other groups come out zero (the call of one
   expert-parallel shard, experimental/gmm_v2/gmm_v2_test.py:44-101).
-  `workspace_out`, if given, receives the int32 workspace the call filled (schedule arrays included)."""
+  `workspace_out`, if given, receives an int32 workspace with the reference's schedule of this call (a pass of its own)."""
   _require_cuda(lhs, rhs, group_sizes, lhs_scale, rhs_scale, rhs_bias, group_offset)
   lib = _lib.load()
   if lhs.dim() != 2 or rhs.dim() != 3:
@@ -326,7 +326,11 @@ def ragged_dot_fwd(lhs, rhs, group_sizes, *, config: KernelConfig, out_dtype: to
     st = launch(pointers, out.data_ptr(), ws.data_ptr(), torch.cuda.current_stream(device).cuda_stream)
   _lib.check(st)
   if workspace_out is not None:
-    workspace_out.append(ws)
+    filled = workspace(m, gs.numel(), config.block_m, device)
+    with _on_device(device):
+      _lib.check(lib.tkx_ragged_dot_schedule_spans(_ptr(gs), gs.numel(), m, config.block_m, config.align_tile,
+                                                   config.grid_tile_width, _ptr(filled), _stream(device)))
+    workspace_out.append(filled)
   _log_launch(ForwardLaunch(pointers, launch, out, new_workspace))
   return out
 
