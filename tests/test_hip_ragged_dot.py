@@ -2351,6 +2351,39 @@ def test_ceiling_probes_run_and_give_plausible_figures(device):
   assert 1.0 < alone < 9.0 and shared > 2 * alone, (alone, shared)
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_repeated_backward_passes_take_remembered_launches(device, dtype):
+  """The cotangents of a repeated training step come from remembered launches: the same bits as a first step's, on new
+  values, on group sizes of other contents and types, and on an expanded (non-contiguous) cotangent."""
+  from tokamax_amd.ragged_dot import hip
+  rng = np.random.default_rng(5)
+  G, m, k, n = 4, 96, 64, 128
+  make = lambda *shape: torch.tensor(rng.normal(0, 1, shape).astype(np.float32), device=device).to(dtype)
+  plans = lambda: len(hip._cotangent_op().__dict__.get("_plans") or ())
+
+  def step(lhs, rhs, gs, dout):
+    lhs, rhs = lhs.clone().requires_grad_(True), rhs.clone().requires_grad_(True)
+    out = tokamax_amd.ragged_dot(lhs, rhs, gs)
+    return (out.detach(), *torch.autograd.grad(out, (lhs, rhs), dout))
+
+  hip._cotangent_op.cache_clear()
+  assert plans() == 0
+  gs = torch.tensor([30, 0, 41, 20], dtype=torch.int32, device=device)
+  step(make(m, k), make(G, k, n), gs, make(m, n))
+  assert plans() == 2  # (one for dlhs, one for drhs)
+  for sizes in ([10, 20, 30, 36], [0, 0, 91, 5]):
+    lhs, rhs, dout, gs = make(m, k), make(G, k, n), make(m, n), torch.tensor(sizes, dtype=torch.int32, device=device)
+    remembered = step(lhs, rhs, gs, dout)
+    assert plans() == 2
+    for other in (gs.to(torch.int64), gs):
+      hip._cotangent_op.cache_clear()
+      for a, b in zip(remembered, step(lhs, rhs, other, dout)):
+        assert torch.equal(a, b)
+  flat = step(lhs, rhs, gs, dout[:1].expand(m, n))
+  for a, b in zip(flat, step(lhs, rhs, gs, dout[:1].repeat(m, 1))):
+    assert torch.equal(a, b)
+
+
 def test_repeated_eager_calls_take_the_remembered_launch(device):
   """The operator's shortcut for repeated eager calls: same bits as the full path, taken only for calls that are one
   forward launch on the caller's own tensors, and never when a gradient is wanted."""

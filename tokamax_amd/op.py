@@ -435,48 +435,73 @@ def infer_device_kind(ba: BoundArguments) -> DeviceKind | None:
   raise ValueError(f"Multiple device kinds found: {kinds}")
 
 
+@dataclasses.dataclass(frozen=True)
+class _VjpCall:
+  """One differentiated call: what `_VjpFunction` needs besides the tensors it is handed."""
+
+  op: Op
+  arguments: dict      # in signature order, None in the place of the tensors that go through autograd
+  names: tuple         # those tensors' arguments
+  config: Any
+  return_residuals: bool
+
+  def full(self, tensors) -> dict:
+    full = dict(self.arguments)
+    full.update(zip(self.names, tensors))
+    return full
+
+
+class _VjpFunction(torch.autograd.Function):
+  """`_fwd` with `op.vjp` as its backward (op.py:276-307). One class for every call: making an autograd.Function
+  subclass (and the class of its backward node) takes the interpreter longer than the small products take the GPU."""
+
+  @staticmethod
+  def forward(ctx, call: _VjpCall, *ts):
+    full = call.full(ts)
+    full["return_residuals"] = True
+    out, residuals = call.op._fwd(config=call.config, **full)  # pylint: disable=protected-access
+    # Inputs and residuals go through save_for_backward, and the output is not kept at all (`vjp` does not use
+    # it): a tensor this function returns, held as a plain attribute of ctx, would close the cycle
+    # out -> grad_fn -> ctx -> out, and the activations would live until the cyclic collector runs.
+    ctx.call = call
+    ctx.has_residuals = residuals is not None
+    ctx.save_for_backward(*ts, *([residuals] if residuals is not None else []))
+    if call.return_residuals:
+      ctx.mark_non_differentiable(residuals)
+      return out, residuals
+    return out
+
+  @staticmethod
+  def backward(ctx, dout, *unused):
+    call = ctx.call
+    saved = ctx.saved_tensors
+    ts, residuals = (saved[:-1], saved[-1]) if ctx.has_residuals else (saved, None)
+    full = call.full(ts)
+    full.pop("return_residuals")
+    pos_names = _positional_names(call.op)
+    args = [full.pop(n) for n in pos_names]
+    with torch.no_grad():
+      grads = call.op.vjp(residuals, None, dout, *args, **full)
+    by_name = dict(grads) if isinstance(grads, dict) else dict(zip(pos_names, grads))
+    return (None, *(by_name.get(n) for n in call.names))
+
+
+_POSITIONAL_NAMES: dict = {}
+
+
+def _positional_names(op: Op) -> tuple:
+  names = _POSITIONAL_NAMES.get(type(op))
+  if names is None:
+    names = tuple(n for n, p in op._fwd_signature.parameters.items()  # pylint: disable=protected-access
+                  if p.kind in (p.POSITIONAL_ONLY, p.POSITIONAL_OR_KEYWORD))
+    _POSITIONAL_NAMES[type(op)] = names
+  return names
+
+
 def _call_with_vjp(op: Op, ba: BoundArguments, config, return_residuals: bool):
-  """Runs `_fwd` under a torch.autograd.Function whose backward is `op.vjp` (op.py:276-307)."""
+  """Runs `_fwd` under `_VjpFunction`."""
   arguments = dict(ba.arguments)
-  names = [k for k, v in arguments.items() if isinstance(v, torch.Tensor) and v.is_floating_point()]
+  names = tuple(k for k, v in arguments.items() if isinstance(v, torch.Tensor) and v.is_floating_point())
   tensors = [arguments[k] for k in names]
-  pos_names = [
-      n for n, p in ba.signature.parameters.items()
-      if p.kind in (p.POSITIONAL_ONLY, p.POSITIONAL_OR_KEYWORD)
-  ]
-
-  class _Fn(torch.autograd.Function):
-
-    @staticmethod
-    def forward(ctx, *ts):
-      full = dict(arguments)
-      full.update(zip(names, ts))
-      bound = BoundArguments(op, full)
-      kwargs = dict(bound.kwargs)
-      kwargs["return_residuals"] = True
-      out, residuals = op._fwd(*bound.args, config=config, **kwargs)  # pylint: disable=protected-access
-      # Inputs and residuals go through save_for_backward, and the output is not kept at all (`vjp` does not use
-      # it): a tensor this function returns, held as a plain attribute of ctx, would close the cycle
-      # out -> grad_fn -> ctx -> out, and the activations would live until the cyclic collector runs.
-      ctx.has_residuals = residuals is not None
-      ctx.save_for_backward(*ts, *([residuals] if residuals is not None else []))
-      if return_residuals:
-        ctx.mark_non_differentiable(residuals)
-        return out, residuals
-      return out
-
-    @staticmethod
-    def backward(ctx, dout, *unused):
-      saved = ctx.saved_tensors
-      ts, residuals = (saved[:-1], saved[-1]) if ctx.has_residuals else (saved, None)
-      full = dict(arguments)
-      full.update(zip(names, ts))
-      bound = BoundArguments(op, full)
-      kwargs = dict(bound.kwargs)
-      kwargs.pop("return_residuals")
-      with torch.no_grad():
-        grads = op.vjp(residuals, None, dout, *bound.args, **kwargs)
-      by_name = dict(grads) if isinstance(grads, dict) else dict(zip(pos_names, grads))
-      return tuple(by_name.get(n) for n in names)
-
-  return _Fn.apply(*tensors)
+  arguments.update(dict.fromkeys(names))
+  return _VjpFunction.apply(_VjpCall(op, arguments, names, config, return_residuals), *tensors)

@@ -552,10 +552,14 @@ def _concrete_operand(x):
 _PLAIN_ARGUMENT_TYPES = (bool, int, float, str, torch.dtype, base.RaggedDotDimensionNumbers)
 
 
+def _sizes_array(group_sizes):
+  return group_sizes.value if type(group_sizes) is base.GroupSizes else group_sizes
+
+
 def _make_plan(records, out, lhs, rhs, group_sizes):
   """The shortcut for calls like the one that left `records` and returned `out`, or None if that call was more than
-  one forward launch on the caller's own buffers."""
-  if len(records) != 1 or not isinstance(records[0], hip_ops.ForwardLaunch) or records[0].out is not out:
+  one launch of a product on the caller's own buffers."""
+  if len(records) != 1 or not isinstance(records[0], hip_ops.Launch) or records[0].out is not out:
     return None
   record = records[0]
   if out.device.index != torch.cuda.current_device():
@@ -593,6 +597,14 @@ def _make_plan(records, out, lhs, rhs, group_sizes):
   return plan
 
 
+@functools.lru_cache(maxsize=None)
+def _cotangent_op() -> "HipRaggedDot":
+  """The op of the two products of every backward pass. One for all of them, so that the configs and the launches it
+  remembers (by shapes, types and arguments) serve the next step: an op made per product chose its tiles anew each
+  time, which at 1024 rows of a numerical study took four times as long as the three products."""
+  return HipRaggedDot()
+
+
 @dataclasses.dataclass(frozen=True)
 class HipRaggedDot(base.RaggedDot):
   """Hand-written HIP ragged dot for gfx950. Physical layout `mk,gkn->mn`, rhs never transposed."""
@@ -605,14 +617,14 @@ class HipRaggedDot(base.RaggedDot):
 
   def __post_init__(self):
     if self.vjp is None:
-      # A fresh op per call avoids infinite recursion (pallas_mosaic_gpu.py:95-100).
-      fn = lambda *a, **kw: HipRaggedDot()(*a, **kw)  # pylint: disable=unnecessary-lambda
+      # An op made at the first backward avoids infinite recursion (pallas_mosaic_gpu.py:95-100).
+      fn = lambda *a, **kw: _cotangent_op()(*a, **kw)  # pylint: disable=unnecessary-lambda
       object.__setattr__(self, "vjp", partial(base.vjp, dlhs_ragged_dot=fn, drhs_ragged_dot=fn))
 
   # -- eager fast path -------------------------------------------------------------------------
   def __call__(self, lhs, rhs, *, return_residuals: bool = False, **kwargs):
     """The operator call (`Op.__call__`) with a shortcut for repeated eager calls: a call that came down to one
-    forward launch on the caller's own tensors (no pass over an operand in front of it, nothing applied to the result
+    launch of a product on the caller's own tensors (no pass over an operand in front of it, nothing applied to the result
     behind it, no gradient wanted) is remembered under the shapes, types and arguments it was made with, and the next
     call of that kind goes straight to the C ABI: allocate the result, pass the addresses. Binding, the choice of a
     config and the routing cost about 45 us of Python per call, more than the small-m kernels take."""
@@ -621,7 +633,7 @@ class HipRaggedDot(base.RaggedDot):
     if key is not None and plans is not None:
       plan = plans.get(key)
       if plan is not None:
-        return plan(lhs, rhs, kwargs["group_sizes"])
+        return plan(lhs, rhs, _sizes_array(kwargs["group_sizes"]))
     if key is None:
       return super().__call__(lhs, rhs, return_residuals=return_residuals, **kwargs)
     log = hip_ops.LAUNCH_LOG
@@ -633,7 +645,7 @@ class HipRaggedDot(base.RaggedDot):
       log.records = outer
     if outer is not None:
       outer.extend(records)
-    plan = _make_plan(records, out, lhs, rhs, kwargs["group_sizes"])
+    plan = _make_plan(records, out, lhs, rhs, _sizes_array(kwargs["group_sizes"]))
     if plan is not None:
       if plans is None or len(plans) > 64:
         plans = {}
@@ -646,10 +658,13 @@ class HipRaggedDot(base.RaggedDot):
     if self.checkify_group_sizes or op.OP_CALL_RECORDER.get() is not None:
       return None
     group_sizes = kwargs.get("group_sizes")
+    parts = []
+    if type(group_sizes) is base.GroupSizes:
+      parts.append(("representative", group_sizes.repr_value_or_total_size))  # (what the choice of a config sees)
+      group_sizes = group_sizes.value
     if type(group_sizes) is not torch.Tensor or not group_sizes.is_cuda:
       return None
     grad = torch.is_grad_enabled()
-    parts = []
     for x in (lhs, rhs):
       if type(x) is torch.Tensor:
         leaves = (x,)
@@ -667,7 +682,8 @@ class HipRaggedDot(base.RaggedDot):
     for name, v in kwargs.items():
       if name == "group_sizes":
         continue
-      if not (v is None or type(v) in _PLAIN_ARGUMENT_TYPES):
+      if not (v is None or type(v) in _PLAIN_ARGUMENT_TYPES
+              or (type(v) is tuple and all(type(x) is precision_lib.Precision for x in v))):
         return None  # (tensors, callables: the full path)
       parts.append((name, v))
     parts.append((op.config_epoch(), config_lib.autotuning_cache_miss_fallback.value,

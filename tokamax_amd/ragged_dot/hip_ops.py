@@ -30,9 +30,9 @@ SCHEDULE_FIELDS = ("group_id", "block_start", "actual_start", "actual_end", "sta
 
 class _LaunchLog(threading.local):
   """What the functions of this module launched while a caller was listening (`records` is a list then): a
-  `ForwardLaunch` for a forward call, None for anything else (a pass over an operand, a quantisation, drhs). The
-  operator's eager fast path reads it to learn whether a call came down to one forward launch on the caller's own
-  tensors, which it can then repeat without the planning in front of it."""
+  `Launch` for a product, None for anything else (a pass over an operand, a quantisation). The operator's eager fast
+  path reads it to learn whether a call came down to one product on the caller's own tensors, which it can then repeat
+  without the planning in front of it."""
   records = None
 
 
@@ -45,8 +45,8 @@ def _log_launch(entry) -> None:
 
 
 @dataclasses.dataclass
-class ForwardLaunch:
-  """One forward launch, repeatable on other buffers of the same shapes: `launch(pointers, out_ptr, ws_ptr, stream)`
+class Launch:
+  """The launch of one product, repeatable on other buffers of the same shapes: `launch(pointers, out_ptr, ws_ptr, stream)`
   with `pointers` in the order of `POINTER_NAMES` (0 for an absent operand) returns the C status."""
 
   POINTER_NAMES = ("lhs", "rhs", "group_sizes", "group_offset", "lhs_scale", "rhs_scale", "rhs_bias")
@@ -331,7 +331,7 @@ def ragged_dot_fwd(lhs, rhs, group_sizes, *, config: KernelConfig, out_dtype: to
       _lib.check(lib.tkx_ragged_dot_schedule_spans(_ptr(gs), gs.numel(), m, config.block_m, config.align_tile,
                                                    config.grid_tile_width, _ptr(filled), _stream(device)))
     workspace_out.append(filled)
-  _log_launch(ForwardLaunch(pointers, launch, out, new_workspace))
+  _log_launch(Launch(pointers, launch, out, new_workspace))
   return out
 
 
@@ -536,7 +536,6 @@ def dequantize(qvalue: torch.Tensor, scale: torch.Tensor, zero_point: torch.Tens
 def ragged_dot_drhs(lhs, dout, group_sizes, num_groups: int, *, config: KernelConfig,
                     out_dtype: torch.dtype) -> torch.Tensor:
   """out[g,k,n] = lhs[rows_g,k]^T . dout[rows_g,n]."""
-  _log_launch(None)
   _require_cuda(lhs, dout, group_sizes)
   lib = _lib.load()
   if lhs.dim() != 2 or dout.dim() != 2 or lhs.shape[0] != dout.shape[0]:
@@ -550,10 +549,17 @@ def ragged_dot_drhs(lhs, dout, group_sizes, num_groups: int, *, config: KernelCo
   m, k = lhs.shape
   n = dout.shape[1]
   out = torch.empty((num_groups, k, n), dtype=out_dtype, device=lhs.device)
-  ws = workspace(m, num_groups, 128, lhs.device)
-  cfg = config.to_c()
-  with _on_device(lhs.device):
-    st = lib.tkx_ragged_dot_drhs(_ptr(lhs), _ptr(dout), _ptr(gs), _ptr(out), _ptr(ws), m, k, n, num_groups,
-                                 dtype_code(lhs.dtype), dtype_code(out_dtype), ctypes.byref(cfg), _stream(lhs.device))
+  device = lhs.device
+  new_workspace = lambda: workspace(m, num_groups, 128, device)
+  ws = new_workspace()
+  cfg, in_code, out_code, drhs = ctypes.byref(config.to_c()), dtype_code(lhs.dtype), dtype_code(out_dtype), lib.tkx_ragged_dot_drhs
+
+  def launch(p, out_ptr, ws_ptr, stream):
+    return drhs(p[0], p[1], p[2], out_ptr, ws_ptr, m, k, n, num_groups, in_code, out_code, cfg, stream)
+
+  pointers = (lhs.data_ptr(), dout.data_ptr(), gs.data_ptr(), 0, 0, 0, 0)
+  with _on_device(device):
+    st = launch(pointers, out.data_ptr(), ws.data_ptr(), torch.cuda.current_stream(device).cuda_stream)
   _lib.check(st)
+  _log_launch(Launch(pointers, launch, out, new_workspace))
   return out
