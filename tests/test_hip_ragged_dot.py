@@ -2233,6 +2233,30 @@ def test_quantize_kernel_bit_exact(shape, tile, qtype, xdtype, device):
   assert torch.equal(as_q.qvalue.view(torch.uint8), qv.view(torch.uint8))
 
 
+@pytest.mark.parametrize("xdtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("qtype", [torch.int8, torch.float8_e4m3fn])
+@pytest.mark.parametrize("shape,tile", [((8193, 1024), 128), ((8195, 1024), 512), ((5, 1016), 1016), ((3, 1032), 1032),
+                                        ((7, 2056), 2056), ((3, 4104), 4104), ((3, 8192), 8192), ((2, 8200), 8200)])
+def test_quantize_rows_held_in_registers(shape, tile, qtype, xdtype, device):
+  """Tiles one row tall, by how many registers hold them (the last one is walked twice), against the oracle's division,
+  bit for bit: with tiles that are nearly zero, nearly the largest float, and mixtures of both with ordinary values
+  (scales whose reciprocal is no normal number take the division itself)."""
+  rng = np.random.default_rng(shape[1] + tile)
+  x = rng.normal(0, 1, shape).astype(np.float32)
+  flat = x.reshape(-1, tile)
+  for row, factor in ((0, 1e-37), (1, 1e25), (2, 1e37), (3, 1e-30)):
+    if row < len(flat):
+      flat[row] *= np.float32(factor)
+  flat[1, 1::2] *= np.float32(1e-30)
+  flat[-1, ::3] = -0.0
+  xt = torch.tensor(x, device=device).to(xdtype)
+  qv, scale = hip_ops.quantize(xt, qtype, (1, tile))
+  want_q, want_s = O.quantize_absmax(_np(xt), _QNAME[qtype], (1, tile))
+  assert np.array_equal(scale.cpu().numpy(), want_s)
+  got_q = qv.view(torch.uint8).cpu().numpy() if qtype == torch.float8_e4m3fn else qv.cpu().numpy()
+  assert np.array_equal(got_q, want_q)
+
+
 @pytest.mark.parametrize("qtype,bound", [(torch.int8, 127.5), (torch.int4, 7.5), (torch.int8, 128.0), (torch.int8, 127.0)])
 @pytest.mark.parametrize("shape,tile", [((96, 256), (1, 128)), ((512, 128), (64, 1)), ((2, 128, 256), (1, 128, 128))])
 def test_quantize_kernel_with_another_bound(shape, tile, qtype, bound, device):
