@@ -1974,6 +1974,32 @@ def test_gated_linear_unit(shape, dtype, device):
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32, torch.float16])
+@pytest.mark.parametrize("out_rows,hidden,reduce", [(1, 8, 1), (3, 2048, 8), (5, 4104, 2), (7, 8200, 1), (1023, 2056, 2),
+                                                    (1024, 4104, 1), (1024, 2056, 3), (2, 16648, 9)])
+def test_row_movement_by_pieces(out_rows, hidden, reduce, dtype, device):
+  """Rows cut into pieces over workgroups (below 1024 output rows), pieces in flight per thread, and one, two, up to
+  eight and more rows per sum: copies bit for bit, sums against f64 within the output type's rounding (and reduce
+  additions in f32). Dropped rows hold infinities that must not reach the result; all of one output row's are dropped."""
+  rng = np.random.default_rng(out_rows + hidden + reduce)
+  rows = 40
+  x = torch.tensor(rng.normal(0, 1, (rows, hidden)).astype(np.float32), device=device).to(dtype)
+  idx = torch.tensor(rng.integers(1, rows, out_rows * reduce).astype(np.int32), device=device)
+  assert torch.equal(tokamax_amd.ragged_gather(x, idx, 0, rows), x[idx.long()])
+  x[0] = float("inf")
+  valid = torch.tensor(rng.integers(0, 4, out_rows * reduce) > 0, device=device)
+  valid[-reduce:] = False
+  idx = torch.where(valid, idx, torch.zeros_like(idx))
+  w = torch.tensor(rng.uniform(0, 1, out_rows * reduce).astype(np.float32), device=device)
+  got = tokamax_amd.ragged_gather_reduce(x, idx, w, valid, reduce)
+  picked = torch.where(valid[:, None], x[idx.long()].double() * w.double()[:, None], 0.0)
+  want = picked.view(out_rows, reduce, hidden).sum(1)
+  bound = picked.abs().view(out_rows, reduce, hidden).sum(1) * reduce * 2.0 ** -23
+  ulp = {torch.bfloat16: 2.0 ** -8, torch.float16: 2.0 ** -11, torch.float32: 2.0 ** -24}[dtype]
+  assert bool(((got.double() - want).abs() <= bound + want.abs() * ulp + (2.0 ** -24 if dtype == torch.float16 else 0.0)).all())
+  assert torch.equal(tokamax_amd.ragged_gather_reduce(x, idx, w, valid.to(torch.int32), reduce), got)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32, torch.float16])
 def test_row_movement_ops(dtype, device):
   """ragged_gather, ragged_scatter (bit-exact copies / zeros) and ragged_gather_reduce (f32 sums, one
   rounding) against the oracle; the token permute -> ragged dot -> weighted un-permute round trip."""

@@ -42,7 +42,8 @@ def _gather_rows(x, indices, *, weights=None, valid=None, start=None, end=None, 
   if weights is not None:
     weights = weights.to(torch.float32).contiguous()
   if valid is not None:
-    valid = valid.to(torch.uint8).contiguous()
+    # (a bool is a byte of 0 or 1 already: no pass over the mask)
+    valid = (valid.view(torch.uint8) if valid.dtype == torch.bool else valid.to(torch.uint8)).contiguous()
   if start is not None:
     start, end = _scalar_i32(start, x.device), _scalar_i32(end, x.device)
   out = torch.empty((out_rows, x.shape[1]), dtype=x.dtype, device=x.device)
