@@ -2401,6 +2401,26 @@ def test_ceiling_probes_run_and_give_plausible_figures(device):
   assert 1.0 < alone < 9.0 and shared > 2 * alone, (alone, shared)
 
 
+@pytest.mark.parametrize("k,n", [(2048, 768), (1024, 768), (2048, 128), (512, 256), (512, 512), (256, 1152), (768, 640)])
+def test_drhs_tiles_dealt_to_the_xcds(k, n, device):
+  """d rhs whose tiles per group divide over the 8 XCDs in each of the ways the launch knows (and two that do not):
+  every tile of every group is written once, with uneven, empty and no rows, against f64 sums (bf16 result: 2^-8 of the
+  value, and f32 sums of at most 300 products)."""
+  rng = np.random.default_rng(k + n)
+  gs = np.array([300, 0, 17, 64, 1, 0], np.int32)
+  m = int(gs.sum()) + 9
+  lhs = torch.tensor(rng.normal(0, 1, (m, k)).astype(np.float32), device=device).to(torch.bfloat16)
+  dout = torch.tensor(rng.normal(0, 1, (m, n)).astype(np.float32), device=device).to(torch.bfloat16)
+  cfg = hip_ops.KernelConfig(256, 128, 32, 2, 2, 3)
+  got = hip_ops.ragged_dot_drhs(lhs, dout, torch.tensor(gs, device=device), len(gs), config=cfg, out_dtype=torch.bfloat16)
+  row = 0
+  for g, size in enumerate(gs):
+    a, b = lhs[row:row + size].double(), dout[row:row + size].double()
+    want, bound = a.t() @ b, a.abs().t() @ b.abs()
+    assert bool(((got[g].double() - want).abs() <= want.abs() * 2.0 ** -8 + bound * 300 * 2.0 ** -23).all())
+    row += size
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 def test_repeated_backward_passes_take_remembered_launches(device, dtype):
   """The cotangents of a repeated training step come from remembered launches: the same bits as a first step's, on new

@@ -99,6 +99,7 @@ struct GemmParams {
   int32_t nb_ext;                   // columns of B (fwd/dlhs): n_ext, or 2 * n_ext for kFwdGlu
   int32_t num_groups;
   int32_t n_tiles, m_tiles;         // tiles along C columns; along C rows (drhs only)
+  int32_t xcd_rows;                 // drhs: XCDs along the rows of a group's tiles (8 / xcd_rows along its columns), or 0
   int32_t real_slots;               // fwd/dlhs: workgroups that may own a task tile (multiple of 8 * kXcdChunk)
   int32_t zero_wgs;                 // fwd/dlhs: workgroups after those that clear the rows of no group
   // Split of the last round (fwd/dlhs, split_k > 1): the launch's tiles beyond the last multiple of `split_cus` are
