@@ -2421,6 +2421,29 @@ def test_drhs_tiles_dealt_to_the_xcds(k, n, device):
     row += size
 
 
+@pytest.mark.parametrize("tiles", [1, 7, 8, 9, 31, 33, 112, 255, 257, 265])
+@pytest.mark.parametrize("split_k", [1, 4])
+def test_tiles_behind_the_last_whole_round(tiles, split_k, device):
+  """Launches whose last round holds any number of tiles, split along the contraction or not: every tile of the result
+  against f64 sums (bf16 result: 2^-8 of the value, and f32 sums of 192 products)."""
+  rng = np.random.default_rng(tiles)
+  gs = np.array([5, 0, 130], np.int32)  # 3 tasks of 128 rows at most: 1 + 2 tiles a column
+  n = 128 * -(-tiles // 3) if tiles > 2 else 128
+  if tiles <= 2:
+    gs = np.array([0, 128 * tiles, 0], np.int32)
+  m, k = int(gs.sum()), 192
+  lhs = torch.tensor(rng.normal(0, 1, (m, k)).astype(np.float32), device=device).to(torch.bfloat16)
+  rhs = torch.tensor(rng.normal(0, 1, (3, k, n)).astype(np.float32), device=device).to(torch.bfloat16)
+  cfg = hip_ops.KernelConfig(128, 128, 64, 2, 2, 4, split_k=split_k)
+  got = hip_ops.ragged_dot_fwd(lhs, rhs, torch.tensor(gs, device=device), config=cfg, out_dtype=torch.bfloat16)
+  row = 0
+  for g, size in enumerate(gs):
+    a, b = lhs[row:row + size].double(), rhs[g].double()
+    want, bound = a @ b, a.abs() @ b.abs()
+    assert bool(((got[row:row + size].double() - want).abs() <= want.abs() * 2.0 ** -8 + bound * 192 * 2.0 ** -23).all())
+    row += size
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 def test_repeated_backward_passes_take_remembered_launches(device, dtype):
   """The cotangents of a repeated training step come from remembered launches: the same bits as a first step's, on new

@@ -802,3 +802,19 @@ def test_config_json_without_split_k_loads_with_the_default():
   assert ctypes.sizeof(c) == 10 * 4 and c.split_k == 1 and c.persistent == 0
   with pytest.raises(ValueError):
     hip.Config(16, 128, 32, 1, 4, 2, 1, 8, 1, -1)
+
+
+@pytest.mark.parametrize("total", [1, 2, 7, 8, 9, 31, 33, 255, 256, 257, 264, 511, 513])
+def test_launch_order_reaches_every_tile_once(total):
+  """The kernel's map from workgroups to list entries: whole rounds of 8 chunks of 32, and the entries behind them in 8
+  equal chunks, reach every entry exactly once from the workgroups that are launched."""
+  slots = -(-total // 256) * 256 + 256
+  seen = []
+  for b in range(slots):
+    idx, xcd = b >> 3, b & 7
+    first, at = idx // 32 * 256, idx % 32
+    share = min(32, (total - first + 7) >> 3)
+    entry = first + xcd * share + at
+    if at < share and entry < total:
+      seen.append(entry)
+  assert sorted(seen) == list(range(total))

@@ -78,7 +78,8 @@ int32_t device_compute_units(int* out);
 enum KernelMode { kFwd = 0, kDlhs = 1, kDrhs = 2, kFwdGlu = 3, kFwdSubK = 4 };
 
 // fwd/dlhs launch order: the tile list is dealt to the 8 XCDs in chunks of this many consecutive
-// tiles (the number of CUs of an XCD: one chunk is what an XCD runs at a time).
+// tiles (the number of CUs of an XCD: one chunk is what an XCD runs at a time), the tiles behind the last whole round of
+// 8 chunks in 8 equal shorter ones.
 constexpr int32_t kXcdChunk = 32;
 
 struct GemmParams {
