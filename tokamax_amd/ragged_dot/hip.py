@@ -952,10 +952,12 @@ class HipRaggedDot(base.RaggedDot):
         shapes = ((256, 256), (128, 256), (128, 128), (64, 128), (32, 128)) if mode == 0 else sorted(
             {(v[0], v[1]) for v in usable if v[0] > 16}, key=lambda t: (-t[0] * t[1], -t[1]))
         want_m, want_n = next((t for t in shapes[:-1] if t[0] <= want_m and tiles(*t) >= _COMPUTE_UNITS), shapes[-1])
-    if mode == 0 and key[1] == _lib.TKX_F32:
+    if mode in (0, 1) and key[1] == _lib.TKX_F32:
       # f32 operands run on the f32 MFMAs at a sixteenth of the bf16 rate: loads never bound them, and the 32-row tile
       # (four of its workgroups share a CU) was the fastest of the three on every measured shape, 128 to 1400 rows
-      # per group (9-47 % ahead of the taller ones).
+      # per group (9-47 % ahead of the taller ones). So for dlhs, on 8 shapes of 5 to 1024 rows per group: 1024 rows over 8
+      # groups, k = 512, n = 1024: 36.0 us on the 64-row tile, 22.7 on this one; 8192 rows over 32, k = 2048, n = 1024:
+      # 338 on the 128-row tile, 303; even with the best other one at worst (64 rows a group, k = 512, n = 2048: 126.1, 126.7).
       want_m, want_n = 32, 128
     # The streaming kernel on int8 weights has a wide form (256 columns per workgroup, two workgroups
     # per CU) that streams 7-9% faster when its workgroups fill the chip evenly, and slower than the
@@ -1011,7 +1013,6 @@ class HipRaggedDot(base.RaggedDot):
     if bm != 16 and mode in (0, 1) and key[1] == key[2] and key[1] in (_lib.TKX_BF16, _lib.TKX_F16):
       # 16-bit operands without scales: the tile that the cost model expects to finish first, with or without the
       # split of the last round (the rules above stay in charge of the choice for the streaming small-m kernel).
-      best = None
       for v in usable:
         if v[0] == 16:
           continue
