@@ -1013,6 +1013,7 @@ class HipRaggedDot(base.RaggedDot):
     if bm != 16 and mode in (0, 1) and key[1] == key[2] and key[1] in (_lib.TKX_BF16, _lib.TKX_F16):
       # 16-bit operands without scales: the tile that the cost model expects to finish first, with or without the
       # split of the last round (the rules above stay in charge of the choice for the streaming small-m kernel).
+      best = None
       for v in usable:
         if v[0] == 16:
           continue
