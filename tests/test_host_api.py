@@ -818,3 +818,14 @@ def test_launch_order_reaches_every_tile_once(total):
     if at < share and entry < total:
       seen.append(entry)
   assert sorted(seen) == list(range(total))
+
+
+@pytest.mark.parametrize("rows, n2, block_m", [(1, 28672, 32), (64, 28672, 32), (100, 28672, 64), (256, 28672, 128),
+                                               (320, 28672, 256), (256, 2816, 32), (900, 11008, 256), (8192, 28672, 256)])
+def test_dense_gated_unit_takes_the_fastest_measured_tile(rows, n2, block_m):
+  """The tile of a gate-up product over one group, k = 4096 (2048 for 2816 columns): the height that measured fastest."""
+  op, dtype = hip.HipRaggedDot(), torch.bfloat16
+  k = 2048 if n2 == 2816 else 4096
+  ba = op.bind(ShapeDtype((rows, k), dtype), ShapeDtype((1, k, n2), dtype), group_sizes=ShapeDtype((1,), torch.int32),
+               fuse_gateup_activation="silu")
+  assert op._get_heuristics_config(ba).block_m == block_m

@@ -1024,6 +1024,16 @@ class HipRaggedDot(base.RaggedDot):
             best = (cost, v, sk)
       if best is not None:
         (bm, bn, bk, wm, wn, ns), modelled_split = best[1], best[2]
+    if mode == 3 and num_groups == 1 and key[1:] == (_lib.TKX_BF16, _lib.TKX_BF16):
+      # Gate-up fusion over one group (the dense gated unit): the launch of the plain product over both halves' columns.
+      # Its tiles are known exactly, start together and end together, so a partial last round counts in full. The rules
+      # above took the 256 x 256 x 32 tile from 224 rows on, however few tiles came of it. On 29 shapes (1 to 8192 rows,
+      # k = 2048 to 8192, 2816 to 28672 columns) this takes the fastest tile or one within 1.5 % of it; k = 4096, 28672
+      # columns: 256 rows 72.5 -> 53.2 us, 1024 rows 193 -> 175, 8192 rows 1431 -> 1308. (With several groups the rules stay:
+      # they are within a few percent on 26 shapes.)
+      fit = dict(_TILE_COST_FIT, tail_floor=1.0)
+      bm, bn, bk, wm, wn, ns = min(usable, key=lambda v: (
+          round(_tile_cost(v, 1, rows, cols, contraction, 1, 0, fit), 3), -v[2], -v[5]))
     # grid_tile_width m-tasks of one group run side by side on an n-panel of its weights (a span never
     # crosses a group, so small groups simply get short spans). With the 32 tiles an XCD runs at a
     # time, 8 wide x 4 n-panels needs the fewest distinct operand panels in its L2; 16 wide measured
