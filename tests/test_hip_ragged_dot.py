@@ -1973,6 +1973,15 @@ def test_gated_linear_unit(shape, dtype, device):
     tokamax_amd.gated_linear_unit(x, w.float(), activation=F.silu)
 
 
+@pytest.mark.parametrize("rows, k, n", [(5, 544, 128), (300, 544, 1408), (256, 2080, 2048)])
+def test_gated_linear_unit_with_a_contraction_of_odd_32s(rows, k, n, device):
+  """k % 64 == 32 has one tile, at few rows as at many."""
+  rng = np.random.default_rng(rows)
+  x = torch.tensor(rng.normal(0, 1, (rows, k)).astype(np.float32)).to(torch.bfloat16).to(device)
+  w = torch.tensor(rng.normal(0, k ** -0.5, (k, 2, n)).astype(np.float32)).to(torch.bfloat16).to(device)
+  _check(tokamax_amd.gated_linear_unit(x, w, activation=torch.nn.functional.silu), O.gated_linear_unit(_np(x), _np(w), O.silu), 3e-3)
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32, torch.float16])
 @pytest.mark.parametrize("out_rows,hidden,reduce", [(1, 8, 1), (3, 2048, 8), (5, 4104, 2), (7, 8200, 1), (1023, 2056, 2),
                                                     (1024, 4104, 1), (1024, 2056, 3), (2, 16648, 9)])

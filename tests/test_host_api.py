@@ -829,3 +829,19 @@ def test_dense_gated_unit_takes_the_fastest_measured_tile(rows, n2, block_m):
   ba = op.bind(ShapeDtype((rows, k), dtype), ShapeDtype((1, k, n2), dtype), group_sizes=ShapeDtype((1,), torch.int32),
                fuse_gateup_activation="silu")
   assert op._get_heuristics_config(ba).block_m == block_m
+
+
+@pytest.mark.parametrize("groups", [1, 8])
+@pytest.mark.parametrize("k", [544, 2080, 4128])
+def test_gateup_tile_has_a_k_step_that_divides_the_contraction(k, groups):
+  """The gate-up kernels take whole k-steps: of the 16-bit tiles only 256 x 256 x 32 serves k % 64 == 32."""
+  op, dtype = hip.HipRaggedDot(), torch.bfloat16
+  for rows in (1, 64, 224, 256, 512, 1024, 2048, 8192):
+    for n2 in (2816, 28672):
+      ba = op.bind(ShapeDtype((rows, k), dtype), ShapeDtype((groups, k, n2), dtype),
+                   group_sizes=ShapeDtype((groups,), torch.int32), fuse_gateup_activation="silu")
+      assert k % op._get_heuristics_config(ba).block_k == 0, (rows, n2)
+  # (a contraction that no k-step divides keeps a config: the gated unit's path through a plain product asks for one)
+  ba = op.bind(ShapeDtype((64, 40), dtype), ShapeDtype((1, 40, 256), dtype), group_sizes=ShapeDtype((1,), torch.int32),
+               fuse_gateup_activation="silu")
+  assert op._get_heuristics_config(ba).block_k

@@ -910,6 +910,10 @@ class HipRaggedDot(base.RaggedDot):
       usable = [v for v in usable if v[0] == 16 or step % v[2] == 0]
       if not usable:
         raise NotImplementedError(f"No hip kernel variant whose k-step divides {step} rows.")
+    if mode == 3:
+      # Gate-up fusion takes whole k-steps (16-bit weights: 64 deep, or 32 in the 256 x 256 x 32 tile, the only one for
+      # k % 64 == 32). Where no variant's divides the contraction the launch declines the call.
+      usable = [v for v in usable if contraction % v[2] == 0] or usable
     # Rows per group decide the m-tile: a tile much taller than a group wastes MFMA work on rows
     # that are masked out at the store; a short tile re-reads the weights more often.
     rows_per_group = rows / max(num_groups, 1) if mode != 2 else rows
