@@ -16,21 +16,29 @@ import pytest
 from tokamax_amd import _lib
 
 LLVM = "/opt/rocm/llvm/bin"
-TOOLS = [os.path.join(LLVM, t) for t in ("llvm-objcopy", "clang-offload-bundler", "llvm-readelf")]
+TOOLS = [os.path.join(LLVM, t) for t in ("llvm-objcopy", "clang-offload-bundler", "llvm-readelf", "llvm-objdump")]
 TARGET = "hipv4-amdgcn-amd-amdhsa--gfx950"
 
 
-def _kernel_metadata(tmp_path):
-  """[(mangled kernel name, scratch bytes per lane, vgprs)] over every code object bundled into the library."""
+def _code_objects(tmp_path):
+  """The gfx950 code objects bundled into the library, one per source file."""
   fat = tmp_path / "fatbin"
   subprocess.run([TOOLS[0], "-O", "binary", "--only-section=.hip_fatbin", _lib.LIB_PATH, str(fat)], check=True)
   blob = fat.read_bytes()
   starts = [m.start() for m in re.finditer(rb"__CLANG_OFFLOAD_BUNDLE__", blob)]  # one bundle per source file
-  rows = []
+  codes = []
   for n, first in enumerate(starts):
     part, code = tmp_path / f"bundle{n}", tmp_path / f"bundle{n}.co"
     part.write_bytes(blob[first:starts[n + 1] if n + 1 < len(starts) else len(blob)])
     subprocess.run([TOOLS[1], "--unbundle", "--type=o", f"--input={part}", f"--targets={TARGET}", f"--output={code}"], check=True)
+    codes.append(code)
+  return codes
+
+
+def _kernel_metadata(tmp_path):
+  """[(mangled kernel name, scratch bytes per lane, vgprs)] over every code object bundled into the library."""
+  rows = []
+  for code in _code_objects(tmp_path):
     notes = subprocess.run([TOOLS[2], "--notes", str(code)], check=True, capture_output=True, text=True).stdout
     name = scratch = None
     for line in notes.splitlines():
@@ -72,3 +80,25 @@ def test_no_kernel_of_the_library_uses_scratch_memory(tmp_path):
   # the 8-wave tiles run two waves per SIMD: 256 registers each
   headline = [v for n, _, v in rows if "GemmKernelILi0ELi1ELi1ELi256ELi256ELi64ELi2ELi4E" in n]
   assert len(headline) >= 6 and max(headline) <= 256
+
+
+@pytest.mark.skipif(not all(os.path.exists(t) for t in TOOLS), reason="ROCm's LLVM tools are not installed")
+def test_matrix_instruction_of_16_bit_tiles(tmp_path):
+  """16x16x32 MFMAs in the forward and dlhs tiles that keep two waves on a SIMD; 32x32x16 where a 4-wave workgroup has
+  its CU to itself and in d rhs, which measured up to 30 % slower on the other form."""
+  name = lambda mode, *tile: "GemmKernelILi%dELi1ELi1E" % mode + "".join(f"Li{t}E" for t in tile)
+  wants = {name(0, 256, 256, 64, 2, 4, 2): "16x16x32", name(1, 128, 256, 64, 2, 4, 3): "16x16x32",
+           name(0, 128, 128, 64, 2, 2, 2): "16x16x32", name(3, 128, 256, 64, 2, 4, 3): "16x16x32",
+           name(0, 128, 256, 64, 2, 2, 3): "32x32x16", name(1, 128, 128, 64, 2, 2, 4): "32x32x16",
+           name(3, 64, 256, 64, 2, 2, 3): "32x32x16", name(2, 128, 128, 64, 2, 2, 4): "32x32x16",
+           name(2, 256, 256, 64, 2, 4, 2): "32x32x16"}
+  seen = {}
+  for code in _code_objects(tmp_path):
+    symbols = subprocess.run([TOOLS[2], "--symbols", "--wide", str(code)], check=True, capture_output=True, text=True).stdout
+    picked = [w.split()[-1] for w in symbols.splitlines() if "gemm_entryI" in w and not w.endswith(".kd")]
+    for tile in wants:
+      for symbol in picked:
+        if tile in symbol:
+          text = subprocess.run([TOOLS[3], "-d", f"--disassemble-symbols={symbol}", str(code)], check=True, capture_output=True, text=True).stdout
+          seen[tile] = set(re.findall(r"v_mfma_f32_(\d+x\d+x\d+)_bf16", text))
+  assert seen == {tile: {form} for tile, form in wants.items()}

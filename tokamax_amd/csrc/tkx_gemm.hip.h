@@ -217,6 +217,7 @@ __device__ __forceinline__ typename Mma<EC, M16>::Frag load_frag(const unsigned 
   typedef typename Mma<EC, M16>::Frag Frag;
   constexpr int KA = Mma<EC, M16>::KA;
   if constexpr (M16) {
+    static_assert(!PAIRED && ES == EC, "16x16 fragments: operands stored in the compute type");
     const int q = lane >> 4, s = lane & 15;
     Frag f;
 #pragma unroll
@@ -224,11 +225,7 @@ __device__ __forceinline__ typename Mma<EC, M16>::Frag load_frag(const unsigned 
       i32x4 v;
       if constexpr (LAYOUT == kKC) {
         // (16 rows further on the swizzle is the same: a constant distance)
-        v = lds_read_b128(tile + (rc_step + 16 * h) * ROW_BYTES,
-                          kc_offset<ROW_BYTES>(rc0 + s, PAIRED ? (kk >> 1) * 8 + 2 * q + (kk & 1) : kk * 4 + q));
-      } else if constexpr (ES == kEI8) {
-        const int krow = kk * KA + 8 * q + (s >> 1), col = rc0 + rc_step + 16 * h + 8 * (s & 1);
-        v = i8x8_to_bf16x8(lds_read_tr8(tile + mc_offset<ROW_BYTES, ES>(krow, col)));
+        v = lds_read_b128(tile + (rc_step + 16 * h) * ROW_BYTES, kc_offset<ROW_BYTES>(rc0 + s, kk * 4 + q));
       } else {
         // (the transposing read of 16-bit elements: see below; a block of 16 lanes covers 4 k-rows of 16 columns)
         const int krow = kk * KA + 8 * q + (s >> 2), col = rc0 + rc_step + 16 * h + 4 * (s & 3);
@@ -739,13 +736,23 @@ struct GemmKernel {
   // NI blocks later. With NI >= 4 that is at least four blocks (sixteen MFMAs, 256 cycles of the matrix pipe for one
   // wave, twice that with the SIMD's other wave) between the LDS read of a fragment and its first use. Smaller wave
   // tiles double-buffer what does not have that distance, which takes an even number of atoms per k-step.
-  // Wave tiles of fewer than four blocks and classic pipelines with 32-deep k-steps keep the 32x32x16 form: their
-  // launches are bound by the operand stream, and the 16x16 form measured even or 2-3 % slower there (a 256-row gated
-  // unit on 256x256x32: 117.1 against 114.2 us).
+  // The 32x32x16 form stays where the 16x16 one measured slower (before and after going back to 32x32, caches flushed
+  // in front of every pass):
+  //  * a 4-wave workgroup that has its CU to itself: one wave per SIMD has nobody to cover a fragment read it waits for,
+  //    and a 16x16 atom waits for twice the bytes before its first MFMA. 128x256x64 on 2x2 waves, 8 groups of 2048 rows,
+  //    k = n = 4096: 701 -> 561 us (981 TFLOP/s); one group of 256 rows, k = 8192, n = 1024: 142 -> 106; 128x128x64 with
+  //    four stages, the first shape: 724 -> 641.
+  //  * d rhs: both fragments come through transposing reads, two to a 16-byte half, with no block order that keeps all of
+  //    them four blocks ahead. One group of 16574 rows, 128x128x64: 169 -> 159 us (warm 163 -> 117); 256x256x64, 8192
+  //    rows, k = n = 2048: 185 -> 165.
+  //  * wave tiles of fewer than four blocks and classic pipelines with 32-deep k-steps, whose launches are bound by the
+  //    operand stream: even or 2-3 % slower.
   static constexpr bool kColsOuter = TM >= 4 || TN < 4;
   static constexpr int NI = kColsOuter ? TM : TN, NO = kColsOuter ? TN : TM;
   static constexpr bool kDoubleInner = NI < 4, kDoubleOuter = (NO - 1) * NI < 4;
-  static constexpr bool M16 = (EA == kEBF16 || EA == kEF16) && EB == EA && TM * TN >= 4 && (BKC % 64 == 0 || SPLIT);
+  static constexpr bool M16 = (EA == kEBF16 || EA == kEF16) && EB == EA && TM * TN >= 4 && (BKC % 64 == 0 || SPLIT) &&
+                              MODE != kDrhs &&
+                              (THREADS > 256 || 2 * NS * (BM + BN) * BK * 2 <= 160 * 1024 /* two on a CU, see kWorkgroupsPerCu */);
   static constexpr int FA_COPIES = (kColsOuter ? kDoubleInner : kDoubleOuter) ? 2 : 1;
   static constexpr int FB_COPIES = (kColsOuter ? kDoubleOuter : kDoubleInner) ? 2 : 1;
   static constexpr int KA = Mma<EC, M16>::KA;
