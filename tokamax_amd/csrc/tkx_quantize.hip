@@ -30,23 +30,36 @@ template <> struct XVec<kEF32> { static constexpr int BYTES = 32; };
 template <> struct XVec<kEBF16> { static constexpr int BYTES = 16; };
 template <> struct XVec<kEF16> { static constexpr int BYTES = 16; };
 
-// 8 consecutive elements of x as f32.
+// 8 consecutive elements of x as they lie in memory, and as f32.
+template <int EX> struct Raw8 { i32x4 w[XVec<EX>::BYTES / 16]; };
 template <int EX>
-__device__ __forceinline__ void load8(const unsigned char* p, float (&v)[8]) {
-  if constexpr (EX == kEF32) {
-    const f32x4 a = *reinterpret_cast<const f32x4*>(p), b = *reinterpret_cast<const f32x4*>(p + 16);
+__device__ __forceinline__ Raw8<EX> load_raw8(const unsigned char* p) {
+  Raw8<EX> r;
 #pragma unroll
-    for (int e = 0; e < 4; ++e) { v[e] = a[e]; v[4 + e] = b[e]; }
+  for (int h = 0; h < XVec<EX>::BYTES / 16; ++h) r.w[h] = *reinterpret_cast<const i32x4*>(p + 16 * h);
+  return r;
+}
+template <int EX>
+__device__ __forceinline__ void widen8(const Raw8<EX>& r, float (&v)[8]) {
+  if constexpr (EX == kEF32) {
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const f32x4 a = __builtin_bit_cast(f32x4, r.w[h]);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) v[4 * h + e] = a[e];
+    }
   } else if constexpr (EX == kEBF16) {
-    const bf16x8 a = *reinterpret_cast<const bf16x8*>(p);
+    const bf16x8 a = __builtin_bit_cast(bf16x8, r.w[0]);
 #pragma unroll
     for (int e = 0; e < 8; ++e) v[e] = (float)a[e];
   } else {
-    const f16x8 a = *reinterpret_cast<const f16x8*>(p);
+    const f16x8 a = __builtin_bit_cast(f16x8, r.w[0]);
 #pragma unroll
     for (int e = 0; e < 8; ++e) v[e] = (float)a[e];
   }
 }
+template <int EX>
+__device__ __forceinline__ void load8(const unsigned char* p, float (&v)[8]) { widen8<EX>(load_raw8<EX>(p), v); }
 
 __device__ __forceinline__ float absmax8(const float (&v)[8]) {
   float m = 0.f;
@@ -111,6 +124,7 @@ __device__ __forceinline__ i32x2 quantize8(const float (&v)[8], float s, bool ne
 #pragma unroll
     for (int e = 0; e < 8; ++e) q[e] = quotient(v[e], s, r);
   } else {
+    asm volatile("");  // (a branch: without it both sides are computed and selected from)
 #pragma unroll
     for (int e = 0; e < 8; ++e) q[e] = v[e] / s;
   }
@@ -120,26 +134,30 @@ __device__ __forceinline__ i32x2 quantize8(const float (&v)[8], float s, bool ne
 // Tiles one row tall. L lanes (a power of two <= 64) own one tile; a wave holds 64 / L tiles of consecutive
 // (row, column-tile) pairs. CH > 0: tiles of at most 8 L CH columns, held in registers (every chunk of 8 loaded before
 // the first is used), U such sets of tiles at a time: x is read once, with CH * U 16-byte loads of a lane in flight.
-// CH == 0: wider tiles, walked twice. Bound by HBM. bf16 to fp8, before (every tile walked twice with one load in flight,
-// the IEEE division) and now: 8192 x 7168 per 128 columns 59.5 -> 48.6 us (3.6 TB/s), 8192 x 4096 per row 34 -> 29 us
-// (3.5 TB/s).
+// CH == 0: wider tiles, walked twice. Bound by HBM, so the chunks are held as they lie in memory (4 registers per 8
+// 16-bit elements; as f32 the 16-chunk form took 217 registers, two waves per SIMD, and lost up to 27 % to walking a tile
+// twice). bf16 to fp8, every tile walked twice against this form, caches flushed in front of every pass: 16384 x 7168 per
+// row 94.9 -> 62.7 us (5.6 TB/s), per 128 columns 104 -> 76.9 (4.6 TB/s), 16384 x 4096 per row 56.7 -> 37.0 (5.4 TB/s).
 template <int EX, int EQ, int CH, int U>
 __global__ __launch_bounds__(kQThreads) void quantize_rows_kernel(const unsigned char* __restrict__ x,
                                                                   unsigned char* __restrict__ q, float* __restrict__ scale,
-                                                                  int64_t rows, int32_t cols, int32_t t_c, int32_t L,
+                                                                  int64_t rows, int32_t cols, int32_t t_c, int32_t lanes,
                                                                   QuantRange qmax) {
   constexpr int XB = XVec<EX>::BYTES;  // bytes of 8 elements of x
+  const int L = CH == 1 ? lanes : 64;  // (a tile of more chunks than lanes has a whole wave: constant distances)
   const int lane = threadIdx.x & 63;
   const int tiles_per_row = cols / t_c;
   const int64_t num_tiles = rows * tiles_per_row;
   const int per_wave = 64 / L;
-  const int64_t wave_id = ((int64_t)blockIdx.x * kQThreads + threadIdx.x) >> 6;
+  int64_t wave_id = ((int64_t)blockIdx.x * kQThreads + threadIdx.x) >> 6;
+  if constexpr (CH != 1) wave_id = (int64_t)blockIdx.x * (kQThreads / 64) + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int64_t num_waves = ((int64_t)gridDim.x * kQThreads) >> 6;
   const int sub = lane / L, l = lane % L;
   const int chunks = t_c / 8;
   for (int64_t t0 = wave_id * per_wave * U; t0 < num_tiles; t0 += num_waves * per_wave * U) {
     float m[U];
-    float v[U][CH > 0 ? CH : 1][8];
+    Raw8<EX> held[U][CH > 0 ? CH : 1];
+    float v[8];
 #pragma unroll
     for (int u = 0; u < U; ++u) {
       // (Tile t's columns begin at element t * t_c: tiles are one row tall and whole in their rows.)
@@ -150,14 +168,13 @@ __global__ __launch_bounds__(kQThreads) void quantize_rows_kernel(const unsigned
 #pragma unroll
         for (int i = 0; i < CH; ++i) {
           const int c = l + i * L;
-#pragma unroll
-          for (int e = 0; e < 8; ++e) v[u][i][e] = 0.f;
-          if (tile < num_tiles && c < chunks) load8<EX>(xr + (int64_t)c * XB, v[u][i]);
+          held[u][i] = Raw8<EX>{};
+          if (tile < num_tiles && c < chunks) held[u][i] = load_raw8<EX>(xr + (int64_t)c * XB);
         }
       } else if (tile < num_tiles) {
         for (int c = l; c < chunks; c += L) {
-          load8<EX>(xr + (int64_t)c * XB, v[u][0]);
-          m[u] = fmaxf(m[u], absmax8(v[u][0]));
+          load8<EX>(xr + (int64_t)c * XB, v);
+          m[u] = fmaxf(m[u], absmax8(v));
         }
       }
     }
@@ -166,7 +183,10 @@ __global__ __launch_bounds__(kQThreads) void quantize_rows_kernel(const unsigned
       const int64_t tile = t0 + u * per_wave + sub;
       if constexpr (CH > 0) {
 #pragma unroll
-        for (int i = 0; i < CH; ++i) m[u] = fmaxf(m[u], absmax8(v[u][i]));
+        for (int i = 0; i < CH; ++i) {
+          widen8<EX>(held[u][i], v);
+          m[u] = fmaxf(m[u], absmax8(v));
+        }
       }
 #pragma unroll
       for (int off = 32; off > 0; off >>= 1)
@@ -181,13 +201,14 @@ __global__ __launch_bounds__(kQThreads) void quantize_rows_kernel(const unsigned
 #pragma unroll
           for (int i = 0; i < CH; ++i) {
             const int c = l + i * L;
-            if (c < chunks) *reinterpret_cast<i32x2*>(qr + c * 8) = quantize8<EQ>(v[u][i], s, near, r, qmax);
+            widen8<EX>(held[u][i], v);
+            if (c < chunks) *reinterpret_cast<i32x2*>(qr + c * 8) = quantize8<EQ>(v, s, near, r, qmax);
           }
         } else {
           const unsigned char* xr = x + tile * t_c * (XB / 8);
           for (int c = l; c < chunks; c += L) {
-            load8<EX>(xr + (int64_t)c * XB, v[u][0]);
-            *reinterpret_cast<i32x2*>(qr + c * 8) = quantize8<EQ>(v[u][0], s, near, r, qmax);
+            load8<EX>(xr + (int64_t)c * XB, v);
+            *reinterpret_cast<i32x2*>(qr + c * 8) = quantize8<EQ>(v, s, near, r, qmax);
           }
         }
       }
