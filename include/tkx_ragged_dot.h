@@ -256,6 +256,11 @@ int32_t tkx_ragged_dot_drhs(const void* lhs, const void* dout, const int32_t* gr
                             void* workspace, int64_t m, int64_t k, int64_t n, int64_t num_groups,
                             int32_t dtype, int32_t out_dtype, const TkxConfig* config, tkx_stream_t stream);
 
+/* Which tile of out (group, row and column of tiles of block_m x block_n) workgroup `workgroup` of such a launch computes.
+ * A host function: the map the kernel uses, for tests and tools. */
+int32_t tkx_ragged_dot_drhs_tile(int64_t workgroup, int64_t k, int64_t n, int32_t block_m, int32_t block_n, int32_t* group,
+                                 int32_t* tile_row, int32_t* tile_column);
+
 /* Weights with several scale blocks along k (the scale tile (1, t_k, 1) with t_k < k of
  * pallas_mosaic_gpu_kernel_sm90_quant.py:91-97; quantization.py:80-83 for the dequantisation):
  *   out[g, kk, c] = qvalue[g, kk, c] * scale[g, kk / scale_block_k, c]

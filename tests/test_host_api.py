@@ -845,3 +845,20 @@ def test_gateup_tile_has_a_k_step_that_divides_the_contraction(k, groups):
   ba = op.bind(ShapeDtype((64, 40), dtype), ShapeDtype((1, 40, 256), dtype), group_sizes=ShapeDtype((1,), torch.int32),
                fuse_gateup_activation="silu")
   assert op._get_heuristics_config(ba).block_k
+
+
+# k, n, tile: dealt to the XCDs or in order. (The wide ones would fetch less than a tenth less and were slower dealt.)
+@pytest.mark.parametrize("k, n, block_m, block_n, dealt", [
+    (2048, 768, 256, 128, True), (1024, 1024, 256, 128, True), (1024, 1024, 128, 128, True), (1016, 12072, 128, 128, False),
+    (432, 8592, 128, 128, False), (432, 8592, 256, 128, False), (4096, 14336, 256, 256, False), (816, 608, 128, 128, False),
+    (100, 100, 128, 128, False)])
+def test_drhs_workgroups_reach_every_tile_once(k, n, block_m, block_n, dealt):
+  lib, groups = _lib.load(), 3
+  m_tiles, n_tiles = -(-k // block_m), -(-n // block_n)
+  out = [ctypes.c_int32() for _ in range(3)]
+  seen = []
+  for b in range(groups * m_tiles * n_tiles):
+    _lib.check(lib.tkx_ragged_dot_drhs_tile(b, k, n, block_m, block_n, *(ctypes.byref(x) for x in out)))
+    seen.append(tuple(x.value for x in out))
+  everything = [(g, r, c) for g in range(groups) for r in range(m_tiles) for c in range(n_tiles)]
+  assert sorted(seen) == everything and (seen != everything) == dealt

@@ -33,6 +33,7 @@ EXPORTED_SYMBOLS = (
     "tkx_ragged_dot_fwd_static_workspace",
     "tkx_ragged_dot_fwd_fused",
     "tkx_ragged_dot_drhs",
+    "tkx_ragged_dot_drhs_tile",
     "tkx_dequantize_weights",
     "tkx_dequantize",
     "tkx_dequantize_zero_point",
@@ -117,6 +118,9 @@ def _declare(lib):
                                            i32, i32, i32, cfgp, vp]
   lib.tkx_ragged_dot_drhs.restype = i32
   lib.tkx_ragged_dot_drhs.argtypes = [vp, vp, vp, vp, vp, i64, i64, i64, i64, i32, i32, cfgp, vp]
+  i32p = ctypes.POINTER(i32)
+  lib.tkx_ragged_dot_drhs_tile.restype = i32
+  lib.tkx_ragged_dot_drhs_tile.argtypes = [i64, i64, i64, i32, i32, i32p, i32p, i32p]
   lib.tkx_dequantize_weights.restype = i32
   lib.tkx_dequantize_weights.argtypes = [vp, vp, vp, i64, i64, i64, i64, i32, i32, vp]
   lib.tkx_dequantize.restype = i32

@@ -500,24 +500,42 @@ int32_t tkx_ragged_dot_fwd_fused(const void* lhs, const void* rhs, const int32_t
                   rhs_scale_blocks, config, stream);
 }
 
-// How a group's m_tiles x n_tiles tiles of d rhs are dealt to the 8 XCDs (GemmParams::xcd_rows). With `rows` XCDs along k
-// and 8 / rows along n, the L2s together fetch every row of the group 8 / rows times from lhs (k wide) and `rows` times
-// from dout (n wide); the split that fetches least, of those that deal every XCD the same number of tiles (0: none
-// does, and the tiles go to the XCDs in order). In order is 1 x 8 where n_tiles is a multiple of 8, which stays unless
-// another split fetches a fifth less. 32768 rows over 128 groups, k = 2048, n = 768 (8 x 6 tiles, 4 x 2 XCDs instead of
-// in order, which fetched twice as much): 213 -> 200 us; 4096 rows over 8 groups, k = 4096, n = 14336 stays in order.
+// How a group's m_tiles x n_tiles tiles of d rhs are dealt to the 8 XCDs (drhs_tile). With `rows` XCDs along k and
+// 8 / rows along n, the L2s together fetch every row of the group 8 / rows times from lhs (k wide) and `rows` times from
+// dout (n wide). In order, a row of tiles lies on min(8, n_tiles) XCDs and a column on as many as n_tiles leaves over by
+// 8, at most m_tiles. The split that fetches least of those that deal every XCD the same number of tiles is taken (else
+// 0, in order) if it fetches a fifth less than in order: neighbouring columns of out written at the same time by
+// neighbouring workgroups are worth something too. Caches flushed: 64 groups of 1000 rows, k = 2048, n = 768, bf16 (8 x 6
+// tiles, 4 x 2 XCDs, fetches half) 322 -> 218 us, k = n = 1024 192 -> 158; k = 432, n = 8592, f32, 64 groups of 400 rows
+// (4 x 68 tiles, would fetch 8 % less) 2026 in order, 2190 dealt; k = 1016, n = 12072, 24 groups of 4 rows (8 x 95, 7 %
+// less) 474 in order, 535 dealt.
 static int32_t drhs_xcd_rows(int64_t k, int64_t n, int32_t m_tiles, int32_t n_tiles) {
+  const int32_t across = n_tiles < 8 ? n_tiles : 8;
+  int32_t column = n_tiles % 8 == 0 ? 1 : n_tiles % 4 == 0 ? 2 : n_tiles % 2 == 0 ? 4 : 8;
+  if (column > m_tiles) column = m_tiles;
+  int64_t fetched = (across * k + column * n) * 4 / 5;
   int32_t best = 0;
-  int64_t fetched = 0;
-  if (n_tiles % 8 == 0) fetched = (8 * k + n) * 4 / 5;
   for (int32_t rows = 1; rows <= 8; rows *= 2) {
     const int64_t f = 8 / rows * k + rows * n;
-    if (m_tiles % rows == 0 && n_tiles % (8 / rows) == 0 && (fetched == 0 || f < fetched)) {
+    if (m_tiles % rows == 0 && n_tiles % (8 / rows) == 0 && f < fetched) {
       best = rows;
       fetched = f;
     }
   }
   return best;
+}
+
+int32_t tkx_ragged_dot_drhs_tile(int64_t workgroup, int64_t k, int64_t n, int32_t block_m, int32_t block_n, int32_t* group,
+                                 int32_t* tile_row, int32_t* tile_column) {
+  if (workgroup < 0 || workgroup > 0x7fffffffLL || k < 1 || n < 1 || k >= (1 << 21) || n >= (1 << 21) || block_m < 1 ||
+      block_n < 1 || !group || !tile_row || !tile_column)
+    return set_error(TKX_ERR_INVALID, "bad argument");
+  const int32_t m_tiles = (int32_t)((k + block_m - 1) / block_m), n_tiles = (int32_t)((n + block_n - 1) / block_n);
+  const DrhsTile t = drhs_tile((int32_t)workgroup, drhs_xcd_rows(k, n, m_tiles, n_tiles), m_tiles, n_tiles);
+  *group = t.group;
+  *tile_row = t.mt;
+  *tile_column = t.nt;
+  return TKX_OK;
 }
 
 int32_t tkx_ragged_dot_drhs(const void* lhs, const void* dout, const int32_t* group_sizes, void* out, void* workspace,

@@ -82,6 +82,28 @@ enum KernelMode { kFwd = 0, kDlhs = 1, kDrhs = 2, kFwdGlu = 3, kFwdSubK = 4 };
 // 8 chunks in 8 equal shorter ones.
 constexpr int32_t kXcdChunk = 32;
 
+// d rhs: the tile of workgroup b, of m_tiles x n_tiles in a group. Workgroup b runs on XCD b % 8. xcd_rows = 0: in order.
+// Else, of a group's tiles, an XCD takes every xcd_rows-th row and every (8 / xcd_rows)-th column of tiles, so that a
+// panel of lhs is fetched into 8 / xcd_rows L2s and one of dout into xcd_rows.
+struct DrhsTile { int32_t group, mt, nt; };
+__host__ __device__ inline DrhsTile drhs_tile(int32_t b, int32_t xcd_rows, int32_t m_tiles, int32_t n_tiles) {
+  const int32_t per_group = m_tiles * n_tiles;
+  DrhsTile t;
+  if (xcd_rows > 0) {
+    const int32_t log2_rows = __builtin_ctz(xcd_rows), xcd = b & 7, i = b >> 3, per_xcd = per_group >> 3;
+    t.group = i / per_xcd;
+    const int32_t r = i - t.group * per_xcd, across = (n_tiles << log2_rows) >> 3, row = r / across;
+    t.mt = (row << log2_rows) + (xcd & (xcd_rows - 1));
+    t.nt = ((r - row * across) << (3 - log2_rows)) + (xcd >> log2_rows);
+  } else {
+    t.group = b / per_group;
+    const int32_t r = b - t.group * per_group;
+    t.mt = r / n_tiles;
+    t.nt = r - t.mt * n_tiles;
+  }
+  return t;
+}
+
 struct GemmParams {
   const void* A;
   const void* B;
@@ -100,7 +122,7 @@ struct GemmParams {
   int32_t nb_ext;                   // columns of B (fwd/dlhs): n_ext, or 2 * n_ext for kFwdGlu
   int32_t num_groups;
   int32_t n_tiles, m_tiles;         // tiles along C columns; along C rows (drhs only)
-  int32_t xcd_rows;                 // drhs: XCDs along the rows of a group's tiles (8 / xcd_rows along its columns), or 0
+  int32_t xcd_rows;                 // drhs: see drhs_tile
   int32_t real_slots;               // fwd/dlhs: workgroups that may own a task tile (multiple of 8 * kXcdChunk)
   int32_t zero_wgs;                 // fwd/dlhs: workgroups after those that clear the rows of no group
   // Split of the last round (fwd/dlhs, split_k > 1): the launch's tiles beyond the last multiple of `split_cus` are

@@ -1017,24 +1017,10 @@ struct GemmKernel {
         if (part + 1 < parts) kc_end = min((int)((int64_t)steps * (part + 1) / parts) * BK, p.k_ext);
       }
     } else {
-      const int per_group = p.m_tiles * p.n_tiles;
-      int mt, nt;
-      if (p.xcd_rows > 0) {
-        // Workgroup b runs on XCD b % 8: of a group's tiles it takes every xcd_rows-th row and every (8 / xcd_rows)-th
-        // column of tiles, so that a panel of lhs is fetched into 8 / xcd_rows L2s and one of dout into xcd_rows.
-        const int log2_rows = __builtin_ctz(p.xcd_rows), xcd = b & 7, i = b >> 3, per_xcd = per_group >> 3;
-        group = i / per_xcd;
-        const int r = i - group * per_xcd, across = (p.n_tiles << log2_rows) >> 3, row = r / across;
-        mt = (row << log2_rows) + (xcd & (p.xcd_rows - 1));
-        nt = ((r - row * across) << (3 - log2_rows)) + (xcd >> log2_rows);
-      } else {
-        group = b / per_group;
-        const int r = b - group * per_group;
-        mt = r / p.n_tiles;
-        nt = r - mt * p.n_tiles;
-      }
-      row0 = mt * BM;
-      col0 = nt * BN;
+      const DrhsTile tile = drhs_tile(b, p.xcd_rows, p.m_tiles, p.n_tiles);
+      group = tile.group;
+      row0 = tile.mt * BM;
+      col0 = tile.nt * BN;
       act_start = row0;
       act_end = min(row0 + BM, p.m_ext);
       GroupScan<1, 1> sc;  // (rows only)
