@@ -193,6 +193,109 @@ def test_tiles_worked_out_from_group_sizes(num_groups, cfg, kind, device):
   assert torch.equal(out, want)
 
 
+def _rows_times_their_group(lhs, rhs, off, m, trans=False):
+  """f32 [m, n]: every row times the matrix of its group (rows [off[g], off[g + 1]) of those below m; others zero)."""
+  want = torch.zeros((m, rhs.shape[1 if trans else 2]), dtype=torch.float32, device=lhs.device)
+  for g in range(rhs.shape[0]):
+    lo, hi = min(int(off[g]), m), min(int(off[g + 1]), m)
+    if hi > lo:
+      want[lo:hi] = lhs[lo:hi].float() @ (rhs[g].float().t() if trans else rhs[g].float())
+  return want
+
+
+def _many_sizes(rng, num_groups, kind):
+  gs = rng.choice([0, 0, 1, 2, 31, 33], num_groups).astype(np.int32)
+  gs[rng.integers(0, num_groups, 4)] = (650, 2100, 300, 129)
+  gs[256:512] = 0  # (a whole chunk of empty groups)
+  gs[-1] = 130
+  if kind == "negative":
+    gs[rng.integers(0, num_groups, 3)] = -(2 ** 31)
+  off = O.group_offsets(gs)
+  return gs, off, max(int(off[-1]) - 300 if kind == "too many rows" else int(off[-1]) + 7, 1) // 4 * 4
+
+
+@pytest.mark.parametrize("num_groups", [385, 1025, 1280, 2051])
+@pytest.mark.parametrize("cfg", [hip_ops.KernelConfig(32, 128, 64, 1, 4, 4), hip_ops.KernelConfig(64, 128, 64, 2, 2, 4, grid_tile_width=3),
+                                 hip_ops.KernelConfig(128, 256, 64, 2, 4, 3, grid_tile_width=2), hip_ops.KernelConfig(256, 256, 64, 2, 4, 2, grid_tile_width=8),
+                                 hip_ops.KernelConfig(128, 128, 64, 2, 2, 4, split_k=4)])
+@pytest.mark.parametrize("kind", ["mixed", "negative", "too many rows"])
+def test_tasks_worked_out_in_front_of_launches_with_many_groups(num_groups, cfg, kind, device):
+  """Forward (from 1025 groups on) and dlhs (from 385 on) of so many groups take their tiles from a kernel in front of
+  the launch: chunks of 256 groups, full, empty and partial, spans of several widths. Exact products of small integers."""
+  rng = np.random.default_rng(num_groups)
+  k, n = 64, 264
+  gs, off, m = _many_sizes(rng, num_groups, kind)
+  lhs = torch.tensor(rng.integers(-2, 3, (m, k)), device=device).to(torch.bfloat16)
+  rhs = torch.tensor(rng.integers(-2, 3, (num_groups, k, n)), device=device).to(torch.bfloat16)
+  dout = torch.tensor(rng.integers(-2, 3, (m, n)), device=device).to(torch.bfloat16)
+  gst = torch.tensor(gs, device=device)
+  out = hip_ops.ragged_dot_fwd(lhs, rhs, gst, config=cfg, out_dtype=torch.float32)
+  assert torch.equal(out, _rows_times_their_group(lhs, rhs, off, m))
+  out = hip_ops.ragged_dot_fwd(dout, rhs, gst, config=cfg, out_dtype=torch.float32, trans_rhs=True)
+  assert torch.equal(out, _rows_times_their_group(dout, rhs, off, m, trans=True))
+
+
+@pytest.mark.parametrize("num_groups", [385, 512, 1281])
+@pytest.mark.parametrize("kind", ["mixed", "negative", "too many rows"])
+def test_drhs_of_many_groups(num_groups, kind, device):
+  """d rhs of more than 384 groups reads the groups' rows from a kernel in front of it. Exact products of small integers."""
+  rng = np.random.default_rng(num_groups)
+  k, n = 72, 136
+  gs, off, m = _many_sizes(rng, num_groups, kind)
+  lhs = torch.tensor(rng.integers(-2, 3, (m, k)), device=device).to(torch.bfloat16)
+  dout = torch.tensor(rng.integers(-2, 3, (m, n)), device=device).to(torch.bfloat16)
+  got = hip_ops.ragged_dot_drhs(lhs, dout, torch.tensor(gs, device=device), num_groups,
+                                config=hip_ops.KernelConfig(128, 128, 64, 2, 2, 4), out_dtype=torch.float32)
+  for g in range(num_groups):
+    lo, hi = min(int(off[g]), m), min(int(off[g + 1]), m)
+    assert torch.equal(got[g], lhs[lo:hi].float().t() @ dout[lo:hi].float()), g
+
+
+@pytest.mark.parametrize("sizes, offset, local", [(2000, 1500, 40), (2000, 0, 300), (1300, 1290, 40), (4000, 700, 1100),
+                                                  (1500, -20, 64), (1500, 1500, 8)])
+def test_group_offset_behind_many_groups(sizes, offset, local, device):
+  """An expert-parallel shard of a job of more than 1024 groups: its first group anywhere, also outside the sizes."""
+  rng = np.random.default_rng(sizes + offset)
+  k, n = 64, 136
+  gs, _, m = _many_sizes(rng, sizes, "mixed")
+  mine = np.array([gs[j] if 0 <= j < sizes else 0 for j in range(offset, offset + local)], np.int64)
+  off = int(gs[:max(min(offset, sizes), 0)].astype(np.int64).sum()) + np.concatenate([[0], np.cumsum(mine)])
+  lhs = torch.tensor(rng.integers(-2, 3, (m, k)), device=device).to(torch.bfloat16)
+  rhs = torch.tensor(rng.integers(-2, 3, (local, k, n)), device=device).to(torch.bfloat16)
+  out = hip_ops.ragged_dot_fwd(lhs, rhs, torch.tensor(gs, device=device), config=hip_ops.KernelConfig(32, 128, 64, 1, 4, 4),
+                               out_dtype=torch.float32, group_offset=torch.tensor([offset], dtype=torch.int32, device=device))
+  assert torch.equal(out, _rows_times_their_group(lhs, rhs, off, m))
+
+
+def test_many_groups_of_int8_rows_with_scales_per_block(device):
+  """The kernels that fetch a tile's lhs scales four rows at a time start their tiles at multiples of four rows, also
+  where a kernel in front works the tiles out. Exact products of small integers, scales of powers of two."""
+  rng = np.random.default_rng(3)
+  num_groups, k, n = 1100, 256, 256
+  gs, off, m = _many_sizes(rng, num_groups, "mixed")
+  lhs = torch.tensor(rng.integers(-2, 3, (m, k)), device=device).to(torch.int8)
+  rhs = torch.tensor(rng.integers(-2, 3, (num_groups, k, n)), device=device).to(torch.int8)
+  lhs_scale = torch.tensor(2.0 ** rng.integers(-2, 3, m), device=device, dtype=torch.float32)
+  for variant in hip._variant_table()[(4, _lib.TKX_I8, _lib.TKX_I8)]:
+    out = hip_ops.ragged_dot_fwd(lhs, rhs, torch.tensor(gs, device=device), config=hip.Config(*variant).to_kernel_config(),
+                                 out_dtype=torch.float32, lhs_scale=lhs_scale,
+                                 rhs_scale=torch.ones((num_groups, 2, n), device=device))
+    assert torch.equal(out, _rows_times_their_group(lhs, rhs, off, m) * lhs_scale[:, None])
+
+
+def test_many_f32_workgroups(device):
+  """f32 launches of more than 8192 workgroups take their tiles from a kernel in front, with few groups too."""
+  rng = np.random.default_rng(4)
+  gs = np.array([0, 30000, 1, 40017, 0, 333], np.int32)
+  off, m, k, n = O.group_offsets(gs), int(gs.sum()) + 40, 32, 520
+  lhs = torch.tensor(rng.integers(-2, 3, (m, k)), device=device).to(torch.float32)
+  rhs = torch.tensor(rng.integers(-2, 3, (len(gs), k, n)), device=device).to(torch.float32)
+  for width in (1, 8):
+    out = hip_ops.ragged_dot_fwd(lhs, rhs, torch.tensor(gs, device=device), out_dtype=torch.float32,
+                                 config=hip_ops.KernelConfig(32, 128, 32, 1, 4, 4, grid_tile_width=width))
+    assert torch.equal(out, _rows_times_their_group(lhs, rhs, off, m))
+
+
 def test_padded(device):
   a, b, gs = _inputs("test_padded", 8, 1024, 128, 256, torch.bfloat16, device, random_groups=True)
   out = tokamax_amd.ragged_dot(a, b, torch.tensor(gs, device=device), preferred_element_type=torch.float32)

@@ -128,6 +128,19 @@ int32_t launch(const Variant* v, const GemmParams& p, int64_t grid, hipStream_t 
   return TKX_OK;
 }
 
+// Whether a kernel in front of a GEMM launch works out its tasks (launch_plan, 5 us and a gap) instead of every wave for
+// itself: with more groups than a few scans of 256 cover, more sizes in front of the first group than a wave adds up in
+// the same time, or, for f32, many workgroups (its tiles are short: the scan is a few percent of a workgroup). us for
+// scans and for the kernel, caches flushed. Forward, 64 rows a group, k = 512, n = 1024, bf16: 768 groups 176 / 179, 1024
+// 236 / 233, 2048 510 / 454, 4096 1224 / 896; dlhs, 32 rows, k = 1024, n = 512: 272 groups 75 / 73, 512 132 / 124, 2048
+// 634 / 432; d rhs of the first: 384 groups 150 / 149, 2048 841 / 748. 32 groups of 2048 rows behind 1500 others 30 / 28,
+// behind 4000 41 / 29. f32: 4096 workgroups even, 8095 764 / 756, 17809 772 / 733 (8 groups of 51572 rows, k = 592, n =
+// 1384), 37418 (k = 272) 921 / 880; 16-bit d rhs of up to 23000 workgroups within 2 % either way.
+bool plan_pays(KernelMode mode, int32_t dtype, int64_t num_groups, int64_t sizes_in_front, int64_t workgroups) {
+  const int64_t many = mode == kDlhs || mode == kDrhs ? 384 : 1024;
+  return num_groups <= kPlanGroups && (num_groups > many || sizes_in_front > 1024 || (dtype == TKX_F32 && workgroups > 8192));
+}
+
 bool valid_out_dtype(int d) { return d == TKX_F32 || d == TKX_BF16 || d == TKX_F16; }
 
 // Device address of `scratch` on the current device, looked up once per device (each GPU holds its own copy of
@@ -422,6 +435,13 @@ int32_t fwd_impl(const void* lhs, const void* rhs, const int32_t* group_sizes, c
   p.zero_wgs = (int32_t)zero_wgs;
   p.split_k = split_k;
   p.split_cus = 1;
+  if (plan_pays(dlhs ? kDlhs : kFwd, lhs_dtype, num_groups, group_offset != nullptr ? num_group_sizes : 0, slots)) {
+    p.plan = static_cast<const int32_t*>(workspace);
+    p.plan_stride = L.tid_size;
+    const bool four_rows = subk && (lhs_dtype == TKX_F8E4M3FN || lhs_dtype == TKX_I8);  // (see GemmKernel::run)
+    const int32_t st = launch_plan(p, false, c.block_m, 32 * c.waves_m, four_rows ? 4 : 1, static_cast<int32_t*>(workspace), stream);
+    if (st != TKX_OK) return st;
+  }
   int64_t split_wgs = 0;
   if (split_k > 1) {
     int cus = 0;
@@ -585,7 +605,13 @@ int32_t tkx_ragged_dot_drhs(const void* lhs, const void* dout, const int32_t* gr
   p.activation = TKX_ACT_NONE;
   p.split_k = 1;
   p.split_cus = 1;
-  return launch(v, p, (int64_t)num_groups * p.m_tiles * p.n_tiles, stream);
+  const int64_t workgroups = (int64_t)num_groups * p.m_tiles * p.n_tiles;
+  if (plan_pays(kDrhs, dtype, num_groups, 0, workgroups)) {
+    p.plan = static_cast<const int32_t*>(workspace);
+    const int32_t st = launch_plan(p, true, 0, 0, 1, static_cast<int32_t*>(workspace), stream);
+    if (st != TKX_OK) return st;
+  }
+  return launch(v, p, workgroups, stream);
 }
 
 int32_t tkx_dequantize_weights(const void* qvalue, const float* scale, void* out, int64_t num_groups, int64_t k,

@@ -71,6 +71,14 @@ int32_t launch_schedule(const int32_t* group_sizes, int64_t G, const int32_t* gr
 int32_t launch_clear_words(int32_t* words, int32_t count, hipStream_t stream);
 int32_t device_compute_units(int* out);
 
+// ---- tasks worked out in front of a GEMM launch -----------------------------------------------------
+constexpr int kPlanArrays = 6;
+constexpr int64_t kPlanGroups = 1 << 18;  // most groups launch_plan serves
+struct GemmParams;
+// Fills `plan` (int32 workspace of a call) for a launch with these parameters: `drhs`, or fwd/dlhs tiles of block_m rows
+// and units of `unit` rows whose first row is a multiple of `align` (1 or 4).
+int32_t launch_plan(const GemmParams& p, bool drhs, int32_t block_m, int32_t unit, int32_t align, int32_t* plan, hipStream_t stream);
+
 // ---- grouped GEMM -----------------------------------------------------------------------------
 // kFwdGlu = forward over weights [gate | up] ([g, k, 2 n_out]) with the epilogue act(gate) * up.
 // kFwdSubK = forward over int8 weights whose scales change along k ([g, k / t_k, n]): the scale row of a
@@ -113,6 +121,12 @@ struct GemmParams {
   const float* b_bias;   // per (group, column of B), added after the scales, or null
   float* c_scale;        // out_dtype fp8: f32 [m_ext, n_ext / 128], one scale per (row, 128 columns) of the result
   const int32_t* group_sizes;       // device, num_global entries; null: one group of all m_ext rows
+  // Null: every wave works its tile out from group_sizes (GroupScan). Else what launch_plan left: drhs: the first row of
+  // every group, and the end; fwd/dlhs: tasks, end of the last group, rows before the first one, then from kWsHeader on
+  // kPlanArrays arrays of plan_stride words, an entry per task: group, first row of the tile, first and end row of the
+  // task, first task and width of its span.
+  const int32_t* plan;
+  int32_t plan_stride;
   const int32_t* group_offset;      // device, one int32, or null: group g is entry offset + g of group_sizes
   int32_t num_global;
   int64_t lda, ldb, ldc;            // leading dimensions, elements

@@ -607,8 +607,9 @@ __device__ __forceinline__ int wave_scan(int x, int limit) {
 }
 
 // The row ranges and tile counts of 256 groups, four to a lane, as every wave of a GEMM launch works them out for itself
-// from the group sizes: one load and two scans of a few hundred cycles, no more than the dependent loads of a
-// precomputed schedule took, and no scheduler kernel in front of the launch (5.5 us and a launch gap per call).
+// from the group sizes: one load and two scans of a few hundred cycles, about what the dependent loads of a
+// precomputed schedule take, and no kernel in front of the launch (5.5 us and a launch gap per call). Calls with many
+// groups have such a kernel (GemmParams::plan): every 256 further groups cost every workgroup another scan.
 // Sizes are device data nobody has checked: each counts as 0 below 0, and rows at or past m do not exist.
 // A group's rows are cut into ceil(rows / BM) tasks of whole units of Q rows (32 rows for every row of waves), as even
 // as they come: the tasks of a group then run at one pace and share its weight panels in L2 to the end.
@@ -647,6 +648,21 @@ struct GroupScan {
     total = __builtin_amdgcn_readlane(tasks_upto, 63);
   }
 };
+
+// Task mt of a group of rows [start, end) that is cut into `tasks`: its tile's first row, its own first and end row.
+struct TaskRows { int row0, first, end; };
+template <int ALIGN>
+__device__ __forceinline__ TaskRows task_rows(int start, int end, int tasks, int mt, int unit) {
+  TaskRows t = {start & -ALIGN, start, end};
+  if (tasks > 1) {
+    const int units = (end - t.row0 + unit - 1) / unit;
+    const int base = units / tasks, more = units - base * tasks;  // the first `more` tasks are one unit taller
+    t.row0 += (mt * base + min(mt, more)) * unit;
+    t.end = min(t.row0 + (base + (mt < more ? 1 : 0)) * unit, end);
+    t.first = max(start, t.row0);
+  }
+  return t;
+}
 
 // ---- the kernel ---------------------------------------------------------------------------------
 // Calls f(integral_constant<int, sel>) for a run-time sel in [I, N].
@@ -882,6 +898,7 @@ struct GemmKernel {
     auto row_block = [&](int i) { return i * WM + wm; };
     const int b = blockIdx.x;
 
+    auto planned = [&](int i) { return __builtin_amdgcn_readfirstlane(p.plan[i]); };
     int group, row0, act_start, act_end, col0, kc_begin, kc_end;
     int part = 0, parts = 1, split_unit = 0;  // (fwd/dlhs) this workgroup contracts part `part` of `parts` of its tile
     if constexpr (MODE != kDrhs) {
@@ -889,14 +906,20 @@ struct GemmKernel {
       typedef GroupScan<BM, SUBP ? 4 : 1> Scan;
       const int offset = p.group_offset != nullptr ? __builtin_amdgcn_readfirstlane(p.group_offset[0]) : 0;
       int lead_rows = 0;  // rows of the groups in front of the first one of this call
-      if (p.group_offset != nullptr) {
-        int rows = 0;
-        for (int j = lane; j < min(max(offset, 0), p.num_global); j += 64) rows = min(rows + min(max(p.group_sizes[j], 0), p.m_ext), p.m_ext);
-        lead_rows = __builtin_amdgcn_readlane(wave_scan(rows, p.m_ext), 63);
-      }
       Scan sc;
-      sc.scan(p, p.m_ext, 0, offset, lane, lead_rows, 0);
-      for (int c = 256; c < p.num_groups; c += 256) sc.scan(p, p.m_ext, c, offset, lane, sc.rows, sc.total);
+      if (p.plan != nullptr) {
+        sc.total = min(planned(0), p.plan_stride);
+        sc.rows = planned(1);
+        lead_rows = planned(2);
+      } else {
+        if (p.group_offset != nullptr) {
+          int rows = 0;
+          for (int j = lane; j < min(max(offset, 0), p.num_global); j += 64) rows = min(rows + min(max(p.group_sizes[j], 0), p.m_ext), p.m_ext);
+          lead_rows = __builtin_amdgcn_readlane(wave_scan(rows, p.m_ext), 63);
+        }
+        sc.scan(p, p.m_ext, 0, offset, lane, lead_rows, 0);
+        for (int c = 256; c < p.num_groups; c += 256) sc.scan(p, p.m_ext, c, offset, lane, sc.rows, sc.total);
+      }
       const int num_tasks = sc.total;
       // Split of the last round: the launch's tiles beyond the last multiple of `split_cus` (a round of workgroups
       // that would leave most CUs idle) are cut along the contraction into `parts` parts. Part 0 is the tile's own
@@ -960,52 +983,58 @@ struct GemmKernel {
         if (L < first_split) parts = 1;
       }
       split_unit = (L - first_split) * parts + part;
-      // The group that owns list entry L (every task owns n_tiles entries), and the entry's place among the group's.
-      int chunk = 0;
-      if (p.num_groups > 256) {
-        sc.scan(p, p.m_ext, 0, offset, lane, lead_rows, 0);
-        while (L >= sc.total * p.n_tiles) sc.scan(p, p.m_ext, chunk += 256, offset, lane, sc.rows, sc.total);
-      }
-      const int owner = __builtin_ctzll(__ballot(L < sc.tasks_upto * p.n_tiles));
-      int tasks = 0, end = 0, first_task = __builtin_amdgcn_readlane(sc.tasks_upto, owner);
-      group = chunk + 4 * owner + 3;
+      int nt;
+      if (p.plan != nullptr) {
+        const int t0 = kWsHeader + L / p.n_tiles;  // some task of the span that holds L (every task owns n_tiles entries)
+        const int first = planned(4 * p.plan_stride + t0), width = planned(5 * p.plan_stride + t0);
+        const int rem = L - first * p.n_tiles;
+        nt = rem / width;
+        const int mt = kWsHeader + first + (rem - nt * width);
+        group = planned(mt);
+        row0 = planned(p.plan_stride + mt);
+        act_start = planned(2 * p.plan_stride + mt);
+        act_end = planned(3 * p.plan_stride + mt);
+      } else {
+        // The group that owns list entry L, and the entry's place among the group's.
+        int chunk = 0;
+        if (p.num_groups > 256) {
+          sc.scan(p, p.m_ext, 0, offset, lane, lead_rows, 0);
+          while (L >= sc.total * p.n_tiles) sc.scan(p, p.m_ext, chunk += 256, offset, lane, sc.rows, sc.total);
+        }
+        const int owner = __builtin_ctzll(__ballot(L < sc.tasks_upto * p.n_tiles));
+        int tasks = 0, end = 0, first_task = __builtin_amdgcn_readlane(sc.tasks_upto, owner);
+        group = chunk + 4 * owner + 3;
 #pragma unroll
-      for (int e = 3; e >= 0; --e) {  // (the lane's groups from its last one back)
-        if (e == 3 || L < first_task * p.n_tiles) {
-          group = chunk + 4 * owner + e;
-          tasks = __builtin_amdgcn_readlane(sc.tasks[e], owner);
-          act_start = __builtin_amdgcn_readlane(sc.start[e], owner);
-          end = __builtin_amdgcn_readlane(sc.end[e], owner);
-          first_task -= tasks;
+        for (int e = 3; e >= 0; --e) {  // (the lane's groups from its last one back)
+          if (e == 3 || L < first_task * p.n_tiles) {
+            group = chunk + 4 * owner + e;
+            tasks = __builtin_amdgcn_readlane(sc.tasks[e], owner);
+            act_start = __builtin_amdgcn_readlane(sc.start[e], owner);
+            end = __builtin_amdgcn_readlane(sc.end[e], owner);
+            first_task -= tasks;
+          }
         }
-      }
-      int rem = L - first_task * p.n_tiles, width = tasks, first = 0;
-      if (tasks > p.grid_tile_width) {
-        const int spans = (tasks + p.grid_tile_width - 1) / p.grid_tile_width;
-        const int base = tasks / spans, wider = tasks - base * spans;  // the first `wider` spans are one task wider
-        const int wide_entries = wider * (base + 1) * p.n_tiles;
-        width = base;
-        if (rem < wide_entries) {
-          width = base + 1;
-        } else {
-          rem -= wide_entries;
-          first = wider * (base + 1);
+        int rem = L - first_task * p.n_tiles, width = tasks, first = 0;
+        if (tasks > p.grid_tile_width) {
+          const int spans = (tasks + p.grid_tile_width - 1) / p.grid_tile_width;
+          const int base = tasks / spans, wider = tasks - base * spans;  // the first `wider` spans are one task wider
+          const int wide_entries = wider * (base + 1) * p.n_tiles;
+          width = base;
+          if (rem < wide_entries) {
+            width = base + 1;
+          } else {
+            rem -= wide_entries;
+            first = wider * (base + 1);
+          }
+          const int span = rem / (width * p.n_tiles);
+          rem -= span * width * p.n_tiles;
+          first += span * width;
         }
-        const int span = rem / (width * p.n_tiles);
-        rem -= span * width * p.n_tiles;
-        first += span * width;
-      }
-      const int nt = rem / width;
-      const int mt = first + (rem - nt * width);
-      row0 = act_start & -(SUBP ? 4 : 1);
-      act_end = end;
-      if (tasks > 1) {
-        constexpr int Q = WM * 32;  // rows of a unit
-        const int units = (end - row0 + Q - 1) / Q;
-        const int base = units / tasks, more = units - base * tasks;  // the first `more` tasks are one unit taller
-        row0 += (mt * base + min(mt, more)) * Q;
-        act_end = min(row0 + (base + (mt < more ? 1 : 0)) * Q, end);
-        act_start = max(act_start, row0);
+        nt = rem / width;
+        const TaskRows rows = task_rows<SUBP ? 4 : 1>(act_start, end, tasks, first + (rem - nt * width), WM * 32);
+        row0 = rows.row0;
+        act_start = rows.first;
+        act_end = rows.end;
       }
       col0 = nt * BNO;
       kc_begin = 0;
@@ -1023,12 +1052,17 @@ struct GemmKernel {
       col0 = tile.nt * BN;
       act_start = row0;
       act_end = min(row0 + BM, p.m_ext);
-      GroupScan<1, 1> sc;  // (rows only)
-      sc.scan(p, p.k_ext, 0, 0, lane, 0, 0);
-      for (int c = 256; c <= group; c += 256) sc.scan(p, p.k_ext, c, 0, lane, sc.rows, 0);
-      const int owner = (group & 255) >> 2, e = group & 3;
-      kc_begin = __builtin_amdgcn_readlane(e < 2 ? (e == 0 ? sc.start[0] : sc.start[1]) : (e == 2 ? sc.start[2] : sc.start[3]), owner);
-      kc_end = __builtin_amdgcn_readlane(e < 2 ? (e == 0 ? sc.end[0] : sc.end[1]) : (e == 2 ? sc.end[2] : sc.end[3]), owner);
+      if (p.plan != nullptr) {
+        kc_begin = planned(group);
+        kc_end = planned(group + 1);
+      } else {
+        GroupScan<1, 1> sc;  // (rows only)
+        sc.scan(p, p.k_ext, 0, 0, lane, 0, 0);
+        for (int c = 256; c <= group; c += 256) sc.scan(p, p.k_ext, c, 0, lane, sc.rows, 0);
+        const int owner = (group & 255) >> 2, e = group & 3;
+        kc_begin = __builtin_amdgcn_readlane(e < 2 ? (e == 0 ? sc.start[0] : sc.start[1]) : (e == 2 ? sc.start[2] : sc.start[3]), owner);
+        kc_end = __builtin_amdgcn_readlane(e < 2 ? (e == 0 ? sc.end[0] : sc.end[1]) : (e == 2 ? sc.end[2] : sc.end[3]), owner);
+      }
     }
 
     const unsigned char* Ab = reinterpret_cast<const unsigned char*>(p.A);

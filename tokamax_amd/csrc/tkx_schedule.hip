@@ -5,6 +5,7 @@
 // the number of tasks that belong to non-empty groups. For callers that want those arrays: the GEMM
 // kernels work out their tiles themselves (tkx_gemm.hip.h, GroupScan).
 #include "tkx_common.h"
+#include "tkx_gemm.hip.h"
 
 namespace tkx {
 namespace {
@@ -146,6 +147,127 @@ __global__ __launch_bounds__(kThreads) void schedule_kernel(const int32_t* __res
   }
 }
 
+// ---- the tasks of a GEMM launch -----------------------------------------------------------------------
+constexpr int kPlanThreads = 256, kPlanWaves = kPlanThreads / 64, kPlanChunks = (int)(kPlanGroups / 256);
+
+// a[0 .. n) += everything in front of it, and `first`: inclusive, saturating at `limit`. One wave.
+__device__ __forceinline__ void scan_in_place(int* a, int n, int first, int limit, int lane) {
+  for (int i = 0; i < n; i += 64) {
+    const int v = min(first + wave_scan(i + lane < n ? a[i + lane] : 0, limit), limit);
+    if (i + lane < n) a[i + lane] = v;
+    first = __builtin_amdgcn_readlane(v, 63);
+  }
+}
+
+// What the waves of a GEMM launch otherwise work out one by one (GroupScan), an entry per task: GemmParams::plan. For
+// launches with so many groups, or so many workgroups, that the work in every one of them costs more than a kernel in
+// front (launch order and row ranges are the same). Every workgroup adds up the groups in chunks of 256, then each wave
+// takes 64 tasks. DRHS: the rows of 256 groups per wave instead.
+template <int BM, int ALIGN, bool DRHS>
+__global__ __launch_bounds__(kPlanThreads) void plan_kernel(const GemmParams p, int32_t unit, int32_t* __restrict__ plan) {
+  __shared__ int rows_before[kPlanChunks + 1], tasks_before[kPlanChunks + 1];  // of every chunk
+  __shared__ int part[kPlanWaves];
+  __shared__ int upto[kPlanWaves][256], starts[kPlanWaves][256], ends[kPlanWaves][256];  // of a wave's current chunk
+  typedef GroupScan<BM, ALIGN> Scan;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int m = DRHS ? p.k_ext : p.m_ext, chunks = (p.num_groups + 255) / 256;
+  const int offset = p.group_offset != nullptr ? __builtin_amdgcn_readfirstlane(p.group_offset[0]) : 0;
+  // Rows of the groups in front of the first one.
+  int rows = 0;
+  for (int j = threadIdx.x; j < min(max(offset, 0), p.num_global); j += kPlanThreads) rows = min(rows + min(max(p.group_sizes[j], 0), m), m);
+  rows = wave_scan(rows, m);
+  if (lane == 63) part[wave] = rows;
+  for (int c = wave; c < chunks; c += kPlanWaves) {
+    Scan sc;
+    sc.scan(p, m, c * 256, offset, lane, 0, 0);
+    if (lane == 0) rows_before[c + 1] = sc.rows;
+  }
+  __syncthreads();
+  int lead = 0;
+  for (int w = 0; w < kPlanWaves; ++w) lead = min(lead + part[w], m);
+  if (wave == 0) {
+    if (lane == 0) rows_before[0] = lead;
+    scan_in_place(rows_before + 1, chunks, lead, m, lane);
+  }
+  __syncthreads();
+  if constexpr (DRHS) {
+    const int c = blockIdx.x * kPlanWaves + wave;
+    if (c < chunks) {
+      Scan sc;
+      sc.scan(p, m, c * 256, offset, lane, rows_before[c], 0);
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        if (c * 256 + 4 * lane + e < p.num_groups) plan[c * 256 + 4 * lane + e] = sc.start[e];
+      if (c == chunks - 1 && lane == 0) plan[p.num_groups] = sc.rows;
+    }
+  } else {
+    for (int c = wave; c < chunks; c += kPlanWaves) {
+      Scan sc;
+      sc.scan(p, m, c * 256, offset, lane, rows_before[c], 0);
+      if (lane == 0) tasks_before[c + 1] = sc.total;
+    }
+    __syncthreads();
+    if (wave == 0) {
+      if (lane == 0) tasks_before[0] = 0;
+      scan_in_place(tasks_before + 1, chunks, 0, 0x7fffffff, lane);
+    }
+    __syncthreads();
+    const int total = min(tasks_before[chunks], p.plan_stride);
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+      plan[0] = total;
+      plan[1] = rows_before[chunks];
+      plan[2] = lead;
+    }
+    const int first = (blockIdx.x * kPlanWaves + wave) * 64, last = min(first + 64, total), task = first + lane;
+    int32_t* const out = plan + kWsHeader;
+    for (int t = first; t < last;) {
+      // The chunk that owns task t: the first one that ends behind it.
+      int lo = 0, hi = chunks - 1;
+      while (lo < hi) {
+        const int mid = (lo + hi) >> 1;
+        if (tasks_before[mid + 1] > t) hi = mid;
+        else lo = mid + 1;
+      }
+      const int c = __builtin_amdgcn_readfirstlane(lo), before = tasks_before[c], behind = min(tasks_before[c + 1], last);
+      Scan sc;
+      sc.scan(p, m, c * 256, offset, lane, rows_before[c], before);
+      int at = sc.tasks_upto - (sc.tasks[0] + sc.tasks[1] + sc.tasks[2] + sc.tasks[3]);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        upto[wave][4 * lane + e] = at += sc.tasks[e];
+        starts[wave][4 * lane + e] = sc.start[e];
+        ends[wave][4 * lane + e] = sc.end[e];
+      }
+      __threadfence_block();
+      if (task >= t && task < behind) {
+        int g = 0, h = 255;  // the first group that ends behind this task
+        while (g < h) {
+          const int mid = (g + h) >> 1;
+          if (upto[wave][mid] > task) h = mid;
+          else g = mid + 1;
+        }
+        const int first_task = g == 0 ? before : upto[wave][g - 1], tasks = upto[wave][g] - first_task, mt = task - first_task;
+        const TaskRows r = task_rows<ALIGN>(starts[wave][g], ends[wave][g], tasks, mt, unit);
+        int span = 0, width = tasks;
+        if (tasks > p.grid_tile_width) {
+          const int spans = (tasks + p.grid_tile_width - 1) / p.grid_tile_width;
+          const int base = tasks / spans, wide = (tasks - base * spans) * (base + 1);  // the first spans are one task wider
+          width = mt < wide ? base + 1 : base;
+          span = mt < wide ? mt / width * width : wide + (mt - wide) / width * width;
+        }
+        out[task] = c * 256 + g;
+        out[p.plan_stride + task] = r.row0;
+        out[2 * p.plan_stride + task] = r.first;
+        out[3 * p.plan_stride + task] = r.end;
+        out[4 * p.plan_stride + task] = first_task + span;
+        out[5 * p.plan_stride + task] = width;
+      }
+      __threadfence_block();
+      t = behind;
+    }
+  }
+}
+
 __global__ __launch_bounds__(kThreads) void clear_words_kernel(int32_t* __restrict__ words, int32_t count) {
   for (int i = threadIdx.x; i < count; i += kThreads) words[i] = 0;
 }
@@ -155,6 +277,26 @@ __global__ __launch_bounds__(kThreads) void clear_words_kernel(int32_t* __restri
 // (a kernel, not a memset: callers may be capturing a graph)
 int32_t launch_clear_words(int32_t* words, int32_t count, hipStream_t stream) {
   clear_words_kernel<<<1, kThreads, 0, stream>>>(words, count);
+  TKX_HIP_CHECK(hipGetLastError());
+  return TKX_OK;
+}
+
+int32_t launch_plan(const GemmParams& p, bool drhs, int32_t block_m, int32_t unit, int32_t align, int32_t* plan, hipStream_t stream) {
+  if (p.num_groups > kPlanGroups) return set_error(TKX_ERR_UNSUPPORTED, "too many groups for the task kernel");
+  auto go = [&](auto kernel, int64_t items) {
+    kernel<<<dim3((unsigned)((items + kPlanThreads - 1) / kPlanThreads)), dim3(kPlanThreads), 0, stream>>>(p, unit, plan);
+  };
+  if (drhs) {
+    go(plan_kernel<1, 1, true>, (int64_t)(p.num_groups + 255) / 256 * 64);  // (a wave per 256 groups)
+  } else {
+#define TKX_PLAN(BM)                                                            \
+  if (block_m == BM) {                                                          \
+    if (align == 4) go(plan_kernel<BM, 4, false>, p.plan_stride);               \
+    else go(plan_kernel<BM, 1, false>, p.plan_stride);                          \
+  } else
+    TKX_PLAN(32) TKX_PLAN(64) TKX_PLAN(128) TKX_PLAN(256) return set_error(TKX_ERR_UNSUPPORTED, "no task kernel for block_m=%d", block_m);
+#undef TKX_PLAN
+  }
   TKX_HIP_CHECK(hipGetLastError());
   return TKX_OK;
 }
