@@ -248,6 +248,10 @@ int32_t tkx_ragged_dot_fwd_fused(const void* lhs, const void* rhs, const int32_t
                                  int32_t lhs_dtype, int32_t rhs_dtype, int32_t out_dtype, int32_t activation,
                                  int32_t gateup, const TkxConfig* config, tkx_stream_t stream);
 
+/* Which entry of a forward / TRANS_RHS launch's list of `tiles` tiles workgroup `workgroup` computes, or -1 (the launch
+ * has enough workgroups for every entry). A host function: the map the kernels use, for tests and tools. */
+int64_t tkx_ragged_dot_launch_order(int64_t workgroup, int64_t tiles);
+
 /* Part (4-drhs): out[G,k,n] = lhs[rows_g, k]^T . dout[rows_g, n], zeros for empty groups.
  * lhs [m,k], dout [m,n] row-major of `dtype` (f32/bf16/f16); out_dtype f32/bf16/f16.
  * Deterministic: one workgroup owns each output tile, no atomics. block_m/block_n of `config`

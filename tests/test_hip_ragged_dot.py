@@ -56,7 +56,7 @@ def _check(actual, expected, tol, rows=None):
 
 
 def _check_spans(ws, m, G, block_m, width, gs):
-  """Launch-order spans: consecutive tasks of one group, at most `width` wide, as even as possible."""
+  """The schedule kernel's spans: consecutive tasks of one group, at most `width` wide, as even as possible."""
   lib = _lib.load()
   tid = lib.tkx_ragged_dot_tid_size(m, G, block_m)
   arr = lambda which: ws[lib.tkx_ragged_dot_workspace_offset(m, G, block_m, which):][:tid].cpu().numpy()
@@ -140,7 +140,9 @@ def test_simple(dtype, device):
 
 
 @pytest.mark.parametrize("width", [1, 3, 8, 16])
-def test_launch_order_spans(width, device):
+def test_schedule_spans_and_products_of_any_width(width, device):
+  """The spans that the schedule kernel lays out for its callers (the products work theirs out themselves), and products
+  with spans of that width."""
   rng = np.random.default_rng(width)
   G, m, k, n = 9, 2048, 128, 256
   gs = np.array([300, 0, 129, 1, 640, 0, 7, 512, 130], np.int32)
@@ -2533,16 +2535,17 @@ def test_drhs_tiles_dealt_to_the_xcds(k, n, device):
     row += size
 
 
-@pytest.mark.parametrize("tiles", [1, 7, 8, 9, 31, 33, 112, 255, 257, 265])
+# (tasks of 128 rows, tiles a task owns): launches of 1, 7, 8, 9, 31 .. 33, 112, 255 .. 257, 264 and 265 tiles, and of 8,
+# 32, 256 and 264 from two tasks.
+@pytest.mark.parametrize("tasks, columns", [(1, t) for t in (1, 7, 8, 9, 31, 32, 33, 112, 255, 256, 257, 264, 265)] +
+                         [(2, t) for t in (4, 16, 128, 132)])
 @pytest.mark.parametrize("split_k", [1, 4])
-def test_tiles_behind_the_last_whole_round(tiles, split_k, device):
+def test_tiles_behind_the_last_whole_round(tasks, columns, split_k, device):
   """Launches whose last round holds any number of tiles, split along the contraction or not: every tile of the result
   against f64 sums (bf16 result: 2^-8 of the value, and f32 sums of 192 products)."""
-  rng = np.random.default_rng(tiles)
-  gs = np.array([5, 0, 130], np.int32)  # 3 tasks of 128 rows at most: 1 + 2 tiles a column
-  n = 128 * -(-tiles // 3) if tiles > 2 else 128
-  if tiles <= 2:
-    gs = np.array([0, 128 * tiles, 0], np.int32)
+  rng = np.random.default_rng(tasks * columns)
+  gs = np.array([128, 0, 0] if tasks == 1 else [5, 0, 128], np.int32)
+  n = 128 * columns
   m, k = int(gs.sum()), 192
   lhs = torch.tensor(rng.normal(0, 1, (m, k)).astype(np.float32), device=device).to(torch.bfloat16)
   rhs = torch.tensor(rng.normal(0, 1, (3, k, n)).astype(np.float32), device=device).to(torch.bfloat16)

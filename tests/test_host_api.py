@@ -804,20 +804,16 @@ def test_config_json_without_split_k_loads_with_the_default():
     hip.Config(16, 128, 32, 1, 4, 2, 1, 8, 1, -1)
 
 
-@pytest.mark.parametrize("total", [1, 2, 7, 8, 9, 31, 33, 255, 256, 257, 264, 511, 513])
+@pytest.mark.parametrize("total", [1, 2, 7, 8, 9, 31, 32, 33, 112, 255, 256, 257, 264, 265, 511, 512, 513])
 def test_launch_order_reaches_every_tile_once(total):
-  """The kernel's map from workgroups to list entries: whole rounds of 8 chunks of 32, and the entries behind them in 8
-  equal chunks, reach every entry exactly once from the workgroups that are launched."""
-  slots = -(-total // 256) * 256 + 256
-  seen = []
-  for b in range(slots):
-    idx, xcd = b >> 3, b & 7
-    first, at = idx // 32 * 256, idx % 32
-    share = min(32, (total - first + 7) >> 3)
-    entry = first + xcd * share + at
-    if at < share and entry < total:
-      seen.append(entry)
-  assert sorted(seen) == list(range(total))
+  """The kernels' map from workgroups to list entries reaches every entry exactly once from the workgroups that are
+  launched (whole rounds of 256), and gives every XCD its equal part of what is behind the last whole round."""
+  lib = _lib.load()
+  entries = [lib.tkx_ragged_dot_launch_order(b, total) for b in range(-(-total // 256) * 256)]
+  assert sorted(e for e in entries if e >= 0) == list(range(total))
+  behind = [sum(e >= total // 256 * 256 for e in entries[xcd::8]) for xcd in range(8)]
+  assert max(behind) == -(-(total % 256) // 8)
+  assert lib.tkx_ragged_dot_launch_order(-(-total // 256) * 256, total) == -1
 
 
 @pytest.mark.parametrize("rows, n2, block_m", [(1, 28672, 32), (64, 28672, 32), (100, 28672, 64), (256, 28672, 128),

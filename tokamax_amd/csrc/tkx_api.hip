@@ -130,15 +130,17 @@ int32_t launch(const Variant* v, const GemmParams& p, int64_t grid, hipStream_t 
 
 // Whether a kernel in front of a GEMM launch works out its tasks (launch_plan, 5 us and a gap) instead of every wave for
 // itself: with more groups than a few scans of 256 cover, more sizes in front of the first group than a wave adds up in
-// the same time, or, for f32, many workgroups (its tiles are short: the scan is a few percent of a workgroup). us for
-// scans and for the kernel, caches flushed. Forward, 64 rows a group, k = 512, n = 1024, bf16: 768 groups 176 / 179, 1024
+// the same time, or many workgroups, of which some have no task (d rhs, where all have: for f32, whose tiles are so short
+// that the scan is a few percent of a workgroup). us for scans and for the kernel, caches flushed. Forward, 64 rows a group, k = 512, n = 1024, bf16: 768 groups 176 / 179, 1024
 // 236 / 233, 2048 510 / 454, 4096 1224 / 896; dlhs, 32 rows, k = 1024, n = 512: 272 groups 75 / 73, 512 132 / 124, 2048
 // 634 / 432; d rhs of the first: 384 groups 150 / 149, 2048 841 / 748. 32 groups of 2048 rows behind 1500 others 30 / 28,
 // behind 4000 41 / 29. f32: 4096 workgroups even, 8095 764 / 756, 17809 772 / 733 (8 groups of 51572 rows, k = 592, n =
-// 1384), 37418 (k = 272) 921 / 880; 16-bit d rhs of up to 23000 workgroups within 2 % either way.
+// 1384), 37418 (k = 272) 921 / 880; 256 rows over 256 groups, Zipf, k = 1296, n = 10952, bf16, 11008 workgroups 461 / 451; 16-bit
+// d rhs of up to 23000 workgroups within 2 % either way.
 bool plan_pays(KernelMode mode, int32_t dtype, int64_t num_groups, int64_t sizes_in_front, int64_t workgroups) {
   const int64_t many = mode == kDlhs || mode == kDrhs ? 384 : 1024;
-  return num_groups <= kPlanGroups && (num_groups > many || sizes_in_front > 1024 || (dtype == TKX_F32 && workgroups > 8192));
+  return num_groups <= kPlanGroups && (num_groups > many || sizes_in_front > 1024 ||
+                                       (workgroups > 8192 && (mode != kDrhs || dtype == TKX_F32)));
 }
 
 bool valid_out_dtype(int d) { return d == TKX_F32 || d == TKX_BF16 || d == TKX_F16; }
@@ -230,8 +232,8 @@ int32_t tkx_ragged_dot_schedule_spans(const int32_t* group_sizes, int64_t num_gr
   if (block_m < 1 || align_tile < 1 || grid_tile_width < 1)
     return set_error(TKX_ERR_INVALID, "block_m, align_tile and grid_tile_width must be positive");
   const WsLayout L = ws_layout(m, num_groups, block_m);
-  return launch_schedule(group_sizes, num_groups, nullptr, num_groups, m, block_m, align_tile, grid_tile_width,
-                         static_cast<int32_t*>(workspace), L, static_cast<hipStream_t>(stream));
+  return launch_schedule(group_sizes, num_groups, block_m, align_tile, grid_tile_width, static_cast<int32_t*>(workspace), L,
+                         static_cast<hipStream_t>(stream));
 }
 
 }  // extern "C"
@@ -418,8 +420,12 @@ int32_t fwd_impl(const void* lhs, const void* rhs, const int32_t* group_sizes, c
   const int64_t out_block_n = gateup ? c.block_n / 2 : c.block_n;  // output columns of a tile
   p.n_tiles = (int32_t)((cols + out_block_n - 1) / out_block_n);
   p.m_tiles = 0;
+  // Tasks there can be: one for every group with rows, and one more for every whole tile of rows. (A workgroup without a
+  // task waits for a CU's LDS and looks at the group sizes before it knows: 32 rows over 256 groups, k = 1296, n = 10952,
+  // bf16, with workgroups for 256 tasks 154 us, for 32 140.)
+  const int64_t most_tasks = m < 1 ? 1 : (m + c.block_m - 1) / c.block_m + (num_groups < m ? num_groups : m) - 1;
   // Whole chunks for every XCD, so that each list entry has a workgroup (see the launch order in run()).
-  const int64_t slots = ((int64_t)L.tid_size * p.n_tiles + 8 * kXcdChunk - 1) / (8 * kXcdChunk) * (8 * kXcdChunk);
+  const int64_t slots = (most_tasks * p.n_tiles + 8 * kXcdChunk - 1) / (8 * kXcdChunk) * (8 * kXcdChunk);
   p.real_slots = (int32_t)slots;
   p.grid_tile_width = c.grid_tile_width;
   p.out_dtype = out_dtype;
@@ -437,7 +443,7 @@ int32_t fwd_impl(const void* lhs, const void* rhs, const int32_t* group_sizes, c
   p.split_cus = 1;
   if (plan_pays(dlhs ? kDlhs : kFwd, lhs_dtype, num_groups, group_offset != nullptr ? num_group_sizes : 0, slots)) {
     p.plan = static_cast<const int32_t*>(workspace);
-    p.plan_stride = L.tid_size;
+    p.plan_stride = (int32_t)most_tasks;
     const bool four_rows = subk && (lhs_dtype == TKX_F8E4M3FN || lhs_dtype == TKX_I8);  // (see GemmKernel::run)
     const int32_t st = launch_plan(p, false, c.block_m, 32 * c.waves_m, four_rows ? 4 : 1, static_cast<int32_t*>(workspace), stream);
     if (st != TKX_OK) return st;
@@ -535,7 +541,7 @@ static int32_t drhs_xcd_rows(int64_t k, int64_t n, int32_t m_tiles, int32_t n_ti
   if (column > m_tiles) column = m_tiles;
   int64_t fetched = (across * k + column * n) * 4 / 5;
   int32_t best = 0;
-  for (int32_t rows = 1; rows <= 8; rows *= 2) {
+  for (int32_t rows = 2; rows <= 8; rows *= 2) {  // (rows = 1 is the order itself)
     const int64_t f = 8 / rows * k + rows * n;
     if (m_tiles % rows == 0 && n_tiles % (8 / rows) == 0 && f < fetched) {
       best = rows;
@@ -543,6 +549,11 @@ static int32_t drhs_xcd_rows(int64_t k, int64_t n, int32_t m_tiles, int32_t n_ti
     }
   }
   return best;
+}
+
+int64_t tkx_ragged_dot_launch_order(int64_t workgroup, int64_t tiles) {
+  if (workgroup < 0 || tiles < 0 || workgroup > 0x7fffff00LL || tiles > 0x7fffff00LL) return -1;
+  return launch_order_entry((int32_t)workgroup, (int32_t)tiles);
 }
 
 int32_t tkx_ragged_dot_drhs_tile(int64_t workgroup, int64_t k, int64_t n, int32_t block_m, int32_t block_n, int32_t* group,

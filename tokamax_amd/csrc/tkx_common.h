@@ -9,9 +9,9 @@
 namespace tkx {
 
 // ---- workspace layout (int32 words) -----------------------------------------------------------
-// What tkx_ragged_dot_schedule fills; the GEMM entry points use the arrival counters and what lies behind them, in calls
-// with split_k > 1.
-// [0] num_tasks  [1] total_rows (end of the last group)  [2] rows before the first group  [kWsHeader ..) group_offsets[G+1]  then eight task arrays of
+// What tkx_ragged_dot_schedule fills; the GEMM entry points use the arrival counters and what lies behind them in calls
+// with split_k > 1, and the words in front of those in calls with a plan (GemmParams::plan, a layout of its own).
+// [0] num_tasks  [1] total_rows (end of the last group)  [2] 0  [kWsHeader ..) group_offsets[G+1]  then eight task arrays of
 // tid_size words each (group_id, block_start, actual_start, actual_end, start_within_block,
 // actual_size, span_first, span_width); every array starts on a 64-word boundary. The last two
 // are not part of the reference's schedule: they cut each group's tasks into spans of at most
@@ -62,12 +62,10 @@ int32_t set_error(int32_t code, const char* fmt, ...);
   } while (0)
 
 // ---- schedule -------------------------------------------------------------------------------------
-// The reference's task arrays (the GEMM kernels do not read them: every wave works out its own tile, GroupScan).
-// `group_offset` (device, one int32; null = 0): the G groups are entries [offset, offset + G) of the
-// `num_global` group sizes.
-int32_t launch_schedule(const int32_t* group_sizes, int64_t G, const int32_t* group_offset, int64_t num_global, int64_t m,
-                        int32_t block_m, int32_t align_tile, int32_t span_width, int32_t* ws, const WsLayout& L,
-                        hipStream_t stream);
+// The reference's task arrays, for callers that want them. The GEMM kernels do not read them: every wave works out its own
+// tile (GroupScan), or launch_plan does.
+int32_t launch_schedule(const int32_t* group_sizes, int64_t G, int32_t block_m, int32_t align_tile, int32_t span_width,
+                        int32_t* ws, const WsLayout& L, hipStream_t stream);
 int32_t launch_clear_words(int32_t* words, int32_t count, hipStream_t stream);
 int32_t device_compute_units(int* out);
 
@@ -89,6 +87,16 @@ enum KernelMode { kFwd = 0, kDlhs = 1, kDrhs = 2, kFwdGlu = 3, kFwdSubK = 4 };
 // tiles (the number of CUs of an XCD: one chunk is what an XCD runs at a time), the tiles behind the last whole round of
 // 8 chunks in 8 equal shorter ones.
 constexpr int32_t kXcdChunk = 32;
+
+// The entry of a launch's list of `total` tiles that workgroup b computes (fwd/dlhs), or -1: whole rounds of 8 chunks, then
+// what is behind them in 8 equal chunks. Workgroup b runs on XCD b % 8.
+__host__ __device__ inline int32_t launch_order_entry(int32_t b, int32_t total) {
+  const int32_t idx = b >> 3, xcd = b & 7;
+  const int32_t first = idx / kXcdChunk * (8 * kXcdChunk), at = idx % kXcdChunk;
+  const int32_t equal = (total - first + 7) >> 3, share = equal < kXcdChunk ? equal : kXcdChunk;
+  const int32_t entry = first + xcd * share + at;
+  return at < share && entry < total ? entry : -1;
+}
 
 // d rhs: the tile of workgroup b, of m_tiles x n_tiles in a group. Workgroup b runs on XCD b % 8. xcd_rows = 0: in order.
 // Else, of a group's tiles, an XCD takes every xcd_rows-th row and every (8 / xcd_rows)-th column of tiles, so that a

@@ -975,11 +975,8 @@ struct GemmKernel {
       // product of 8192 rows 279 -> 265; training step of 4096 rows over 8 groups 1575 -> 1462; 192 rows over int4
       // weights 77 -> 72.5.
       if (L < 0) {
-        const int idx = b >> 3, xcd = b & 7;
-        const int first = idx / kXcdChunk * (8 * kXcdChunk), at = idx % kXcdChunk;
-        const int share = min(kXcdChunk, (total - first + 7) >> 3);
-        L = first + xcd * share + at;
-        if (at >= share || L >= total) return;
+        L = launch_order_entry(b, total);
+        if (L < 0) return;
         if (L < first_split) parts = 1;
       }
       split_unit = (L - first_split) * parts + part;
