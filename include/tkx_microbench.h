@@ -19,6 +19,11 @@ int32_t tkxmb_mfma_bf16(const void* operands, int32_t iters, void* sink, void* s
 /* FLOP of one such launch on the current device. */
 int64_t tkxmb_mfma_bf16_flops(int32_t iters);
 
+/* The same loop on v_mfma_f32_16x16x32_bf16, four to a 32x32 block and 32 deep (the larger 16-bit tiles' form), and its
+ * FLOP per launch. */
+int32_t tkxmb_mfma_bf16_16x16(const void* operands, int32_t iters, void* sink, void* stream);
+int64_t tkxmb_mfma_bf16_16x16_flops(int32_t iters);
+
 /* The same loop on v_mfma_scale_f32_32x32x64_f8f6f4 with e4m3fn operands and no block scales (`operands`: 64 KB
  * of fp8 bytes), and its FLOP per launch. */
 int32_t tkxmb_mfma_fp8(const void* operands, int32_t iters, void* sink, void* stream);

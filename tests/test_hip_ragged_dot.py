@@ -2515,6 +2515,13 @@ def test_ceiling_probes_run_and_give_plausible_figures(device):
   assert 1.0 < alone < 9.0 and shared > 2 * alone, (alone, shared)
 
 
+def test_probe_of_the_16x16_matrix_instruction(device):
+  """The loop on 16x16x32 MFMAs stays below the published peak and slows down on random operands like the other form."""
+  from tokamax_amd import microbench
+  zeros, random = (microbench.mfma_bf16_tflops(data, device, iters=2000, form="16x16x32") for data in ("zeros", "random"))
+  assert 800 < random < zeros < 2600, (random, zeros)
+
+
 @pytest.mark.parametrize("k,n", [(2048, 768), (1024, 768), (2048, 128), (512, 256), (512, 512), (256, 1152), (768, 640)])
 def test_drhs_tiles_dealt_to_the_xcds(k, n, device):
   """d rhs whose tiles per group divide over the 8 XCDs in each of the ways the launch knows (and two that do not):

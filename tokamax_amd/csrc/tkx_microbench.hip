@@ -6,6 +6,8 @@
 //    published dense peak assumes the nominal shader clock; under a sustained MFMA load the clock settles lower, and
 //    how much lower depends on the operand bits (the same instruction stream runs about 30 % faster on all-zero
 //    operands than on random ones). A GEMM on real data is bounded by the random-data figure.
+//    tkxmb_mfma_bf16_16x16: the same on v_mfma_f32_16x16x32_bf16, four to a 32x32x32 block product, as the larger 16-bit
+//    tiles issue them.
 //  * tkxmb_operand_stream: the operand stream of a tiled GEMM without its arithmetic: workgroups stream HBM-resident
 //    panels into LDS with global_load_lds_dwordx4, `share` workgroups of one XCD reading the same panel at a time,
 //    as the tiles next to a GEMM tile share its operand panels through their XCD's L2.
@@ -55,6 +57,44 @@ __global__ __launch_bounds__(kThreads) void mfma_loop(const i32x4* src, float* o
     for (int j = 0; j < NB; ++j)
       for (int e = 0; e < 16; ++e) s += acc[i][j][e];
   if (s == 12345.f) out[0] = s;  // keeps the loop alive
+}
+
+// The same loop on 16x16x32 MFMAs: every 32x32 block is 2 x 2 of them, 32 deep, its fragments two halves of 16 rows
+// (columns).
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+__global__ __launch_bounds__(kThreads) void mfma16_loop(const i32x4* src, float* out, int iters) {
+  constexpr int NA = 4, NB = 2;
+  bf16x8 a[NA][2], b[NB][2];
+  for (int h = 0; h < 2; ++h) {
+    for (int i = 0; i < NA; ++i) a[i][h] = __builtin_bit_cast(bf16x8, src[(threadIdx.x * (1 + 2 * h) + kThreads * i + 77 * h) % kOperandWords]);
+    for (int i = 0; i < NB; ++i) b[i][h] = __builtin_bit_cast(bf16x8, src[(threadIdx.x * (7 - 2 * h) + kThreads * i + 1234 * (1 + h)) % kOperandWords]);
+  }
+  f32x4 acc[NA][NB][4];
+  for (int i = 0; i < NA; ++i)
+    for (int j = 0; j < NB; ++j)
+      for (int t = 0; t < 4; ++t) acc[i][j][t] = f32x4{0.f, 0.f, 0.f, 0.f};
+  for (int it = 0; it < iters; ++it) {
+#pragma unroll
+    for (int j = 0; j < NB; ++j)
+#pragma unroll
+      for (int i = 0; i < NA; ++i)
+#pragma unroll
+        for (int t = 0; t < 4; ++t)
+          acc[i][j][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b[j][t & 1], a[i][t >> 1], acc[i][j][t], 0, 0, 0);
+    if ((it & 3) == 3) {
+      for (int h = 0; h < 2; ++h) {
+        const bf16x8 t = a[0][h];
+        for (int i = 0; i + 1 < NA; ++i) a[i][h] = a[i + 1][h];
+        a[NA - 1][h] = t;
+      }
+    }
+  }
+  float s = 0;
+  for (int i = 0; i < NA; ++i)
+    for (int j = 0; j < NB; ++j)
+      for (int t = 0; t < 4; ++t)
+        for (int e = 0; e < 4; ++e) s += acc[i][j][t][e];
+  if (s == 12345.f) out[0] = s;
 }
 
 // The same loop on the fp8 (e4m3fn) form of the MFMA, 32x32x64 with 32-byte fragments and no block scales.
@@ -126,6 +166,16 @@ int32_t tkxmb_mfma_bf16(const void* operands, int32_t iters, void* sink, void* s
   int cus = 0;
   if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, 0) != hipSuccess) return 3;
   mfma_loop<<<cus, kThreads, 0, static_cast<hipStream_t>(stream)>>>(static_cast<const i32x4*>(operands), static_cast<float*>(sink), iters);
+  return hipGetLastError() == hipSuccess ? 0 : 3;
+}
+
+int64_t tkxmb_mfma_bf16_16x16_flops(int32_t iters) { return 2 * tkxmb_mfma_bf16_flops(iters); }  // blocks 32 deep, not 16
+
+int32_t tkxmb_mfma_bf16_16x16(const void* operands, int32_t iters, void* sink, void* stream) {
+  if (operands == nullptr || sink == nullptr || iters < 1) return 1;
+  int cus = 0;
+  if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, 0) != hipSuccess) return 3;
+  mfma16_loop<<<cus, kThreads, 0, static_cast<hipStream_t>(stream)>>>(static_cast<const i32x4*>(operands), static_cast<float*>(sink), iters);
   return hipGetLastError() == hipSuccess ? 0 : 3;
 }
 

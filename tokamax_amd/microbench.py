@@ -11,7 +11,8 @@ import os
 import torch
 
 LIB_PATH = os.path.join(os.path.dirname(os.path.abspath(__file__)), "lib", "libtkx_microbench.so")
-EXPORTED_SYMBOLS = ("tkxmb_mfma_bf16", "tkxmb_mfma_bf16_flops", "tkxmb_mfma_fp8", "tkxmb_mfma_fp8_flops", "tkxmb_operand_stream", "tkxmb_operand_stream_bytes")
+EXPORTED_SYMBOLS = ("tkxmb_mfma_bf16", "tkxmb_mfma_bf16_flops", "tkxmb_mfma_bf16_16x16", "tkxmb_mfma_bf16_16x16_flops",
+                    "tkxmb_mfma_fp8", "tkxmb_mfma_fp8_flops", "tkxmb_operand_stream", "tkxmb_operand_stream_bytes")
 
 _lib = None
 
@@ -25,6 +26,8 @@ def load():
     i32, i64, vp = ctypes.c_int32, ctypes.c_int64, ctypes.c_void_p
     lib.tkxmb_mfma_bf16.restype, lib.tkxmb_mfma_bf16.argtypes = i32, [vp, i32, vp, vp]
     lib.tkxmb_mfma_bf16_flops.restype, lib.tkxmb_mfma_bf16_flops.argtypes = i64, [i32]
+    lib.tkxmb_mfma_bf16_16x16.restype, lib.tkxmb_mfma_bf16_16x16.argtypes = i32, [vp, i32, vp, vp]
+    lib.tkxmb_mfma_bf16_16x16_flops.restype, lib.tkxmb_mfma_bf16_16x16_flops.argtypes = i64, [i32]
     lib.tkxmb_mfma_fp8.restype, lib.tkxmb_mfma_fp8.argtypes = i32, [vp, i32, vp, vp]
     lib.tkxmb_mfma_fp8_flops.restype, lib.tkxmb_mfma_fp8_flops.argtypes = i64, [i32]
     lib.tkxmb_operand_stream.restype, lib.tkxmb_operand_stream.argtypes = i32, [vp, i64, i32, i32, vp]
@@ -48,9 +51,12 @@ def _timed(launch, repeats: int) -> float:
   return sorted(times)[len(times) // 2]
 
 
-def mfma_bf16_tflops(data: str, device, iters: int = 20000, repeats: int = 3) -> float:
-  """TFLOP/s of the register-resident bf16 MFMA loop on operands that are all `"zeros"` or `"random"` (normal)."""
+def mfma_bf16_tflops(data: str, device, iters: int = 20000, repeats: int = 3, form: str = "32x32x16") -> float:
+  """TFLOP/s of the register-resident bf16 MFMA loop on operands that are all `"zeros"` or `"random"` (normal); `form`:
+  the instruction, `"32x32x16"` or `"16x16x32"` (whose iterations are twice as long)."""
   lib = load()
+  probe, flops = ((lib.tkxmb_mfma_bf16, lib.tkxmb_mfma_bf16_flops) if form == "32x32x16"
+                  else (lib.tkxmb_mfma_bf16_16x16, lib.tkxmb_mfma_bf16_16x16_flops))
   gen = torch.Generator(device=device).manual_seed(0)
   operands = (torch.zeros(32768, device=device, dtype=torch.bfloat16) if data == "zeros"
               else torch.randn(32768, device=device, generator=gen).to(torch.bfloat16))
@@ -58,10 +64,10 @@ def mfma_bf16_tflops(data: str, device, iters: int = 20000, repeats: int = 3) ->
   stream = torch.cuda.current_stream(device).cuda_stream
 
   def launch():
-    if lib.tkxmb_mfma_bf16(operands.data_ptr(), iters, sink.data_ptr(), stream) != 0:
-      raise RuntimeError("tkxmb_mfma_bf16 failed")
+    if probe(operands.data_ptr(), iters, sink.data_ptr(), stream) != 0:
+      raise RuntimeError("the bf16 MFMA probe failed")
 
-  return lib.tkxmb_mfma_bf16_flops(iters) / _timed(launch, repeats) / 1e9
+  return flops(iters) / _timed(launch, repeats) / 1e9
 
 
 def mfma_fp8_tflops(data: str, device, iters: int = 10000, repeats: int = 3) -> float:
