@@ -68,10 +68,11 @@ __device__ __forceinline__ void set4(Acc4& c, int t, f32x4 v) { c.q[t] = v; }
 
 // MFMA flavour chosen by the A element kind: contraction elements per 32x32 atom and fragment bytes.
 // M16 (bf16, f16): a 32x32 block is four 16x16x32 MFMAs, 32 deep, instead of one 32x32x16. Both forms have the same
-// nominal rate, but under a sustained load of random operands the chip's power limit sets the clock, and the 16x16
-// form spends less on its accumulators (a quarter of their register traffic per product): a register-resident loop
-// of it holds 1770 TFLOP/s on all CUs where 32x32x16 holds 1537, with two waves per SIMD. (fp8: 3330 against 3400
-// TFLOP/s for 16x16x128 and 32x32x64; those kernels keep the 32x32 form.) In the GEMM, whose other bound is the operand
+// nominal rate (and reach it on operands of zeros: 2160 and 2180 TFLOP/s), but under a sustained load of random operands
+// the chip's power limit sets the clock, and the 16x16 form spends less on its accumulators (a quarter of their register
+// traffic per product): a register-resident loop of it holds 1746-1786 TFLOP/s on all CUs where 32x32x16 holds 1542-1629,
+// with two waves per SIMD (tkx_microbench.hip, the two in turn). (fp8: 3330 against 3400 TFLOP/s for 16x16x128 and
+// 32x32x64; those kernels keep the 32x32 form.) In the GEMM, whose other bound is the operand
 // stream: the gate-up product of 16384 rows, k = 4096, 2 n = 28672 over 8 groups 3074 -> 2907 us (1325 TFLOP/s), the
 // down product 1560 -> 1484 us, a 256-expert prefill (65536 rows, k = 7168, n = 2048) 2289 -> 2192 us.
 template <int EA, bool M16 = false> struct Mma;
