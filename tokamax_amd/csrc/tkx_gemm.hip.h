@@ -899,6 +899,8 @@ struct GemmKernel {
     auto row_block = [&](int i) { return i * WM + wm; };
     const int b = blockIdx.x;
 
+    // (The ways that few launches take stand behind the kernel: with the plan's in the middle of the code in front of the
+    // first load, a training step of three kernels that take turns was 1 % slower, 535 against 530 us; this way even.)
     auto planned = [&](int i) { return __builtin_amdgcn_readfirstlane(p.plan[i]); };
     int group, row0, act_start, act_end, col0, kc_begin, kc_end;
     int part = 0, parts = 1, split_unit = 0;  // (fwd/dlhs) this workgroup contracts part `part` of `parts` of its tile
@@ -908,12 +910,12 @@ struct GemmKernel {
       const int offset = p.group_offset != nullptr ? __builtin_amdgcn_readfirstlane(p.group_offset[0]) : 0;
       int lead_rows = 0;  // rows of the groups in front of the first one of this call
       Scan sc;
-      if (p.plan != nullptr) {
+      if (__builtin_expect(p.plan != nullptr, 0)) {
         sc.total = min(planned(0), p.plan_stride);
         sc.rows = planned(1);
         lead_rows = planned(2);
       } else {
-        if (p.group_offset != nullptr) {
+        if (__builtin_expect(p.group_offset != nullptr, 0)) {
           int rows = 0;
           for (int j = lane; j < min(max(offset, 0), p.num_global); j += 64) rows = min(rows + min(max(p.group_sizes[j], 0), p.m_ext), p.m_ext);
           lead_rows = __builtin_amdgcn_readlane(wave_scan(rows, p.m_ext), 63);
@@ -972,9 +974,9 @@ struct GemmKernel {
       // share panels in their XCD's L2, and neighbouring chunks share the span's lhs panels in the
       // memory-side cache. The tiles behind the last whole round of 8 chunks go to the XCDs in 8 equal chunks: whole
       // ones would leave some XCDs, their L2s and their share of the way to memory idle (112 tiles: four of eight).
-      // Before and now: dense gated unit of 256 rows (112 tiles) 110 -> 101 us, of 17 rows 65.4 -> 39.8; 32-expert fp8
-      // product of 8192 rows 279 -> 265; training step of 4096 rows over 8 groups 1575 -> 1462; 192 rows over int4
-      // weights 77 -> 72.5.
+      // Before and now: dense gated unit of 256 rows on 256x256x32 (112 tiles) 110 -> 101 us, of 17 rows, k = 4096, 28672
+      // columns, on weights that the memory-side cache held 65.4 -> 39.8; 32-expert fp8 product of 8192 rows 279 -> 265;
+      // training step of 4096 rows over 8 groups 1575 -> 1462; 192 rows over int4 weights 77 -> 72.5.
       if (L < 0) {
         L = launch_order_entry(b, total);
         if (L < 0) return;
@@ -982,7 +984,7 @@ struct GemmKernel {
       }
       split_unit = (L - first_split) * parts + part;
       int nt;
-      if (p.plan != nullptr) {
+      if (__builtin_expect(p.plan != nullptr, 0)) {
         const int t0 = kWsHeader + L / p.n_tiles;  // some task of the span that holds L (every task owns n_tiles entries)
         const int first = planned(4 * p.plan_stride + t0), width = planned(5 * p.plan_stride + t0);
         const int rem = L - first * p.n_tiles;
@@ -995,7 +997,7 @@ struct GemmKernel {
       } else {
         // The group that owns list entry L, and the entry's place among the group's.
         int chunk = 0;
-        if (p.num_groups > 256) {
+        if (__builtin_expect(p.num_groups > 256, 0)) {
           sc.scan(p, p.m_ext, 0, offset, lane, lead_rows, 0);
           while (L >= sc.total * p.n_tiles) sc.scan(p, p.m_ext, chunk += 256, offset, lane, sc.rows, sc.total);
         }
@@ -1050,7 +1052,7 @@ struct GemmKernel {
       col0 = tile.nt * BN;
       act_start = row0;
       act_end = min(row0 + BM, p.m_ext);
-      if (p.plan != nullptr) {
+      if (__builtin_expect(p.plan != nullptr, 0)) {
         kc_begin = planned(group);
         kc_end = planned(group + 1);
       } else {
