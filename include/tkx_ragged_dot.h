@@ -83,7 +83,9 @@ typedef struct TkxConfig {
   int32_t waves_n;         /* wavefronts along n in a workgroup */
   int32_t grid_tile_width; /* most m-tasks (of one group) that share an n-panel in launch order (L2 reuse);
                               unused by the streaming small-m kernel (block_m == 16) */
-  int32_t align_tile;      /* task starts are aligned down to this many rows (reference default 8) */
+  int32_t align_tile;      /* >= 1. Row alignment of task starts in tkx_ragged_dot_schedule (reference default 8). The products
+                              start a group's first task at its first row, kernels that fold lhs scales in per k-block at
+                              the multiple of four rows below; those still decline a value that is no multiple of 4 */
   int32_t num_stages;      /* LDS stages of block_k contraction elements kept in flight */
   int32_t split_k;         /* workgroups that share the contraction of one output tile (the reference's split_k,
                               pallas_mosaic_gpu_common.py:53, pallas_triton.py:41-48). 0 and 1: no split. Above 1, on the
@@ -96,7 +98,7 @@ typedef struct TkxConfig {
                               result): only the tiles of the launch's last, partial round of workgroups are split, into
                               floor(CUs / their number) parts, at most split_k, so that a launch of 1.25 rounds costs
                               1.25 rounds instead of 2; `workspace` then is tkx_ragged_dot_split_workspace_bytes long and
-                              needs no clearing (the schedule kernel clears the counters). Parts are added in the order
+                              needs no clearing (a small kernel in front of the launch clears the counters). Parts are added in the order
                               of their index whoever arrives last: results are reproducible run to run. */
   int32_t persistent;      /* the reference's `persistent` (pallas_mosaic_gpu_common.py:55): resident workgroups that share
                               the work out evenly instead of one workgroup per tile and nothing else. 0: off. 1 (the
@@ -147,7 +149,7 @@ int64_t tkx_ragged_dot_tid_size(int64_t m, int64_t num_groups, int32_t block_m);
 /* Bytes of device workspace needed by schedule/fwd/drhs for these sizes (int32 arrays, 256-aligned). */
 int64_t tkx_ragged_dot_workspace_bytes(int64_t m, int64_t num_groups, int32_t block_m);
 
-/* Bytes of workspace of a tiled forward / TRANS_RHS call with config->split_k > 1: the schedule arrays, then one f32
+/* Bytes of workspace of a tiled forward / TRANS_RHS call with config->split_k > 1: room for the tasks and the arrival counters, then one f32
  * partial tile (block_m x block_n) for each of at most 256 parts. */
 int64_t tkx_ragged_dot_split_workspace_bytes(int64_t m, int64_t num_groups, int32_t block_m, int32_t block_n);
 
@@ -162,7 +164,8 @@ int64_t tkx_ragged_dot_workspace_offset(int64_t m, int64_t num_groups, int32_t b
 
 /* Part (1): group-offset prefix sum + tile schedule, one small kernel on `stream`.
  * group_sizes: device int32[G] (negative entries count as 0). Fills `workspace`. (For callers that want the reference's
- * arrays. The forward and backward kernels do not read them: every wave works out its own tile from group_sizes.) */
+ * arrays. The forward and backward entry points do not read them: every wave works out its own tile from group_sizes, or,
+ * with many groups, a small kernel in front of the launch leaves the tasks in the workspace, in a layout of its own.) */
 int32_t tkx_ragged_dot_schedule(const int32_t* group_sizes, int64_t num_groups, int64_t m, int32_t block_m,
                                 int32_t align_tile, void* workspace, tkx_stream_t stream);
 /* ... with launch-order spans of up to grid_tile_width tasks. */
@@ -202,12 +205,13 @@ int32_t tkx_ragged_dot_fwd_fp8_out(const void* lhs, const void* rhs, const int32
 
 /* tkx_ragged_dot_fwd for callers that cannot hand over a workspace they allocated: code under HIP graph capture,
  * tight serving loops, harnesses that forbid hipMalloc. It has no counterpart in the reference (XLA owns every buffer
- * there). Same arguments and results as tkx_ragged_dot_fwd, without `workspace`: the schedule arrays live in a
+ * there). Same arguments and results as tkx_ragged_dot_fwd, without `workspace`: its place is taken by a
  * 256 KiB device array inside the library (one copy per GPU, held until the process ends), which limits
  * tkx_ragged_dot_workspace_bytes(m, num_groups, block_m) to 262144, i.e. about cdiv(m, block_m) + num_groups <= 8100;
  * larger problems return TKX_ERR_UNSUPPORTED, and so does config->split_k > 1 (its arrival counters need a workspace
  * that was cleared). The call allocates and frees nothing. All calls on one GPU share that
- * array: two of them that overlap in time (different streams or threads) race; calls on one stream are ordered.
+ * array: two of them that overlap in time (different streams or threads) race where both write it (calls with many groups
+ * do, see tkx_ragged_dot_schedule); calls on one stream are ordered.
  * The first call on a device looks the array's address up (hipGetSymbolAddress), and the first call of a kernel on a
  * device raises that kernel's limit of dynamic LDS (hipFuncSetAttribute): both are remembered in fixed tables (no host
  * allocation either) and should happen outside capture, i.e. make one eager call per (device, config) first. */

@@ -37,7 +37,9 @@ class Config:
 
   (block_m, block_n, block_k, waves_m, waves_n, num_stages) selects a precompiled kernel variant;
   `grid_tile_width` m-tasks share one n-panel of rhs in launch order (L2 reuse);
-  `align_tile` is the row alignment of task starts (the reference's `align_tile`, default 8);
+  `align_tile` is the row alignment of task starts in the schedule the library lays out for callers that read it (the
+  reference's `align_tile`, default 8); the products start a group's first task at its first row (with lhs scales per
+  k-block: at the multiple of four rows below) whatever it says;
   `split_k` workgroups share the contraction of one output tile (the reference's field of that name): on the streaming
   small-m kernel (block_m == 16) every tile is split; on a tiled forward / dlhs kernel of at least 128 rows only the
   tiles of the launch's last, partial round of workgroups are, into at most that many parts;
@@ -1031,10 +1033,13 @@ class HipRaggedDot(base.RaggedDot):
     if mode == 3 and num_groups == 1 and key[1:] == (_lib.TKX_BF16, _lib.TKX_BF16):
       # Gate-up fusion over one group (the dense gated unit): the launch of the plain product over both halves' columns.
       # Its tiles are known exactly, start together and end together, so a partial last round counts in full. The rules
-      # above took the 256 x 256 x 32 tile from 224 rows on, however few tiles came of it. On 29 shapes (1 to 8192 rows,
-      # k = 2048 to 8192, 2816 to 28672 columns) this takes the fastest tile or one within 1.5 % of it; k = 4096, 28672
-      # columns: 256 rows 72.5 -> 53.2 us, 1024 rows 193 -> 175, 8192 rows 1431 -> 1308. (With several groups the rules stay:
-      # they are within a few percent on 26 shapes.)
+      # above took the 256 x 256 x 32 tile from 224 rows on, however few tiles came of it. On 119 shapes (1 to 8192 rows,
+      # seven widths of k = 1024 to 8192; weights rotated past the memory-side cache, as a layer's are) this takes the
+      # fastest tile or one within 1.5 % of it on 113, and one within 5.3 % on the others, where few 256-row tiles leave
+      # one round that the deeper pipeline of 256 x 256 x 32 streams faster. k = 4096, 28672 columns: 256 rows 93.6 -> 74.8
+      # us (74.4 -> 58.4 on weights the memory-side cache holds), 1024 rows 203 -> 194, 8192 rows 1488 -> 1362.
+      # With several groups the rules stay so far: on 40 shapes (2 to 256 groups, even and Zipf sizes, caches flushed) they
+      # are 7 % behind the fastest tile on average and 38 % at worst (2 groups of 150 rows), this model 2 % on average.
       fit = dict(_TILE_COST_FIT, tail_floor=1.0)
       bm, bn, bk, wm, wn, ns = min(usable, key=lambda v: (
           round(_tile_cost(v, 1, rows, cols, contraction, 1, 0, fit), 3), -v[2], -v[5]))
