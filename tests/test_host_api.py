@@ -804,15 +804,17 @@ def test_config_json_without_split_k_loads_with_the_default():
     hip.Config(16, 128, 32, 1, 4, 2, 1, 8, 1, -1)
 
 
-@pytest.mark.parametrize("total", [1, 2, 7, 8, 9, 31, 32, 33, 112, 255, 256, 257, 264, 265, 511, 512, 513])
+@pytest.mark.parametrize("total", [1, 2, 7, 8, 9, 31, 32, 33, 112, 255, 256, 257, 264, 265, 511, 512, 513, 3071, 3072,
+                                   3073, 4032])
 def test_launch_order_reaches_every_tile_once(total):
   """The kernels' map from workgroups to list entries reaches every entry exactly once from the workgroups that are
-  launched (whole rounds of 256), and gives every XCD its equal part of what is behind the last whole round."""
+  launched (whole rounds of 256), and gives every XCD its equal part of what is behind the last whole round in a launch
+  of at most 12 rounds, chunks of 32 in a longer one."""
   lib = _lib.load()
   entries = [lib.tkx_ragged_dot_launch_order(b, total) for b in range(-(-total // 256) * 256)]
   assert sorted(e for e in entries if e >= 0) == list(range(total))
   behind = [sum(e >= total // 256 * 256 for e in entries[xcd::8]) for xcd in range(8)]
-  assert max(behind) == -(-(total % 256) // 8)
+  assert max(behind) == (-(-(total % 256) // 8) if total <= 12 * 256 else min(total % 256, 32))
   assert lib.tkx_ragged_dot_launch_order(-(-total // 256) * 256, total) == -1
 
 

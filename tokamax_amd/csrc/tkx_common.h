@@ -84,16 +84,17 @@ int32_t launch_plan(const GemmParams& p, bool drhs, int32_t block_m, int32_t uni
 enum KernelMode { kFwd = 0, kDlhs = 1, kDrhs = 2, kFwdGlu = 3, kFwdSubK = 4 };
 
 // fwd/dlhs launch order: the tile list is dealt to the 8 XCDs in chunks of this many consecutive
-// tiles (the number of CUs of an XCD: one chunk is what an XCD runs at a time), the tiles behind the last whole round of
-// 8 chunks in 8 equal shorter ones.
-constexpr int32_t kXcdChunk = 32;
+// tiles (the number of CUs of an XCD: one chunk is what an XCD runs at a time). In a launch of at most kEqualTailRounds
+// rounds of 8 chunks the tiles behind the last whole round go out in 8 equal shorter chunks.
+constexpr int32_t kXcdChunk = 32, kEqualTailRounds = 12;
 
 // The entry of a launch's list of `total` tiles that workgroup b computes (fwd/dlhs), or -1: whole rounds of 8 chunks, then
-// what is behind them in 8 equal chunks. Workgroup b runs on XCD b % 8.
+// what is behind them, in 8 equal chunks if the launch is short. Workgroup b runs on XCD b % 8.
 __host__ __device__ inline int32_t launch_order_entry(int32_t b, int32_t total) {
   const int32_t idx = b >> 3, xcd = b & 7;
   const int32_t first = idx / kXcdChunk * (8 * kXcdChunk), at = idx % kXcdChunk;
-  const int32_t equal = (total - first + 7) >> 3, share = equal < kXcdChunk ? equal : kXcdChunk;
+  const int32_t equal = (total - first + 7) >> 3;
+  const int32_t share = total <= kEqualTailRounds * 8 * kXcdChunk && equal < kXcdChunk ? equal : kXcdChunk;
   const int32_t entry = first + xcd * share + at;
   return at < share && entry < total ? entry : -1;
 }

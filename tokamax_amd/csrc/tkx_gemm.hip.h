@@ -972,10 +972,14 @@ struct GemmKernel {
       // ceil(tasks / grid_tile_width) spans of nearly equal width); inside a span its m-tasks take
       // an n-panel of the group's weights back to back, then the next n-panel: the tiles of a chunk
       // share panels in their XCD's L2, and neighbouring chunks share the span's lhs panels in the
-      // memory-side cache. The tiles behind the last whole round of 8 chunks go to the XCDs in 8 equal chunks: whole
-      // ones would leave some XCDs, their L2s and their share of the way to memory idle (112 tiles: four of eight).
-      // Before and now: dense gated unit of 256 rows on 256x256x32 (112 tiles) 110 -> 101 us, of 17 rows, k = 4096, 28672
-      // columns, on weights that the memory-side cache held 65.4 -> 39.8; 32-expert fp8 product of 8192 rows 279 -> 265;
+      // memory-side cache. In a launch of few rounds the tiles behind the last whole round of 8 chunks go to the XCDs in
+      // 8 equal chunks: whole ones would leave some XCDs, their L2s and their share of the way to memory idle (112 tiles:
+      // four of eight). In a long one that is a small part, and the XCDs are not at the same point of the list by then.
+      // Whole and equal chunks, products of 7168 columns over k = 4096 in 256 x 256 tiles: 4.4 rounds bf16 516 and 495 us,
+      // int8 298 and 284; 7.9 rounds 16-bit ones 1 to 2 % apart; 15.8 rounds fp8 843 and 869, int8 917 and 927, the
+      // 16-bit ones alike. Between, at 8.8 and 10.5 rounds, both are within 1.5 %, the equal ones mostly the faster.
+      // Whole and equal chunks, short launches: dense gated unit of 256 rows on 256x256x32 (112 tiles) 110 -> 101 us, of
+      // 17 rows, k = 4096, 28672 columns, on weights that the memory-side cache held 65.4 -> 39.8; 32-expert fp8 product of 8192 rows 279 -> 265;
       // training step of 4096 rows over 8 groups 1575 -> 1462; 192 rows over int4 weights 77 -> 72.5.
       if (L < 0) {
         L = launch_order_entry(b, total);
