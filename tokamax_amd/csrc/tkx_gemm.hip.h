@@ -128,14 +128,18 @@ __device__ __forceinline__ f32x16 mma_atom(const typename Mma<EA>::Frag& first, 
 
 // ---- LDS tile addressing ------------------------------------------------------------------------
 // Contraction-contiguous tile: [rows][ROW_BYTES], 16-byte chunks XOR-swizzled by the row so that the
-// 16 lanes of one ds_read_b128 phase (16 consecutive rows, one chunk each: 256 bytes, every bank
-// once) touch distinct banks. A row covers CPR of the 16 chunk slots of a 256-byte bank line, so
-// the swizzle has to tell apart the 16 / CPR rows that start on the same slot: with 4 chunks per
-// row those are rows r, r + 4, r + 8, r + 12 (row bits 2 and 3), with 8 chunks per row r, r + 2, ...
+// 16 lanes of one ds_read_b128 phase (256 bytes, every bank once) touch distinct banks. A row covers CPR of the 16
+// chunk slots of a 256-byte bank line, so the swizzle has to tell apart the 16 / CPR rows that start on the same slot:
+// with 4 chunks per row those are rows r, r + 4, r + 8, r + 12 (row bits 2 and 3), with 8 chunks per row r, r + 2, ...,
+// r + 14 (row bits 1 to 3). A phase is not 16 consecutive lanes: it takes lanes from both of the 16-lane blocks of a
+// half-wave, which read one chunk of 32 rows in a 32x32 fragment, but chunks c and c ^ 1 of the same 16 rows in a 16x16
+// one. (row >> 1) & 7 keeps rows 2 r and 2 r + 1 on neighbouring values, so the chunks that c ^ 1 moves away from are the
+// ones it moves to, whichever rows the phase takes from which block.
 template <int ROW_BYTES>
 __device__ __forceinline__ int kc_swizzle(int row) {
   constexpr int CPR = ROW_BYTES / 16;
   if constexpr (CPR == 4) return (row >> 2) & 3;
+  else if constexpr (CPR == 8) return (row >> 1) & 7;
   else return ((row & 7) ^ ((row >> 3) & 1)) & (CPR - 1);
 }
 template <int ROW_BYTES>
@@ -144,13 +148,15 @@ __device__ __forceinline__ int kc_offset(int row, int chunk) {
 }
 
 // Row/column-contiguous tile: [BK rows of k][ROW_BYTES], 32-byte granules XOR-swizzled by k.
-// E selects the pattern that suits the read instruction used for that element size.
+// E selects the pattern that suits the read instruction used for that element size. 16-bit elements: the 32 lanes of a
+// transposing read's phase take 4 k-rows of two neighbouring granules in a 32x32 fragment, k-rows r .. r + 3 and
+// r + 8 .. r + 11 of one granule in a 16x16 one, hence row bits 0, 1 and 3.
 template <int ROW_BYTES, int E>
 __device__ __forceinline__ int mc_swizzle(int krow) {
   constexpr int NG = ROW_BYTES / 32;
   int f;
   if constexpr (E == kEF32) f = ((krow >> 2) & 1) << 2;
-  else if constexpr (E == kEBF16 || E == kEF16) f = ((krow & 3) << 1) ^ ((krow >> 1) & 1);
+  else if constexpr (E == kEBF16 || E == kEF16) f = ((krow & 3) << 1) | ((krow >> 3) & 1);
   else f = krow & 7;
   return f & (NG - 1);
 }
@@ -430,7 +436,8 @@ struct DirectLoader {
   // is a multiple of 8 the per-lane offsets of a wave's instructions differ by a wave-uniform
   // stride: one per-lane offset is kept and the stride goes into the scalar base pointer.
   static constexpr int ROWS_PER_INSTR_STEP = NWAVES * 1024 / ROW_BYTES;
-  static constexpr bool STRIDED = LAYOUT == kMC && (NWAVES * 1024) % ROW_BYTES == 0 && ROWS_PER_INSTR_STEP % 8 == 0;
+  static constexpr bool STRIDED = LAYOUT == kMC && (NWAVES * 1024) % ROW_BYTES == 0 &&
+                                  ROWS_PER_INSTR_STEP % (ES == kEBF16 || ES == kEF16 ? 16 : 8) == 0;
   static constexpr int NOFF = STRIDED ? 1 : PER;
 
   uint32_t voff[NOFF];  // per-lane byte offset from the wave-uniform base pointer of a k-step
