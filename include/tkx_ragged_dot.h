@@ -252,6 +252,17 @@ int32_t tkx_ragged_dot_fwd_fused(const void* lhs, const void* rhs, const int32_t
                                  int32_t lhs_dtype, int32_t rhs_dtype, int32_t out_dtype, int32_t activation,
                                  int32_t gateup, const TkxConfig* config, tkx_stream_t stream);
 
+/* tkx_ragged_dot_fwd_fused without gate-up fusion for weight scales that `rhs_scale_cols` columns share: rhs_scale is
+ * f32[G, rhs_scale_blocks, n / rhs_scale_cols] (4-byte aligned). 1: that call. 128: fp8 x fp8 with more than one scale
+ * block along k (the 128 x 128 block form of fp8 weights) and n % 128 == 0; the results are bit for bit those of the same
+ * scales repeated over their columns. */
+int32_t tkx_ragged_dot_fwd_scale_tiles(const void* lhs, const void* rhs, const int32_t* group_sizes,
+                                       const int32_t* group_offset, const float* lhs_scale, const float* rhs_scale,
+                                       const float* rhs_bias, void* out, void* workspace, int64_t m, int64_t k, int64_t n,
+                                       int64_t num_groups, int64_t num_group_sizes, int64_t rhs_scale_blocks,
+                                       int64_t rhs_scale_cols, int32_t lhs_dtype, int32_t rhs_dtype, int32_t out_dtype,
+                                       int32_t activation, const TkxConfig* config, tkx_stream_t stream);
+
 /* Which entry of a forward / TRANS_RHS launch's list of `tiles` tiles workgroup `workgroup` computes, or -1 (the launch
  * has enough workgroups for every entry). A host function: the map the kernels use, for tests and tools. */
 int64_t tkx_ragged_dot_launch_order(int64_t workgroup, int64_t tiles);
@@ -337,6 +348,12 @@ int32_t tkx_row_sums_fp8(const void* x, float* sums, int64_t rows, int64_t cols,
 int32_t tkx_quantize(const void* x, void* qvalue, float* scale, int64_t rows, int64_t cols, int64_t scale_block_rows,
                      int64_t scale_block_cols, int32_t x_dtype, int32_t q_dtype, float qmax, float bound,
                      tkx_stream_t stream);
+
+/* tkx_quantize with tiles one row tall and the scales laid out f32 [cols / scale_block_cols, rows], the form in which the
+ * products with scale blocks along k read the lhs scales. Fewer than 2^31 tiles. */
+int32_t tkx_quantize_scales_transposed(const void* x, void* qvalue, float* scale, int64_t rows, int64_t cols,
+                                       int64_t scale_block_cols, int32_t x_dtype, int32_t q_dtype, float qmax, float bound,
+                                       tkx_stream_t stream);
 
 /* The token permute / un-permute steps either side of the ragged dot in an MoE layer, one kernel:
  *   out[j, :] = sum over r < reduce_group_size of keep(g) * weights[g] * x[indices[g], :],  g = j * reduce_group_size + r

@@ -2702,3 +2702,43 @@ def test_timing_tool_collects_every_kind_of_problem(tmp_path, device):
   assert sorted(e["mode"] for e in entries) == [0] * 14 + [1, 2]
   for e in entries:
     assert 1.0 <= tile_cost.heuristics_gap(e) < 3.0, e["shape"]
+
+
+# ---- weight scales per 128 columns, read as they are ---------------------------------------------------------
+@pytest.mark.parametrize("variant", [(128, 256, 128, 2, 4, 3), (64, 256, 128, 2, 2, 3), (32, 256, 128, 1, 4, 3)])
+@pytest.mark.parametrize("k,n,t_k,sizes", [
+    (256, 128, 128, (1, 0, 39)),         # half a tile of columns, a group of one row, an empty one, rows of no group
+    (384, 384, 128, (128, 64, 4)),       # an odd number of 128-column blocks
+    (1024, 640, 256, (130, 61)),         # scale blocks of two k-steps
+    (2048, 256, 1024, (33, 95)),
+])
+def test_fp8_weight_scales_per_128_columns(variant, k, n, t_k, sizes, device):
+  """Block scales [g, k/t_k, n/128] give the bits of the same scales repeated over their columns."""
+  rng = np.random.default_rng(k + n)
+  G, m = len(sizes), max(sum(sizes) + 7, 8 * len(sizes) + 1) // 4 * 4 + 4
+  gs = torch.tensor(sizes, dtype=torch.int32, device=device)
+  f8 = torch.float8_e4m3fn
+  x = torch.tensor(rng.normal(0, 1, (m, k)).astype(np.float32)).to(device).to(f8)
+  w = torch.tensor(rng.normal(0, 1, (G, k, n)).astype(np.float32)).to(device).to(f8)
+  xs = torch.tensor(rng.uniform(0.5, 2, (m, k // t_k)).astype(np.float32), device=device)
+  # (a view behind one float: the scales need no more than their own alignment)
+  ws = torch.tensor(rng.uniform(0.5, 2, G * (k // t_k) * (n // 128) + 1).astype(np.float32), device=device)[1:].view(G, k // t_k, n // 128)
+  op = hip.HipRaggedDot(config=hip.Config(*variant))
+  lhs = tokamax_amd.QArray(x, xs)
+  out = op(lhs, tokamax_amd.QArray(w, ws), group_sizes=gs, preferred_element_type=torch.bfloat16)
+  rep = op(lhs, tokamax_amd.QArray(w, ws.repeat_interleave(128, dim=2)), group_sizes=gs, preferred_element_type=torch.bfloat16)
+  assert torch.equal(out.view(torch.int16), rep.view(torch.int16))
+  xf = _np(x) * np.repeat(_np(xs), t_k, axis=1)
+  wf = _np(w) * np.repeat(np.repeat(_np(ws), t_k, axis=1), 128, axis=2)
+  want = O.ragged_dot(xf, wf, np.asarray(sizes, np.int32), acc_dtype=np.float64, out_dtype="f64")
+  _check(out, want, 2e-3, rows=sum(sizes))  # (one rounding of the result to bf16)
+  assert torch.count_nonzero(out[sum(sizes):]) == 0
+
+
+@pytest.mark.parametrize("rows,cols,t_c", [(1, 16, 8), (5, 384, 128), (3, 2048, 1024), (2, 17408, 8704), (4099, 256, 128)])
+def test_quantised_scales_laid_out_by_block(rows, cols, t_c, device):
+  x = torch.randn(rows, cols, device=device, dtype=torch.bfloat16)
+  q, s = hip_ops.quantize(x, torch.float8_e4m3fn, (1, t_c))
+  qt, st = hip_ops.quantize(x, torch.float8_e4m3fn, (1, t_c), scale_by_block=True)
+  assert st.shape == s.shape and st.t().is_contiguous() and torch.equal(st, s)
+  assert torch.equal(q.view(torch.uint8), qt.view(torch.uint8))

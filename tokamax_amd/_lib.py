@@ -32,6 +32,7 @@ EXPORTED_SYMBOLS = (
     "tkx_ragged_dot_fwd",
     "tkx_ragged_dot_fwd_static_workspace",
     "tkx_ragged_dot_fwd_fused",
+    "tkx_ragged_dot_fwd_scale_tiles",
     "tkx_ragged_dot_launch_order",
     "tkx_ragged_dot_drhs",
     "tkx_ragged_dot_drhs_tile",
@@ -39,6 +40,7 @@ EXPORTED_SYMBOLS = (
     "tkx_dequantize",
     "tkx_dequantize_zero_point",
     "tkx_quantize",
+    "tkx_quantize_scales_transposed",
     "tkx_ragged_gather_rows",
     "tkx_ragged_dot_num_variants",
     "tkx_ragged_dot_variant",
@@ -117,6 +119,9 @@ def _declare(lib):
   lib.tkx_ragged_dot_fwd_fused.restype = i32
   lib.tkx_ragged_dot_fwd_fused.argtypes = [vp, vp, vp, vp, vp, vp, vp, vp, vp, i64, i64, i64, i64, i64, i64, i32, i32,
                                            i32, i32, i32, cfgp, vp]
+  lib.tkx_ragged_dot_fwd_scale_tiles.restype = i32
+  lib.tkx_ragged_dot_fwd_scale_tiles.argtypes = [vp, vp, vp, vp, vp, vp, vp, vp, vp, i64, i64, i64, i64, i64, i64, i64, i32,
+                                                 i32, i32, i32, cfgp, vp]
   lib.tkx_ragged_dot_drhs.restype = i32
   lib.tkx_ragged_dot_drhs.argtypes = [vp, vp, vp, vp, vp, i64, i64, i64, i64, i32, i32, cfgp, vp]
   lib.tkx_ragged_dot_launch_order.restype = i64
@@ -132,6 +137,8 @@ def _declare(lib):
   lib.tkx_dequantize_zero_point.argtypes = [vp, vp, vp, vp, i64, i64, i64, i64, i32, i32, vp]
   lib.tkx_quantize.restype = i32
   lib.tkx_quantize.argtypes = [vp, vp, vp, i64, i64, i64, i64, i32, i32, ctypes.c_float, ctypes.c_float, vp]
+  lib.tkx_quantize_scales_transposed.restype = i32
+  lib.tkx_quantize_scales_transposed.argtypes = [vp, vp, vp, i64, i64, i64, i32, i32, ctypes.c_float, ctypes.c_float, vp]
   lib.tkx_ragged_gather_rows.restype = i32
   lib.tkx_ragged_gather_rows.argtypes = [vp, vp, vp, vp, vp, vp, vp, i64, i64, i64, i64, i32, vp]
   lib.tkx_ragged_dot_num_variants.restype = i32

@@ -117,7 +117,7 @@ int32_t prepare(const void* fn, int32_t smem_bytes) {
 }
 
 int32_t launch(const Variant* v, const GemmParams& p, int64_t grid, hipStream_t stream) {
-  const void* fn = p.c_scale != nullptr ? v->fn_fp8_out : p.split_k > 1 ? v->fn_split : v->fn;
+  const void* fn = p.c_scale != nullptr ? v->fn_fp8_out : p.split_k > 1 ? v->fn_split : p.wide_scales ? v->fn_wide_scales : v->fn;
   int32_t st = prepare(fn, v->smem_bytes);
   if (st != TKX_OK) return st;
   if (grid <= 0 || grid > 0x7fffffffLL) return set_error(TKX_ERR_INVALID, "grid size %lld out of range", (long long)grid);
@@ -242,12 +242,14 @@ namespace {
 // Forward / dlhs launcher behind both public forward entry points. `gateup`: rhs is [g, k, n] =
 // [gate | up] and out is [m, n/2] = act(lhs.gate + bias) * (lhs.up + bias), `activation` naming act.
 // `group_offset` (device, one int32, or null) and `num_group_sizes`: the num_groups groups of rhs are
-// entries [offset, offset + num_groups) of the num_group_sizes group sizes.
+// entries [offset, offset + num_groups) of the num_group_sizes group sizes. `rhs_scale_cols`: columns that share an rhs
+// scale (1, or 128: the block form of fp8 weights under fp8 activations).
 int32_t fwd_impl(const void* lhs, const void* rhs, const int32_t* group_sizes, const int32_t* group_offset,
                  const float* lhs_scale, const float* rhs_scale, const float* rhs_bias, void* out, void* workspace,
                  int64_t m, int64_t k, int64_t n, int64_t num_groups, int64_t num_group_sizes, int32_t lhs_dtype,
                  int32_t rhs_dtype, int32_t out_dtype, int32_t mode, int32_t activation, bool gateup,
-                 int64_t rhs_scale_blocks, const TkxConfig* config, tkx_stream_t stream_, float* out_scale = nullptr) {
+                 int64_t rhs_scale_blocks, const TkxConfig* config, tkx_stream_t stream_, float* out_scale = nullptr,
+                 int64_t rhs_scale_cols = 1) {
   hipStream_t stream = static_cast<hipStream_t>(stream_);
   if (!lhs || !rhs || !out || !workspace || !config) return set_error(TKX_ERR_INVALID, "null pointer argument");
   // (no group sizes: a single group that owns every row; the tiled kernels only)
@@ -348,9 +350,12 @@ int32_t fwd_impl(const void* lhs, const void* rhs, const int32_t* group_sizes, c
   if ((n * rb) % 16 != 0 || (dlhs && (n * lb) % 16 != 0)) return set_error(TKX_ERR_UNSUPPORTED, "n*sizeof(elem) must be a multiple of 16");
   if ((cols * ob) % 16 != 0 || cols % 8 != 0) return set_error(TKX_ERR_UNSUPPORTED, "output row size must be a multiple of 8 elements");
   if (((uintptr_t)lhs | (uintptr_t)rhs | (uintptr_t)out | (uintptr_t)workspace) % 16 != 0 ||
-      (rhs_scale && (uintptr_t)rhs_scale % 16 != 0))
+      (rhs_scale && (uintptr_t)rhs_scale % (rhs_scale_cols == 1 ? 16 : 4) != 0))
     return set_error(TKX_ERR_UNSUPPORTED, "pointers must be 16-byte aligned");
 
+  if (rhs_scale_cols != 1 && (rhs_scale_cols != 128 || !subk || v->fn_wide_scales == nullptr || n % 128 != 0))
+    return set_error(TKX_ERR_UNSUPPORTED, "an rhs scale per 128 columns needs fp8 x fp8 operands, scale blocks along k and n %% 128 == 0"
+                                          " (n=%lld columns per scale=%lld)", (long long)n, (long long)rhs_scale_cols);
   if (out_scale != nullptr && (v->fn == nullptr || v->fn_fp8_out == nullptr))
     return set_error(TKX_ERR_UNSUPPORTED, "this kernel variant cannot quantise its result (bf16 or fp8 forward tiles whose"
                                           " wave columns tile 128 output columns can)");
@@ -432,6 +437,7 @@ int32_t fwd_impl(const void* lhs, const void* rhs, const int32_t* group_sizes, c
   p.activation = activation;
   p.scale_blocks = subk ? (int32_t)rhs_scale_blocks : 1;
   p.log2_block_rows = log2_block_rows;
+  p.wide_scales = rhs_scale_cols != 1;
   if (slots > 0x7fffff00LL) return set_error(TKX_ERR_UNSUPPORTED, "too many tiles");
   // Extra workgroups zero the rows past the last group (and before the first, with a group offset);
   // they exit at once when there are none.
@@ -524,6 +530,21 @@ int32_t tkx_ragged_dot_fwd_fused(const void* lhs, const void* rhs, const int32_t
   return fwd_impl(lhs, rhs, group_sizes, group_offset, lhs_scale, rhs_scale, rhs_bias, out, workspace, m, k, n, num_groups,
                   num_group_sizes, lhs_dtype, rhs_dtype, out_dtype, TKX_MODE_DEFAULT, activation, gateup == 1,
                   rhs_scale_blocks, config, stream);
+}
+
+int32_t tkx_ragged_dot_fwd_scale_tiles(const void* lhs, const void* rhs, const int32_t* group_sizes, const int32_t* group_offset,
+                                       const float* lhs_scale, const float* rhs_scale, const float* rhs_bias, void* out,
+                                       void* workspace, int64_t m, int64_t k, int64_t n, int64_t num_groups,
+                                       int64_t num_group_sizes, int64_t rhs_scale_blocks, int64_t rhs_scale_cols,
+                                       int32_t lhs_dtype, int32_t rhs_dtype, int32_t out_dtype, int32_t activation,
+                                       const TkxConfig* config, tkx_stream_t stream) {
+  if (rhs_scale_blocks < 1 || rhs_scale_cols < 1) return set_error(TKX_ERR_INVALID, "rhs_scale_blocks and rhs_scale_cols must be >= 1");
+  if (rhs_scale == nullptr) return set_error(TKX_ERR_INVALID, "null pointer argument");
+  if (group_offset != nullptr && (uintptr_t)group_offset % 4 != 0)
+    return set_error(TKX_ERR_INVALID, "group_offset must be 4-byte aligned");
+  return fwd_impl(lhs, rhs, group_sizes, group_offset, lhs_scale, rhs_scale, rhs_bias, out, workspace, m, k, n, num_groups,
+                  num_group_sizes, lhs_dtype, rhs_dtype, out_dtype, TKX_MODE_DEFAULT, activation, false, rhs_scale_blocks,
+                  config, stream, nullptr, rhs_scale_cols);
 }
 
 // How a group's m_tiles x n_tiles tiles of d rhs are dealt to the 8 XCDs (drhs_tile). With `rows` XCDs along k and
@@ -713,9 +734,12 @@ int32_t tkx_row_sums_fp8(const void* x, float* sums, int64_t rows, int64_t cols,
   return launch_row_sums_fp8(x, sums, rows, cols, chunk_cols != cols, static_cast<hipStream_t>(stream));
 }
 
-int32_t tkx_quantize(const void* x, void* qvalue, float* scale, int64_t rows, int64_t cols, int64_t scale_block_rows,
-                     int64_t scale_block_cols, int32_t x_dtype, int32_t q_dtype, float qmax, float bound,
-                     tkx_stream_t stream) {
+}  // extern "C"
+
+namespace {
+int32_t quantize_impl(const void* x, void* qvalue, float* scale, int64_t rows, int64_t cols, int64_t scale_block_rows,
+                      int64_t scale_block_cols, int32_t x_dtype, int32_t q_dtype, float qmax, float bound, bool scale_t,
+                      tkx_stream_t stream) {
   if (!x || !qvalue || !scale) return set_error(TKX_ERR_INVALID, "null pointer argument");
   if (rows < 1 || cols < 1 || scale_block_rows < 1 || scale_block_cols < 1)
     return set_error(TKX_ERR_INVALID, "bad sizes rows=%lld cols=%lld block=%lldx%lld", (long long)rows, (long long)cols,
@@ -751,8 +775,25 @@ int32_t tkx_quantize(const void* x, void* qvalue, float* scale, int64_t rows, in
     if (q_dtype != TKX_I8) return set_error(TKX_ERR_INVALID, "a bound above qmax belongs to the integer types");
     range.lo = -qmax - 1.f;
   }
-  return launch_quantize(x, qvalue, scale, rows, cols, scale_block_rows, scale_block_cols, x_dtype, q_dtype, range,
+  if (scale_t && (scale_block_rows != 1 || rows * (cols / scale_block_cols) > 0x7fffffffLL))
+    return set_error(TKX_ERR_UNSUPPORTED, "transposed scales come with tiles one row tall, fewer than 2^31 of them");
+  return launch_quantize(x, qvalue, scale, rows, cols, scale_block_rows, scale_block_cols, x_dtype, q_dtype, range, scale_t,
                          static_cast<hipStream_t>(stream));
+}
+}  // namespace
+
+extern "C" {
+
+int32_t tkx_quantize(const void* x, void* qvalue, float* scale, int64_t rows, int64_t cols, int64_t scale_block_rows,
+                     int64_t scale_block_cols, int32_t x_dtype, int32_t q_dtype, float qmax, float bound,
+                     tkx_stream_t stream) {
+  return quantize_impl(x, qvalue, scale, rows, cols, scale_block_rows, scale_block_cols, x_dtype, q_dtype, qmax, bound, false, stream);
+}
+
+int32_t tkx_quantize_scales_transposed(const void* x, void* qvalue, float* scale, int64_t rows, int64_t cols,
+                                       int64_t scale_block_cols, int32_t x_dtype, int32_t q_dtype, float qmax, float bound,
+                                       tkx_stream_t stream) {
+  return quantize_impl(x, qvalue, scale, rows, cols, 1, scale_block_cols, x_dtype, q_dtype, qmax, bound, true, stream);
 }
 
 int32_t tkx_ragged_gather_rows(const void* x, const int32_t* indices, const float* weights, const uint8_t* valid,

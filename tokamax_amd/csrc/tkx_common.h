@@ -158,6 +158,7 @@ struct GemmParams {
   int32_t grid_tile_width;
   int32_t out_dtype, activation;
   int32_t scale_blocks, log2_block_rows;  // kFwdSubK: b_scale is [g, scale_blocks, n]; rows of k per block = 1 << log2
+  int32_t wide_scales;  // ... or, not 0: [g, scale_blocks, n / 128]
 };
 
 struct Variant {
@@ -169,6 +170,7 @@ struct Variant {
   int32_t split_b; // > 0: the split pipeline (that many B stages of block_k / 2; num_stages A stages of block_k)
   const void* fn_fp8_out;  // the same kernel storing fp8 with one scale per (row, 128 columns) (GemmParams::c_scale), or null
   const void* fn_split;    // the same kernel splitting the tiles of the last round along the contraction (GemmParams::split_k), or null
+  const void* fn_wide_scales;  // the same kernel with weight scales per (k-block, 128 columns) (GemmParams::wide_scales), or null
 };
 
 // ---- decode (small-m streaming kernel; int8 or 16-bit weights) -----------------------------------
@@ -207,10 +209,11 @@ int32_t launch_dequant(const void* q, const float* scale, const float* zero_poin
 
 // ---- absmax quantisation to int8 / fp8 with block scales (the inverse pass) -------------------------
 // scale[R, C] = absmax of tile (R, C) / bound (1 for an all-zero tile); q = convert(clip(x / scale)). x f32, bf16 or f16.
-// `bound`: what the tile's absmax is divided by; values are clipped to [lo, hi] after the division.
+// `bound`: what the tile's absmax is divided by; values are clipped to [lo, hi] after the division. `scale_t` (t_r == 1):
+// the scales are laid out [cols / t_c, rows].
 struct QuantRange { float bound, lo, hi; };
 int32_t launch_quantize(const void* x, void* q, float* scale, int64_t rows, int64_t cols, int64_t t_r, int64_t t_c,
-                        int32_t x_dtype, int32_t q_dtype, QuantRange range, hipStream_t stream);
+                        int32_t x_dtype, int32_t q_dtype, QuantRange range, bool scale_t, hipStream_t stream);
 
 // ---- row gather with optional mask, weight and reduction (token permute / un-permute) -------------
 int32_t launch_gather_rows(const void* x, const int32_t* indices, const float* weights, const unsigned char* valid,

@@ -408,6 +408,11 @@ __device__ __forceinline__ void direct_load_16(const unsigned char* sbase, uint3
   asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds), "v"(voff), "s"(sbase)
                : "memory", "m0");
 }
+// 4 bytes per lane: LDS[lds + 4*lane] <- *(sbase + voff)
+__device__ __forceinline__ void direct_load_4(const unsigned char* sbase, uint32_t voff, unsigned lds) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, %2" ::"s"(lds), "v"(voff), "s"(sbase)
+               : "memory", "m0");
+}
 // Workgroup barrier that also orders direct-to-LDS loads: a wave's loads count on vmcnt, and other
 // waves read the bytes they deposit, so every wave must drain vmcnt BEFORE it arrives at the
 // barrier (the compiler only guards a wave's own later LDS reads).
@@ -891,9 +896,15 @@ struct GemmKernel {
   // its own so that the plain one carries none of its code or registers.
   // Kernels that can split the tiles of a launch's last round along the contraction (GemmParams::split_k).
   static constexpr bool SPLITK = (MODE == kFwd || MODE == kDlhs) && BM >= 128;
+  // Kernels that take weight scales per 128 columns (the block form of fp8 weights).
+  static constexpr bool WIDE_SCALES = SUBP && EA == kEF8 && EB == kEF8 && 128 % WTN == 0;
   // SK: the instantiation that does (a kernel of its own, like the quantising one).
-  template <bool QO = false, bool SK = false>
+  // WB: the instantiation for weight scales per (k-block, 128 columns), [g, scale_blocks, n / 128]: one scale for all
+  // columns of a wave, so that folding a k-step in takes one multiply-add per element and one product per row instead of
+  // a product and a multiply-add per element.
+  template <bool QO = false, bool SK = false, bool WB = false>
   static __device__ __forceinline__ void run(const GemmParams& p, unsigned char* smem) {
+    static_assert(!WB || WIDE_SCALES, "this kernel takes one weight scale per column");
     static_assert(!QO || QOUT, "this kernel has no quantising epilogue");
     static_assert(!SK || (SPLITK && !QO), "this kernel has no split of the last round");
     const int tid = threadIdx.x, lane = tid & 63;
@@ -1276,9 +1287,10 @@ struct GemmKernel {
       // (kFwdSubK) scales of this tile's columns: row `block` of the group's [scale_blocks, n] table; lanes past
       // the last column re-read the last four (their products are never stored).
       const unsigned char* const gS0 =
-          SUBK ? reinterpret_cast<const unsigned char*>(p.b_scale + (int64_t)group * p.scale_blocks * p.nb_ext) : nullptr;
+          SUBK ? reinterpret_cast<const unsigned char*>(p.b_scale + (int64_t)group * p.scale_blocks * (WB ? p.nb_ext >> 7 : p.nb_ext)) : nullptr;
       constexpr int SCALE_LANES = 64 / NLOAD;  // lanes of a wave that fetch 16 bytes of the scale row each
-      const uint32_t scale_voff = SUBK ? (uint32_t)min(col0 + 4 * (wave * SCALE_LANES + lane), p.nb_ext - 4) * 4u : 0u;
+      const uint32_t scale_voff = WB ? (uint32_t)(min(col0 + wn * WTN, p.nb_ext - 1) >> 7) * 4u
+                                  : SUBK ? (uint32_t)min(col0 + 4 * (wave * SCALE_LANES + lane), p.nb_ext - 4) * 4u : 0u;
       // (fp8 x fp8) lhs scales [scale_blocks, m]: the BM rows of the tile, 4 per lane; chunks past the last row
       // re-read the last four (m and row0 are multiples of 4, so a chunk is all inside or all outside).
       constexpr int XS_LANES = BM / 4 / NLOAD;
@@ -1290,7 +1302,7 @@ struct GemmKernel {
         sp.b = uniform_pointer(gB0 + step * stepB);
         sp.s = nullptr;
         if constexpr (SUBK)
-          sp.s = uniform_pointer(gS0 + (int64_t)((kc_begin + step * BK) >> p.log2_block_rows) * p.nb_ext * 4);
+          sp.s = uniform_pointer(gS0 + (int64_t)((kc_begin + step * BK) >> p.log2_block_rows) * (WB ? p.nb_ext >> 7 : p.nb_ext) * 4);
         if constexpr (SUBP) {
           const int64_t block = (kc_begin + step * BK) >> p.log2_block_rows;
           sp.x = uniform_pointer(reinterpret_cast<const unsigned char*>(p.a_scale) + block * p.m_ext * 4);
@@ -1308,7 +1320,11 @@ struct GemmKernel {
         else if (q < DirA::PER + DirB::PER) db.issue_one(q - DirA::PER, sp.b, sp.lds + StageA::BYTES, wave);
         else if (SUBK && q == DirA::PER + DirB::PER) {
           const unsigned dst = SUBP ? sp.ring : sp.lds + StageA::BYTES + StageB::BYTES;
-          if (lane < SCALE_LANES) direct_load_16(sp.s, scale_voff, dst + wave * (SCALE_LANES * 16));
+          if constexpr (WB) {
+            if (lane == 0) direct_load_4(sp.s, scale_voff, dst + wave * 4);  // (the scale of the wave's own columns)
+          } else if (lane < SCALE_LANES) {
+            direct_load_16(sp.s, scale_voff, dst + wave * (SCALE_LANES * 16));
+          }
         } else if (SUBP && q == DirA::PER + DirB::PER + 1) {
           if (lane < XS_LANES) direct_load_16(sp.x, xs_voff, sp.ring + BN * 4 + wave * (XS_LANES * 16));
         } else if (SUBP && I4F && q == DirA::PER + DirB::PER + 2) {
@@ -1574,6 +1590,20 @@ struct GemmKernel {
                   xoff[i] = -8.f * xs[i] * *reinterpret_cast<const float*>(slot + (BN + BM) * 4 + 4 * (row_block(i) * 32 + (lane & 31)));
                   xs[i] *= 512.f;
                 }
+              }
+              if constexpr (WB) {
+                const float ws = *reinterpret_cast<const float*>(slot + wave * 4);
+#pragma unroll
+                for (int i = 0; i < TM; ++i) {
+                  xs[i] *= ws;
+#pragma unroll
+                  for (int j = 0; j < TN; ++j)
+                    if (i < NV) {
+#pragma unroll
+                      for (int e = 0; e < 16; ++e) acc[i][j][e] += pacc[i][j][e] * xs[i];
+                    }
+                }
+                return;  // (the last statement of a k-step)
               }
 #pragma unroll
               for (int j = 0; j < TN; ++j)
@@ -2006,6 +2036,17 @@ __global__ __launch_bounds__(K::THREADS, K::kWavesPerSimd) void gemm_entry_split
   extern __shared__ __attribute__((aligned(1024))) unsigned char tkx_smem[];
   K::template run<false, true>(p, tkx_smem);
 }
+template <class K>
+__global__ __launch_bounds__(K::THREADS, K::kWavesPerSimd) void gemm_entry_wide_scales(const GemmParams p) {
+  extern __shared__ __attribute__((aligned(1024))) unsigned char tkx_smem[];
+  K::template run<false, false, true>(p, tkx_smem);
+}
+// The entry that takes weight scales per 128 columns, of a kernel that has one, else null.
+template <class K>
+const void* wide_scales_entry() {
+  if constexpr (K::WIDE_SCALES) return reinterpret_cast<const void*>(&gemm_entry_wide_scales<K>);
+  else return nullptr;
+}
 // The entry that splits the last round of a kernel that has one, else null.
 template <class K>
 const void* split_entry() {
@@ -2024,7 +2065,7 @@ const void* fp8_out_entry() {
     MODE, EA, EB, BM, BN, BK, WM, WN, NS, ::tkx::GemmKernel<MODE, EA, EB, BM, BN, BK, WM, WN, NS, HB>::SMEM_BYTES, \
         reinterpret_cast<const void*>(&::tkx::gemm_entry<::tkx::GemmKernel<MODE, EA, EB, BM, BN, BK, WM, WN, NS, HB>>), HB, \
         ::tkx::fp8_out_entry<::tkx::GemmKernel<MODE, EA, EB, BM, BN, BK, WM, WN, NS, HB>>(),                      \
-        ::tkx::split_entry<::tkx::GemmKernel<MODE, EA, EB, BM, BN, BK, WM, WN, NS, HB>>()                         \
+        ::tkx::split_entry<::tkx::GemmKernel<MODE, EA, EB, BM, BN, BK, WM, WN, NS, HB>>(), nullptr                \
   }
 
 #define TKX_VARIANT(MODE, EA, EB, BM, BN, BK, WM, WN, NS)                                            \
@@ -2032,7 +2073,8 @@ const void* fp8_out_entry() {
     MODE, EA, EB, BM, BN, BK, WM, WN, NS, ::tkx::GemmKernel<MODE, EA, EB, BM, BN, BK, WM, WN, NS>::SMEM_BYTES, \
         reinterpret_cast<const void*>(&::tkx::gemm_entry<::tkx::GemmKernel<MODE, EA, EB, BM, BN, BK, WM, WN, NS>>), 0, \
         ::tkx::fp8_out_entry<::tkx::GemmKernel<MODE, EA, EB, BM, BN, BK, WM, WN, NS>>(),                       \
-        ::tkx::split_entry<::tkx::GemmKernel<MODE, EA, EB, BM, BN, BK, WM, WN, NS>>()                          \
+        ::tkx::split_entry<::tkx::GemmKernel<MODE, EA, EB, BM, BN, BK, WM, WN, NS>>(),                         \
+        ::tkx::wide_scales_entry<::tkx::GemmKernel<MODE, EA, EB, BM, BN, BK, WM, WN, NS>>()                    \
   }
 
 }  // namespace tkx

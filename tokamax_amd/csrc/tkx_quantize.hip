@@ -142,7 +142,7 @@ template <int EX, int EQ, int CH, int U>
 __global__ __launch_bounds__(kQThreads) void quantize_rows_kernel(const unsigned char* __restrict__ x,
                                                                   unsigned char* __restrict__ q, float* __restrict__ scale,
                                                                   int64_t rows, int32_t cols, int32_t t_c, int32_t lanes,
-                                                                  QuantRange qmax) {
+                                                                  QuantRange qmax, bool scale_t) {
   constexpr int XB = XVec<EX>::BYTES;  // bytes of 8 elements of x
   const int L = CH == 1 ? lanes : 64;  // (a tile of more chunks than lanes has a whole wave: constant distances)
   const int lane = threadIdx.x & 63;
@@ -195,7 +195,14 @@ __global__ __launch_bounds__(kQThreads) void quantize_rows_kernel(const unsigned
       const bool near = __all(has_reciprocal(s));
       const float r = 1.f / s;
       if (tile < num_tiles) {
-        if (l == 0) scale[tile] = s;
+        if (l == 0) {
+          int64_t at = tile;
+          if (scale_t) {  // [cols / t_c, rows], the form in which the products with scale blocks along k read them
+            const uint32_t row = (uint32_t)tile / (uint32_t)tiles_per_row;  // (fewer than 2^31 tiles)
+            at = (int64_t)((uint32_t)tile - row * (uint32_t)tiles_per_row) * rows + row;
+          }
+          scale[at] = s;
+        }
         unsigned char* qr = q + tile * t_c;
         if constexpr (CH > 0) {
 #pragma unroll
@@ -220,13 +227,13 @@ __global__ __launch_bounds__(kQThreads) void quantize_rows_kernel(const unsigned
 // of 16-bit elements, 8 of f32), more sets of tiles at a time where a tile is short.
 template <int EX, int EQ>
 void launch_rows(int per_lane, int64_t tiles, int L, const unsigned char* x, unsigned char* q, float* scale, int64_t rows,
-                 int32_t cols, int32_t t_c, QuantRange range, hipStream_t stream) {
+                 int32_t cols, int32_t t_c, QuantRange range, bool scale_t, hipStream_t stream) {
   auto go = [&](auto kernel, int sets) {
     const int64_t per_workgroup = (int64_t)(64 / L) * sets * (kQThreads / 64);
     int64_t grid = (tiles + per_workgroup - 1) / per_workgroup;
     if (grid > 256 * 16) grid = 256 * 16;
     if (grid < 1) grid = 1;
-    kernel<<<dim3((unsigned)grid), dim3(kQThreads), 0, stream>>>(x, q, scale, rows, cols, t_c, (int32_t)L, range);
+    kernel<<<dim3((unsigned)grid), dim3(kQThreads), 0, stream>>>(x, q, scale, rows, cols, t_c, (int32_t)L, range, scale_t);
   };
   // (Four sets at a time need so many tiles that every SIMD still gets waves of its own.)
   const bool many = tiles / (64 / L) >= 256 * 4 * 4 * 4;
@@ -376,7 +383,7 @@ __global__ __launch_bounds__(kQThreads) void quantize_tiles_kernel(const unsigne
 
 template <int EX>
 int32_t launch_for_x(const void* x, void* q, float* scale, int64_t rows, int64_t cols, int64_t t_r, int64_t t_c,
-                     int32_t q_dtype, QuantRange qmax, hipStream_t stream) {
+                     int32_t q_dtype, QuantRange qmax, bool scale_t, hipStream_t stream) {
   const auto* xb = static_cast<const unsigned char*>(x);
   auto* qb = static_cast<unsigned char*>(q);
   if (t_r == 1) {
@@ -385,9 +392,9 @@ int32_t launch_for_x(const void* x, void* q, float* scale, int64_t rows, int64_t
     const int64_t tiles = rows * (cols / t_c);
     const int per_lane = (chunks + L - 1) / L;
     if (q_dtype == TKX_I8)
-      launch_rows<EX, kEI8>(per_lane, tiles, L, xb, qb, scale, rows, (int32_t)cols, (int32_t)t_c, qmax, stream);
+      launch_rows<EX, kEI8>(per_lane, tiles, L, xb, qb, scale, rows, (int32_t)cols, (int32_t)t_c, qmax, scale_t, stream);
     else
-      launch_rows<EX, kEF8>(per_lane, tiles, L, xb, qb, scale, rows, (int32_t)cols, (int32_t)t_c, qmax, stream);
+      launch_rows<EX, kEF8>(per_lane, tiles, L, xb, qb, scale, rows, (int32_t)cols, (int32_t)t_c, qmax, scale_t, stream);
   } else if (t_c != 1 && !((t_c & (t_c - 1)) == 0 && t_c >= 8 && t_c <= 256)) {
     const int64_t num_tiles = (rows / t_r) * (cols / t_c), chunks = rows * (cols / 8);
     int64_t grid = (chunks + kQThreads - 1) / kQThreads;
@@ -416,10 +423,10 @@ int32_t launch_for_x(const void* x, void* q, float* scale, int64_t rows, int64_t
 }  // namespace
 
 int32_t launch_quantize(const void* x, void* q, float* scale, int64_t rows, int64_t cols, int64_t t_r, int64_t t_c,
-                        int32_t x_dtype, int32_t q_dtype, QuantRange qmax, hipStream_t stream) {
-  if (x_dtype == TKX_F32) return launch_for_x<kEF32>(x, q, scale, rows, cols, t_r, t_c, q_dtype, qmax, stream);
-  if (x_dtype == TKX_BF16) return launch_for_x<kEBF16>(x, q, scale, rows, cols, t_r, t_c, q_dtype, qmax, stream);
-  return launch_for_x<kEF16>(x, q, scale, rows, cols, t_r, t_c, q_dtype, qmax, stream);
+                        int32_t x_dtype, int32_t q_dtype, QuantRange qmax, bool scale_t, hipStream_t stream) {
+  if (x_dtype == TKX_F32) return launch_for_x<kEF32>(x, q, scale, rows, cols, t_r, t_c, q_dtype, qmax, scale_t, stream);
+  if (x_dtype == TKX_BF16) return launch_for_x<kEBF16>(x, q, scale, rows, cols, t_r, t_c, q_dtype, qmax, scale_t, stream);
+  return launch_for_x<kEF16>(x, q, scale, rows, cols, t_r, t_c, q_dtype, qmax, scale_t, stream);
 }
 
 }  // namespace tkx

@@ -236,6 +236,25 @@ def _per_column_rhs_scale(rhs):
   return QArray(rhs.qvalue, scale, rhs.zero_point, rhs.qtype)
 
 
+def _shapes_of(x):
+  """A quantised operand's shapes and types, for plans that need no more."""
+  if not isinstance(x, QArray) or not isinstance(x.scale, torch.Tensor):
+    return x
+  return QArray(ShapeDtype(tuple(x.qvalue.shape), x.qvalue.dtype), ShapeDtype(tuple(x.scale.shape), x.scale.dtype),
+                x.zero_point, x.qtype)
+
+
+def _kernels_read_scale_tiles(lhs, rhs) -> bool:
+  """Whether the fp8 x fp8 kernels for scale blocks along k read weight scales per 128 columns ([g, k/t_k, n/128], the
+  128 x 128 block form) as they are. Repeated over their columns first, the scales of 32 x 7168 x 2048 weights took a pass of
+  5 us, and every k-step of a tile twice the vector work (a scale per element instead of one per row)."""
+  if not (isinstance(lhs, QArray) and isinstance(rhs, QArray) and rhs.qvalue.dtype == torch.float8_e4m3fn
+          and lhs.qvalue.dtype == torch.float8_e4m3fn):
+    return False
+  g, _, n = rhs.qvalue.shape
+  return rhs.scale.shape[0] == g and rhs.scale.shape[2] * 128 == n
+
+
 def _per_row_lhs_scale(lhs):
   """A quantised lhs [m, k] whose scale rows are shared by runs of consecutive lhs rows ([m / t_m, blocks]: tiles
   several rows tall, one scale per tensor) with each scale row repeated for its lhs rows. Works on tensors and on shapes."""
@@ -449,8 +468,10 @@ def _route(lhs, rhs, *, dims, precision, rhs_scale, fuse_gateup_activation, pref
   lhs_dt, rhs_dt = _dtype_of(lhs), _dtype_of(rhs)
   widen_lhs = widen_rhs = native = False
   if mode == 0:
-    lhs, rhs = _per_row_lhs_scale(lhs), _per_column_rhs_scale(rhs)
-    widen_lhs, widen_rhs, native = _widening_plan(lhs, rhs, allow_native=not gateup)
+    lhs = _per_row_lhs_scale(lhs)
+    widen_lhs, widen_rhs, native = _widening_plan(lhs, _per_column_rhs_scale(_shapes_of(rhs)), allow_native=not gateup)
+    if not (native and not widen_lhs and _kernels_read_scale_tiles(lhs, rhs)):
+      rhs = _per_column_rhs_scale(rhs)
     if (gateup and isinstance(rhs, QArray) and not widen_rhs and rhs.qvalue.dtype in (torch.int8, torch.float8_e4m3fn)
         and rhs.qvalue.shape[2] % 32):
       # Gate-up fusion reads the up half of a weight row n / 2 elements in, which is a whole 16-byte piece of one-byte
@@ -549,6 +570,18 @@ def _concrete_operand(x):
   """An `AsQArray` quantised on the device; an operand with a zero point dequantised to bf16 (quantization.py:85-93:
   none of the kernels takes a zero point)."""
   return quantization.as_array_or_qarray_without_zero_point(x)
+
+
+def _concrete_lhs(lhs, rhs):
+  """`_concrete_operand` for an lhs: where it is quantised to 8 bits per (row, k-block) for weights with as many scale
+  blocks along k, its scales come in the order the kernels read them in (another order took a transposing copy of 7 us at
+  8192 rows of 56 blocks)."""
+  if (isinstance(lhs, AsQArray) and lhs.calibration_method == "absmax" and isinstance(rhs, QArray) and lhs.ndim == 2
+      and lhs.tile_shape[0] == 1 and lhs.scale_shape[1] > 1 and len(rhs.scale.shape) == 3
+      and rhs.scale.shape[1] == lhs.scale_shape[1]):
+    qvalue, scale = hip_ops.quantize(lhs.value, lhs.qtype, lhs.tile_shape, scale_by_block=True)
+    return QArray(qvalue, scale, None, lhs.qtype)
+  return _concrete_operand(lhs)
 
 
 _PLAIN_ARGUMENT_TYPES = (bool, int, float, str, torch.dtype, base.RaggedDotDimensionNumbers)
@@ -738,7 +771,8 @@ class HipRaggedDot(base.RaggedDot):
       raise NotImplementedError("group_offset needs the default dimension numbers.")
 
     # Quantise / dequantise what the kernels cannot take as it is, then plan the call on shapes and types.
-    lhs, rhs = _concrete_operand(lhs), _concrete_operand(rhs)
+    rhs = _concrete_operand(rhs)
+    lhs = _concrete_lhs(lhs, rhs)
     rhs = _settle_packed_int4(lhs, rhs, dims=ragged_dot_dimension_numbers,
                               plain=rhs_bias is None and fuse_gateup_activation is None and rhs_scale is None,
                               gateup=fuse_gateup_activation is not None)

@@ -202,8 +202,8 @@ def ragged_dot_fwd(lhs, rhs, group_sizes, *, config: KernelConfig, out_dtype: to
                    gateup: bool = False, group_offset=None, workspace_out: list | None = None) -> torch.Tensor:
   """out[m,n] = lhs[m,k] . rhs[g,k,n]   (trans_rhs: out[m,k] = lhs[m,n] . rhs[g,k,n]^T).
 
-  `rhs_scale` is [g,n] / [g,1,n], or [g,blocks,n] with `blocks` scale blocks along k (streaming small-m
-  kernel only). `rhs_bias` ([g,n] or [g,1,n]) is added to the scaled result before the activation. `gateup`: rhs
+  `rhs_scale` is [g,n] / [g,1,n], or [g,blocks,n] with `blocks` scale blocks along k, or (fp8 x fp8) [g,blocks,n/128] with
+  a scale per block of k and 128 columns. `rhs_bias` ([g,n] or [g,1,n]) is added to the scaled result before the activation. `gateup`: rhs
   columns are [gate | up] and out[m,n/2] = activation(gate part) * (up part) (base.py:211-217).
   `group_offset` (device int32 tensor of one element): `group_sizes` covers every group of the job, rhs holds the
   groups [offset, offset + g) of them, and the rows of all other groups come out zero (the call of one
@@ -272,12 +272,14 @@ def ragged_dot_fwd(lhs, rhs, group_sizes, *, config: KernelConfig, out_dtype: to
       lhs_scale = lhs_scale.to(torch.float32).contiguous().view(-1)
     if lhs_scale.numel() != m * lhs_scale_blocks:
       raise NotImplementedError("lhs scale must be one f32 per row (or per row and k-block)")
-  scale_blocks = 1
+  scale_blocks = scale_cols = 1
   if rhs_scale is not None:
     if rhs_scale.dim() == 3 and rhs_scale.shape[1] > 1:
       scale_blocks = int(rhs_scale.shape[1])
+      if rhs_scale.shape[2] * 128 == n:
+        scale_cols = 128
     rhs_scale = rhs_scale.to(torch.float32).contiguous().view(-1)
-    if rhs_scale.numel() != G * scale_blocks * n or k % scale_blocks:
+    if rhs_scale.numel() * scale_cols != G * scale_blocks * n or k % scale_blocks:
       raise NotImplementedError("rhs scale must be one f32 per (group, column) or per (group, k-block, column)")
   if lhs_scale_blocks != 1 and lhs_scale_blocks != scale_blocks:
     raise NotImplementedError("lhs and rhs scales must have the same number of blocks along k")
@@ -314,6 +316,14 @@ def ragged_dot_fwd(lhs, rhs, group_sizes, *, config: KernelConfig, out_dtype: to
 
     def launch(p, out_ptr, ws_ptr, stream):
       return fwd(p[0], p[1], p[2], p[4], p[5], out_ptr, ws_ptr, m, k, n, G, a_code, b_code, o_code, mode, act_code, cfg, stream)
+  elif scale_cols != 1:
+    if gateup:
+      raise NotImplementedError("gate-up fusion takes one rhs scale per (group, column)")
+    num_sizes, tiles = gs.numel(), lib.tkx_ragged_dot_fwd_scale_tiles
+
+    def launch(p, out_ptr, ws_ptr, stream):
+      return tiles(p[0], p[1], p[2], p[3], p[4], p[5], p[6], out_ptr, ws_ptr, m, k, n, G, num_sizes, scale_blocks,
+                   scale_cols, a_code, b_code, o_code, act_code, cfg, stream)
   else:
     num_sizes, glu = gs.numel(), 1 if gateup else 0
     fused = lib.tkx_ragged_dot_fwd_fused
@@ -361,7 +371,8 @@ for _bits in range(2, 8):
     _QMAX[getattr(torch, f"int{_bits}")] = float(2 ** (_bits - 1) - 1)  # sub-byte integers live in int8 storage
 
 
-def quantize(x: torch.Tensor, qtype: torch.dtype, tile_shape, bound: float | None = None) -> tuple[torch.Tensor, torch.Tensor]:
+def quantize(x: torch.Tensor, qtype: torch.dtype, tile_shape, bound: float | None = None,
+             scale_by_block: bool = False) -> tuple[torch.Tensor, torch.Tensor]:
   """(qvalue, scale) of the absmax quantisation of `x` with one scale per tile of `tile_shape`
   (`qwix.quantize(x, qtype, tiled_axes=dict(enumerate(tile_shape)))`, quantization.py:65-78):
   scale = absmax(tile) / bound (1 for an all-zero tile), qvalue = round_to_nearest_even(x / scale), saturated at qmax.
@@ -370,7 +381,9 @@ def quantize(x: torch.Tensor, qtype: torch.dtype, tile_shape, bound: float | Non
   x f32, bf16 or f16: [rows, cols] with tiles one row tall and a multiple of 8 columns wide, or several rows tall and
   1 column or a multiple of 8 columns wide; or weights [g, k, n] with a tile (1, t_k, t_n) (taken as g * k rows) or a
   tile (t_g, k, t_n) of whole groups (one scale per tensor: (g, k, n)). qtype int8, fp8 (e4m3fn) or a sub-byte integer
-  (int4: values in [-7, 7], kept in int8 storage)."""
+  (int4: values in [-7, 7], kept in int8 storage).
+  `scale_by_block` (x [rows, cols], tiles one row tall): the scales lie in memory block by block, [cols / t_c, rows], as
+  the products with scale blocks along k read them; the tensor returned is the [rows, cols / t_c] view of that."""
   _log_launch(None)
   _require_cuda(x)
   lib = _lib.load()
@@ -394,6 +407,13 @@ def quantize(x: torch.Tensor, qtype: torch.dtype, tile_shape, bound: float | Non
   x = x.contiguous()
   storage = torch.float8_e4m3fn if qtype == torch.float8_e4m3fn else torch.int8
   qvalue = torch.empty(x.shape, dtype=storage, device=x.device)
+  if scale_by_block and x.dim() == 2 and t_r == 1 and rows * (cols // t_c) < 2**31:
+    scale = torch.empty((cols // t_c, rows), dtype=torch.float32, device=x.device)
+    with _on_device(x.device):
+      _lib.check(lib.tkx_quantize_scales_transposed(
+          _ptr(x), _ptr(qvalue), _ptr(scale), rows, cols, t_c, dtype_code(x.dtype), dtype_code(storage),
+          ctypes.c_float(_QMAX[qtype]), ctypes.c_float(0.0 if bound is None else bound), _stream(x.device)))
+    return qvalue, scale.t()
   scale = torch.empty(tuple(d // t for d, t in zip(x.shape, tile_shape)), dtype=torch.float32, device=x.device)
   with _on_device(x.device):
     st = lib.tkx_quantize(_ptr(x), _ptr(qvalue), _ptr(scale), rows, cols, t_r, t_c, dtype_code(x.dtype), dtype_code(storage),
