@@ -2742,3 +2742,33 @@ def test_quantised_scales_laid_out_by_block(rows, cols, t_c, device):
   qt, st = hip_ops.quantize(x, torch.float8_e4m3fn, (1, t_c), scale_by_block=True)
   assert st.shape == s.shape and st.t().is_contiguous() and torch.equal(st, s)
   assert torch.equal(q.view(torch.uint8), qt.view(torch.uint8))
+
+
+# ---- weights that no cache holds to the next call ------------------------------------------------------------
+@pytest.mark.parametrize("variant,gateup", [((256, 256, 64, 2, 4, 3), False), ((128, 256, 64, 2, 4, 3), False),
+                                            ((32, 128, 64, 1, 4, 4), False), ((64, 256, 64, 2, 2, 3), True)])
+def test_large_weights_give_the_bits_of_their_parts(variant, gateup, device):
+  """Past 256 MB the weights of a group with one task are loaded past the caches: groups of one task, of several, of one
+  row, empty ones and rows of no group against the same groups in two calls on smaller weights."""
+  G, k, n = 34, 2048, 2048
+  assert G * k * n * 2 >= 256 << 20 > (G // 2) * k * n * 2
+  gen = torch.Generator(device=device).manual_seed(3)
+  sizes = ([5, 0, 300, 1, 33, 128] * 6)[:G]
+  m = sum(sizes) + 11
+  lhs = torch.randn(m, k, device=device, generator=gen).to(torch.bfloat16)
+  rhs = (torch.randn(G, k, n, device=device, generator=gen) * k ** -0.5).to(torch.bfloat16)
+  gs = torch.tensor(sizes, dtype=torch.int32, device=device)
+  op = hip.HipRaggedDot(config=hip.Config(*variant))
+  kw = dict(fuse_gateup_activation="silu") if gateup else {}
+  out = op(lhs, rhs, group_sizes=gs, **kw)
+  half, rows = G // 2, sum(sizes[:G // 2])
+  first = op(lhs[:rows], rhs[:half], group_sizes=gs[:half], **kw)
+  second = op(lhs[rows:], rhs[half:], group_sizes=gs[half:], **kw)
+  assert torch.equal(out, torch.cat([first, second]))
+  if not gateup:
+    back = hip.HipRaggedDot(config=hip.Config(128, 256, 64, 2, 4, 3))
+    dims = base.TRANS_RHS_RAGGED_DOT_DIM_NUMS
+    grad = back(out, rhs, group_sizes=gs, ragged_dot_dimension_numbers=dims)
+    parts = [back(out[:rows], rhs[:half], group_sizes=gs[:half], ragged_dot_dimension_numbers=dims),
+             back(out[rows:], rhs[half:], group_sizes=gs[half:], ragged_dot_dimension_numbers=dims)]
+    assert torch.equal(grad, torch.cat(parts))

@@ -143,6 +143,11 @@ bool plan_pays(KernelMode mode, int32_t dtype, int64_t num_groups, int64_t sizes
                                        (workgroups > 8192 && (mode != kDrhs || dtype == TKX_F32)));
 }
 
+// Bytes of the memory-side cache. Weights of at least as many are not there any more when the next call wants them, and are
+// loaded past it where one task of a group reads them, i.e. once (GemmKernel::run): allocating every line there and in L2 is
+// what a product bound by them loses a tenth of its rate to.
+constexpr int64_t kMemorySideCache = 256 << 20;
+
 bool valid_out_dtype(int d) { return d == TKX_F32 || d == TKX_BF16 || d == TKX_F16; }
 
 // Device address of `scratch` on the current device, looked up once per device (each GPU holds its own copy of
@@ -438,6 +443,7 @@ int32_t fwd_impl(const void* lhs, const void* rhs, const int32_t* group_sizes, c
   p.scale_blocks = subk ? (int32_t)rhs_scale_blocks : 1;
   p.log2_block_rows = log2_block_rows;
   p.wide_scales = rhs_scale_cols != 1;
+  p.stream_weights = num_groups * p.b_group_stride * rb >= kMemorySideCache;
   if (slots > 0x7fffff00LL) return set_error(TKX_ERR_UNSUPPORTED, "too many tiles");
   // Extra workgroups zero the rows past the last group (and before the first, with a group offset);
   // they exit at once when there are none.

@@ -158,6 +158,7 @@ struct GemmParams {
   int32_t grid_tile_width;
   int32_t out_dtype, activation;
   int32_t scale_blocks, log2_block_rows;  // kFwdSubK: b_scale is [g, scale_blocks, n]; rows of k per block = 1 << log2
+  int32_t stream_weights;  // fwd/dlhs: the weights of a group with one task are loaded with the non-temporal policy
   int32_t wide_scales;  // ... or, not 0: [g, scale_blocks, n / 128]
 };
 

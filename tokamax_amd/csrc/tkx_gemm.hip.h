@@ -157,7 +157,7 @@ __device__ __forceinline__ int mc_swizzle(int krow) {
   int f;
   if constexpr (E == kEF32) f = ((krow >> 2) & 1) << 2;
   else if constexpr (E == kEBF16 || E == kEF16) f = ((krow & 3) << 1) | ((krow >> 3) & 1);
-  else f = krow & 7;
+  else f = NG < 8 ? krow >> 1 : krow & 7;  // (rows of 128 bytes: two to a bank line)
   return f & (NG - 1);
 }
 template <int ROW_BYTES, int E>
@@ -408,6 +408,14 @@ __device__ __forceinline__ void direct_load_16(const unsigned char* sbase, uint3
   asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds), "v"(voff), "s"(sbase)
                : "memory", "m0");
 }
+// The same; `once`, not 0: with the non-temporal policy, which leaves nothing of the line behind in L2 and in the memory-side
+// cache. (Branches inside the statement: a compile-time choice would be a second copy of the k loop.)
+__device__ __forceinline__ void direct_load_16(const unsigned char* sbase, uint32_t voff, unsigned lds, int once) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_cmp_eq_u32 %3, 0\n\ts_cbranch_scc1 .Ltkx_keep%=\n\tglobal_load_lds_dwordx4 %1, %2 nt\n\t"
+               "s_branch .Ltkx_done%=\n.Ltkx_keep%=:\n\tglobal_load_lds_dwordx4 %1, %2\n.Ltkx_done%=:" ::"s"(lds), "v"(voff),
+               "s"(sbase), "s"(once)
+               : "memory", "m0", "scc");
+}
 // 4 bytes per lane: LDS[lds + 4*lane] <- *(sbase + voff)
 __device__ __forceinline__ void direct_load_4(const unsigned char* sbase, uint32_t voff, unsigned lds) {
   asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, %2" ::"s"(lds), "v"(voff), "s"(sbase)
@@ -497,15 +505,15 @@ struct DirectLoader {
 
   // Instruction i (0 <= i < PER) of this wave's share: `base` = wave-uniform pointer of the k-step,
   // `tile_lds` = LDS byte address of the destination tile (wave-uniform).
-  __device__ __forceinline__ void issue_one(int i, const unsigned char* base, unsigned tile_lds, int wave) const {
+  // ONCE: the kernel has loads that may be of lines nobody else reads (`once`).
+  template <bool ONCE = false>
+  __device__ __forceinline__ void issue_one(int i, const unsigned char* base, unsigned tile_lds, int wave, int once = 0) const {
     const int j = i * NWAVES + wave;
     if (INSTRS % NWAVES != 0 && j >= INSTRS) return;
-    if constexpr (STRIDED) direct_load_16(base + i * stride, voff[0], tile_lds + j * 1024);
-    else direct_load_16(base, voff[i], tile_lds + j * 1024);
-  }
-  __device__ __forceinline__ void issue(const unsigned char* base, unsigned tile_lds, int wave) const {
-#pragma unroll
-    for (int i = 0; i < PER; ++i) issue_one(i, base, tile_lds, wave);
+    const unsigned char* const from = STRIDED ? base + i * stride : base;
+    const uint32_t off = voff[STRIDED ? 0 : i];
+    if constexpr (ONCE) direct_load_16(from, off, tile_lds + j * 1024, once);
+    else direct_load_16(from, off, tile_lds + j * 1024);
   }
 };
 
@@ -735,9 +743,9 @@ struct GemmKernel {
   static constexpr bool SUBP = SUBK && (EA == kEF8 || EA == kEI8);
   static_assert(!SUBK || ((EB == kEI8 || EB == kEF8 || EB == kEI4) &&
                           (EA == kEBF16 || (SUBP && EB == EA) || (EA == kEF8 && EB == kEI4 && BK == 128) ||
-                           (EA == kEI8 && EB == kEI4)) && BN == 256),
+                           (EA == kEI8 && EB == kEI4)) && (BN == 256 || BN == 128)),
                 "per-k-block scales: bf16 lhs with int8, packed int4 or fp8 weights, fp8 x fp8, int8 x int8 or fp8 x packed int4"
-                " (whose row sums come per 128-deep k-step); one 1 KB scale row per k-step");
+                " (whose row sums come per 128-deep k-step); one scale row of 512 or 1024 bytes per k-step");
   static constexpr int BNO = GLU ? BN / 2 : BN;  // output columns of a tile
   static constexpr int EC = EA;  // MFMA type follows A; B may be stored narrower (int8 weights)
   // Packed int4 weights: a B stage is a byte tile of half the depth; a lane's transposing read of 8 bytes of its
@@ -818,6 +826,7 @@ struct GemmKernel {
   static constexpr int NLOAD = WM * WN;
   typedef DirectLoader<LA, EA, BM, BK, NLOAD> DirA;
   typedef DirectLoader<LB, EBS, BN, BKB, NLOAD> DirB;
+  static constexpr bool ONCE = MODE != kDrhs;
   static constexpr int SCALE_BYTES = (SUBK && !SUBP) ? BN * 4 : 0;  // kFwdSubK: the k-step's scale row behind its two tiles
   static constexpr int STAGE_BYTES = StageA::BYTES + StageB::BYTES + SCALE_BYTES;
   // fp8 x fp8: the scales of a k-step (BN weight-column scales, then BM lhs-row scales) are still needed when its
@@ -921,6 +930,7 @@ struct GemmKernel {
     // first load, a training step of three kernels that take turns was 1 % slower, 535 against 530 us; this way even.)
     auto planned = [&](int i) { return __builtin_amdgcn_readfirstlane(p.plan[i]); };
     int group, row0, act_start, act_end, col0, kc_begin, kc_end;
+    int once = 0;  // (fwd/dlhs) not 0: this task is its group's only one, so that nobody else reads its panels of weights
     int part = 0, parts = 1, split_unit = 0;  // (fwd/dlhs) this workgroup contracts part `part` of `parts` of its tile
     if constexpr (MODE != kDrhs) {
       // (kFwdSubK with lhs scales: a tile's scales are fetched four rows at a time)
@@ -1057,6 +1067,7 @@ struct GemmKernel {
         row0 = rows.row0;
         act_start = rows.first;
         act_end = rows.end;
+        if (tasks == 1) once = p.stream_weights;
       }
       col0 = nt * BNO;
       kc_begin = 0;
@@ -1185,7 +1196,7 @@ struct GemmKernel {
         da.issue_one(q, uniform_pointer(gA0 + dstep * stepA), smem_lds + stage * A_BYTES, wave);
       };
       auto issue_b = [&](int q, int step, int stage) {
-        db.issue_one(q, uniform_pointer(gB0 + step * stepB), smem_lds + B_REGION + stage * B_BYTES, wave);
+        db.template issue_one<ONCE>(q, uniform_pointer(gB0 + step * stepB), smem_lds + B_REGION + stage * B_BYTES, wave, once);
       };
       // Prologue, in the order of the steady state (steps -LOOK .. -1).
 #pragma unroll
@@ -1233,7 +1244,7 @@ struct GemmKernel {
                                                      [&] { barrier_after_direct_loads<(ODD ? kOdd : kEven)>(); },
                                                      [&](int q) {
                                                        if (ODD && q < PA) da.issue_one(q, src_a, dst_a, wave);
-                                                       else db.issue_one(q - (ODD ? PA : 0), src_b, dst_b, wave);
+                                                       else db.template issue_one<ONCE>(q - (ODD ? PA : 0), src_b, dst_b, wave, once);
                                                      });
           } else {
             // (After the last step the reads fetch fragments nobody uses, from LDS that is there.)
@@ -1246,7 +1257,7 @@ struct GemmKernel {
                                      }
                                      if (kt + HB < nfull) {
 #pragma unroll
-                                       for (int q = 0; q < PB; ++q) db.issue_one(q, src_b, dst_b, wave);
+                                       for (int q = 0; q < PB; ++q) db.template issue_one<ONCE>(q, src_b, dst_b, wave, once);
                                      }
                                    },
                                    [](int) {});
@@ -1288,7 +1299,7 @@ struct GemmKernel {
       // the last column re-read the last four (their products are never stored).
       const unsigned char* const gS0 =
           SUBK ? reinterpret_cast<const unsigned char*>(p.b_scale + (int64_t)group * p.scale_blocks * (WB ? p.nb_ext >> 7 : p.nb_ext)) : nullptr;
-      constexpr int SCALE_LANES = 64 / NLOAD;  // lanes of a wave that fetch 16 bytes of the scale row each
+      constexpr int SCALE_LANES = BN / 4 / NLOAD;  // lanes of a wave that fetch 16 bytes of the scale row each
       const uint32_t scale_voff = WB ? (uint32_t)(min(col0 + wn * WTN, p.nb_ext - 1) >> 7) * 4u
                                   : SUBK ? (uint32_t)min(col0 + 4 * (wave * SCALE_LANES + lane), p.nb_ext - 4) * 4u : 0u;
       // (fp8 x fp8) lhs scales [scale_blocks, m]: the BM rows of the tile, 4 per lane; chunks past the last row
@@ -1317,7 +1328,7 @@ struct GemmKernel {
       };
       auto issue_slot = [&](int q, const StepPtrs& sp) {
         if (q < DirA::PER) da.issue_one(q, sp.a, sp.lds, wave);
-        else if (q < DirA::PER + DirB::PER) db.issue_one(q - DirA::PER, sp.b, sp.lds + StageA::BYTES, wave);
+        else if (q < DirA::PER + DirB::PER) db.template issue_one<ONCE>(q - DirA::PER, sp.b, sp.lds + StageA::BYTES, wave, once);
         else if (SUBK && q == DirA::PER + DirB::PER) {
           const unsigned dst = SUBP ? sp.ring : sp.lds + StageA::BYTES + StageB::BYTES;
           if constexpr (WB) {
