@@ -743,9 +743,9 @@ struct GemmKernel {
   static constexpr bool SUBP = SUBK && (EA == kEF8 || EA == kEI8);
   static_assert(!SUBK || ((EB == kEI8 || EB == kEF8 || EB == kEI4) &&
                           (EA == kEBF16 || (SUBP && EB == EA) || (EA == kEF8 && EB == kEI4 && BK == 128) ||
-                           (EA == kEI8 && EB == kEI4)) && (BN == 256 || BN == 128)),
+                           (EA == kEI8 && EB == kEI4)) && BN == 256),
                 "per-k-block scales: bf16 lhs with int8, packed int4 or fp8 weights, fp8 x fp8, int8 x int8 or fp8 x packed int4"
-                " (whose row sums come per 128-deep k-step); one scale row of 512 or 1024 bytes per k-step");
+                " (whose row sums come per 128-deep k-step); one 1 KB scale row per k-step");
   static constexpr int BNO = GLU ? BN / 2 : BN;  // output columns of a tile
   static constexpr int EC = EA;  // MFMA type follows A; B may be stored narrower (int8 weights)
   // Packed int4 weights: a B stage is a byte tile of half the depth; a lane's transposing read of 8 bytes of its

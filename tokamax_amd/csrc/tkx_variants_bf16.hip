@@ -28,7 +28,9 @@ static const Variant kVariants[] = {
     GLU(256, 256, 64, 2, 4, 2),
     GLU(128, 256, 64, 2, 4, 3),
     GLU(64, 256, 64, 2, 2, 3),
+    GLU(64, 128, 64, 2, 2, 3),
     GLU(32, 256, 64, 1, 4, 3),
+    GLU(32, 128, 64, 1, 2, 3),
     DRHS(256, 256, 64, 2, 4, 2),
     DRHS(256, 256, 32, 2, 4, 4),
     DRHS(128, 256, 64, 2, 4, 3),

@@ -950,6 +950,10 @@ class HipRaggedDot(base.RaggedDot):
       # Gate-up fusion takes whole k-steps (16-bit weights: 64 deep, or 32 in the 256 x 256 x 32 tile, the only one for
       # k % 64 == 32). Where no variant's divides the contraction the launch declines the call.
       usable = [v for v in usable if contraction % v[2] == 0] or usable
+    narrow = []  # (gate-up over one group: see below)
+    if mode == 3 and key[1:] == (_lib.TKX_BF16, _lib.TKX_BF16):
+      narrow = [v for v in usable if v[1] == 128]
+      usable = [v for v in usable if v[1] != 128] or usable
     # Rows per group decide the m-tile: a tile much taller than a group wastes MFMA work on rows
     # that are masked out at the store; a short tile re-reads the weights more often.
     rows_per_group = rows / max(num_groups, 1) if mode != 2 else rows
@@ -990,7 +994,7 @@ class HipRaggedDot(base.RaggedDot):
       if tiles(want_m, want_n) < _COMPUTE_UNITS // 2:
         # (gate-up fusion and scales per k-block have 256-column tiles only: of the shapes there are)
         shapes = ((256, 256), (128, 256), (128, 128), (64, 128), (32, 128)) if mode == 0 else sorted(
-            {(v[0], v[1]) for v in usable if v[0] > 16}, key=lambda t: (-t[0] * t[1], -t[1]))
+            {(v[0], v[1]) for v in usable if v[0] > 16 and v[1] == 256}, key=lambda t: (-t[0] * t[1], -t[1]))
         want_m, want_n = next((t for t in shapes[:-1] if t[0] <= want_m and tiles(*t) >= _COMPUTE_UNITS), shapes[-1])
     if mode in (0, 1) and key[1] == _lib.TKX_F32:
       # f32 operands run on the f32 MFMAs at a sixteenth of the bf16 rate: loads never bound them, and the 32-row tile
@@ -1075,8 +1079,13 @@ class HipRaggedDot(base.RaggedDot):
       # With several groups the rules stay so far: on 40 shapes (2 to 256 groups, even and Zipf sizes, caches flushed) they
       # are 7 % behind the fastest tile on average and 38 % at worst (2 groups of 150 rows), this model 2 % on average.
       fit = dict(_TILE_COST_FIT, tail_floor=1.0)
-      bm, bn, bk, wm, wn, ns = min(usable, key=lambda v: (
-          round(_tile_cost(v, 1, rows, cols, contraction, 1, 0, fit), 3), -v[2], -v[5]))
+      cost = lambda v: (round(_tile_cost(v, 1, rows, cols, contraction, 1, 0, fit), 3), -v[2], -v[5])
+      bm, bn, bk, wm, wn, ns = min(usable, key=cost)
+      if narrow and bm <= 64 and -(-rows // bm) * -(-cols // bn) < 0.85 * _COMPUTE_UNITS:
+        # Few rows, bound by the weights: such a launch leaves CUs without a workgroup, and a CU streams weights at no more than 45 to 50 GB/s: tiles of half
+        # the columns bring in more of them. k = 4096, 28672 columns, 1 to 32 rows: 58.4-59.9 -> 47.3-48.1 us; k = 2048,
+        # 8192 columns, 32 and 128 rows: 26.9 -> 20.4, 26.0 -> 20.4. (Where the wide tiles fill the chip they stay.)
+        bm, bn, bk, wm, wn, ns = min(narrow, key=cost)
     # grid_tile_width m-tasks of one group run side by side on an n-panel of its weights (a span never
     # crosses a group, so small groups simply get short spans). With the 32 tiles an XCD runs at a
     # time, 8 wide x 4 n-panels needs the fewest distinct operand panels in its L2; 16 wide measured
