@@ -143,10 +143,15 @@ bool plan_pays(KernelMode mode, int32_t dtype, int64_t num_groups, int64_t sizes
                                        (workgroups > 8192 && (mode != kDrhs || dtype == TKX_F32)));
 }
 
-// Bytes of the memory-side cache. Weights of at least as many are not there any more when the next call wants them, and are
-// loaded past it where one task of a group reads them, i.e. once (GemmKernel::run): allocating every line there and in L2 is
-// what a product bound by them loses a tenth of its rate to.
+// Bytes of the memory-side cache. Where the groups that m rows can reach have at least as many bytes of weights, these are not
+// there any more when the next call wants them, and are loaded past it where one task of a group reads them, i.e. once
+// (GemmKernel::run): allocating every line there and in L2 is what a product bound by them loses a tenth of its rate to. (Four
+// tokens over 128 experts of 805 MB reach 32 of them, 201 MB: the expert block 97 us with its weights kept, 107 past the
+// caches.)
+// Whole lines only: of a line that two tiles share both fetch all of it then (1312 rows over 32 groups, k = 2560, rows of
+// 4816 bytes, fp8: 122 -> 129 us).
 constexpr int64_t kMemorySideCache = 256 << 20;
+constexpr int64_t kLineBytes = 128;
 
 bool valid_out_dtype(int d) { return d == TKX_F32 || d == TKX_BF16 || d == TKX_F16; }
 
@@ -443,7 +448,8 @@ int32_t fwd_impl(const void* lhs, const void* rhs, const int32_t* group_sizes, c
   p.scale_blocks = subk ? (int32_t)rhs_scale_blocks : 1;
   p.log2_block_rows = log2_block_rows;
   p.wide_scales = rhs_scale_cols != 1;
-  p.stream_weights = num_groups * p.b_group_stride * rb >= kMemorySideCache;
+  p.stream_weights = (num_groups < m ? num_groups : m) * p.b_group_stride * rb >= kMemorySideCache &&
+                     (uintptr_t)rhs % kLineBytes == 0 && n * rb % kLineBytes == 0 && (!gateup || cols * rb % kLineBytes == 0);
   if (slots > 0x7fffff00LL) return set_error(TKX_ERR_UNSUPPORTED, "too many tiles");
   // Extra workgroups zero the rows past the last group (and before the first, with a group offset);
   // they exit at once when there are none.

@@ -826,7 +826,9 @@ struct GemmKernel {
   static constexpr int NLOAD = WM * WN;
   typedef DirectLoader<LA, EA, BM, BK, NLOAD> DirA;
   typedef DirectLoader<LB, EBS, BN, BKB, NLOAD> DirB;
-  static constexpr bool ONCE = MODE != kDrhs;
+  // Kernels whose weights may be lines that nobody else reads. (Packed int4 weights are bound by their conversion: 2 to 5 % for
+  // the choice at every load, nothing gained.)
+  static constexpr bool ONCE = MODE != kDrhs && EB != kEI4;
   static constexpr int SCALE_BYTES = (SUBK && !SUBP) ? BN * 4 : 0;  // kFwdSubK: the k-step's scale row behind its two tiles
   static constexpr int STAGE_BYTES = StageA::BYTES + StageB::BYTES + SCALE_BYTES;
   // fp8 x fp8: the scales of a k-step (BN weight-column scales, then BM lhs-row scales) are still needed when its
