@@ -2772,3 +2772,56 @@ def test_large_weights_give_the_bits_of_their_parts(variant, gateup, device):
     parts = [back(out[:rows], rhs[:half], group_sizes=gs[:half], ragged_dot_dimension_numbers=dims),
              back(out[rows:], rhs[half:], group_sizes=gs[half:], ragged_dot_dimension_numbers=dims)]
     assert torch.equal(grad, torch.cat(parts))
+
+
+@pytest.mark.parametrize("kind", ["fp8", "fp8_k128", "grad", "grad_lhs_only", "grad_trans_rhs"])
+def test_repeated_calls_behind_a_quantisation_or_under_autograd_are_remembered(kind, device):
+  """A second call of a kind (activations quantised on the way, a gradient wanted) takes the remembered launch: the bits of
+  a first call on the same values, whatever changed since: values, group sizes, which operand wants its gradient."""
+  gen = torch.Generator(device=device).manual_seed(17)
+  G, m, k, n = 4, 96, 256, 256
+  trans = kind == "grad_trans_rhs"
+  kw = dict(ragged_dot_dimension_numbers=base.TRANS_RHS_RAGGED_DOT_DIM_NUMS) if trans else {}
+
+  def inputs(sizes):
+    lhs = torch.randn(m, n if trans else k, device=device, generator=gen).to(torch.bfloat16)
+    rhs = (torch.randn(G, k, n, device=device, generator=gen) * k ** -0.5).to(torch.bfloat16)
+    dout = torch.randn(m, k if trans else n, device=device, generator=gen).to(torch.bfloat16)
+    return lhs, rhs, dout, torch.tensor(sizes, dtype=torch.int32, device=device)
+
+  def call(op, lhs, rhs, dout, gs):
+    if kind.startswith("fp8"):
+      tiled = {1: 128} if kind == "fp8_k128" else None
+      w = tokamax_amd.AsQArray(rhs, torch.float8_e4m3fn, tiled_axes={0: 1, 1: 128, 2: 128} if tiled else {0: 1, 2: 1}).as_qarray()
+      a = tokamax_amd.AsQArray(lhs, torch.float8_e4m3fn, channelwise_axes=(0,), tiled_axes=tiled)
+      return (op(a, w, group_sizes=gs, preferred_element_type=torch.bfloat16),)
+    lhs, rhs = lhs.clone().requires_grad_(True), rhs.clone().requires_grad_(kind != "grad_lhs_only")
+    out = op(lhs, rhs, group_sizes=gs, **kw)
+    assert out.requires_grad
+    out.backward(dout)
+    assert (rhs.grad is not None) == rhs.requires_grad
+    return (out.detach(), lhs.grad) + ((rhs.grad,) if rhs.requires_grad else ())
+
+  op = hip.HipRaggedDot()
+  call(op, *inputs([30, 0, 41, 20]))
+  assert len(op.__dict__["_plans"]) == 1
+  for sizes in ([30, 0, 41, 25], [0, 96, 0, 0], [1, 2, 3, 4]):
+    given = inputs(sizes)
+    got = call(op, *given)
+    assert len(op.__dict__["_plans"]) == 1
+    for a, b in zip(got, call(hip.HipRaggedDot(), *given)):
+      assert torch.equal(a, b)
+  if kind.startswith("grad"):
+    # an activation given as a callable, and no gradient wanted: ways of their own
+    lhs, rhs, dout, gs = given
+    assert not op(lhs, rhs, group_sizes=gs, **kw).requires_grad
+    with torch.no_grad():
+      assert not op(lhs.clone().requires_grad_(True), rhs, group_sizes=gs, **kw).requires_grad
+    # tensors saved for the backward pass go through the caller's hooks, both times alike
+    seen = []
+    with torch.autograd.graph.saved_tensors_hooks(lambda t: seen.append(t.shape) or t, lambda t: t):
+      call(op, *given)
+      again = list(seen)
+      seen.clear()
+      call(hip.HipRaggedDot(), *given)
+    assert again == seen

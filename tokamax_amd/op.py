@@ -444,6 +444,7 @@ class _VjpCall:
   names: tuple         # those tensors' arguments
   config: Any
   return_residuals: bool
+  forward: Any = None  # what `_fwd` does with the tensors, where the caller has that at hand: tensors -> the result
 
   def full(self, tensors) -> dict:
     full = dict(self.arguments)
@@ -457,9 +458,12 @@ class _VjpFunction(torch.autograd.Function):
 
   @staticmethod
   def forward(ctx, call: _VjpCall, *ts):
-    full = call.full(ts)
-    full["return_residuals"] = True
-    out, residuals = call.op._fwd(config=call.config, **full)  # pylint: disable=protected-access
+    if call.forward is not None:
+      out = residuals = call.forward(*ts)
+    else:
+      full = call.full(ts)
+      full["return_residuals"] = True
+      out, residuals = call.op._fwd(config=call.config, **full)  # pylint: disable=protected-access
     # Inputs and residuals go through save_for_backward, and the output is not kept at all (`vjp` does not use
     # it): a tensor this function returns, held as a plain attribute of ctx, would close the cycle
     # out -> grad_fn -> ctx -> out, and the activations would live until the cyclic collector runs.
@@ -505,3 +509,9 @@ def _call_with_vjp(op: Op, ba: BoundArguments, config, return_residuals: bool):
   tensors = [arguments[k] for k in names]
   arguments.update(dict.fromkeys(names))
   return _VjpFunction.apply(_VjpCall(op, arguments, names, config, return_residuals), *tensors)
+
+
+def call_with_vjp(op: Op, arguments: dict, names: tuple, forward, *tensors):
+  """`_call_with_vjp` for a caller that has bound such a call before and knows how to run it: `arguments` in signature
+  order with None in the place of `names`, `forward(*tensors)` the result (which is its own residual)."""
+  return _VjpFunction.apply(_VjpCall(op, arguments, names, None, False, forward), *tensors)

@@ -593,21 +593,26 @@ def _sizes_array(group_sizes):
 
 def _make_plan(records, out, lhs, rhs, group_sizes):
   """The shortcut for calls like the one that left `records` and returned `out`, or None if that call was more than
-  one launch of a product on the caller's own buffers."""
-  if len(records) != 1 or not isinstance(records[0], hip_ops.Launch) or records[0].out is not out:
+  one launch of a product on the caller's own buffers and on what its `AsQArray` operands were quantised to."""
+  if not records or not isinstance(records[-1], hip_ops.Launch) or type(out) is not torch.Tensor:
     return None
-  record = records[0]
+  record, quantised = records[-1], records[:-1]
+  if record.out.data_ptr() != out.data_ptr() or record.out.shape != out.shape or record.out.dtype != out.dtype:
+    return None
   if out.device.index != torch.cuda.current_device():
     return None  # (the launch ran under a device guard; the shortcut has none)
 
-  def leaves(lhs, rhs, group_sizes):
-    return ((lhs,) if type(lhs) is torch.Tensor else (lhs.qvalue, lhs.scale)) + \
-           ((rhs,) if type(rhs) is torch.Tensor else (rhs.qvalue, rhs.scale)) + (group_sizes,)
-
-  given = [t.data_ptr() for t in leaves(lhs, rhs, group_sizes)]
+  by_source = {id(r.source): r for r in quantised if isinstance(r, hip_ops.Quantised)}
+  operands = [by_source.get(id(x.value)) if type(x) is AsQArray else None for x in (lhs, rhs)]
+  if len(quantised) != sum(r is not None for r in operands) or len(quantised) != sum(type(x) is AsQArray for x in (lhs, rhs)):
+    return None  # (a pass over an operand that is not its quantisation)
+  arguments = tuple(None if r is None else r.arguments for r in operands)
+  parts = lambda x: (x,) if type(x) is torch.Tensor else (x.qvalue, x.scale)
+  given = [t.data_ptr() for x, r in zip((lhs, rhs), operands) for t in parts(r if r is not None else x)]
+  given.append(group_sizes.data_ptr())
   if 0 in given or len(set(given)) != len(given):
     return None
-  source = []  # for every pointer of the launch: which of the caller's tensors it was, -1 for an absent operand
+  source = []  # for every pointer of the launch: which of the call's tensors it was, -1 for an absent operand
   for p in record.pointers:
     if p == 0:
       source.append(-1)
@@ -620,7 +625,10 @@ def _make_plan(records, out, lhs, rhs, group_sizes):
   shape, dtype, device = tuple(out.shape), out.dtype, out.device
 
   def plan(lhs, rhs, group_sizes):
-    tensors = leaves(lhs, rhs, group_sizes)
+    tensors = ()
+    for x, args in ((lhs, arguments[0]), (rhs, arguments[1])):
+      tensors += parts(x) if args is None else hip_ops.quantize(x.value, **args)
+    tensors += (group_sizes,)
     result = torch.empty(shape, dtype=dtype, device=device)
     ws = new_workspace()
     status = launch([0 if i < 0 else tensors[i].data_ptr() for i in source], result.data_ptr(), ws.data_ptr(),
@@ -628,6 +636,21 @@ def _make_plan(records, out, lhs, rhs, group_sizes):
     if status != 0:
       _lib.check(status)
     return result
+
+  return plan
+
+
+def _make_differentiated_plan(ba, forward):
+  """The shortcut for differentiated calls like `ba`, whose forward is one launch (`forward`, a plan as above)."""
+  self, template, representative = ba.op, dict(ba.arguments), None
+  if type(template["group_sizes"]) is GroupSizes:
+    representative = template["group_sizes"].repr_value_or_total_size
+  template.update(lhs=None, rhs=None, group_sizes=None)
+
+  def plan(lhs, rhs, group_sizes):
+    wrapped = group_sizes if representative is None else GroupSizes(group_sizes, representative)
+    return op.call_with_vjp(self, dict(template, group_sizes=wrapped), ("lhs", "rhs"),
+                            lambda a, b: forward(a, b, group_sizes), lhs, rhs)
 
   return plan
 
@@ -659,18 +682,19 @@ class HipRaggedDot(base.RaggedDot):
   # -- eager fast path -------------------------------------------------------------------------
   def __call__(self, lhs, rhs, *, return_residuals: bool = False, **kwargs):
     """The operator call (`Op.__call__`) with a shortcut for repeated eager calls: a call that came down to one
-    launch of a product on the caller's own tensors (no pass over an operand in front of it, nothing applied to the result
-    behind it, no gradient wanted) is remembered under the shapes, types and arguments it was made with, and the next
-    call of that kind goes straight to the C ABI: allocate the result, pass the addresses. Binding, the choice of a
-    config and the routing cost about 45 us of Python per call, more than the small-m kernels take."""
+    launch of a product on the caller's own tensors, or on what `AsQArray` operands were quantised to (no other pass over an
+    operand in front of it, nothing applied to the result behind it, plain arguments only), is remembered under the shapes,
+    types and arguments it was made with, and the next call of that kind goes straight to the C ABI: quantise, allocate the
+    result, pass the addresses. Where a gradient is wanted that happens inside the same autograd function as ever. Binding,
+    the choice of a config and the routing cost about 45 us of Python per call, more than the small-m kernels take."""
     key = None if return_residuals else self._plan_key(lhs, rhs, kwargs)
+    if key is None:
+      return super().__call__(lhs, rhs, return_residuals=return_residuals, **kwargs)
     plans = self.__dict__.get("_plans")
-    if key is not None and plans is not None:
+    if plans is not None:
       plan = plans.get(key)
       if plan is not None:
         return plan(lhs, rhs, _sizes_array(kwargs["group_sizes"]))
-    if key is None:
-      return super().__call__(lhs, rhs, return_residuals=return_residuals, **kwargs)
     log = hip_ops.LAUNCH_LOG
     outer, log.records = log.records, []
     try:
@@ -681,6 +705,9 @@ class HipRaggedDot(base.RaggedDot):
     if outer is not None:
       outer.extend(records)
     plan = _make_plan(records, out, lhs, rhs, _sizes_array(kwargs["group_sizes"]))
+    if plan is not None and out.grad_fn is not None:
+      both = type(lhs) is torch.Tensor and type(rhs) is torch.Tensor
+      plan = _make_differentiated_plan(self.bind(lhs, rhs, **kwargs), plan) if both else None
     if plan is not None:
       if plans is None or len(plans) > 64:
         plans = {}
@@ -702,7 +729,14 @@ class HipRaggedDot(base.RaggedDot):
     grad = torch.is_grad_enabled()
     for x in (lhs, rhs):
       if type(x) is torch.Tensor:
-        leaves = (x,)
+        if not x.is_cuda:
+          return None
+        parts.append((x.shape, x.dtype, x.is_contiguous(), grad and x.requires_grad))
+        continue
+      if type(x) is AsQArray:
+        leaves = (x.value,)
+        parts.append((x.qtype, tuple(x.channelwise_axes), x.tiled_axes and tuple(sorted(x.tiled_axes.items())),
+                      x.calibration_method))
       elif type(x) is QArray and x.zero_point is None:
         leaves = (x.qvalue, x.scale)
         parts.append(x.qtype)
@@ -712,8 +746,8 @@ class HipRaggedDot(base.RaggedDot):
         if type(t) is not torch.Tensor or not t.is_cuda or (grad and t.requires_grad):
           return None
         parts.append((t.shape, t.dtype, t.is_contiguous()))
-    parts.append((group_sizes.shape, group_sizes.dtype, group_sizes.is_contiguous(), lhs.device if type(lhs) is torch.Tensor
-                  else lhs.qvalue.device))
+    device = lhs.device if type(lhs) is torch.Tensor else lhs.value.device if type(lhs) is AsQArray else lhs.qvalue.device
+    parts.append((group_sizes.shape, group_sizes.dtype, group_sizes.is_contiguous(), device, self.vjp is not None))
     for name, v in kwargs.items():
       if name == "group_sizes":
         continue

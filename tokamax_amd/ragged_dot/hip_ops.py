@@ -30,9 +30,9 @@ SCHEDULE_FIELDS = ("group_id", "block_start", "actual_start", "actual_end", "sta
 
 class _LaunchLog(threading.local):
   """What the functions of this module launched while a caller was listening (`records` is a list then): a
-  `Launch` for a product, None for anything else (a pass over an operand, a quantisation). The operator's eager fast
-  path reads it to learn whether a call came down to one product on the caller's own tensors, which it can then repeat
-  without the planning in front of it."""
+  `Launch` for a product, a `Quantised` for a quantisation, None for anything else (another pass over an operand). The
+  operator's eager fast path reads it to learn whether a call came down to one product on the caller's own tensors, or on
+  their quantised forms, which it can then repeat without the planning in front of it."""
   records = None
 
 
@@ -54,6 +54,16 @@ class Launch:
   launch: object
   out: torch.Tensor        # the result it returned (for the caller to recognise it)
   new_workspace: object    # () -> the int32 workspace tensor of a repeat
+
+
+@dataclasses.dataclass
+class Quantised:
+  """A call of `quantize`: what it was given and what came of it."""
+
+  source: torch.Tensor
+  arguments: dict          # everything but the source
+  qvalue: torch.Tensor
+  scale: torch.Tensor
 
 
 def dtype_code(dtype: torch.dtype) -> int:
@@ -384,7 +394,7 @@ def quantize(x: torch.Tensor, qtype: torch.dtype, tile_shape, bound: float | Non
   (int4: values in [-7, 7], kept in int8 storage).
   `scale_by_block` (x [rows, cols], tiles one row tall): the scales lie in memory block by block, [cols / t_c, rows], as
   the products with scale blocks along k read them; the tensor returned is the [rows, cols / t_c] view of that."""
-  _log_launch(None)
+  source, arguments = x, dict(qtype=qtype, tile_shape=tuple(tile_shape), bound=bound, scale_by_block=scale_by_block)
   _require_cuda(x)
   lib = _lib.load()
   if qtype not in _QMAX:
@@ -413,12 +423,14 @@ def quantize(x: torch.Tensor, qtype: torch.dtype, tile_shape, bound: float | Non
       _lib.check(lib.tkx_quantize_scales_transposed(
           _ptr(x), _ptr(qvalue), _ptr(scale), rows, cols, t_c, dtype_code(x.dtype), dtype_code(storage),
           ctypes.c_float(_QMAX[qtype]), ctypes.c_float(0.0 if bound is None else bound), _stream(x.device)))
+    _log_launch(Quantised(source, arguments, qvalue, scale.t()))
     return qvalue, scale.t()
   scale = torch.empty(tuple(d // t for d, t in zip(x.shape, tile_shape)), dtype=torch.float32, device=x.device)
   with _on_device(x.device):
     st = lib.tkx_quantize(_ptr(x), _ptr(qvalue), _ptr(scale), rows, cols, t_r, t_c, dtype_code(x.dtype), dtype_code(storage),
                           ctypes.c_float(_QMAX[qtype]), ctypes.c_float(0.0 if bound is None else bound), _stream(x.device))
   _lib.check(st)
+  _log_launch(Quantised(source, arguments, qvalue, scale))
   return qvalue, scale
 
 
