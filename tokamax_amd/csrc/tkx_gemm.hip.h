@@ -134,17 +134,18 @@ __device__ __forceinline__ f32x16 mma_atom(const typename Mma<EA>::Frag& first, 
 // r + 14 (row bits 1 to 3). A phase is not 16 consecutive lanes: it takes lanes from both of the 16-lane blocks of a
 // half-wave, which read one chunk of 32 rows in a 32x32 fragment, but chunks c and c ^ 1 of the same 16 rows in a 16x16
 // one. (row >> 1) & 7 keeps rows 2 r and 2 r + 1 on neighbouring values, so the chunks that c ^ 1 moves away from are the
-// ones it moves to, whichever rows the phase takes from which block.
-template <int ROW_BYTES>
+// ones it moves to, whichever rows the phase takes from which block. (32x32 fragments have no conflicts with either form;
+// theirs is the one they had: 192 rows over 8 groups of packed int4 weights 75.6 us with it, 76.9 with the other.)
+template <int ROW_BYTES, bool M16>
 __device__ __forceinline__ int kc_swizzle(int row) {
   constexpr int CPR = ROW_BYTES / 16;
   if constexpr (CPR == 4) return (row >> 2) & 3;
-  else if constexpr (CPR == 8) return (row >> 1) & 7;
+  else if constexpr (CPR == 8 && M16) return (row >> 1) & 7;
   else return ((row & 7) ^ ((row >> 3) & 1)) & (CPR - 1);
 }
-template <int ROW_BYTES>
+template <int ROW_BYTES, bool M16>
 __device__ __forceinline__ int kc_offset(int row, int chunk) {
-  return row * ROW_BYTES + ((chunk ^ kc_swizzle<ROW_BYTES>(row)) << 4);
+  return row * ROW_BYTES + ((chunk ^ kc_swizzle<ROW_BYTES, M16>(row)) << 4);
 }
 
 // Row/column-contiguous tile: [BK rows of k][ROW_BYTES], 32-byte granules XOR-swizzled by k.
@@ -232,7 +233,7 @@ __device__ __forceinline__ typename Mma<EC, M16>::Frag load_frag(const unsigned 
       i32x4 v;
       if constexpr (LAYOUT == kKC) {
         // (16 rows further on the swizzle is the same: a constant distance)
-        v = lds_read_b128(tile + (rc_step + 16 * h) * ROW_BYTES, kc_offset<ROW_BYTES>(rc0 + s, kk * 4 + q));
+        v = lds_read_b128(tile + (rc_step + 16 * h) * ROW_BYTES, kc_offset<ROW_BYTES, M16>(rc0 + s, kk * 4 + q));
       } else {
         // (the transposing read of 16-bit elements: see below; a block of 16 lanes covers 4 k-rows of 16 columns)
         const int krow = kk * KA + 8 * q + (s >> 2), col = rc0 + rc_step + 16 * h + 4 * (s & 3);
@@ -250,14 +251,14 @@ __device__ __forceinline__ typename Mma<EC, M16>::Frag load_frag(const unsigned 
     tile += rc_step * ROW_BYTES;
     if constexpr (EC == kEF8) {
       const int c0 = kk * 4 + q * 2;
-      i32x4 lo = lds_read_b128(tile, kc_offset<ROW_BYTES>(row, c0));
-      i32x4 hi = lds_read_b128(tile, kc_offset<ROW_BYTES>(row, c0 + 1));
+      i32x4 lo = lds_read_b128(tile, kc_offset<ROW_BYTES, M16>(row, c0));
+      i32x4 hi = lds_read_b128(tile, kc_offset<ROW_BYTES, M16>(row, c0 + 1));
       Frag f;
       f[0] = lo[0]; f[1] = lo[1]; f[2] = lo[2]; f[3] = lo[3];
       f[4] = hi[0]; f[5] = hi[1]; f[6] = hi[2]; f[7] = hi[3];
       return f;
     } else {
-      return lds_read_b128(tile, kc_offset<ROW_BYTES>(row, PAIRED ? (kk >> 1) * 4 + 2 * q + (kk & 1) : kk * 2 + q));
+      return lds_read_b128(tile, kc_offset<ROW_BYTES, M16>(row, PAIRED ? (kk >> 1) * 4 + 2 * q + (kk & 1) : kk * 2 + q));
     }
   } else {
     rc0 += rc_step;
@@ -434,7 +435,7 @@ __device__ __forceinline__ void barrier_after_direct_loads() {
   __syncthreads();
 }
 
-template <int LAYOUT, int ES, int RC /* rows or cols of C covered */, int BK, int NWAVES>
+template <int LAYOUT, int ES, int RC /* rows or cols of C covered */, int BK, int NWAVES, bool M16>
 struct DirectLoader {
   static constexpr int ESZ = elem_bytes(ES);
   static constexpr int ROW_BYTES = (LAYOUT == kKC) ? BK * ESZ : RC * ESZ;
@@ -483,7 +484,7 @@ struct DirectLoader {
       const int off = j * 1024 + lane * 16;
       const int row = off / ROW_BYTES, pc = (off % ROW_BYTES) >> 4;
       if constexpr (LAYOUT == kKC) {
-        const int lc = pc ^ kc_swizzle<ROW_BYTES>(row);
+        const int lc = pc ^ kc_swizzle<ROW_BYTES, M16>(row);
         int grow = rc0 + row;
         grow = grow < rc_hi ? grow : rc_hi - 1;
         grow = (grow > rc_lo ? grow : rc_lo) - rc0;
@@ -520,7 +521,7 @@ struct DirectLoader {
 // ---- global -> register -> LDS, masked path (a partial last k-step) ---------------------------
 // One operand tile moved in 16-byte chunks; chunk q of the tile belongs to thread (q % THREADS).
 // Contraction indices at or past `k_hi` are zero-filled.
-template <int LAYOUT, int ES, int RC, int BK, int THREADS>
+template <int LAYOUT, int ES, int RC, int BK, int THREADS, bool M16>
 struct TileStage {
   static constexpr int ESZ = elem_bytes(ES);
   static constexpr int ROW_BYTES = (LAYOUT == kKC) ? BK * ESZ : RC * ESZ;
@@ -548,7 +549,7 @@ struct TileStage {
         row = row < rc_ext ? row : rc_ext - 1;
         const int kcol = kc0 + c * (16 / ESZ);
         if (kcol < k_hi) v = *reinterpret_cast<const i32x4*>(base + ((int64_t)row * ld + kcol) * ESZ);
-        off = kc_offset<ROW_BYTES>(r, c);
+        off = kc_offset<ROW_BYTES, M16>(r, c);
       } else {
         const int krow = kc0 + r;
         int colb = rc0 * ESZ + c * 16;
@@ -820,12 +821,12 @@ struct GemmKernel {
                         (I4I && (MODE == kFwd || MODE == kFwdGlu || MODE == kFwdSubK))) && !SPLIT),
                 "packed int4 weights: forward with bf16, fp8 or int8 activations");
   static constexpr int BKB = I4 ? BKC / 2 : BKC;  // rows of a B stage
-  typedef TileStage<LA, EA, BM, BK, THREADS> StageA;
-  typedef TileStage<LB, EBS, BN, BKB, THREADS> StageB;
+  typedef TileStage<LA, EA, BM, BK, THREADS, M16> StageA;
+  typedef TileStage<LB, EBS, BN, BKB, THREADS, M16> StageB;
   // Every wave takes an equal share of a k-step's direct-to-LDS loads.
   static constexpr int NLOAD = WM * WN;
-  typedef DirectLoader<LA, EA, BM, BK, NLOAD> DirA;
-  typedef DirectLoader<LB, EBS, BN, BKB, NLOAD> DirB;
+  typedef DirectLoader<LA, EA, BM, BK, NLOAD, M16> DirA;
+  typedef DirectLoader<LB, EBS, BN, BKB, NLOAD, M16> DirB;
   // Kernels whose weights may be lines that nobody else reads. (Packed int4 weights are bound by their conversion: 2 to 5 % for
   // the choice at every load, nothing gained.)
   static constexpr bool ONCE = MODE != kDrhs && EB != kEI4;
@@ -1656,7 +1657,7 @@ struct GemmKernel {
     }
     // (gate-up, per-k-block-scale and packed-int4 problems are taken only with whole k-steps)
     if constexpr (!GLU && !SUBK && !I4) if (tail) {
-      typedef TileStage<LA, EA, BM, BKC, THREADS> TailA;  // (an A tile as deep as a compute step)
+      typedef TileStage<LA, EA, BM, BKC, THREADS, M16> TailA;  // (an A tile as deep as a compute step)
       for (int kc0 = kc_begin + nmain * BKC; kc0 < kc_end; kc0 += BKC) {
         if (kc0 > kc_begin) __syncthreads();  // the tile's last reads of the LDS written below are done
         TailA::copy(Ab, p.lda, row0, p.m_ext, kc0, kc_end, smem, tid);
