@@ -172,6 +172,7 @@ struct Variant {
   const void* fn_fp8_out;  // the same kernel storing fp8 with one scale per (row, 128 columns) (GemmParams::c_scale), or null
   const void* fn_split;    // the same kernel splitting the tiles of the last round along the contraction (GemmParams::split_k), or null
   const void* fn_wide_scales;  // the same kernel with weight scales per (k-block, 128 columns) (GemmParams::wide_scales), or null
+  const void* fn_once;  // the same kernel with the weights of a group's only task loaded past the caches (GemmParams::stream_weights), or null
 };
 
 // ---- decode (small-m streaming kernel; int8 or 16-bit weights) -----------------------------------

@@ -827,9 +827,9 @@ struct GemmKernel {
   static constexpr int NLOAD = WM * WN;
   typedef DirectLoader<LA, EA, BM, BK, NLOAD, M16> DirA;
   typedef DirectLoader<LB, EBS, BN, BKB, NLOAD, M16> DirB;
-  // Kernels whose weights may be lines that nobody else reads. (Packed int4 weights are bound by their conversion: 2 to 5 % for
-  // the choice at every load, nothing gained.)
-  static constexpr bool ONCE = MODE != kDrhs && EB != kEI4;
+  // Kernels that have an instantiation for weights whose lines nobody else reads (`ON` of run()). (Packed int4 weights are
+  // bound by their conversion, f32 products by the MFMAs, and so are scales per k-block.)
+  static constexpr bool ONCE = (MODE == kFwd || MODE == kFwdGlu || MODE == kDlhs) && EB != kEI4 && EB != kEF32;
   static constexpr int SCALE_BYTES = (SUBK && !SUBP) ? BN * 4 : 0;  // kFwdSubK: the k-step's scale row behind its two tiles
   static constexpr int STAGE_BYTES = StageA::BYTES + StageB::BYTES + SCALE_BYTES;
   // fp8 x fp8: the scales of a k-step (BN weight-column scales, then BM lhs-row scales) are still needed when its
@@ -914,9 +914,12 @@ struct GemmKernel {
   // WB: the instantiation for weight scales per (k-block, 128 columns), [g, scale_blocks, n / 128]: one scale for all
   // columns of a wave, so that folding a k-step in takes one multiply-add per element and one product per row instead of
   // a product and a multiply-add per element.
-  template <bool QO = false, bool SK = false, bool WB = false>
+  // ON: the instantiation that loads the weights of a group's only task past the caches (GemmParams::stream_weights; a
+  // kernel of its own because the choice at every load costs the long launches 0.5 to 0.9 %).
+  template <bool QO = false, bool SK = false, bool WB = false, bool ON = false>
   static __device__ __forceinline__ void run(const GemmParams& p, unsigned char* smem) {
     static_assert(!WB || WIDE_SCALES, "this kernel takes one weight scale per column");
+    static_assert(!ON || (ONCE && !QO && !SK && !WB), "this kernel has no loads past the caches");
     static_assert(!QO || QOUT, "this kernel has no quantising epilogue");
     static_assert(!SK || (SPLITK && !QO), "this kernel has no split of the last round");
     const int tid = threadIdx.x, lane = tid & 63;
@@ -1070,8 +1073,9 @@ struct GemmKernel {
         row0 = rows.row0;
         act_start = rows.first;
         act_end = rows.end;
-        if (tasks == 1) once = p.stream_weights;
+        if (ON) once = tasks == 1;
       }
+      if (ON) once = __builtin_amdgcn_readfirstlane(once);  // (in a scalar register, whatever the compiler knows of it)
       col0 = nt * BNO;
       kc_begin = 0;
       kc_end = p.k_ext;
@@ -1199,7 +1203,7 @@ struct GemmKernel {
         da.issue_one(q, uniform_pointer(gA0 + dstep * stepA), smem_lds + stage * A_BYTES, wave);
       };
       auto issue_b = [&](int q, int step, int stage) {
-        db.template issue_one<ONCE>(q, uniform_pointer(gB0 + step * stepB), smem_lds + B_REGION + stage * B_BYTES, wave, once);
+        db.template issue_one<ON>(q, uniform_pointer(gB0 + step * stepB), smem_lds + B_REGION + stage * B_BYTES, wave, once);
       };
       // Prologue, in the order of the steady state (steps -LOOK .. -1).
 #pragma unroll
@@ -1247,7 +1251,7 @@ struct GemmKernel {
                                                      [&] { barrier_after_direct_loads<(ODD ? kOdd : kEven)>(); },
                                                      [&](int q) {
                                                        if (ODD && q < PA) da.issue_one(q, src_a, dst_a, wave);
-                                                       else db.template issue_one<ONCE>(q - (ODD ? PA : 0), src_b, dst_b, wave, once);
+                                                       else db.template issue_one<ON>(q - (ODD ? PA : 0), src_b, dst_b, wave, once);
                                                      });
           } else {
             // (After the last step the reads fetch fragments nobody uses, from LDS that is there.)
@@ -1260,7 +1264,7 @@ struct GemmKernel {
                                      }
                                      if (kt + HB < nfull) {
 #pragma unroll
-                                       for (int q = 0; q < PB; ++q) db.template issue_one<ONCE>(q, src_b, dst_b, wave, once);
+                                       for (int q = 0; q < PB; ++q) db.template issue_one<ON>(q, src_b, dst_b, wave, once);
                                      }
                                    },
                                    [](int) {});
@@ -1331,7 +1335,7 @@ struct GemmKernel {
       };
       auto issue_slot = [&](int q, const StepPtrs& sp) {
         if (q < DirA::PER) da.issue_one(q, sp.a, sp.lds, wave);
-        else if (q < DirA::PER + DirB::PER) db.template issue_one<ONCE>(q - DirA::PER, sp.b, sp.lds + StageA::BYTES, wave, once);
+        else if (q < DirA::PER + DirB::PER) db.template issue_one<ON>(q - DirA::PER, sp.b, sp.lds + StageA::BYTES, wave, once);
         else if (SUBK && q == DirA::PER + DirB::PER) {
           const unsigned dst = SUBP ? sp.ring : sp.lds + StageA::BYTES + StageB::BYTES;
           if constexpr (WB) {
@@ -2055,6 +2059,17 @@ __global__ __launch_bounds__(K::THREADS, K::kWavesPerSimd) void gemm_entry_wide_
   extern __shared__ __attribute__((aligned(1024))) unsigned char tkx_smem[];
   K::template run<false, false, true>(p, tkx_smem);
 }
+template <class K>
+__global__ __launch_bounds__(K::THREADS, K::kWavesPerSimd) void gemm_entry_once(const GemmParams p) {
+  extern __shared__ __attribute__((aligned(1024))) unsigned char tkx_smem[];
+  K::template run<false, false, false, true>(p, tkx_smem);
+}
+// The entry that loads weights read once past the caches, of a kernel that has one, else null.
+template <class K>
+const void* once_entry() {
+  if constexpr (K::ONCE) return reinterpret_cast<const void*>(&gemm_entry_once<K>);
+  else return nullptr;
+}
 // The entry that takes weight scales per 128 columns, of a kernel that has one, else null.
 template <class K>
 const void* wide_scales_entry() {
@@ -2079,7 +2094,8 @@ const void* fp8_out_entry() {
     MODE, EA, EB, BM, BN, BK, WM, WN, NS, ::tkx::GemmKernel<MODE, EA, EB, BM, BN, BK, WM, WN, NS, HB>::SMEM_BYTES, \
         reinterpret_cast<const void*>(&::tkx::gemm_entry<::tkx::GemmKernel<MODE, EA, EB, BM, BN, BK, WM, WN, NS, HB>>), HB, \
         ::tkx::fp8_out_entry<::tkx::GemmKernel<MODE, EA, EB, BM, BN, BK, WM, WN, NS, HB>>(),                      \
-        ::tkx::split_entry<::tkx::GemmKernel<MODE, EA, EB, BM, BN, BK, WM, WN, NS, HB>>(), nullptr                \
+        ::tkx::split_entry<::tkx::GemmKernel<MODE, EA, EB, BM, BN, BK, WM, WN, NS, HB>>(), nullptr,               \
+        ::tkx::once_entry<::tkx::GemmKernel<MODE, EA, EB, BM, BN, BK, WM, WN, NS, HB>>()                          \
   }
 
 #define TKX_VARIANT(MODE, EA, EB, BM, BN, BK, WM, WN, NS)                                            \
@@ -2088,7 +2104,8 @@ const void* fp8_out_entry() {
         reinterpret_cast<const void*>(&::tkx::gemm_entry<::tkx::GemmKernel<MODE, EA, EB, BM, BN, BK, WM, WN, NS>>), 0, \
         ::tkx::fp8_out_entry<::tkx::GemmKernel<MODE, EA, EB, BM, BN, BK, WM, WN, NS>>(),                       \
         ::tkx::split_entry<::tkx::GemmKernel<MODE, EA, EB, BM, BN, BK, WM, WN, NS>>(),                         \
-        ::tkx::wide_scales_entry<::tkx::GemmKernel<MODE, EA, EB, BM, BN, BK, WM, WN, NS>>()                    \
+        ::tkx::wide_scales_entry<::tkx::GemmKernel<MODE, EA, EB, BM, BN, BK, WM, WN, NS>>(),                   \
+        ::tkx::once_entry<::tkx::GemmKernel<MODE, EA, EB, BM, BN, BK, WM, WN, NS>>()                           \
   }
 
 }  // namespace tkx
