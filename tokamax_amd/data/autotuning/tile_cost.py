@@ -6,7 +6,8 @@ without the split of the last round): entries `{"shape": [rows, contraction, col
 waves_n, num_stages, split_k, microseconds], ...]}`; entries of bf16 activations over quantised weights (one scale per
 (group, column)) carry `"rhs": "int8"` or `"int4"` (packed two to a byte), fp8 x fp8 entries `"rhs": "fp8"`, int8 x int8
 entries `"rhs": "int8x8"`, fp8 activations over packed int4 weights `"fp8i4"` (`"fp8i4k"`: weight scales per 128 k rows, `"fp8i4glu"`: gate-up fusion), int8 activations over them `"int8i4"` / `"int8i4k"` / `"int8i4glu"`, bf16 gate-up fusion `"glu"`, int8 weights with scales per 128 k rows `"int8k"`, f32 operands `"f32"`; mode 2 is
-drhs with `"shape": [m, k, n, groups]`. The constants are fitted to the bf16 entries;
+drhs with `"shape": [m, k, n, groups]`. Forward, dlhs and `"glu"` entries of bf16 operands are timed with cold caches
+(`time_cold`), on even to Zipf group sizes; the others with warm ones. The constants are fitted to the bf16 entries;
 the others are what the rules for quantised weights in `HipRaggedDot._get_heuristics_config` were set by and are
 checked against.
 
@@ -20,10 +21,12 @@ checked against.
 from __future__ import annotations
 
 import argparse
+import functools
 import json
 import math
 import os
 import random
+import statistics
 
 from tokamax_amd.ragged_dot import hip
 
@@ -167,6 +170,21 @@ def refit(entries: list[dict], start: dict, iterations: int, seed: int = 0) -> d
   return best
 
 
+def time_cold(fn, iterations: int) -> float:
+  """Median time (us) of a call whose operands no cache holds, as between the layers of a model: a pass over 640 MB goes in
+  front of every one."""
+  import torch  # pylint: disable=g-import-not-at-top
+  flush = torch.empty(160 << 20, dtype=torch.int32, device="cuda")
+  events = [(torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)) for _ in range(iterations)]
+  for start, end in events:
+    flush.fill_(0)
+    start.record()
+    fn()
+    end.record()
+  torch.cuda.synchronize()
+  return statistics.median(start.elapsed_time(end) for start, end in events) * 1e3
+
+
 def collect(specs: list[str], iterations: int, path: str | None = None) -> None:
   """Times every tiled and streaming variant on the problems `specs` name and adds the entries to the timings file of
   this device (or to `path`)."""
@@ -174,7 +192,6 @@ def collect(specs: list[str], iterations: int, path: str | None = None) -> None:
   import torch  # pylint: disable=g-import-not-at-top
   import tokamax_amd  # pylint: disable=g-import-not-at-top
   from tokamax_amd import op as op_lib  # pylint: disable=g-import-not-at-top
-  from tokamax_amd.autotuning import autotuner as autotuner_lib  # pylint: disable=g-import-not-at-top
   from tokamax_amd.autotuning import cache as cache_lib  # pylint: disable=g-import-not-at-top
   from tokamax_amd.ragged_dot import base  # pylint: disable=g-import-not-at-top
 
@@ -182,7 +199,6 @@ def collect(specs: list[str], iterations: int, path: str | None = None) -> None:
   path = path or timings_path(cache_lib.device_dir_name(op_lib.device_kind(device)))
   os.makedirs(os.path.dirname(path), exist_ok=True)
   entries = load(path) if os.path.exists(path) else []
-  tuner = autotuner_lib.Autotuner(iterations=iterations, warmup=2)
   op = tokamax_amd.HipRaggedDot()
   gen = torch.Generator(device=device).manual_seed(1)
   def array(shape, dtype, top):
@@ -205,10 +221,18 @@ def collect(specs: list[str], iterations: int, path: str | None = None) -> None:
     lhs, rhs, kwargs = arguments(entry, array)
     bound = op.bind(lhs, rhs, group_sizes=group_sizes, **kwargs)
     configs = {c for c in bound.autotuning_configs if c.block_m == 16 or c.grid_tile_width == 8}
-    data = tuner.autotune(
-        lambda c: (lambda: tokamax_amd.HipRaggedDot(config=c)(lhs, rhs, group_sizes=group_sizes, **kwargs)), configs
-    )
-    us = {c: d.median_evaluation_time_ms * 1e3 for c, d in data.items() if hasattr(d, "median_evaluation_time_ms")}
+    order, us, declined = list(configs), {}, set()
+    for c in order + order[::-1]:  # (twice, the second time in reverse: the clock depends on what ran just before)
+      if c in declined:
+        continue
+      fn = functools.partial(tokamax_amd.HipRaggedDot(config=c), lhs, rhs, group_sizes=group_sizes, **kwargs)
+      try:
+        if c not in us:
+          fn()
+      except (NotImplementedError, ValueError):
+        declined.add(c)
+        continue
+      us[c] = min(time_cold(fn, iterations), us.get(c, math.inf))
     streaming = [t for c, t in us.items() if c.block_m == 16]
     entry.update(
         streaming_best_us=round(min(streaming), 2) if streaming else None,

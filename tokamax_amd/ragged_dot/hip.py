@@ -12,6 +12,7 @@ from __future__ import annotations
 
 import dataclasses
 import functools
+import math
 from functools import partial
 from typing import ClassVar
 
@@ -89,21 +90,31 @@ def _tiled_split_pays(mode: int, block_m: int, block_n: int, rows: int, cols: in
 
 # Constants of `_tile_cost`, fitted by tokamax_amd/data/autotuning/tile_cost.py to the timings beside it.
 _TILE_COST_FIT = dict(
-    mfma_flop_per_us=6.142e6,    # a CU's MFMA rate on a full tile
-    load_byte_per_us=59.31e3,    # a CU's rate of bringing operand slices into LDS
-    partial_block=1.475,         # 32-row blocks' worth of rows that a task costs beyond the rows it has
-    four_wave_factor=1.033,      # MFMA time of a 4-wave tile against an 8-wave one
-    in_flight_full=64.97,        # contraction elements in flight from which loads run at their full rate
-    in_flight_exponent=1.802,
-    fixed_us=3.348,              # per tile: start-up and epilogue
-    fixed_area_us=3.636,         # ... more per 256x256 of output
-    shared_cu_mfma=1.396,        # two workgroups on a CU: each k-step takes 2x this (MFMA bound)
-    shared_cu_load=0.9206,       # ... or 2x this (load bound)
-    tail_floor=0.4117,           # a partial round behind full ones costs at least this share of a round
-    exchange_us=26.43,           # price of splitting the last round along the contraction
-    group_straddle=0.8914,       # extra tiles per group at an arbitrary row offset
-    short_piece=1.526,           # time of loading 64-byte pieces of rows against 128-byte ones
+    mfma_flop_per_us=7.408e6,    # a CU's MFMA rate on a full tile
+    load_byte_per_us=58.790e3,   # a CU's rate of bringing operand slices into LDS
+    partial_block=2.218,         # 32-row blocks' worth of rows that a task costs beyond the rows it has
+    four_wave_factor=0.9076,     # MFMA time of a 4-wave tile against an 8-wave one
+    in_flight_full=72.82,        # contraction elements in flight from which loads run at their full rate
+    in_flight_exponent=1.501,
+    fixed_us=3.345,              # per tile: start-up and epilogue
+    fixed_area_us=4.088,         # ... more per 256x256 of output
+    shared_cu_mfma=1.481,        # two workgroups on a CU: each k-step takes 2x this (MFMA bound)
+    shared_cu_load=0.9356,       # ... or 2x this (load bound)
+    tail_floor=0.8865,           # a partial round behind full ones costs at least this share of a round
+    exchange_us=38.0,            # price of splitting the last round along the contraction
+    group_straddle=0.6284,       # extra tiles per group at an arbitrary row offset
+    listed_straddle=0.5,         # ... that there are (a group's last task is half full on average); the rest is what they cost
+    short_piece=1.434,           # time of loading 64-byte pieces of rows against 128-byte ones
+    cold_weights=0.05984,        # a panel of weights that no task has loaded yet: so much longer than one that L2 holds
+    dlhs_fixed=1.019,            # dlhs: a tile's start-up and epilogue against a forward launch's
 )
+# ... and for the kernels on 32x32 MFMAs (quantised operands, f32), whose rate and pipelines the constants above, fitted to
+# 16-bit tiles of which most run on the 16x16 ones, do not describe; also for the dense gated unit, where the choice by these
+# was measured on 119 shapes.
+_TILE_COST_FIT_32X32 = dict(
+    mfma_flop_per_us=6.142e6, load_byte_per_us=59.31e3, partial_block=1.475, four_wave_factor=1.033, in_flight_full=64.97,
+    in_flight_exponent=1.802, fixed_us=3.348, fixed_area_us=3.636, shared_cu_mfma=1.396, shared_cu_load=0.9206,
+    tail_floor=0.4117, exchange_us=26.43, group_straddle=0.8914, listed_straddle=0.8914, short_piece=1.526, cold_weights=0.0, dlhs_fixed=1.0)
 
 
 def _tile_cost(variant, split_k: int, rows: int, cols: int, contraction: int, num_groups: int, mode: int = 0,
@@ -113,17 +124,20 @@ def _tile_cost(variant, split_k: int, rows: int, cols: int, contraction: int, nu
   wave that holds them) and the time to bring its operand slices into LDS, which a pipeline with less than about 65
   contraction elements in flight stretches; a tile also pays a fixed time (start-up and epilogue, growing with its
   area). Shapes whose LDS lets two 4-wave workgroups share a CU run two tiles at a time at less than half the pace
-  each, so that their fixed times overlap. A group of r rows at an arbitrary offset touches about r / block_m + 0.89
+  each, so that their fixed times overlap. A group of r rows costs about r / block_m + 0.63
   tiles. A partial round behind full ones overlaps with them in part; with `split_k` its tiles are cut into parts at
   the price of the exchange.
-  The constants were fitted to the measured times of every compiled variant on 122 shapes (m = 256 .. 262144, k and
-  n = 256 .. 14336, 2 .. 256 groups, forward and dlhs; 2852 timings): the variant this picks is within 4 % of the
-  fastest one on average and 31 % at worst on those shapes. On 12 further shapes that no fit has seen it is within
-  6 % on average and 24 % at worst (8 % and 48 % before the term for 64-byte pieces, which one of them prompted),
-  against 21 % and 52 % for rules on rows per group alone; an earlier fit to 110 of the shapes was within 10 % and 47 %
-  on the 12 others, against 30 % and 77 % for those rules."""
+  The constants were fitted to the measured times of every compiled variant, caches cold, on 270 shapes (m = 32 .. 262144,
+  k and n = 256 .. 16384, 2 .. 256 groups of even to Zipf sizes, forward and dlhs; 6914 timings): the variant this picks is
+  within 2.8 % of the fastest one on average and 24 % at worst, most of it at 8 to 64 rows per group (1 to 2 % from 128 on).
+  The constants before, fitted to warm timings when all tiles ran on 32x32 MFMAs, are 4.7 % and 36 % behind on these. A
+  training product of 4096 rows over 8 groups, k = 4096, n = 14336: 475 -> 452 us; dlhs of 32768 rows over 128, contraction
+  768, 2048 columns: 198 -> 169; 236 rows over 8, k = 1552, n = 9624: 62.4 -> 56.4."""
   bm, bn, bk, wm, wn, ns = variant
-  tasks = min(rows / bm + fit["group_straddle"] * num_groups, -(-rows // bm) + num_groups - 1)
+  touched = num_groups * -math.expm1(-rows / num_groups) if num_groups > 1 else 1  # (groups that any of the rows fall into)
+  tasks = min(rows / bm + fit["group_straddle"] * touched, -(-rows // bm) + touched - 1)
+  if num_groups > 1:
+    tasks = max(tasks, touched)
   tiles = tasks * -(-cols // bn)
   four_waves = wm * wn == 4
   two_per_cu = four_waves and 2 * ns * (bm * 2 + bn * rhs_bytes) * bk <= 160 * 1024
@@ -136,9 +150,10 @@ def _tile_cost(variant, split_k: int, rows: int, cols: int, contraction: int, nu
   # (a 32-element slice of an operand that is contiguous along the contraction, as the lhs is and in dlhs the weights
   # are too, is read in 64-byte pieces)
   short = fit["short_piece"] if bk < 64 else 1.0
-  load_us = (bm * 2 * short + bn * rhs_bytes * (short if mode == 1 else 1.0)) * bk / fit["load_byte_per_us"] / in_flight
+  first = 1.0 + fit["cold_weights"] * touched / tasks
+  load_us = (bm * 2 * short + bn * rhs_bytes * first * (short if mode == 1 else 1.0)) * bk / fit["load_byte_per_us"] / in_flight
   steps = -(-contraction // bk)
-  fixed_us = fit["fixed_us"] + fit["fixed_area_us"] * bm * bn / 65536
+  fixed_us = (fit["fixed_us"] + fit["fixed_area_us"] * bm * bn / 65536) * (fit["dlhs_fixed"] if mode == 1 else 1.0)
   alone_us = steps * max(mma_us, load_us) + fixed_us
   if two_per_cu:
     tile_us = steps * 2 * max(fit["shared_cu_mfma"] * mma_us, fit["shared_cu_load"] * load_us) + fixed_us
@@ -154,7 +169,7 @@ def _tile_cost(variant, split_k: int, rows: int, cols: int, contraction: int, nu
       # (not behind a round of paired 8-wave workgroups: those start together and end together)
       last *= fit["tail_floor"] + (1 - fit["tail_floor"]) * rest / slots
     if split_k > 1:
-      beyond = int(tiles) % _COMPUTE_UNITS
+      beyond = int(min(rows / bm + fit["listed_straddle"] * touched, tasks) * -(-cols // bn)) % _COMPUTE_UNITS
       parts = min(split_k, _COMPUTE_UNITS // beyond) if beyond > 0 else 1
       if parts > 1:
         last = last / parts + fit["exchange_us"]
@@ -984,7 +999,7 @@ class HipRaggedDot(base.RaggedDot):
       # Gate-up fusion takes whole k-steps (16-bit weights: 64 deep, or 32 in the 256 x 256 x 32 tile, the only one for
       # k % 64 == 32). Where no variant's divides the contraction the launch declines the call.
       usable = [v for v in usable if contraction % v[2] == 0] or usable
-    narrow = []  # (gate-up over one group: see below)
+    narrow = []  # (gate-up: the model below takes them into account, the rules do not)
     if mode == 3 and key[1:] == (_lib.TKX_BF16, _lib.TKX_BF16):
       narrow = [v for v in usable if v[1] == 128]
       usable = [v for v in usable if v[1] != 128] or usable
@@ -1110,16 +1125,20 @@ class HipRaggedDot(base.RaggedDot):
       # fastest tile or one within 1.5 % of it on 113, and one within 5.3 % on the others, where few 256-row tiles leave
       # one round that the deeper pipeline of 256 x 256 x 32 streams faster. k = 4096, 28672 columns: 256 rows 93.6 -> 74.8
       # us (74.4 -> 58.4 on weights the memory-side cache holds), 1024 rows 203 -> 194, 8192 rows 1488 -> 1362.
-      # With several groups the rules stay so far: on 40 shapes (2 to 256 groups, even and Zipf sizes, caches flushed) they
-      # are 7 % behind the fastest tile on average and 38 % at worst (2 groups of 150 rows), this model 2 % on average.
-      fit = dict(_TILE_COST_FIT, tail_floor=1.0)
+      fit = dict(_TILE_COST_FIT_32X32, tail_floor=1.0)
       cost = lambda v: (round(_tile_cost(v, 1, rows, cols, contraction, 1, 0, fit), 3), -v[2], -v[5])
       bm, bn, bk, wm, wn, ns = min(usable, key=cost)
       if narrow and bm <= 64 and -(-rows // bm) * -(-cols // bn) < 0.85 * _COMPUTE_UNITS:
-        # Few rows, bound by the weights: such a launch leaves CUs without a workgroup, and a CU streams weights at no more than 45 to 50 GB/s: tiles of half
-        # the columns bring in more of them. k = 4096, 28672 columns, 1 to 32 rows: 58.4-59.9 -> 47.3-48.1 us; k = 2048,
-        # 8192 columns, 32 and 128 rows: 26.9 -> 20.4, 26.0 -> 20.4. (Where the wide tiles fill the chip they stay.)
+        # Few rows, bound by the weights: such a launch leaves CUs without a workgroup, and a CU streams weights at no more
+        # than 45 to 50 GB/s: tiles of half the columns bring in more of them. k = 4096, 28672 columns, 1 to 32 rows:
+        # 58.4-59.9 -> 47.3-48.1 us; k = 2048, 8192 columns, 32 and 128 rows: 26.9 -> 20.4, 26.0 -> 20.4. (Where the wide
+        # tiles fill the chip they stay.)
         bm, bn, bk, wm, wn, ns = min(narrow, key=cost)
+    elif mode == 3 and key[1:] == (_lib.TKX_BF16, _lib.TKX_BF16):
+      # ... and over several groups. On 44 shapes of 12 rows per group or more (5 to 256 groups, even to Zipf sizes, caches
+      # flushed) the rules above are 5.7 % behind the fastest tile on average and 20 % at worst, the model 1.9 % and 17 %.
+      bm, bn, bk, wm, wn, ns = min(usable + narrow, key=lambda v: (
+          round(_tile_cost(v, 1, rows, cols, contraction, num_groups), 3), -v[2], -v[5]))
     # grid_tile_width m-tasks of one group run side by side on an n-panel of its weights (a span never
     # crosses a group, so small groups simply get short spans). With the 32 tiles an XCD runs at a
     # time, 8 wide x 4 n-panels needs the fewest distinct operand panels in its L2; 16 wide measured
@@ -1146,7 +1165,7 @@ class HipRaggedDot(base.RaggedDot):
       if pairs_of_four and (wm, wn) == (1, 4):
         shares = 2 * ns * (bm + bn * 0.5) * bk <= 160 * 1024
       estimate = lambda sk: _tile_cost(v, sk, rows, cols, contraction // narrow, num_groups, mode,
-                                       rhs_bytes=2.0 if narrow == 2 else rb, shares_cu=shares)
+                                       _TILE_COST_FIT_32X32, 2.0 if narrow == 2 else rb, shares)
       if key[1] == _lib.TKX_F32 or estimate(4) < estimate(1):
         split_k = 4
     return Config(block_m=bm, block_n=bn, block_k=bk, waves_m=wm, waves_n=wn, num_stages=ns, grid_tile_width=width,
