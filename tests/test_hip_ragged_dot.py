@@ -2825,3 +2825,21 @@ def test_repeated_calls_behind_a_quantisation_or_under_autograd_are_remembered(k
       seen.clear()
       call(hip.HipRaggedDot(), *given)
     assert again == seen
+
+
+@pytest.mark.parametrize("rows", [1, 31, 33, 128, 300])
+def test_one_group_without_group_sizes_owns_every_row(rows, device):
+  """A tiled launch over one group may leave the group sizes out (the dense gated unit does): the bits of the launch with
+  them, on every kind of tile of the gate-up and of the plain product, edges of tiles among the rows."""
+  gen = torch.Generator(device=device).manual_seed(rows)
+  k, n = 192, 512
+  x = torch.randn(rows, k, device=device, generator=gen).to(torch.bfloat16)
+  w = (torch.randn(1, k, n, device=device, generator=gen) * k ** -0.5).to(torch.bfloat16)
+  gs = torch.tensor([rows], dtype=torch.int32, device=device)
+  for variant, gateup in (((32, 128, 64, 1, 2, 3), True), ((64, 256, 64, 2, 2, 3), True), ((256, 256, 64, 2, 4, 2), True),
+                          ((32, 128, 64, 1, 4, 4), False), ((256, 256, 64, 2, 4, 3), False)):
+    kw = dict(config=hip.Config(*variant).to_kernel_config(), out_dtype=torch.bfloat16, gateup=gateup,
+              activation="silu" if gateup else None)
+    assert torch.equal(hip_ops.ragged_dot_fwd(x, w, None, **kw), hip_ops.ragged_dot_fwd(x, w, gs, **kw)), variant
+  with pytest.raises(ValueError):
+    hip_ops.ragged_dot_fwd(x, w.expand(2, k, n), None, **kw)

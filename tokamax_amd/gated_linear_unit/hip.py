@@ -73,13 +73,15 @@ class HipGatedLinearUnit(op.Op):
     x2 = x.reshape(-1, k)
     rows = x2.shape[0]
     rhs = fused.reshape(1, k, 2 * n)
-    gs = torch.full((1,), rows, dtype=torch.int32, device=x.device)
     name = None if activation is None else ragged_hip._fused_activation_name(activation)  # pylint: disable=protected-access
     kcfg = config.to_kernel_config()
     if activation is None or name is not None:
-      out = hip_ops.ragged_dot_fwd(x2, rhs, gs, config=kcfg, out_dtype=x.dtype, activation=name, gateup=True)
+      # (The kernel knows that its one group owns every row: filling in a group size for it was a launch in front. 256 rows,
+      # k = 4096, 28672 columns 76.5 -> 74.5 us; 2 rows, k = 3776, 31936 columns 48.1 -> 41.5; 5 rows, small 47.8 -> 41.6.)
+      out = hip_ops.ragged_dot_fwd(x2, rhs, None, config=kcfg, out_dtype=x.dtype, activation=name, gateup=True)
     else:
       # A callable with no in-kernel twin: gate and up in one f32 GEMM, the rest in torch on f32.
+      gs = torch.full((1,), rows, dtype=torch.int32, device=x.device)
       both = hip_ops.ragged_dot_fwd(x2, rhs, gs, config=self._plain_config(x2, rhs, gs), out_dtype=torch.float32)
       out = (activation(both[:, :n]) * both[:, n:]).to(x.dtype)
     return out.reshape(*lead, n), None

@@ -212,6 +212,7 @@ def ragged_dot_fwd(lhs, rhs, group_sizes, *, config: KernelConfig, out_dtype: to
                    gateup: bool = False, group_offset=None, workspace_out: list | None = None) -> torch.Tensor:
   """out[m,n] = lhs[m,k] . rhs[g,k,n]   (trans_rhs: out[m,k] = lhs[m,n] . rhs[g,k,n]^T).
 
+  `group_sizes` None (tiled kernels, one group, no `group_offset`): the group owns every row.
   `rhs_scale` is [g,n] / [g,1,n], or [g,blocks,n] with `blocks` scale blocks along k, or (fp8 x fp8) [g,blocks,n/128] with
   a scale per block of k and 128 columns. `rhs_bias` ([g,n] or [g,1,n]) is added to the scaled result before the activation. `gateup`: rhs
   columns are [gate | up] and out[m,n/2] = activation(gate part) * (up part) (base.py:211-217).
@@ -224,15 +225,17 @@ def ragged_dot_fwd(lhs, rhs, group_sizes, *, config: KernelConfig, out_dtype: to
   if lhs.dim() != 2 or rhs.dim() != 3:
     raise ValueError(f"expected lhs [m,k] and rhs [g,k,n], got {tuple(lhs.shape)} and {tuple(rhs.shape)}")
   lhs, rhs = lhs.contiguous(), rhs.contiguous()
-  gs = _group_sizes_i32(group_sizes)
   G, k, n = rhs.shape
+  gs = None if group_sizes is None else _group_sizes_i32(group_sizes)
+  if gs is None and (G != 1 or group_offset is not None or config.block_m == 16 or workspace_out is not None):
+    raise ValueError("group_sizes may be left out for one group in a tiled kernel only")
   if rhs.dtype == torch.uint8:
     k *= 2  # packed int4: a byte row holds two contraction rows
     if trans_rhs:
       raise NotImplementedError("packed int4 weights take the default dimension numbers; unpack_int4 them first")
   m = lhs.shape[0]
   if group_offset is None:
-    if gs.numel() != G:
+    if gs is not None and gs.numel() != G:
       raise ValueError(f"group_sizes has {gs.numel()} entries, rhs has {G} groups")
   else:
     if trans_rhs:
@@ -329,13 +332,13 @@ def ragged_dot_fwd(lhs, rhs, group_sizes, *, config: KernelConfig, out_dtype: to
   elif scale_cols != 1:
     if gateup:
       raise NotImplementedError("gate-up fusion takes one rhs scale per (group, column)")
-    num_sizes, tiles = gs.numel(), lib.tkx_ragged_dot_fwd_scale_tiles
+    num_sizes, tiles = G if gs is None else gs.numel(), lib.tkx_ragged_dot_fwd_scale_tiles
 
     def launch(p, out_ptr, ws_ptr, stream):
       return tiles(p[0], p[1], p[2], p[3], p[4], p[5], p[6], out_ptr, ws_ptr, m, k, n, G, num_sizes, scale_blocks,
                    scale_cols, a_code, b_code, o_code, act_code, cfg, stream)
   else:
-    num_sizes, glu = gs.numel(), 1 if gateup else 0
+    num_sizes, glu = G if gs is None else gs.numel(), 1 if gateup else 0
     fused = lib.tkx_ragged_dot_fwd_fused
 
     def launch(p, out_ptr, ws_ptr, stream):
