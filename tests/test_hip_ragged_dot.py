@@ -2843,3 +2843,26 @@ def test_one_group_without_group_sizes_owns_every_row(rows, device):
     assert torch.equal(hip_ops.ragged_dot_fwd(x, w, None, **kw), hip_ops.ragged_dot_fwd(x, w, gs, **kw)), variant
   with pytest.raises(ValueError):
     hip_ops.ragged_dot_fwd(x, w.expand(2, k, n), None, **kw)
+
+
+def test_large_weights_with_scale_tiles_give_the_bits_of_their_parts(device):
+  """As `test_large_weights_give_the_bits_of_their_parts`, for fp8 weights with a scale per 128 x 128 block."""
+  G, k, n = 34, 2048, 4096
+  assert G * k * n >= 256 << 20 > (G // 2) * k * n
+  gen = torch.Generator(device=device).manual_seed(4)
+  sizes = ([4, 0, 300, 8, 32, 128] * 6)[:G]
+  m = sum(sizes)
+  f8 = torch.float8_e4m3fn
+  lhs = tokamax_amd.QArray(torch.randn(m, k, device=device, generator=gen).to(f8),
+                           torch.rand(k // 128, m, device=device, generator=gen).t(), None, f8)
+  w = torch.cat([torch.randn(1, k, n, device=device, generator=gen).to(f8).view(torch.uint8) for _ in range(G)]).view(f8)
+  scale = torch.rand(G, k // 128, n // 128, device=device, generator=gen) * k ** -0.5
+  gs = torch.tensor(sizes, dtype=torch.int32, device=device)
+  part = lambda a, b, g0, g1: (tokamax_amd.QArray(lhs.qvalue[a:b], lhs.scale[a:b], None, f8),
+                               tokamax_amd.QArray(w[g0:g1], scale[g0:g1], None, f8), gs[g0:g1])
+  half, rows = G // 2, sum(sizes[:G // 2])
+  for variant in ((128, 256, 128, 2, 4, 3), (64, 256, 128, 2, 2, 3), (32, 256, 128, 1, 4, 3)):
+    op = hip.HipRaggedDot(config=hip.Config(*variant))
+    call = lambda a, b, g: op(a, b, group_sizes=g, preferred_element_type=torch.bfloat16)
+    whole = call(*part(0, m, 0, G))
+    assert torch.equal(whole, torch.cat([call(*part(0, rows, 0, half)), call(*part(rows, m, half, G))])), variant

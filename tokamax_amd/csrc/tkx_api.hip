@@ -117,8 +117,10 @@ int32_t prepare(const void* fn, int32_t smem_bytes) {
 }
 
 int32_t launch(const Variant* v, const GemmParams& p, int64_t grid, hipStream_t stream) {
-  const void* fn = p.c_scale != nullptr ? v->fn_fp8_out : p.split_k > 1 ? v->fn_split : p.wide_scales ? v->fn_wide_scales
-                   : p.stream_weights && v->fn_once != nullptr ? v->fn_once : v->fn;
+  // (fn_once reads the scales like fn_wide_scales does where there is one)
+  const bool once = p.stream_weights && v->fn_once != nullptr && (p.wide_scales != 0) == (v->fn_wide_scales != nullptr);
+  const void* fn = p.c_scale != nullptr ? v->fn_fp8_out : p.split_k > 1 ? v->fn_split : once ? v->fn_once
+                   : p.wide_scales ? v->fn_wide_scales : v->fn;
   int32_t st = prepare(fn, v->smem_bytes);
   if (st != TKX_OK) return st;
   if (grid <= 0 || grid > 0x7fffffffLL) return set_error(TKX_ERR_INVALID, "grid size %lld out of range", (long long)grid);

@@ -152,18 +152,19 @@ __device__ __forceinline__ int kc_offset(int row, int chunk) {
 // E selects the pattern that suits the read instruction used for that element size. 16-bit elements: the 32 lanes of a
 // transposing read's phase take 4 k-rows of two neighbouring granules in a 32x32 fragment, k-rows r .. r + 3 and
 // r + 8 .. r + 11 of one granule in a 16x16 one, hence row bits 0, 1 and 3.
-template <int ROW_BYTES, int E>
+template <int ROW_BYTES, int E, bool M16>
 __device__ __forceinline__ int mc_swizzle(int krow) {
   constexpr int NG = ROW_BYTES / 32;
   int f;
   if constexpr (E == kEF32) f = ((krow >> 2) & 1) << 2;
-  else if constexpr (E == kEBF16 || E == kEF16) f = ((krow & 3) << 1) | ((krow >> 3) & 1);
+  else if constexpr ((E == kEBF16 || E == kEF16) && M16) f = ((krow & 3) << 1) | ((krow >> 3) & 1);
+  else if constexpr (E == kEBF16 || E == kEF16) f = ((krow & 3) << 1) ^ ((krow >> 1) & 1);
   else f = NG < 8 ? krow >> 1 : krow & 7;  // (rows of 128 bytes: two to a bank line)
   return f & (NG - 1);
 }
-template <int ROW_BYTES, int E>
+template <int ROW_BYTES, int E, bool M16>
 __device__ __forceinline__ int mc_offset(int krow, int byte_in_row) {
-  const int g = (byte_in_row >> 5) ^ mc_swizzle<ROW_BYTES, E>(krow);
+  const int g = (byte_in_row >> 5) ^ mc_swizzle<ROW_BYTES, E, M16>(krow);
   return krow * ROW_BYTES + (g << 5) + (byte_in_row & 31);
 }
 
@@ -237,8 +238,8 @@ __device__ __forceinline__ typename Mma<EC, M16>::Frag load_frag(const unsigned 
       } else {
         // (the transposing read of 16-bit elements: see below; a block of 16 lanes covers 4 k-rows of 16 columns)
         const int krow = kk * KA + 8 * q + (s >> 2), col = rc0 + rc_step + 16 * h + 4 * (s & 3);
-        const i32x2 lo = lds_read_tr16(tile + mc_offset<ROW_BYTES, ES>(krow, col * 2));
-        const i32x2 hi = lds_read_tr16(tile + mc_offset<ROW_BYTES, ES>(krow + 4, col * 2));
+        const i32x2 lo = lds_read_tr16(tile + mc_offset<ROW_BYTES, ES, M16>(krow, col * 2));
+        const i32x2 hi = lds_read_tr16(tile + mc_offset<ROW_BYTES, ES, M16>(krow + 4, col * 2));
         v = i32x4{lo[0], lo[1], hi[0], hi[1]};
       }
 #pragma unroll
@@ -268,7 +269,7 @@ __device__ __forceinline__ typename Mma<EC, M16>::Frag load_frag(const unsigned 
       Frag f;
 #pragma unroll
       for (int t = 0; t < 4; ++t)
-        f[t] = *reinterpret_cast<const int*>(tile + mc_offset<ROW_BYTES, ES>(kb + 4 * q + t, col * 4));
+        f[t] = *reinterpret_cast<const int*>(tile + mc_offset<ROW_BYTES, ES, M16>(kb + 4 * q + t, col * 4));
       return f;
     } else if constexpr (ES == kEBF16 || ES == kEF16) {
       // ds_read_b64_tr_b16: in each block of 16 lanes, lane s supplies the address of 4 consecutive
@@ -276,8 +277,8 @@ __device__ __forceinline__ typename Mma<EC, M16>::Frag load_frag(const unsigned 
       const int blk = lane >> 4, s = lane & 15;
       const int krow = kb + 8 * (blk >> 1) + (s >> 2);
       const int col = rc0 + 16 * (blk & 1) + 4 * (s & 3);
-      const i32x2 l2 = lds_read_tr16(tile + mc_offset<ROW_BYTES, ES>(krow, col * 2));
-      const i32x2 h2 = lds_read_tr16(tile + mc_offset<ROW_BYTES, ES>(krow + 4, col * 2));
+      const i32x2 l2 = lds_read_tr16(tile + mc_offset<ROW_BYTES, ES, M16>(krow, col * 2));
+      const i32x2 h2 = lds_read_tr16(tile + mc_offset<ROW_BYTES, ES, M16>(krow + 4, col * 2));
       Frag f;
       f[0] = l2[0]; f[1] = l2[1]; f[2] = h2[0]; f[3] = h2[1];
       return f;
@@ -291,7 +292,7 @@ __device__ __forceinline__ typename Mma<EC, M16>::Frag load_frag(const unsigned 
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
           const int krow = kb + 32 * (blk >> 1) + 8 * j + (s >> 1);
-          const i32x2 v = lds_read_tr8(tile + mc_offset<ROW_BYTES, ES>(krow, col));
+          const i32x2 v = lds_read_tr8(tile + mc_offset<ROW_BYTES, ES, M16>(krow, col));
           f[2 * j] = v[0];
           f[2 * j + 1] = v[1];
         }
@@ -299,15 +300,15 @@ __device__ __forceinline__ typename Mma<EC, M16>::Frag load_frag(const unsigned 
       } else if constexpr (EC == kEI8) {
         // 16 contraction values per lane: k rows 16 (l / 32) .. + 15 of the atom.
         const int krow = kb + 16 * (blk >> 1) + (s >> 1);
-        const i32x2 lo = lds_read_tr8(tile + mc_offset<ROW_BYTES, ES>(krow, col));
-        const i32x2 hi = lds_read_tr8(tile + mc_offset<ROW_BYTES, ES>(krow + 8, col));
+        const i32x2 lo = lds_read_tr8(tile + mc_offset<ROW_BYTES, ES, M16>(krow, col));
+        const i32x2 hi = lds_read_tr8(tile + mc_offset<ROW_BYTES, ES, M16>(krow + 8, col));
         Frag f;
         f[0] = lo[0]; f[1] = lo[1]; f[2] = hi[0]; f[3] = hi[1];
         return f;
       } else {
         static_assert(EC == kEBF16 && ES == kEI8, "1-byte storage feeds fp8, int8 or bf16(int8) MFMAs only");
         const int krow = kb + 8 * (blk >> 1) + (s >> 1);
-        const i32x2 v = lds_read_tr8(tile + mc_offset<ROW_BYTES, ES>(krow, col));
+        const i32x2 v = lds_read_tr8(tile + mc_offset<ROW_BYTES, ES, M16>(krow, col));
         return i8x8_to_bf16x8(v);
       }
     }
@@ -446,12 +447,12 @@ struct DirectLoader {
   static_assert(BYTES % 1024 == 0, "tile must be a whole number of wave-wide 16-byte loads");
 
   // Rows between two consecutive instructions of one wave. In the row/column-contiguous layout the
-  // rows are contraction indices (never clamped) and the swizzle repeats every 8 rows, so when this
+  // rows are contraction indices (never clamped) and the swizzle repeats every 8 (16-bit elements of M16: 16) rows, so when this
   // is a multiple of 8 the per-lane offsets of a wave's instructions differ by a wave-uniform
   // stride: one per-lane offset is kept and the stride goes into the scalar base pointer.
   static constexpr int ROWS_PER_INSTR_STEP = NWAVES * 1024 / ROW_BYTES;
   static constexpr bool STRIDED = LAYOUT == kMC && (NWAVES * 1024) % ROW_BYTES == 0 &&
-                                  ROWS_PER_INSTR_STEP % (ES == kEBF16 || ES == kEF16 ? 16 : 8) == 0;
+                                  ROWS_PER_INSTR_STEP % (M16 ? 16 : 8) == 0;
   static constexpr int NOFF = STRIDED ? 1 : PER;
 
   uint32_t voff[NOFF];  // per-lane byte offset from the wave-uniform base pointer of a k-step
@@ -490,7 +491,7 @@ struct DirectLoader {
         grow = (grow > rc_lo ? grow : rc_lo) - rc0;
         voff[i] = (uint32_t)(grow * (int)ld * ESZ + lc * 16);
       } else {
-        const int lc = ((((pc >> 1) ^ mc_swizzle<ROW_BYTES, ES>(row))) << 1) | (pc & 1);
+        const int lc = ((((pc >> 1) ^ mc_swizzle<ROW_BYTES, ES, M16>(row))) << 1) | (pc & 1);
         int colb = rc0 * ESZ + lc * 16;
         if (glu_tn > 0) {
           const int c = lc * (16 / ESZ), blk = c >> 5, half = glu_tn >> 1;
@@ -556,7 +557,7 @@ struct TileStage {
         const int lim = rc_ext * ESZ - 16;
         colb = colb < lim ? colb : lim;
         if (krow < k_hi) v = *reinterpret_cast<const i32x4*>(base + (int64_t)krow * ld * ESZ + colb);
-        off = mc_offset<ROW_BYTES, ES>(r, c * 16);
+        off = mc_offset<ROW_BYTES, ES, M16>(r, c * 16);
       }
       *reinterpret_cast<i32x4*>(tile + off) = v;
     }
@@ -828,7 +829,7 @@ struct GemmKernel {
   typedef DirectLoader<LA, EA, BM, BK, NLOAD, M16> DirA;
   typedef DirectLoader<LB, EBS, BN, BKB, NLOAD, M16> DirB;
   // Kernels that have an instantiation for weights whose lines nobody else reads (`ON` of run()). (Packed int4 weights are
-  // bound by their conversion, f32 products by the MFMAs, and so are scales per k-block.)
+  // bound by their conversion, f32 products by the MFMAs; with scales per k-block the form for 128 columns has one only.)
   static constexpr bool ONCE = (MODE == kFwd || MODE == kFwdGlu || MODE == kDlhs) && EB != kEI4 && EB != kEF32;
   static constexpr int SCALE_BYTES = (SUBK && !SUBP) ? BN * 4 : 0;  // kFwdSubK: the k-step's scale row behind its two tiles
   static constexpr int STAGE_BYTES = StageA::BYTES + StageB::BYTES + SCALE_BYTES;
@@ -919,7 +920,7 @@ struct GemmKernel {
   template <bool QO = false, bool SK = false, bool WB = false, bool ON = false>
   static __device__ __forceinline__ void run(const GemmParams& p, unsigned char* smem) {
     static_assert(!WB || WIDE_SCALES, "this kernel takes one weight scale per column");
-    static_assert(!ON || (ONCE && !QO && !SK && !WB), "this kernel has no loads past the caches");
+    static_assert(!ON || ((ONCE || WB) && !QO && !SK), "this kernel has no loads past the caches");
     static_assert(!QO || QOUT, "this kernel has no quantising epilogue");
     static_assert(!SK || (SPLITK && !QO), "this kernel has no split of the last round");
     const int tid = threadIdx.x, lane = tid & 63;
@@ -1142,8 +1143,8 @@ struct GemmKernel {
       const int blk = lane >> 4, s_ = lane & 15;
       const int col = wn * WTN + j * 32 + 16 * (blk & 1) + 8 * (s_ & 1);
       const int krow = kk * (KA / 2) + 16 * (blk >> 1) + (s_ >> 1);
-      const i32x2 lo = lds_read_tr8(stage + StageA::BYTES + mc_offset<StageB::ROW_BYTES, EBS>(krow, col));
-      const i32x2 hi = lds_read_tr8(stage + StageA::BYTES + mc_offset<StageB::ROW_BYTES, EBS>(krow + 8, col));
+      const i32x2 lo = lds_read_tr8(stage + StageA::BYTES + mc_offset<StageB::ROW_BYTES, EBS, M16>(krow, col));
+      const i32x2 hi = lds_read_tr8(stage + StageA::BYTES + mc_offset<StageB::ROW_BYTES, EBS, M16>(krow + 8, col));
       return i32x4{lo[0], lo[1], hi[0], hi[1]};
     };
     // (int8 activations over packed int4 weights) the 8 bytes that hold the 16 contraction entries of the lane's half
@@ -1152,14 +1153,14 @@ struct GemmKernel {
       const int blk = lane >> 4, s_ = lane & 15;
       const int col = wn * WTN + j * 32 + 16 * (blk & 1) + 8 * (s_ & 1);
       const int krow = kk * (KA / 2) + 8 * (blk >> 1) + (s_ >> 1);
-      return lds_read_tr8(stage + StageA::BYTES + mc_offset<StageB::ROW_BYTES, EBS>(krow, col));
+      return lds_read_tr8(stage + StageA::BYTES + mc_offset<StageB::ROW_BYTES, EBS, M16>(krow, col));
     };
     auto load_b_frag = [&](const unsigned char* stage, int j, int kk) -> Frag {
       if constexpr (SUBK && !SUBP) {
         const int blk = lane >> 4, s_ = lane & 15;
         const int col = wn * WTN + j * 32 + 16 * (blk & 1) + 8 * (s_ & 1);
         const int krow = kk * KA + 8 * (blk >> 1) + (s_ >> 1);
-        const i32x2 v = lds_read_tr8(stage + StageA::BYTES + mc_offset<StageB::ROW_BYTES, EB>(krow, col));
+        const i32x2 v = lds_read_tr8(stage + StageA::BYTES + mc_offset<StageB::ROW_BYTES, EB, M16>(krow, col));
         const float scale = *reinterpret_cast<const float*>(stage + StageA::BYTES + StageB::BYTES +
                                                             4 * (wn * WTN + j * 32 + (lane & 31)));
         if constexpr (EB == kEI8) return i8x8_to_bf16x8_scaled(v, scale);
@@ -1454,7 +1455,7 @@ struct GemmKernel {
                     const int blk = lane >> 4, s_ = lane & 15;
                     const int col = wn * WTN + j * 32 + 16 * (blk & 1) + 8 * (s_ & 1);
                     const int krow = (kk >> 1) * 16 + 8 * (blk >> 1) + (s_ >> 1);
-                    raw[j] = lds_read_tr8(stage + StageA::BYTES + mc_offset<StageB::ROW_BYTES, EBS>(krow, col));
+                    raw[j] = lds_read_tr8(stage + StageA::BYTES + mc_offset<StageB::ROW_BYTES, EBS, M16>(krow, col));
                   }
                 }
               } else {
@@ -2064,10 +2065,17 @@ __global__ __launch_bounds__(K::THREADS, K::kWavesPerSimd) void gemm_entry_once(
   extern __shared__ __attribute__((aligned(1024))) unsigned char tkx_smem[];
   K::template run<false, false, false, true>(p, tkx_smem);
 }
-// The entry that loads weights read once past the caches, of a kernel that has one, else null.
+template <class K>
+__global__ __launch_bounds__(K::THREADS, K::kWavesPerSimd) void gemm_entry_wide_scales_once(const GemmParams p) {
+  extern __shared__ __attribute__((aligned(1024))) unsigned char tkx_smem[];
+  K::template run<false, false, true, true>(p, tkx_smem);
+}
+// The entry that loads weights read once past the caches (with scales per 128 columns: that form of them), of a kernel that
+// has one, else null.
 template <class K>
 const void* once_entry() {
   if constexpr (K::ONCE) return reinterpret_cast<const void*>(&gemm_entry_once<K>);
+  else if constexpr (K::WIDE_SCALES) return reinterpret_cast<const void*>(&gemm_entry_wide_scales_once<K>);
   else return nullptr;
 }
 // The entry that takes weight scales per 128 columns, of a kernel that has one, else null.

@@ -639,11 +639,16 @@ def _make_plan(records, out, lhs, rhs, group_sizes):
   launch, new_workspace = record.launch, record.new_workspace
   shape, dtype, device = tuple(out.shape), out.dtype, out.device
 
-  def plan(lhs, rhs, group_sizes):
+  def operands_of(lhs, rhs):
     tensors = ()
     for x, args in ((lhs, arguments[0]), (rhs, arguments[1])):
       tensors += parts(x) if args is None else hip_ops.quantize(x.value, **args)
-    tensors += (group_sizes,)
+    return tensors
+
+  plain = type(lhs) is torch.Tensor and type(rhs) is torch.Tensor
+
+  def plan(lhs, rhs, group_sizes):
+    tensors = (lhs, rhs, group_sizes) if plain else (*operands_of(lhs, rhs), group_sizes)
     result = torch.empty(shape, dtype=dtype, device=device)
     ws = new_workspace()
     status = launch([0 if i < 0 else tensors[i].data_ptr() for i in source], result.data_ptr(), ws.data_ptr(),
