@@ -151,6 +151,8 @@ bool plan_pays(KernelMode mode, int32_t dtype, int64_t num_groups, int64_t sizes
 // (GemmKernel::run): allocating every line there and in L2 is what a product bound by them loses a tenth of its rate to. (Four
 // tokens over 128 experts of 805 MB reach 32 of them, 201 MB: the expert block 97 us with its weights kept, 107 past the
 // caches.)
+// Where the mean group has four tiles of rows or more, hardly a group has a task alone: the kernel without the choice
+// (16384 rows over 8 groups, gate-up: 0.5 to 0.9 %).
 // Whole lines only: of a line that two tiles share both fetch all of it then (1312 rows over 32 groups, k = 2560, rows of
 // 4816 bytes, fp8: 122 -> 129 us).
 constexpr int64_t kMemorySideCache = 256 << 20;
@@ -451,7 +453,7 @@ int32_t fwd_impl(const void* lhs, const void* rhs, const int32_t* group_sizes, c
   p.scale_blocks = subk ? (int32_t)rhs_scale_blocks : 1;
   p.log2_block_rows = log2_block_rows;
   p.wide_scales = rhs_scale_cols != 1;
-  p.stream_weights = (num_groups < m ? num_groups : m) * p.b_group_stride * rb >= kMemorySideCache &&
+  p.stream_weights = (num_groups < m ? num_groups : m) * p.b_group_stride * rb >= kMemorySideCache && m < 4 * c.block_m * num_groups &&
                      (uintptr_t)rhs % kLineBytes == 0 && n * rb % kLineBytes == 0 && (!gateup || cols * rb % kLineBytes == 0);
   if (slots > 0x7fffff00LL) return set_error(TKX_ERR_UNSUPPORTED, "too many tiles");
   // Extra workgroups zero the rows past the last group (and before the first, with a group offset);
