@@ -2866,3 +2866,27 @@ def test_large_weights_with_scale_tiles_give_the_bits_of_their_parts(device):
     call = lambda a, b, g: op(a, b, group_sizes=g, preferred_element_type=torch.bfloat16)
     whole = call(*part(0, m, 0, G))
     assert torch.equal(whole, torch.cat([call(*part(0, rows, 0, half)), call(*part(rows, m, half, G))])), variant
+
+
+def test_remembered_launches_read_scales_in_the_order_they_lie_in(device):
+  """lhs scales per (row, k-block) held block by block are read as they are; the same scales in other orders of the same
+  shape, given to the op that remembers that launch, give the bits of an op that remembers nothing."""
+  gen = torch.Generator(device=device).manual_seed(5)
+  G, m, k, n = 2, 64, 512, 256
+  f8 = torch.float8_e4m3fn
+  x = torch.randn(m, k, device=device, generator=gen).to(f8)
+  w = tokamax_amd.QArray(torch.randn(G, k, n, device=device, generator=gen).to(f8),
+                         torch.rand(G, k // 128, n // 128, device=device, generator=gen) + 0.5)
+  gs = torch.tensor([40, 24], dtype=torch.int32, device=device)
+  scale = torch.rand(m, k // 128, device=device, generator=gen) + 0.5
+  by_block = scale.t().contiguous().t()
+  tall = torch.rand(k // 128, 2 * m, device=device, generator=gen).t()
+  tall[:m] = scale
+  wide = torch.rand(m, 2 * k // 128, device=device, generator=gen)
+  wide[:, :k // 128] = scale
+  op = hip.HipRaggedDot()
+  call = lambda op, s: op(tokamax_amd.QArray(x, s), w, group_sizes=gs, preferred_element_type=torch.bfloat16)
+  want = call(op, by_block)
+  assert len(op.__dict__["_plans"]) == 1
+  for s in (by_block.clone(memory_format=torch.preserve_format), tall[:m], wide[:, :k // 128], scale):
+    assert torch.equal(s, scale) and torch.equal(call(op, s), want) and torch.equal(call(hip.HipRaggedDot(), s), want)

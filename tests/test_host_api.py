@@ -860,3 +860,28 @@ def test_drhs_workgroups_reach_every_tile_once(k, n, block_m, block_n, dealt):
     seen.append(tuple(x.value for x in out))
   everything = [(g, r, c) for g in range(groups) for r in range(m_tiles) for c in range(n_tiles)]
   assert sorted(seen) == everything and (seen != everything) == dealt
+
+
+@pytest.fixture
+def remembered_key(monkeypatch):
+  """The key under which `HipRaggedDot` remembers a launch, of tensors that only claim to be on a GPU."""
+  monkeypatch.setattr(torch.Tensor, "is_cuda", property(lambda t: True), raising=False)
+  monkeypatch.setattr(torch.cuda, "current_device", lambda: 0)
+  sizes = torch.zeros(2, dtype=torch.int32)
+  return lambda lhs, rhs, **kw: hip.HipRaggedDot()._plan_key(lhs, rhs, dict(group_sizes=sizes, **kw))
+
+
+def test_remembered_launches_tell_the_orders_of_an_operand_apart(remembered_key):
+  """Some operands that are not contiguous go to the kernels without a copy (lhs scales held block by block), so a launch
+  remembered for one order must not serve another: it passes the address on and the kernel reads its own order there."""
+  m, blocks, k, n = 8, 2, 256, 16
+  x, rhs = torch.zeros(m, k, dtype=torch.int8), torch.zeros(2, k, n, dtype=torch.bfloat16)
+  by_block = lambda: torch.zeros(blocks, m).t()
+  orders = [torch.zeros(m, blocks), by_block(), torch.zeros(blocks, 2 * m).t()[:m], torch.zeros(m, 2 * blocks)[:, :blocks],
+            torch.zeros(1, 1).expand(m, blocks)]
+  keys = [remembered_key(tokamax_amd.QArray(x, s), rhs) for s in orders]
+  assert None not in keys and len(set(keys)) == len(orders)
+  assert keys[1] == remembered_key(tokamax_amd.QArray(x, by_block()), rhs)
+  wide = torch.zeros(m, 2 * k, dtype=torch.bfloat16)
+  keys = [remembered_key(a, rhs) for a in (wide[:, :k], wide[:, ::2], torch.zeros(k, m, dtype=torch.bfloat16).t())]
+  assert None not in keys and len(set(keys)) == 3

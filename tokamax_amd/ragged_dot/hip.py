@@ -602,6 +602,13 @@ def _concrete_lhs(lhs, rhs):
 _PLAIN_ARGUMENT_TYPES = (bool, int, float, str, torch.dtype, base.RaggedDotDimensionNumbers)
 
 
+def _layout(t: torch.Tensor):
+  """What a remembered launch has to know of where a tensor's elements lie: None if they are contiguous, else the strides.
+  (Some orders besides the contiguous one go to the kernels without a copy, scales held block by block among them, so that
+  "not contiguous" alone would let one of those stand for every other.)"""
+  return None if t.is_contiguous() else t.stride()
+
+
 def _sizes_array(group_sizes):
   return group_sizes.value if type(group_sizes) is base.GroupSizes else group_sizes
 
@@ -751,7 +758,7 @@ class HipRaggedDot(base.RaggedDot):
       if type(x) is torch.Tensor:
         if not x.is_cuda:
           return None
-        parts.append((x.shape, x.dtype, x.is_contiguous(), grad and x.requires_grad))
+        parts.append((x.shape, x.dtype, _layout(x), grad and x.requires_grad))
         continue
       if type(x) is AsQArray:
         leaves = (x.value,)
@@ -765,9 +772,9 @@ class HipRaggedDot(base.RaggedDot):
       for t in leaves:
         if type(t) is not torch.Tensor or not t.is_cuda or (grad and t.requires_grad):
           return None
-        parts.append((t.shape, t.dtype, t.is_contiguous()))
+        parts.append((t.shape, t.dtype, _layout(t)))
     device = lhs.device if type(lhs) is torch.Tensor else lhs.value.device if type(lhs) is AsQArray else lhs.qvalue.device
-    parts.append((group_sizes.shape, group_sizes.dtype, group_sizes.is_contiguous(), device, self.vjp is not None))
+    parts.append((group_sizes.shape, group_sizes.dtype, _layout(group_sizes), device, self.vjp is not None))
     for name, v in kwargs.items():
       if name == "group_sizes":
         continue
