@@ -2890,3 +2890,23 @@ def test_remembered_launches_read_scales_in_the_order_they_lie_in(device):
   assert len(op.__dict__["_plans"]) == 1
   for s in (by_block.clone(memory_format=torch.preserve_format), tall[:m], wide[:, :k // 128], scale):
     assert torch.equal(s, scale) and torch.equal(call(op, s), want) and torch.equal(call(hip.HipRaggedDot(), s), want)
+
+
+def test_empty_tiled_axes_mean_no_tiles(device):
+  """An `AsQArray` with an empty mapping for its tiles, first call and repeated ones: the bits of the same call with None."""
+  gen = torch.Generator(device=device).manual_seed(6)
+  G, m, k, n = 2, 64, 256, 256
+  f8 = torch.float8_e4m3fn
+  x = torch.randn(m, k, device=device, generator=gen).to(torch.bfloat16)
+  w = torch.randn(G, k, n, device=device, generator=gen).to(torch.bfloat16)
+  gs = torch.tensor([40, 24], dtype=torch.int32, device=device)
+  op = hip.HipRaggedDot()
+
+  def call(op, tiled):
+    return op(tokamax_amd.AsQArray(x, f8, channelwise_axes=(0,), tiled_axes=tiled),
+              tokamax_amd.AsQArray(w, f8, channelwise_axes=(0, 2), tiled_axes=tiled), group_sizes=gs,
+              preferred_element_type=torch.bfloat16)
+
+  want = call(hip.HipRaggedDot(), None)
+  for tiled in ({}, {}, None):
+    assert torch.equal(call(op, tiled), want)

@@ -885,3 +885,15 @@ def test_remembered_launches_tell_the_orders_of_an_operand_apart(remembered_key)
   wide = torch.zeros(m, 2 * k, dtype=torch.bfloat16)
   keys = [remembered_key(a, rhs) for a in (wide[:, :k], wide[:, ::2], torch.zeros(k, m, dtype=torch.bfloat16).t())]
   assert None not in keys and len(set(keys)) == 3
+
+
+@pytest.mark.parametrize("tiled", [None, {}, {1: 128}, {0: 1, 1: 0.5}])
+def test_remembered_launches_have_a_key_for_every_way_to_name_tiles(remembered_key, tiled):
+  """`tiled_axes` of an `AsQArray` may be None, empty (both: no tiles) or a mapping; each call has a key that hashes."""
+  f8 = torch.float8_e4m3fn
+  x, w = torch.zeros(8, 256, dtype=torch.bfloat16), torch.zeros(2, 256, 16, dtype=torch.bfloat16)
+  as_lhs = lambda t: tokamax_amd.AsQArray(x, f8, channelwise_axes=(0,), tiled_axes=t)
+  as_rhs = lambda t: tokamax_amd.AsQArray(w, f8, channelwise_axes=(0, 2), tiled_axes=t)
+  keys = {remembered_key(as_lhs(tiled), w), remembered_key(x, as_rhs(tiled)), remembered_key(as_lhs(tiled), as_rhs(tiled))}
+  assert len(keys) == 3 and None not in keys
+  assert (remembered_key(as_lhs(tiled), w) == remembered_key(as_lhs(None), w)) == (not tiled)

@@ -762,7 +762,7 @@ class HipRaggedDot(base.RaggedDot):
         continue
       if type(x) is AsQArray:
         leaves = (x.value,)
-        parts.append((x.qtype, tuple(x.channelwise_axes), x.tiled_axes and tuple(sorted(x.tiled_axes.items())),
+        parts.append((x.qtype, tuple(x.channelwise_axes), tuple(sorted(x.tiled_axes.items())) if x.tiled_axes else None,
                       x.calibration_method))
       elif type(x) is QArray and x.zero_point is None:
         leaves = (x.qvalue, x.scale)
