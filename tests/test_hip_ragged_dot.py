@@ -2910,3 +2910,25 @@ def test_empty_tiled_axes_mean_no_tiles(device):
   want = call(hip.HipRaggedDot(), None)
   for tiled in ({}, {}, None):
     assert torch.equal(call(op, tiled), want)
+
+
+@pytest.mark.parametrize("groups", [1, 8])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+def test_calls_without_rows_are_refused_by_the_library(dtype, groups, device):
+  """Zero rows: a `ValueError` of the library's argument check, whatever product it is, and nothing is launched."""
+  k, n = 256, 512
+  w = torch.zeros(groups, k, n, dtype=dtype, device=device)
+  gs = torch.zeros(groups, dtype=torch.int32, device=device)
+  empty = lambda cols: torch.zeros(0, cols, dtype=dtype, device=device)
+  op = hip.HipRaggedDot()
+  with pytest.raises(ValueError):
+    op(empty(k), w, group_sizes=gs)
+  with pytest.raises(ValueError):
+    op(empty(n), w, group_sizes=gs, ragged_dot_dimension_numbers=base.TRANS_RHS_RAGGED_DOT_DIM_NUMS)
+  with pytest.raises(ValueError):
+    op(empty(k), empty(n), group_sizes=gs, ragged_dot_dimension_numbers=base.RAGGED_CONTRACTING_DOT_DIM_NUMS)
+  if dtype == torch.bfloat16:
+    with pytest.raises(ValueError):
+      op(empty(k), w, group_sizes=gs, fuse_gateup_activation="silu")
+    with pytest.raises(ValueError):
+      tokamax_amd.gated_linear_unit(empty(k), w[0].view(k, 2, n // 2), activation=torch.nn.functional.silu)

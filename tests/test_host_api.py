@@ -897,3 +897,20 @@ def test_remembered_launches_have_a_key_for_every_way_to_name_tiles(remembered_k
   keys = {remembered_key(as_lhs(tiled), w), remembered_key(x, as_rhs(tiled)), remembered_key(as_lhs(tiled), as_rhs(tiled))}
   assert len(keys) == 3 and None not in keys
   assert (remembered_key(as_lhs(tiled), w) == remembered_key(as_lhs(None), w)) == (not tiled)
+
+
+@pytest.mark.parametrize("kind, dtype", [("gate_up", torch.bfloat16)] + [
+    (kind, dtype) for kind in ("forward", "dlhs", "drhs") for dtype in (torch.bfloat16, torch.float16, torch.float32)])
+@pytest.mark.parametrize("groups", [1, 8, 256])
+@pytest.mark.parametrize("rows", [0, 1])
+def test_heuristics_choose_a_tile_for_few_rows_and_none(rows, groups, dtype, kind):
+  """A call without rows gets a config like any other (the library refuses it then, with an error of its own)."""
+  dims = dict(dlhs=base.TRANS_RHS_RAGGED_DOT_DIM_NUMS, drhs=base.RAGGED_CONTRACTING_DOT_DIM_NUMS).get(kind)
+  kw = {} if dims is None else dict(ragged_dot_dimension_numbers=dims)
+  if kind == "gate_up":
+    kw = dict(fuse_gateup_activation="silu")
+  rhs = ShapeDtype((rows, 256) if kind == "drhs" else (groups, 256, 256), dtype)
+  op = hip.HipRaggedDot()
+  config = op._get_heuristics_config(
+      op.bind(ShapeDtype((rows, 256), dtype), rhs, group_sizes=ShapeDtype((groups,), torch.int32), **kw))
+  assert config.block_m >= 16 and config.block_n >= 128

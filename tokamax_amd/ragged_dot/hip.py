@@ -134,6 +134,7 @@ def _tile_cost(variant, split_k: int, rows: int, cols: int, contraction: int, nu
   training product of 4096 rows over 8 groups, k = 4096, n = 14336: 475 -> 452 us; dlhs of 32768 rows over 128, contraction
   768, 2048 columns: 198 -> 169; 236 rows over 8, k = 1552, n = 9624: 62.4 -> 56.4."""
   bm, bn, bk, wm, wn, ns = variant
+  rows = max(rows, 1)  # (a call without rows gets a config as well: the library is the one to refuse it)
   touched = num_groups * -math.expm1(-rows / num_groups) if num_groups > 1 else 1  # (groups that any of the rows fall into)
   tasks = min(rows / bm + fit["group_straddle"] * touched, -(-rows // bm) + touched - 1)
   if num_groups > 1:
