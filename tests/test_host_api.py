@@ -914,3 +914,15 @@ def test_heuristics_choose_a_tile_for_few_rows_and_none(rows, groups, dtype, kin
   config = op._get_heuristics_config(
       op.bind(ShapeDtype((rows, 256), dtype), rhs, group_sizes=ShapeDtype((groups,), torch.int32), **kw))
   assert config.block_m >= 16 and config.block_n >= 128
+
+
+def test_gated_unit_declines_a_streaming_config(monkeypatch):
+  """A config of the streaming small-m kernel, which has no gate-up fusion: not implemented, so that a caller's next
+  implementation gets the call."""
+  from tokamax_amd.ragged_dot import hip_ops
+  monkeypatch.setattr(hip_ops, "_require_cuda", lambda *tensors: None)
+  from tokamax_amd.gated_linear_unit import hip as glu_hip
+  x, w = torch.zeros(4, 1024, dtype=torch.bfloat16), torch.zeros(1024, 2, 128, dtype=torch.bfloat16)
+  with pytest.raises(NotImplementedError):
+    glu_hip.HipGatedLinearUnit()._fwd(x, w, activation=None, precision=precision_lib.canonicalize_precision(None),
+                                      return_residuals=False, config=hip.Config(16, 128, 32, 1, 4, 2, 1, 8))

@@ -227,8 +227,10 @@ def ragged_dot_fwd(lhs, rhs, group_sizes, *, config: KernelConfig, out_dtype: to
   lhs, rhs = lhs.contiguous(), rhs.contiguous()
   G, k, n = rhs.shape
   gs = None if group_sizes is None else _group_sizes_i32(group_sizes)
-  if gs is None and (G != 1 or group_offset is not None or config.block_m == 16 or workspace_out is not None):
-    raise ValueError("group_sizes may be left out for one group in a tiled kernel only")
+  if gs is None and (G != 1 or group_offset is not None or workspace_out is not None):
+    raise ValueError("group_sizes may be left out for one group only")
+  if gs is None and config.block_m == 16:
+    raise NotImplementedError("the streaming small-m kernel needs group_sizes (and has no gate-up fusion)")
   if rhs.dtype == torch.uint8:
     k *= 2  # packed int4: a byte row holds two contraction rows
     if trans_rhs:
