@@ -926,3 +926,37 @@ def test_gated_unit_declines_a_streaming_config(monkeypatch):
   with pytest.raises(NotImplementedError):
     glu_hip.HipGatedLinearUnit()._fwd(x, w, activation=None, precision=precision_lib.canonicalize_precision(None),
                                       return_residuals=False, config=hip.Config(16, 128, 32, 1, 4, 2, 1, 8))
+
+
+# m, groups, scale blocks of the weights along k, gate-up fusion: whether the kernels read the lhs scales per k-block
+@pytest.mark.parametrize("m, groups, blocks, gate_up, native", [
+    (64, 2, 2, False, True), (16, 2, 2, False, False), (62, 2, 2, False, False), (64, 2, 2, True, False), (64, 2, 1, False, False)])
+def test_lhs_scales_are_laid_out_as_they_are_read(m, groups, blocks, gate_up, native, monkeypatch):
+  """An lhs quantised on the way in with several scales per row: by block where the product folds them in per k-block, row by
+  row where the lhs is widened (whose pass would copy the other order first)."""
+  from tokamax_amd.ragged_dot import hip_ops
+  k, n, f8, read = 256, 256, torch.float8_e4m3fn, []
+
+  def quantize(x, qtype, tile_shape, bound=None, scale_by_block=False):
+    shape = [d // t for d, t in zip(x.shape, tile_shape)]
+    return x.to(f8), torch.ones(shape[::-1]).t() if scale_by_block else torch.ones(shape)
+
+  def dequantize(qvalue, scale, zero_point=None):
+    read.append(("pass", tuple(scale.shape), scale.is_contiguous()))
+    return qvalue.to(torch.bfloat16)
+
+  def product(lhs, rhs, sizes, *, lhs_scale=None, **kw):
+    if lhs_scale is not None:
+      read.append(("product", tuple(lhs_scale.shape), lhs_scale.t().is_contiguous()))
+    return torch.zeros(m, n // 2 if gate_up else n)
+
+  for fake in (quantize, dequantize):
+    monkeypatch.setattr(hip_ops, fake.__name__, fake)
+  monkeypatch.setattr(hip_ops, "ragged_dot_fwd", product)
+  lhs = tokamax_amd.AsQArray(torch.zeros(m, k, dtype=torch.bfloat16), f8, channelwise_axes=(0,), tiled_axes={1: 128})
+  rhs = tokamax_amd.QArray(torch.zeros(groups, k, n).to(f8), torch.ones(groups, blocks, n // 128 if blocks > 1 else n))
+  op = hip.HipRaggedDot()
+  arguments = op.bind(lhs, rhs, group_sizes=torch.zeros(groups, dtype=torch.int32), preferred_element_type=torch.bfloat16,
+                      fuse_gateup_activation="silu" if gate_up else None).arguments
+  op._fwd(config=hip.Config(32, 256, 128, 1, 4, 3), **dict(arguments, return_residuals=False))
+  assert read[0] == ("product" if native else "pass", (m, k // 128), True)

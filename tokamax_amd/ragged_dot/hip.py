@@ -588,16 +588,10 @@ def _concrete_operand(x):
   return quantization.as_array_or_qarray_without_zero_point(x)
 
 
-def _concrete_lhs(lhs, rhs):
-  """`_concrete_operand` for an lhs: where it is quantised to 8 bits per (row, k-block) for weights with as many scale
-  blocks along k, its scales come in the order the kernels read them in (another order took a transposing copy of 7 us at
-  8192 rows of 56 blocks)."""
-  if (isinstance(lhs, AsQArray) and lhs.calibration_method == "absmax" and isinstance(rhs, QArray) and lhs.ndim == 2
-      and lhs.tile_shape[0] == 1 and lhs.scale_shape[1] > 1 and len(rhs.scale.shape) == 3
-      and rhs.scale.shape[1] == lhs.scale_shape[1]):
-    qvalue, scale = hip_ops.quantize(lhs.value, lhs.qtype, lhs.tile_shape, scale_by_block=True)
-    return QArray(qvalue, scale, None, lhs.qtype)
-  return _concrete_operand(lhs)
+def _scales_per_row_and_block(x) -> bool:
+  """Whether `x` is to be quantised with several scales per row: the form of which there are two orders in memory."""
+  return (isinstance(x, AsQArray) and x.calibration_method == "absmax" and x.ndim == 2 and x.tile_shape[0] == 1
+          and x.scale_shape[1] > 1)
 
 
 _PLAIN_ARGUMENT_TYPES = (bool, int, float, str, torch.dtype, base.RaggedDotDimensionNumbers)
@@ -832,9 +826,12 @@ class HipRaggedDot(base.RaggedDot):
     if group_offset is not None and ragged_dot_dimension_numbers != base.DEFAULT_RAGGED_DOT_DIM_NUMS:
       raise NotImplementedError("group_offset needs the default dimension numbers.")
 
-    # Quantise / dequantise what the kernels cannot take as it is, then plan the call on shapes and types.
+    # Quantise / dequantise what the kernels cannot take as it is, then plan the call on shapes and types. An lhs with
+    # several scales per row is planned on first: the kernels that fold scales in per k-block read them block by block (in the
+    # other order a transposing copy of 7 us at 8192 rows of 56 blocks), the pass that widens it row by row.
     rhs = _concrete_operand(rhs)
-    lhs = _concrete_lhs(lhs, rhs)
+    to_quantise = lhs if _scales_per_row_and_block(lhs) else None
+    lhs = _concrete_operand(lhs) if to_quantise is None else lhs.abstract_qarray()
     rhs = _settle_packed_int4(lhs, rhs, dims=ragged_dot_dimension_numbers,
                               plain=rhs_bias is None and fuse_gateup_activation is None and rhs_scale is None,
                               gateup=fuse_gateup_activation is not None)
@@ -842,6 +839,10 @@ class HipRaggedDot(base.RaggedDot):
                    rhs_scale=rhs_scale, fuse_gateup_activation=fuse_gateup_activation,
                    preferred_element_type=preferred_element_type)
     lhs, rhs, preferred_element_type = route.lhs, route.rhs, route.preferred_element_type
+    if to_quantise is not None:
+      qvalue, scale = hip_ops.quantize(to_quantise.value, to_quantise.qtype, to_quantise.tile_shape,
+                                       scale_by_block=not route.widen_lhs)
+      lhs = QArray(qvalue, scale, None, to_quantise.qtype)
     mode = _MODE_OF_DIMS[ragged_dot_dimension_numbers]
 
     lhs_scale = rhs_scale_ = None
