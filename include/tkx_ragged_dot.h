@@ -267,6 +267,12 @@ int32_t tkx_ragged_dot_fwd_scale_tiles(const void* lhs, const void* rhs, const i
  * has enough workgroups for every entry). A host function: the map the kernels use, for tests and tools. */
 int64_t tkx_ragged_dot_launch_order(int64_t workgroup, int64_t tiles);
 
+/* 1 if a forward (`gateup`: with gate-up fusion) or TRANS_RHS launch of these sizes, its rhs on a 128-byte line, takes the
+ * kernel that loads weights which one workgroup reads past the caches, 0 if not (also where there is no such launch). A host
+ * function: the rule the launches go by, for tests and tools. */
+int32_t tkx_ragged_dot_streams_weights(int64_t m, int64_t k, int64_t n, int64_t num_groups, int32_t lhs_dtype,
+                                       int32_t rhs_dtype, int32_t mode, int32_t gateup, const TkxConfig* config);
+
 /* Part (4-drhs): out[G,k,n] = lhs[rows_g, k]^T . dout[rows_g, n], zeros for empty groups.
  * lhs [m,k], dout [m,n] row-major of `dtype` (f32/bf16/f16); out_dtype f32/bf16/f16.
  * Deterministic: one workgroup owns each output tile, no atomics. block_m/block_n of `config`

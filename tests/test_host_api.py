@@ -960,3 +960,29 @@ def test_lhs_scales_are_laid_out_as_they_are_read(m, groups, blocks, gate_up, na
                       fuse_gateup_activation="silu" if gate_up else None).arguments
   op._fwd(config=hip.Config(32, 256, 128, 1, 4, 3), **dict(arguments, return_residuals=False))
   assert read[0] == ("product" if native else "pass", (m, k // 128), True)
+
+
+def _streams_weights(dtype, mode, variant, m, k, n, groups, gate_up=False, split_k=1):
+  code = dict(bf16=_lib.TKX_BF16, f16=_lib.TKX_F16, f32=_lib.TKX_F32)[dtype]
+  config = hip.Config(*variant, split_k=split_k).to_kernel_config().to_c()
+  return _lib.load().tkx_ragged_dot_streams_weights(m, k, n, groups, code, code, mode, int(gate_up), ctypes.byref(config))
+
+
+def test_weights_are_loaded_past_the_caches_in_whole_lines():
+  """The loads that leave nothing of a line behind are for loads of whole 128-byte lines: a TRANS_RHS k-step of 32 16-bit
+  elements is half of one, whose other half the next k-step would fetch again."""
+  wide = dict(m=2048, k=2048, n=2048, groups=32)  # (256 MB of weights, groups of a fraction of a tile)
+  for v in _lib.variants(0):
+    variant = tuple(v[f] for f in ("block_m", "block_n", "block_k", "waves_m", "waves_n", "num_stages"))
+    for dtype, code in (("bf16", _lib.TKX_BF16), ("f16", _lib.TKX_F16), ("f32", _lib.TKX_F32)):
+      if v["lhs_dtype"] != code or v["rhs_dtype"] != code or v["mode"] not in (0, 1, 3) or v["block_m"] == 16:
+        continue
+      whole = dtype != "f32" and (v["mode"] != 1 or v["block_k"] >= 64)
+      mode = _lib.TKX_MODE_TRANS_RHS if v["mode"] == 1 else _lib.TKX_MODE_DEFAULT
+      assert _streams_weights(dtype, mode, variant, gate_up=v["mode"] == 3, **wide) == whole, (dtype, v)
+  tile = (128, 256, 64, 2, 4, 3)
+  takes = lambda **kw: _streams_weights("bf16", _lib.TKX_MODE_DEFAULT, tile, **dict(wide, **kw))
+  assert takes() and not takes(split_k=4)
+  assert not takes(groups=31) and not takes(m=31) and takes(m=32)      # weights that the cache holds, of the groups reached
+  assert not takes(n=2112 - 8) and takes(n=2112)                       # rows of whole lines
+  assert takes(m=4 * 128 * 32 - 1) and not takes(m=4 * 128 * 32)       # groups of four tiles

@@ -34,6 +34,7 @@ EXPORTED_SYMBOLS = (
     "tkx_ragged_dot_fwd_fused",
     "tkx_ragged_dot_fwd_scale_tiles",
     "tkx_ragged_dot_launch_order",
+    "tkx_ragged_dot_streams_weights",
     "tkx_ragged_dot_drhs",
     "tkx_ragged_dot_drhs_tile",
     "tkx_dequantize_weights",
@@ -124,6 +125,8 @@ def _declare(lib):
                                                  i32, i32, i32, cfgp, vp]
   lib.tkx_ragged_dot_drhs.restype = i32
   lib.tkx_ragged_dot_drhs.argtypes = [vp, vp, vp, vp, vp, i64, i64, i64, i64, i32, i32, cfgp, vp]
+  lib.tkx_ragged_dot_streams_weights.restype = i32
+  lib.tkx_ragged_dot_streams_weights.argtypes = [i64, i64, i64, i64, i32, i32, i32, i32, cfgp]
   lib.tkx_ragged_dot_launch_order.restype = i64
   lib.tkx_ragged_dot_launch_order.argtypes = [i64, i64]
   i32p = ctypes.POINTER(i32)

@@ -118,7 +118,7 @@ int32_t prepare(const void* fn, int32_t smem_bytes) {
 
 int32_t launch(const Variant* v, const GemmParams& p, int64_t grid, hipStream_t stream) {
   // (fn_once reads the scales like fn_wide_scales does where there is one)
-  const bool once = p.stream_weights && v->fn_once != nullptr && (p.wide_scales != 0) == (v->fn_wide_scales != nullptr);
+  const bool once = p.stream_weights && (p.wide_scales != 0) == (v->fn_wide_scales != nullptr);
   const void* fn = p.c_scale != nullptr ? v->fn_fp8_out : p.split_k > 1 ? v->fn_split : once ? v->fn_once
                    : p.wide_scales ? v->fn_wide_scales : v->fn;
   int32_t st = prepare(fn, v->smem_bytes);
@@ -146,17 +146,23 @@ bool plan_pays(KernelMode mode, int32_t dtype, int64_t num_groups, int64_t sizes
                                        (workgroups > 8192 && (mode != kDrhs || dtype == TKX_F32)));
 }
 
-// Bytes of the memory-side cache. Where the groups that m rows can reach have at least as many bytes of weights, these are not
-// there any more when the next call wants them, and are loaded past it where one task of a group reads them, i.e. once
-// (GemmKernel::run): allocating every line there and in L2 is what a product bound by them loses a tenth of its rate to. (Four
-// tokens over 128 experts of 805 MB reach 32 of them, 201 MB: the expert block 97 us with its weights kept, 107 past the
-// caches.)
+// Whether a forward / dlhs launch takes the kernel that loads the weights of a group's only task past the caches
+// (GemmKernel::run). The bytes of the memory-side cache: where the groups that m rows can reach have at least as many bytes of
+// weights, these are not there any more when the next call wants them, and allocating every line there and in L2 is what a
+// product bound by them loses a tenth of its rate to. (Four tokens over 128 experts of 805 MB reach 32 of them, 201 MB: the
+// expert block 97 us with its weights kept, 107 past the caches.)
 // Where the mean group has four tiles of rows or more, hardly a group has a task alone: the kernel without the choice
 // (16384 rows over 8 groups, gate-up: 0.5 to 0.9 %).
 // Whole lines only: of a line that two tiles share both fetch all of it then (1312 rows over 32 groups, k = 2560, rows of
-// 4816 bytes, fp8: 122 -> 129 us).
+// 4816 bytes, fp8: 122 -> 129 us). `up_offset_bytes`: from the gate to the up half of a row. (Tiles whose loads take less than
+// a line of a row have no such kernel: GemmKernel::ONCE.)
 constexpr int64_t kMemorySideCache = 256 << 20;
 constexpr int64_t kLineBytes = 128;
+bool streams_weights(const Variant& v, int64_t m, int64_t num_groups, int64_t group_bytes, int64_t row_bytes,
+                     int64_t up_offset_bytes) {
+  return v.fn_once != nullptr && (num_groups < m ? num_groups : m) * group_bytes >= kMemorySideCache &&
+         m < 4 * v.block_m * num_groups && row_bytes % kLineBytes == 0 && up_offset_bytes % kLineBytes == 0;
+}
 
 bool valid_out_dtype(int d) { return d == TKX_F32 || d == TKX_BF16 || d == TKX_F16; }
 
@@ -453,8 +459,8 @@ int32_t fwd_impl(const void* lhs, const void* rhs, const int32_t* group_sizes, c
   p.scale_blocks = subk ? (int32_t)rhs_scale_blocks : 1;
   p.log2_block_rows = log2_block_rows;
   p.wide_scales = rhs_scale_cols != 1;
-  p.stream_weights = (num_groups < m ? num_groups : m) * p.b_group_stride * rb >= kMemorySideCache && m < 4 * c.block_m * num_groups &&
-                     (uintptr_t)rhs % kLineBytes == 0 && n * rb % kLineBytes == 0 && (!gateup || cols * rb % kLineBytes == 0);
+  p.stream_weights = (uintptr_t)rhs % kLineBytes == 0 &&
+                     streams_weights(*v, m, num_groups, p.b_group_stride * rb, n * rb, gateup ? cols * rb : 0);
   if (slots > 0x7fffff00LL) return set_error(TKX_ERR_UNSUPPORTED, "too many tiles");
   // Extra workgroups zero the rows past the last group (and before the first, with a group offset);
   // they exit at once when there are none.
@@ -592,6 +598,15 @@ static int32_t drhs_xcd_rows(int64_t k, int64_t n, int32_t m_tiles, int32_t n_ti
 int64_t tkx_ragged_dot_launch_order(int64_t workgroup, int64_t tiles) {
   if (workgroup < 0 || tiles < 0 || workgroup > 0x7fffff00LL || tiles > 0x7fffff00LL) return -1;
   return launch_order_entry((int32_t)workgroup, (int32_t)tiles);
+}
+
+int32_t tkx_ragged_dot_streams_weights(int64_t m, int64_t k, int64_t n, int64_t num_groups, int32_t lhs_dtype,
+                                       int32_t rhs_dtype, int32_t mode, int32_t gateup, const TkxConfig* config) {
+  if (config == nullptr || m < 1 || k < 1 || n < 1 || num_groups < 1) return 0;
+  const Variant* v = find_variant(mode == TKX_MODE_TRANS_RHS ? kDlhs : gateup ? kFwdGlu : kFwd, lhs_dtype, rhs_dtype, *config);
+  if (v == nullptr || config->split_k > 1) return 0;
+  const int64_t rb = dtype_bytes(rhs_dtype);
+  return streams_weights(*v, m, num_groups, k * n * rb, n * rb, gateup ? n / 2 * rb : 0) ? 1 : 0;
 }
 
 int32_t tkx_ragged_dot_drhs_tile(int64_t workgroup, int64_t k, int64_t n, int32_t block_m, int32_t block_n, int32_t* group,

@@ -829,8 +829,10 @@ struct GemmKernel {
   typedef DirectLoader<LA, EA, BM, BK, NLOAD, M16> DirA;
   typedef DirectLoader<LB, EBS, BN, BKB, NLOAD, M16> DirB;
   // Kernels that have an instantiation for weights whose lines nobody else reads (`ON` of run()). (Packed int4 weights are
-  // bound by their conversion, f32 products by the MFMAs; with scales per k-block the form for 128 columns has one only.)
-  static constexpr bool ONCE = (MODE == kFwd || MODE == kFwdGlu || MODE == kDlhs) && EB != kEI4 && EB != kEF32;
+  // bound by their conversion, f32 products by the MFMAs; with scales per k-block the form for 128 columns has one only; and a
+  // k-step of half a line along the weights' rows would have each line fetched twice.)
+  static constexpr bool ONCE = (MODE == kFwd || MODE == kFwdGlu || (MODE == kDlhs && StageB::ROW_BYTES >= 128)) &&
+                               EB != kEI4 && EB != kEF32;
   static constexpr int SCALE_BYTES = (SUBK && !SUBP) ? BN * 4 : 0;  // kFwdSubK: the k-step's scale row behind its two tiles
   static constexpr int STAGE_BYTES = StageA::BYTES + StageB::BYTES + SCALE_BYTES;
   // fp8 x fp8: the scales of a k-step (BN weight-column scales, then BM lhs-row scales) are still needed when its
