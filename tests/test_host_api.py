@@ -986,3 +986,41 @@ def test_weights_are_loaded_past_the_caches_in_whole_lines():
   assert not takes(groups=31) and not takes(m=31) and takes(m=32)      # weights that the cache holds, of the groups reached
   assert not takes(n=2112 - 8) and takes(n=2112)                       # rows of whole lines
   assert takes(m=4 * 128 * 32 - 1) and not takes(m=4 * 128 * 32)       # groups of four tiles
+
+
+def test_calls_of_several_launches_are_looked_at_once(remembered_key, monkeypatch):
+  """A call that took more than one launch (a pass over an operand in front of the product) goes the full way each time, and
+  is not examined for a shortcut again; a call of another kind is."""
+  from tokamax_amd.ragged_dot import hip_ops
+  examined, make_plan = [], hip._make_plan
+  monkeypatch.setattr(hip, "_make_plan", lambda *a: examined.append(a[1]) or make_plan(*a))
+
+  def full_path(self, lhs, rhs, *, return_residuals=False, **kw):
+    out = torch.zeros(lhs.shape[0], rhs.shape[2])
+    hip_ops._log_launch(None)
+    hip_ops._log_launch(hip_ops.Launch((1,) * 7, None, out, None))
+    return out
+
+  monkeypatch.setattr(op_lib.Op, "__call__", full_path)
+  op, sizes = hip.HipRaggedDot(), torch.zeros(2, dtype=torch.int32)
+  rhs = torch.zeros(2, 64, 128, dtype=torch.bfloat16)
+  for m, count in ((8, 1), (8, 1), (8, 1), (16, 2), (8, 2)):
+    out = op(torch.zeros(m, 64, dtype=torch.bfloat16), rhs, group_sizes=sizes)
+    assert out.shape == (m, 128) and len(examined) == count and "_plans" not in op.__dict__
+
+
+def test_scales_are_planned_on_shapes_only_where_they_may_stay_as_they_are(monkeypatch):
+  """Weight scales per 128 columns are taken as they are by fp8 x fp8 kernels alone: for other activations they are repeated
+  and planned on once."""
+  made = []
+  monkeypatch.setattr(hip, "_shapes_of", lambda x, f=hip._shapes_of: made.append(x) or f(x))
+  f8 = torch.float8_e4m3fn
+  rhs = tokamax_amd.QArray(torch.zeros(2, 256, 256).to(f8), torch.ones(2, 2, 2))
+  route = lambda lhs, rhs: hip._route(lhs, rhs, dims=base.DEFAULT_RAGGED_DOT_DIM_NUMS, precision=precision_lib.canonicalize_precision(None),
+                                      rhs_scale=None, fuse_gateup_activation=None, preferred_element_type=torch.bfloat16)
+  wide = route(torch.zeros(64, 256, dtype=torch.bfloat16), rhs)
+  assert not made and wide.native_k_blocks and tuple(wide.rhs.scale.shape) == (2, 2, 256)
+  blocks = lambda m: tokamax_amd.QArray(torch.zeros(m, 256).to(f8), torch.ones(m, 2))
+  native, widened = route(blocks(64), rhs), route(blocks(16), rhs)
+  assert native.native_k_blocks and not native.widen_lhs and native.rhs.scale is rhs.scale
+  assert widened.widen_lhs and tuple(widened.rhs.scale.shape) == (2, 2, 256)

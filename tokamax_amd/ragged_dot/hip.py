@@ -485,8 +485,12 @@ def _route(lhs, rhs, *, dims, precision, rhs_scale, fuse_gateup_activation, pref
   widen_lhs = widen_rhs = native = False
   if mode == 0:
     lhs = _per_row_lhs_scale(lhs)
-    widen_lhs, widen_rhs, native = _widening_plan(lhs, _per_column_rhs_scale(_shapes_of(rhs)), allow_native=not gateup)
-    if not (native and not widen_lhs and _kernels_read_scale_tiles(lhs, rhs)):
+    tiles = _kernels_read_scale_tiles(lhs, rhs)
+    if not tiles:
+      rhs = _per_column_rhs_scale(rhs)
+    widen_lhs, widen_rhs, native = _widening_plan(lhs, _per_column_rhs_scale(_shapes_of(rhs)) if tiles else rhs,
+                                                  allow_native=not gateup)
+    if tiles and not (native and not widen_lhs):
       rhs = _per_column_rhs_scale(rhs)
     if (gateup and isinstance(rhs, QArray) and not widen_rhs and rhs.qvalue.dtype in (torch.int8, torch.float8_e4m3fn)
         and rhs.qvalue.shape[2] % 32):
@@ -588,10 +592,13 @@ def _concrete_operand(x):
   return quantization.as_array_or_qarray_without_zero_point(x)
 
 
-def _scales_per_row_and_block(x) -> bool:
-  """Whether `x` is to be quantised with several scales per row: the form of which there are two orders in memory."""
-  return (isinstance(x, AsQArray) and x.calibration_method == "absmax" and x.ndim == 2 and x.tile_shape[0] == 1
-          and x.scale_shape[1] > 1)
+def _block_scale_tile(x):
+  """The tile of an `x` to be quantised with several scales per row, the form of which there are two orders in memory; else
+  None."""
+  if not isinstance(x, AsQArray) or x.calibration_method != "absmax" or x.ndim != 2:
+    return None
+  tile = x.tile_shape
+  return tile if tile[0] == 1 and tile[1] < x.shape[1] else None
 
 
 _PLAIN_ARGUMENT_TYPES = (bool, int, float, str, torch.dtype, base.RaggedDotDimensionNumbers)
@@ -608,21 +615,28 @@ def _sizes_array(group_sizes):
   return group_sizes.value if type(group_sizes) is base.GroupSizes else group_sizes
 
 
+# What `_make_plan` says of calls that are more than one launch, however often they are made.
+_FULL_PATH = object()
+
+
 def _make_plan(records, out, lhs, rhs, group_sizes):
-  """The shortcut for calls like the one that left `records` and returned `out`, or None if that call was more than
-  one launch of a product on the caller's own buffers and on what its `AsQArray` operands were quantised to."""
+  """The shortcut for calls like the one that left `records` and returned `out`; `_FULL_PATH` if such calls are more than
+  one launch of a product on the caller's own buffers and on what its `AsQArray` operands were quantised to; None if this one
+  does not tell (empty or shared buffers)."""
   if not records or not isinstance(records[-1], hip_ops.Launch) or type(out) is not torch.Tensor:
-    return None
+    return _FULL_PATH
   record, quantised = records[-1], records[:-1]
+  if len(quantised) != (type(lhs) is AsQArray) + (type(rhs) is AsQArray):
+    return _FULL_PATH  # (a pass over an operand that is not its quantisation)
   if record.out.data_ptr() != out.data_ptr() or record.out.shape != out.shape or record.out.dtype != out.dtype:
-    return None
+    return _FULL_PATH
   if out.device.index != torch.cuda.current_device():
     return None  # (the launch ran under a device guard; the shortcut has none)
 
   by_source = {id(r.source): r for r in quantised if isinstance(r, hip_ops.Quantised)}
   operands = [by_source.get(id(x.value)) if type(x) is AsQArray else None for x in (lhs, rhs)]
-  if len(quantised) != sum(r is not None for r in operands) or len(quantised) != sum(type(x) is AsQArray for x in (lhs, rhs)):
-    return None  # (a pass over an operand that is not its quantisation)
+  if len(quantised) != sum(r is not None for r in operands):
+    return None  # (one array given for both, or a quantisation of something else)
   arguments = tuple(None if r is None else r.arguments for r in operands)
   parts = lambda x: (x,) if type(x) is torch.Tensor else (x.qvalue, x.scale)
   given = [t.data_ptr() for x, r in zip((lhs, rhs), operands) for t in parts(r if r is not None else x)]
@@ -636,7 +650,7 @@ def _make_plan(records, out, lhs, rhs, group_sizes):
     elif p in given:
       source.append(given.index(p))
     else:
-      return None  # (a buffer this call made itself: a widened or repeated operand, converted group sizes)
+      return _FULL_PATH  # (a buffer this call made itself: a widened or repeated operand, converted group sizes)
   source = tuple(source)
   launch, new_workspace = record.launch, record.new_workspace
   shape, dtype, device = tuple(out.shape), out.dtype, out.device
@@ -717,6 +731,9 @@ class HipRaggedDot(base.RaggedDot):
       plan = plans.get(key)
       if plan is not None:
         return plan(lhs, rhs, _sizes_array(kwargs["group_sizes"]))
+    longer = self.__dict__.get("_longer_calls")  # (keys of the calls that are more than one launch: nothing to learn again)
+    if longer is not None and key in longer:
+      return super().__call__(lhs, rhs, **kwargs)
     log = hip_ops.LAUNCH_LOG
     outer, log.records = log.records, []
     try:
@@ -727,10 +744,15 @@ class HipRaggedDot(base.RaggedDot):
     if outer is not None:
       outer.extend(records)
     plan = _make_plan(records, out, lhs, rhs, _sizes_array(kwargs["group_sizes"]))
-    if plan is not None and out.grad_fn is not None:
+    if plan is not None and plan is not _FULL_PATH and out.grad_fn is not None:
       both = type(lhs) is torch.Tensor and type(rhs) is torch.Tensor
-      plan = _make_differentiated_plan(self.bind(lhs, rhs, **kwargs), plan) if both else None
-    if plan is not None:
+      plan = _make_differentiated_plan(self.bind(lhs, rhs, **kwargs), plan) if both else _FULL_PATH
+    if plan is _FULL_PATH:
+      if longer is None or len(longer) > 64:
+        longer = set()
+        object.__setattr__(self, "_longer_calls", longer)
+      longer.add(key)
+    elif plan is not None:
       if plans is None or len(plans) > 64:
         plans = {}
         object.__setattr__(self, "_plans", plans)
@@ -830,8 +852,8 @@ class HipRaggedDot(base.RaggedDot):
     # several scales per row is planned on first: the kernels that fold scales in per k-block read them block by block (in the
     # other order a transposing copy of 7 us at 8192 rows of 56 blocks), the pass that widens it row by row.
     rhs = _concrete_operand(rhs)
-    to_quantise = lhs if _scales_per_row_and_block(lhs) else None
-    lhs = _concrete_operand(lhs) if to_quantise is None else lhs.abstract_qarray()
+    tile, to_quantise = _block_scale_tile(lhs), lhs
+    lhs = _concrete_operand(lhs) if tile is None else lhs.abstract_qarray()
     rhs = _settle_packed_int4(lhs, rhs, dims=ragged_dot_dimension_numbers,
                               plain=rhs_bias is None and fuse_gateup_activation is None and rhs_scale is None,
                               gateup=fuse_gateup_activation is not None)
@@ -839,9 +861,8 @@ class HipRaggedDot(base.RaggedDot):
                    rhs_scale=rhs_scale, fuse_gateup_activation=fuse_gateup_activation,
                    preferred_element_type=preferred_element_type)
     lhs, rhs, preferred_element_type = route.lhs, route.rhs, route.preferred_element_type
-    if to_quantise is not None:
-      qvalue, scale = hip_ops.quantize(to_quantise.value, to_quantise.qtype, to_quantise.tile_shape,
-                                       scale_by_block=not route.widen_lhs)
+    if tile is not None:
+      qvalue, scale = hip_ops.quantize(to_quantise.value, to_quantise.qtype, tile, scale_by_block=not route.widen_lhs)
       lhs = QArray(qvalue, scale, None, to_quantise.qtype)
     mode = _MODE_OF_DIMS[ragged_dot_dimension_numbers]
 
