@@ -1009,18 +1009,42 @@ def test_calls_of_several_launches_are_looked_at_once(remembered_key, monkeypatc
     assert out.shape == (m, 128) and len(examined) == count and "_plans" not in op.__dict__
 
 
-def test_scales_are_planned_on_shapes_only_where_they_may_stay_as_they_are(monkeypatch):
-  """Weight scales per 128 columns are taken as they are by fp8 x fp8 kernels alone: for other activations they are repeated
-  and planned on once."""
-  made = []
-  monkeypatch.setattr(hip, "_shapes_of", lambda x, f=hip._shapes_of: made.append(x) or f(x))
+def test_bound_arguments_list_every_tensor_once():
   f8 = torch.float8_e4m3fn
-  rhs = tokamax_amd.QArray(torch.zeros(2, 256, 256).to(f8), torch.ones(2, 2, 2))
-  route = lambda lhs, rhs: hip._route(lhs, rhs, dims=base.DEFAULT_RAGGED_DOT_DIM_NUMS, precision=precision_lib.canonicalize_precision(None),
-                                      rhs_scale=None, fuse_gateup_activation=None, preferred_element_type=torch.bfloat16)
-  wide = route(torch.zeros(64, 256, dtype=torch.bfloat16), rhs)
-  assert not made and wide.native_k_blocks and tuple(wide.rhs.scale.shape) == (2, 2, 256)
-  blocks = lambda m: tokamax_amd.QArray(torch.zeros(m, 256).to(f8), torch.ones(m, 2))
-  native, widened = route(blocks(64), rhs), route(blocks(16), rhs)
-  assert native.native_k_blocks and not native.widen_lhs and native.rhs.scale is rhs.scale
-  assert widened.widen_lhs and tuple(widened.rhs.scale.shape) == (2, 2, 256)
+  x, sizes = torch.zeros(8, 256), torch.zeros(2, dtype=torch.int32)
+  q = tokamax_amd.QArray(torch.zeros(2, 256, 16).to(f8), torch.ones(2, 1, 16))
+  ba = hip.HipRaggedDot().bind(tokamax_amd.AsQArray(x, f8, channelwise_axes=(0,), tiled_axes={1: 128}), q, group_sizes=sizes)
+  assert [id(t) for t in ba.tensors] == [id(t) for t in (x, q.qvalue, q.scale, sizes)]
+
+
+@pytest.mark.parametrize("m, groups, gate_up, tile", [(64, 2, False, (1, 128)), (16, 2, False, None), (62, 2, False, None),
+                                                       (64, 2, True, None)])
+def test_calls_whose_lhs_is_surely_widened_are_not_planned_on_shapes(m, groups, gate_up, tile):
+  f8 = torch.float8_e4m3fn
+  rhs = tokamax_amd.QArray(torch.zeros(groups, 256, 16).to(f8), torch.ones(groups, 2, 16))
+  lhs = lambda **kw: tokamax_amd.AsQArray(torch.zeros(m, 256), f8, channelwise_axes=(0,), **kw)
+  assert hip._block_scale_tile(lhs(tiled_axes={1: 128}), rhs, gate_up) == tile
+  assert hip._block_scale_tile(lhs(), rhs, gate_up) is None and hip._block_scale_tile(lhs(), rhs.qvalue, gate_up) is None
+
+
+def test_weight_scales_are_repeated_where_no_kernel_reads_them_per_128_columns():
+  """Weight scales per 128 columns are taken as they are by the fp8 x fp8 kernels for scale blocks alone, also where the plan
+  is made on shapes; a form that tiles nothing is refused."""
+  f8 = torch.float8_e4m3fn
+  values = lambda *shape: torch.zeros(shape).to(f8)
+  rhs = tokamax_amd.QArray(values(2, 256, 256), torch.ones(2, 2, 2))
+  route = lambda lhs, rhs, **kw: hip._route(lhs, rhs, **dict(dict(
+      dims=base.DEFAULT_RAGGED_DOT_DIM_NUMS, precision=precision_lib.canonicalize_precision(None), rhs_scale=None,
+      fuse_gateup_activation=None, preferred_element_type=torch.bfloat16), **kw))
+  blocks = lambda m: tokamax_amd.QArray(values(m, 256), torch.ones(m, 2))
+  shapes = lambda q: tokamax_amd.QArray(*(ShapeDtype(tuple(t.shape), t.dtype) for t in (q.qvalue, q.scale)))
+  bf16 = torch.zeros(64, 256, dtype=torch.bfloat16)
+  for of in (lambda q: q, shapes):
+    native, few, fused, wide = (route(of(blocks(64)), of(rhs)), route(of(blocks(16)), of(rhs)),
+                                route(of(blocks(64)), of(rhs), fuse_gateup_activation="silu"), route(bf16, of(rhs)))
+    assert native.native_k_blocks and not native.widen_lhs and tuple(native.rhs.scale.shape) == (2, 2, 2)
+    assert few.native_k_blocks and few.widen_lhs and tuple(few.rhs.scale.shape) == (2, 2, 256)
+    assert fused.widen_lhs and fused.widen_rhs and tuple(fused.rhs.scale.shape) == (2, 2, 256)
+    assert wide.native_k_blocks and tuple(wide.rhs.scale.shape) == (2, 2, 256)
+  with pytest.raises(NotImplementedError):
+    route(blocks(64), tokamax_amd.QArray(values(2, 256, 256), torch.ones(2, 3, 2)))

@@ -96,6 +96,9 @@ class AsQArray:
   dtype = property(lambda self: self.value.dtype)
   ndim = property(lambda self: len(self.value.shape))
 
+  def _leaves(self):
+    return (self.value,)
+
   def _key(self):
     tiled = None if self.tiled_axes is None else tuple(sorted(self.tiled_axes.items()))
     value = self.value if not isinstance(self.value, torch.Tensor) else id(self.value)  # (arrays compare by identity)

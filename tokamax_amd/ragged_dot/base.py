@@ -50,6 +50,9 @@ class RaggedDotDimensionNumbers:
     object.__setattr__(self, "lhs_ragged_dimensions", tuple(int(i) for i in self.lhs_ragged_dimensions))
     object.__setattr__(self, "rhs_group_dimensions", tuple(int(i) for i in self.rhs_group_dimensions))
 
+  def _leaves(self):
+    return ()  # (no arrays)
+
   def _to_jsonable(self):
     return dict(
         dot_dimension_numbers=[[list(d) for d in pair] for pair in self.dot_dimension_numbers],

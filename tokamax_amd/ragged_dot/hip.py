@@ -216,12 +216,12 @@ def _fused_activation_name(activation) -> str | None:
     return None
 
 
-def _scale_blocks_along_k(q: QArray) -> int | None:
-  """Number of scale blocks along k of a quantised rhs [g,k,n] (scale [g, blocks, n]), or None if the
+def _scale_blocks_along_k(q: QArray, scale_cols: int = 1) -> int | None:
+  """Number of scale blocks along k of a quantised rhs [g,k,n] (scale [g, blocks, n / scale_cols]), or None if the
   scale has another form."""
   g, k, n = q.qvalue.shape
   shape = tuple(q.scale.shape)
-  if len(shape) != 3 or shape[0] != g or shape[2] != n or shape[1] < 1 or k % shape[1] != 0:
+  if len(shape) != 3 or shape[0] != g or shape[2] * scale_cols != n or shape[1] < 1 or k % shape[1] != 0:
     return None
   return shape[1]
 
@@ -250,14 +250,6 @@ def _per_column_rhs_scale(rhs):
   else:
     scale = ShapeDtype((g, rhs.scale.shape[1], n), rhs.scale.dtype)
   return QArray(rhs.qvalue, scale, rhs.zero_point, rhs.qtype)
-
-
-def _shapes_of(x):
-  """A quantised operand's shapes and types, for plans that need no more."""
-  if not isinstance(x, QArray) or not isinstance(x.scale, torch.Tensor):
-    return x
-  return QArray(ShapeDtype(tuple(x.qvalue.shape), x.qvalue.dtype), ShapeDtype(tuple(x.scale.shape), x.scale.dtype),
-                x.zero_point, x.qtype)
 
 
 def _kernels_read_scale_tiles(lhs, rhs) -> bool:
@@ -314,8 +306,13 @@ def _widening_pass_takes(q: QArray) -> bool:
   return t_c == 1 or t_c % 16 == 0
 
 
-def _widening_plan(lhs, rhs, allow_native: bool = True) -> tuple[bool, bool, bool]:
-  """(widen lhs, widen rhs, native k-blocks): how a pair of (possibly quantised) operands reaches the kernels.
+# Up to so many rows per group on average, an lhs quantised like its weights is widened for the streaming small-m kernel.
+_WIDENED_ROWS_PER_GROUP = 8
+
+
+def _widening_plan(lhs, rhs, allow_native: bool = True, rhs_scale_cols: int = 1) -> tuple[bool, bool, bool]:
+  """(widen lhs, widen rhs, native k-blocks): how a pair of (possibly quantised) operands reaches the kernels
+  (`rhs_scale_cols`: with every rhs scale repeated over that many columns).
 
   * One scale per lhs row and one per (group, column): applied in the kernels' epilogue (bf16 x int8, fp8 x fp8,
     int8 x int8), nothing is widened.
@@ -342,7 +339,7 @@ def _widening_plan(lhs, rhs, allow_native: bool = True) -> tuple[bool, bool, boo
       lhs_blocks = 0
     widen_lhs = lhs_blocks != 1 or _dtype_of(lhs) == torch.int8  # (unless int8 meets int8 below)
   if rhs_q:
-    blocks = _scale_blocks_along_k(rhs)
+    blocks = _scale_blocks_along_k(rhs, rhs_scale_cols)
     if blocks is None and not _rhs_scale_tiles(rhs) and not _widening_pass_takes(rhs):
       raise NotImplementedError("rhs scale must have shape [g,1,n], [g,k/t_k,n] or [g,k/t_k,n/t_n] with 16 | t_n, got"
                                 f" {tuple(rhs.scale.shape)}")
@@ -362,7 +359,7 @@ def _widening_plan(lhs, rhs, allow_native: bool = True) -> tuple[bool, bool, boo
     # (Groups of a few rows are better off with a widened lhs and the streaming small-m kernel, below.)
     if both_int8 and blocks == 1 and k % 16 == 0:
       return False, False, False  # one scale per row and per column: the plain int8 MFMA variants, scales in the epilogue
-    if shape_ok and m % 4 == 0 and rhs.qvalue.shape[2] % 16 == 0 and m > 8 * rhs.qvalue.shape[0]:
+    if shape_ok and m % 4 == 0 and rhs.qvalue.shape[2] % 16 == 0 and m > _WIDENED_ROWS_PER_GROUP * rhs.qvalue.shape[0]:
       return False, False, True
   if rhs_q and allow_native and blocks is not None and rhs.qvalue.dtype in (torch.int8, torch.float8_e4m3fn):
     # Kernels of their own (bf16 lhs; 256-column tiles) for int8 weights with several scale blocks along k and
@@ -488,8 +485,7 @@ def _route(lhs, rhs, *, dims, precision, rhs_scale, fuse_gateup_activation, pref
     tiles = _kernels_read_scale_tiles(lhs, rhs)
     if not tiles:
       rhs = _per_column_rhs_scale(rhs)
-    widen_lhs, widen_rhs, native = _widening_plan(lhs, _per_column_rhs_scale(_shapes_of(rhs)) if tiles else rhs,
-                                                  allow_native=not gateup)
+    widen_lhs, widen_rhs, native = _widening_plan(lhs, rhs, not gateup, 128 if tiles else 1)
     if tiles and not (native and not widen_lhs):
       rhs = _per_column_rhs_scale(rhs)
     if (gateup and isinstance(rhs, QArray) and not widen_rhs and rhs.qvalue.dtype in (torch.int8, torch.float8_e4m3fn)
@@ -592,10 +588,12 @@ def _concrete_operand(x):
   return quantization.as_array_or_qarray_without_zero_point(x)
 
 
-def _block_scale_tile(x):
-  """The tile of an `x` to be quantised with several scales per row, the form of which there are two orders in memory; else
-  None."""
-  if not isinstance(x, AsQArray) or x.calibration_method != "absmax" or x.ndim != 2:
+def _block_scale_tile(x, rhs, gateup):
+  """The tile of an `x` to be quantised with several scales per row, the form of which there are two orders in memory, if the
+  product may be one that reads them block by block; else None. (That is for `_widening_plan` to say; calls of which it surely
+  is not true are spared a plan on shapes: 6 us of 120.)"""
+  if (not isinstance(x, AsQArray) or x.calibration_method != "absmax" or x.ndim != 2 or not isinstance(rhs, QArray) or gateup
+      or x.shape[0] % 4 or (x.shape[0] <= _WIDENED_ROWS_PER_GROUP * rhs.shape[0] and not rhs.packed)):
     return None
   tile = x.tile_shape
   return tile if tile[0] == 1 and tile[1] < x.shape[1] else None
@@ -723,17 +721,16 @@ class HipRaggedDot(base.RaggedDot):
     types and arguments it was made with, and the next call of that kind goes straight to the C ABI: quantise, allocate the
     result, pass the addresses. Where a gradient is wanted that happens inside the same autograd function as ever. Binding,
     the choice of a config and the routing cost about 45 us of Python per call, more than the small-m kernels take."""
-    key = None if return_residuals else self._plan_key(lhs, rhs, kwargs)
-    if key is None:
+    call = None if return_residuals else self._call_key(lhs, rhs, kwargs)
+    longer = self.__dict__.get("_longer_calls")  # (calls that are more than one launch: nothing to learn again)
+    if call is None or (longer is not None and call in longer):
       return super().__call__(lhs, rhs, return_residuals=return_residuals, **kwargs)
+    key = (call, self._config_key())
     plans = self.__dict__.get("_plans")
     if plans is not None:
       plan = plans.get(key)
       if plan is not None:
         return plan(lhs, rhs, _sizes_array(kwargs["group_sizes"]))
-    longer = self.__dict__.get("_longer_calls")  # (keys of the calls that are more than one launch: nothing to learn again)
-    if longer is not None and key in longer:
-      return super().__call__(lhs, rhs, **kwargs)
     log = hip_ops.LAUNCH_LOG
     outer, log.records = log.records, []
     try:
@@ -751,7 +748,7 @@ class HipRaggedDot(base.RaggedDot):
       if longer is None or len(longer) > 64:
         longer = set()
         object.__setattr__(self, "_longer_calls", longer)
-      longer.add(key)
+      longer.add(call)
     elif plan is not None:
       if plans is None or len(plans) > 64:
         plans = {}
@@ -761,6 +758,17 @@ class HipRaggedDot(base.RaggedDot):
 
   def _plan_key(self, lhs, rhs, kwargs):
     """What a remembered launch depends on, or None for a call that always takes the full path."""
+    call = self._call_key(lhs, rhs, kwargs)
+    return None if call is None else (call, self._config_key())
+
+  @staticmethod
+  def _config_key():
+    """The part of it that the choice of a config depends on beside the call."""
+    return (config_lib.autotuning_cache_miss_fallback.value, config_lib.ignore_autotuning_cache.value,
+            id(op.AUTOTUNING_CACHE_OVERLAY_STACK.get()), torch.cuda.current_device())
+
+  def _call_key(self, lhs, rhs, kwargs):
+    """The part of it that the call itself makes up (and the state of the cached configs), or None."""
     if self.checkify_group_sizes or op.OP_CALL_RECORDER.get() is not None:
       return None
     group_sizes = kwargs.get("group_sizes")
@@ -799,9 +807,7 @@ class HipRaggedDot(base.RaggedDot):
               or (type(v) is tuple and all(type(x) is precision_lib.Precision for x in v))):
         return None  # (tensors, callables: the full path)
       parts.append((name, v))
-    parts.append((op.config_epoch(), config_lib.autotuning_cache_miss_fallback.value,
-                  config_lib.ignore_autotuning_cache.value, id(op.AUTOTUNING_CACHE_OVERLAY_STACK.get()),
-                  torch.cuda.current_device()))
+    parts.append(op.config_epoch())
     return tuple(parts)
 
   # -- forward ---------------------------------------------------------------------------------
@@ -852,7 +858,7 @@ class HipRaggedDot(base.RaggedDot):
     # several scales per row is planned on first: the kernels that fold scales in per k-block read them block by block (in the
     # other order a transposing copy of 7 us at 8192 rows of 56 blocks), the pass that widens it row by row.
     rhs = _concrete_operand(rhs)
-    tile, to_quantise = _block_scale_tile(lhs), lhs
+    tile, to_quantise = _block_scale_tile(lhs, rhs, gateup), lhs
     lhs = _concrete_operand(lhs) if tile is None else lhs.abstract_qarray()
     rhs = _settle_packed_int4(lhs, rhs, dims=ragged_dot_dimension_numbers,
                               plain=rhs_bias is None and fuse_gateup_activation is None and rhs_scale is None,
