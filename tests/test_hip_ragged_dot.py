@@ -2601,7 +2601,7 @@ def test_repeated_backward_passes_take_remembered_launches(device, dtype):
 
 def test_repeated_eager_calls_take_the_remembered_launch(device):
   """The operator's shortcut for repeated eager calls: same bits as the full path, taken only for calls that are one
-  forward launch on the caller's own tensors, and never when a gradient is wanted."""
+  forward launch on the caller's own tensors; where a gradient is wanted, inside the autograd function."""
   rng = np.random.default_rng(11)
   G, m, k, n = 8, 64, 1024, 256
   gs = np.array([3, 0, 9, 1, 0, 20, 7, 5], np.int32)
@@ -2641,7 +2641,7 @@ def test_repeated_eager_calls_take_the_remembered_launch(device):
   c = op(lhs2, q, group_sizes=gst, preferred_element_type=torch.bfloat16, activation=torch.relu)
   assert torch.equal(c, torch.relu(out2))
   assert len(plans) <= n_before + 1  # (the k-block call may be one launch of a variant of its own; the others are not)
-  # a gradient: the full path with its custom VJP
+  # a gradient: the custom VJP
   lhs_g = lhs.float().clone().to(torch.bfloat16).requires_grad_(True)
   w = torch.tensor(rng.normal(0, k ** -0.5, (G, k, n)).astype(np.float32), device=device).to(torch.bfloat16)
   op(lhs_g.detach(), w, group_sizes=gst)
@@ -2812,8 +2812,25 @@ def test_repeated_calls_behind_a_quantisation_or_under_autograd_are_remembered(k
     for a, b in zip(got, call(hip.HipRaggedDot(), *given)):
       assert torch.equal(a, b)
   if kind.startswith("grad"):
-    # an activation given as a callable, and no gradient wanted: ways of their own
     lhs, rhs, dout, gs = given
+    # an activation given as a callable: the full path both times, and no plan of its own
+    before = dict(op.__dict__["_plans"])
+    both = []
+    for fresh in (op, op, hip.HipRaggedDot()):
+      a, b = lhs.clone().requires_grad_(True), rhs.clone().requires_grad_(True)
+      out = fresh(a, b, group_sizes=gs, activation=torch.relu, **kw)
+      both.append((out.detach(), *torch.autograd.grad(out, (a, b), dout)))
+    assert op.__dict__["_plans"] == before
+    assert all(torch.equal(x, y) for other in both[1:] for x, y in zip(both[0], other))
+    # the operator that remembers one set of operands that want their gradients, given another
+    for wanted in ((True, False), (False, True), (True, True), (False, True), (True, False)):
+      results = []
+      for fresh in (op, hip.HipRaggedDot()):
+        a, b = lhs.clone().requires_grad_(wanted[0]), rhs.clone().requires_grad_(wanted[1])
+        out = fresh(a, b, group_sizes=gs, **kw)
+        results.append((out.detach(), *torch.autograd.grad(out, [t for t, w in zip((a, b), wanted) if w], dout)))
+      assert all(torch.equal(x, y) for x, y in zip(*results)), wanted
+    # no gradient wanted: a way of its own
     assert not op(lhs, rhs, group_sizes=gs, **kw).requires_grad
     with torch.no_grad():
       assert not op(lhs.clone().requires_grad_(True), rhs, group_sizes=gs, **kw).requires_grad

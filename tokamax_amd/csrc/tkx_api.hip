@@ -156,6 +156,9 @@ bool plan_pays(KernelMode mode, int32_t dtype, int64_t num_groups, int64_t sizes
 // Whole lines only: of a line that two tiles share both fetch all of it then (1312 rows over 32 groups, k = 2560, rows of
 // 4816 bytes, fp8: 122 -> 129 us). `up_offset_bytes`: from the gate to the up half of a row. (Tiles whose loads take less than
 // a line of a row have no such kernel: GemmKernel::ONCE.)
+// Behind a plan no task says whether it is its group's only one, so that every load keeps its line there; the kernel without
+// the choice is no faster for such launches (128x256x64 over 64 groups, 4096 x 14336, with the choice and without: 12160 rows
+// 1862 and 1869 us, gate-up 1941 and 1948; 16000 rows, k = 2048, 1078 both).
 constexpr int64_t kMemorySideCache = 256 << 20;
 constexpr int64_t kLineBytes = 128;
 bool streams_weights(const Variant& v, int64_t m, int64_t num_groups, int64_t group_bytes, int64_t row_bytes,

@@ -2,8 +2,8 @@
 
 `activation(x @ weights[:, 0]) * (x @ weights[:, 1])` (tokamax/_src/ops/gated_linear_unit/base.py:60-120).
 Fused weights `[K, 2, N]` are, row by row, `[gate | up]`: exactly the `[1, K, 2N]` weight layout of the
-ragged dot's gate-up mode with a single group that owns every row, so this op is that kernel with
-`group_sizes = [M]`; the product is formed on the f32 accumulators and rounded once to `x.dtype`, as
+ragged dot's gate-up mode with a single group that owns every row, so this op is that kernel without
+group sizes; the product is formed on the f32 accumulators and rounded once to `x.dtype`, as
 the reference does (base.py:108-118).
 """
 

@@ -602,11 +602,10 @@ def _block_scale_tile(x, rhs, gateup):
 _PLAIN_ARGUMENT_TYPES = (bool, int, float, str, torch.dtype, base.RaggedDotDimensionNumbers)
 
 
-def _layout(t: torch.Tensor):
-  """What a remembered launch has to know of where a tensor's elements lie: None if they are contiguous, else the strides.
-  (Some orders besides the contiguous one go to the kernels without a copy, scales held block by block among them, so that
-  "not contiguous" alone would let one of those stand for every other.)"""
-  return None if t.is_contiguous() else t.stride()
+def _config_state():
+  """What the choice of a config depends on beside the call and the cached configs."""
+  return (config_lib.autotuning_cache_miss_fallback.value, config_lib.ignore_autotuning_cache.value,
+          id(op.AUTOTUNING_CACHE_OVERLAY_STACK.get()), torch.cuda.current_device())
 
 
 def _sizes_array(group_sizes):
@@ -725,7 +724,7 @@ class HipRaggedDot(base.RaggedDot):
     longer = self.__dict__.get("_longer_calls")  # (calls that are more than one launch: nothing to learn again)
     if call is None or (longer is not None and call in longer):
       return super().__call__(lhs, rhs, return_residuals=return_residuals, **kwargs)
-    key = (call, self._config_key())
+    key = (call, *_config_state())
     plans = self.__dict__.get("_plans")
     if plans is not None:
       plan = plans.get(key)
@@ -759,16 +758,12 @@ class HipRaggedDot(base.RaggedDot):
   def _plan_key(self, lhs, rhs, kwargs):
     """What a remembered launch depends on, or None for a call that always takes the full path."""
     call = self._call_key(lhs, rhs, kwargs)
-    return None if call is None else (call, self._config_key())
-
-  @staticmethod
-  def _config_key():
-    """The part of it that the choice of a config depends on beside the call."""
-    return (config_lib.autotuning_cache_miss_fallback.value, config_lib.ignore_autotuning_cache.value,
-            id(op.AUTOTUNING_CACHE_OVERLAY_STACK.get()), torch.cuda.current_device())
+    return None if call is None else (call, *_config_state())
 
   def _call_key(self, lhs, rhs, kwargs):
-    """The part of it that the call itself makes up (and the state of the cached configs), or None."""
+    """The part of it that the call itself makes up (and the state of the cached configs), or None. (Strides of what is not
+    contiguous: some orders besides the contiguous one go to the kernels without a copy, scales held block by block among
+    them, and must not stand for every other.)"""
     if self.checkify_group_sizes or op.OP_CALL_RECORDER.get() is not None:
       return None
     group_sizes = kwargs.get("group_sizes")
@@ -783,7 +778,7 @@ class HipRaggedDot(base.RaggedDot):
       if type(x) is torch.Tensor:
         if not x.is_cuda:
           return None
-        parts.append((x.shape, x.dtype, _layout(x), grad and x.requires_grad))
+        parts.append((x.shape, x.dtype, x.is_contiguous() or x.stride(), grad and x.requires_grad))
         continue
       if type(x) is AsQArray:
         leaves = (x.value,)
@@ -797,9 +792,10 @@ class HipRaggedDot(base.RaggedDot):
       for t in leaves:
         if type(t) is not torch.Tensor or not t.is_cuda or (grad and t.requires_grad):
           return None
-        parts.append((t.shape, t.dtype, _layout(t)))
+        parts.append((t.shape, t.dtype, t.is_contiguous() or t.stride()))
     device = lhs.device if type(lhs) is torch.Tensor else lhs.value.device if type(lhs) is AsQArray else lhs.qvalue.device
-    parts.append((group_sizes.shape, group_sizes.dtype, _layout(group_sizes), device, self.vjp is not None))
+    parts.append((group_sizes.shape, group_sizes.dtype, group_sizes.is_contiguous() or group_sizes.stride(), device,
+                  self.vjp is not None))
     for name, v in kwargs.items():
       if name == "group_sizes":
         continue
