@@ -7,9 +7,9 @@ waves_n, num_stages, split_k, microseconds], ...]}`; entries of bf16 activations
 (group, column)) carry `"rhs": "int8"` or `"int4"` (packed two to a byte), fp8 x fp8 entries `"rhs": "fp8"`, int8 x int8
 entries `"rhs": "int8x8"`, fp8 activations over packed int4 weights `"fp8i4"` (`"fp8i4k"`: weight scales per 128 k rows, `"fp8i4glu"`: gate-up fusion), int8 activations over them `"int8i4"` / `"int8i4k"` / `"int8i4glu"`, bf16 gate-up fusion `"glu"`, int8 weights with scales per 128 k rows `"int8k"`, f32 operands `"f32"`; mode 2 is
 drhs with `"shape": [m, k, n, groups]`. Forward, dlhs and `"glu"` entries of bf16 operands are timed with cold caches
-(`time_cold`), on even to Zipf group sizes; the others with warm ones. The constants are fitted to the bf16 entries;
-the others are what the rules for quantised weights in `HipRaggedDot._get_heuristics_config` were set by and are
-checked against.
+(`time_cold`), on the group sizes that `collect` draws or on others (even, Zipf), which an entry does not say; the others
+with warm ones. The constants are fitted to bf16 entries; those marked `"unseen": true` are kept out of the fit. The others
+are what the rules for quantised weights in `HipRaggedDot._get_heuristics_config` were set by and are checked against.
 
   python -m tokamax_amd.data.autotuning.tile_cost check              # how far the model's pick is from the fastest
   python -m tokamax_amd.data.autotuning.tile_cost fit [--iterations N]  # refit; prints the constants to paste
@@ -263,7 +263,7 @@ def main() -> None:
     collect(args.shapes, args.iterations or 6)
     return
   entries = load()
-  label = lambda e: "drhs" if e["mode"] == 2 else e.get("rhs", "bf16")
+  label = lambda e: "drhs" if e["mode"] == 2 else "unseen bf16" if e.get("unseen") else e.get("rhs", "bf16")
   others = [e for e in entries if label(e) != "bf16"]
   entries = [e for e in entries if label(e) == "bf16"]  # (what the model is fitted to: forward and dlhs of bf16 operands)
   if args.command == "fit":
@@ -277,6 +277,11 @@ def main() -> None:
   mean, worst = summary(gaps(entries, current))
   print(f"{len(entries)} shapes, {sum(len(e['timings']) for e in entries)} timings: the model's pick is "
         f"{100 * mean:.1f} % above the fastest variant on average, {100 * worst:.0f} % at worst")
+  for low, high in ((0, 8), (8, 16), (16, 64), (64, 128), (128, 512), (512, math.inf)):
+    some = [e for e in entries if low <= e["shape"][0] / e["shape"][3] < high]
+    if some:
+      mean, worst = summary(gaps(some, current))
+      print(f"  {len(some)} of {low} to {high} rows per group: {100 * mean:.1f} %, {100 * worst:.0f} % at worst")
   for kind in ["bf16"] + sorted({label(e) for e in others}):
     some = [e for e in others if label(e) == kind] if kind != "bf16" else entries
     mean, worst = summary([heuristics_gap(e) for e in some])

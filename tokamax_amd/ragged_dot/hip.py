@@ -127,10 +127,13 @@ def _tile_cost(variant, split_k: int, rows: int, cols: int, contraction: int, nu
   each, so that their fixed times overlap. A group of r rows costs about r / block_m + 0.63
   tiles. A partial round behind full ones overlaps with them in part; with `split_k` its tiles are cut into parts at
   the price of the exchange.
+  A workgroup of two waves (a gate-up tile) is counted like one of eight.
   The constants were fitted to the measured times of every compiled variant, caches cold, on 270 shapes (m = 32 .. 262144,
-  k and n = 256 .. 16384, 2 .. 256 groups of even to Zipf sizes, forward and dlhs; 6914 timings): the variant this picks is
-  within 2.8 % of the fastest one on average and 24 % at worst, most of it at 8 to 64 rows per group (1 to 2 % from 128 on).
-  The constants before, fitted to warm timings when all tiles ran on 32x32 MFMAs, are 4.7 % and 36 % behind on these. A
+  k and n = 256 .. 16384, 2 .. 256 groups, forward and dlhs; 6812 timings): the variant this picks is within 2.8 % of the
+  fastest one on average and 24 % at worst, 3 to 4 % at 8 to 512 rows per group and 1 % beyond; the config the heuristics hand
+  out, streaming kernel included, 3.3 % and 24 %. On 60 shapes that no fit has seen the config is 4.6 % and 33 % behind; refits
+  to re-timed dlhs shapes and 48 more were 5 to 6 % behind there and are not used. The constants before, fitted to warm timings
+  when all tiles ran on 32x32 MFMAs, are 4.5 % and 62 % behind on the 270, 4.7 % and 37 % on the 60. A
   training product of 4096 rows over 8 groups, k = 4096, n = 14336: 475 -> 452 us; dlhs of 32768 rows over 128, contraction
   768, 2048 columns: 198 -> 169; 236 rows over 8, k = 1552, n = 9624: 62.4 -> 56.4."""
   bm, bn, bk, wm, wn, ns = variant
@@ -1172,8 +1175,8 @@ class HipRaggedDot(base.RaggedDot):
         # tiles fill the chip they stay.)
         bm, bn, bk, wm, wn, ns = min(narrow, key=cost)
     elif mode == 3 and key[1:] == (_lib.TKX_BF16, _lib.TKX_BF16):
-      # ... and over several groups. On 44 shapes of 12 rows per group or more (5 to 256 groups, even to Zipf sizes, caches
-      # flushed) the rules above are 5.7 % behind the fastest tile on average and 20 % at worst, the model 1.9 % and 17 %.
+      # ... and over several groups. On 80 shapes (5 to 256 groups, caches flushed) the rules above are 7.3 % behind the fastest
+      # tile on average and 37 % at worst, the model 2.0 % and 22 %; of 12 rows per group or more (62) 8.4 %, 1.5 %.
       bm, bn, bk, wm, wn, ns = min(usable + narrow, key=lambda v: (
           round(_tile_cost(v, 1, rows, cols, contraction, num_groups), 3), -v[2], -v[5]))
     # grid_tile_width m-tasks of one group run side by side on an n-panel of its weights (a span never
